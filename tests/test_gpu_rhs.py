@@ -49,6 +49,24 @@ def test_tiled_fp64_matches_oracle(orc, ws, shape, kind, tile):
     assert err <= TOL_FP64
 
 
+@pytest.mark.parametrize("ratio", [1e1, 1e4, 1e8])
+def test_tiled_fp64_across_strong_jumps(orc, ws, ratio):
+    """Spherical blasts: the FP64 candidates are the central one plus fourth differences, so
+    beside a jump every candidate passes through values of the jump's size (up to 1e12 times
+    the quiet side's for the energy flux).  The drop-in bar holds as on any other state:
+    each face keeps an error of a few ulp of the largest value in its window."""
+    from windstencil_amd import initial as I
+    nx, ny, nz = 37, 21, 18
+    prims = I.blast(nx, ny, nz, 5, ratio)
+    ref = oracle_du(orc, prims)
+    for tile in W.TILE_SHAPES:
+        ctx = make_ctx(nx, ny, nz)
+        ctx.set_tile_shape(tile)
+        err = rel_l2(gpu_du_comput(ctx, upload_state(prims)), ref)
+        log(f"  blast ratio {ratio:g} tile {tile}: rel L2 {err:.3e}")
+        assert err <= TOL_FP64
+
+
 @pytest.mark.parametrize("shape", [(4, 4, 4), (4, 9, 5), (7, 4, 6), (5, 6, 4), (129, 65, 33)])
 def test_smallest_and_ragged_extents(orc, ws, shape):
     """Extents at the minimum the periodic halo allows (4 cells, where the halo is the

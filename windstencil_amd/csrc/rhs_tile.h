@@ -285,6 +285,9 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
     const int line = t / TL::T, seg = t % TL::T;
     const int f0 = seg * K;                               // first face of this thread
     const bool active = (t < TL::NT) && (line >= g.lo_across) && (line < g.lim_across) && (f0 <= g.lim_line);
+    // face fluxes: times FS in the FP64 form (weno_k leaves its values times kFace; the flux
+    // difference of phase 3 divides by it)
+    constexpr double FS = MIX ? 1.0 : kFace;
     double Fv[5][K];
     // one-sided closures (BND): global index of the tile's first cell along the line
     const int n_dom = DIR == 0 ? k.nx : DIR == 1 ? k.ny : k.nz;
@@ -310,12 +313,12 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
                 double pv, mv;
                 const bool cp = closure_p(cellP, n_dom, fg, lo, hi, pv);
                 const bool cm = closure_m(cellM, n_dom, fg, lo, hi, mv);
-                if (cp || cm) Fv[m][j] = (cp ? pv : wenoP()) + (cm ? mv : wenoM());
+                if (cp || cm) Fv[m][j] = FS * ((cp ? pv : wenoP()) + (cm ? mv : wenoM()));
                 if (BND && nr_hi && fg == n_dom) {
                     double a = 0.0, b = 0.0;
                     closure_p(cellP, n_dom, n_dom - 1, lo, hi, a);
                     closure_p(cellP, n_dom, n_dom, lo, hi, b);
-                    nfix[m] = b - a;
+                    nfix[m] = FS * (b - a);
                 }
             };
             // a stored face f (f <= lim_line) reads only points f..f+7, all written in
@@ -341,12 +344,12 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
 #pragma unroll
                 for (int j = 0; j < K; ++j) {
                     const double den = dP[j] * dM[j];
-                    Fv[m][j] = (bP[j] + bM[j]) + fma(nP[j], dM[j], nM[j] * dP[j]) * recip_nr(den);
+                    Fv[m][j] = fma(fma(nP[j], dM[j], nM[j] * dP[j]), recip_nr(den), bP[j] + bM[j]);
                 }
                 if (near)
 #pragma unroll
                     for (int j = 0; j < K; ++j)
-                        closed(j, [&] { return bP[j] + nP[j] / dP[j]; }, [&] { return bM[j] + nM[j] / dM[j]; });
+                        closed(j, [&] { return (bP[j] + nP[j] / dP[j]) / kFace; }, [&] { return (bM[j] + nM[j] / dM[j]) / kFace; });
             }
         }
         // Faces whose FP32 weights left FP32's range (strong discontinuities of the split
@@ -367,13 +370,13 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
                         auto cellP = [&](int cg) { return sp[m * TL::QS + TL::pidx(line, cg - gl0 + LAP)]; };
                         auto cellM = [&](int cg) { return sp[(5 + m) * TL::QS + TL::pidx(line, cg - gl0 + LAP)]; };
                         double pv, mv;
-                        if (!closure_p(cellP, n_dom, fg, lo, hi, pv)) { face64<false>(qp + j, nP, dP, bP); pv = bP + nP / dP; }
-                        if (!closure_m(cellM, n_dom, fg, lo, hi, mv)) { face64<true>(qm + j, nM, dM, bM); mv = bM + nM / dM; }
+                        if (!closure_p(cellP, n_dom, fg, lo, hi, pv)) { face64<false>(qp + j, nP, dP, bP); pv = (bP + nP / dP) / kFace; }
+                        if (!closure_m(cellM, n_dom, fg, lo, hi, mv)) { face64<true>(qm + j, nM, dM, bM); mv = (bM + nM / dM) / kFace; }
                         val = pv + mv;
                     } else {
                         face64<false>(qp + j, nP, dP, bP);
                         face64<true>(qm + j, nM, dM, bM);
-                        val = (bP + bM) + fma(nP, dM, nM * dP) * recip_nr(dP * dM);
+                        val = fma(fma(nP, dM, nM * dP), recip_nr(dP * dM), bP + bM) / kFace;
                     }
 #pragma unroll
                     for (int q = 0; q < 5; ++q)
@@ -420,7 +423,7 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
     __syncthreads();
 
     // ---- phase 3: flux difference of each cell ---------------------------------------------
-    const double scale0 = -k.rh[DIR];
+    const double scale0 = -k.rh[DIR] / FS;
     const double sdt = STG ? (sa.dt_dev ? *sa.dt_dev : sa.dt) : 0.0;
     double cfl_max = 0.0;
 #pragma unroll
@@ -452,7 +455,7 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
                 double a = 0.0, b = 0.0;
                 closure_m(cellM, n_dom, 0, lo, hi, a);
                 closure_m(cellM, n_dom, 1, lo, hi, b);
-                val = scale * (b - a);
+                val = scale * (FS * (b - a));
             } else if (last_only_p) {
                 val = scale * nfix_lds[l * 5 + m];
             }

@@ -179,30 +179,31 @@ __device__ __forceinline__ void plane_conserved(const CellPrims &p, double cv, d
 // ---------------------------------------------------------------------------
 
 // Nonlinear weights are homogeneous of degree four in (eps + S_k), so the indicators may be
-// scaled freely.  The FP64 form scales them by 1/(720*39): the second-difference term
-// (780*36/720 = 39 in units of the 720 term) gets coefficient 1, the first-derivative
-// term 1/39 (folded into the candidates' difference coefficients as 1/sqrt(39)), the
-// third-difference term 39.05/39, and eps becomes 2.592e-6/(720*39).  The FP32 form keeps
-// the 1/720 scale (eps 3.6e-9): at 1/(720*39) the product of four (eps + S) factors of a
-// smooth window would fall below FP32's normal range.
+// scaled freely.  The FP64 form scales them by 1/(781*36): the third-difference term
+// (781*36 D3^2) becomes a plain square, the first-derivative term (720) takes
+// sqrt(720/(781*36)) in its coefficients and the second-difference term (780*36)
+// sqrt(780/781), and eps becomes 2.592e-6/(781*36).  The FP32 form keeps the 1/720 scale
+// (eps 3.6e-9): at 1/(781*36) the product of four (eps + S) factors of a smooth window would
+// fall below FP32's normal range.
 constexpr double kD0 = 0.0401954833730;
 constexpr double kD1 = 0.2493800006710;
 constexpr double kD2 = 0.4802686256260;
 constexpr double kD3 = 0.2009775476730;
 constexpr double kD4 = 0.0291783426580;
-constexpr double kEps39 = 2.592e-6 / (720.0 * 39.0);
-constexpr double kC39 = 39.05 / 39.0;
-constexpr double kA39 = 0.16012815380508713;   // 1/sqrt(39)
+constexpr double kEpsS = 2.592e-6 / (781.0 * 36.0);
+constexpr double kAS = 0.160025606145638858;    // sqrt(720 / (781 * 36))
+constexpr double kBS = 0.999359590072005084;    // sqrt(780 / 781)
+// linear weights over the central one
+constexpr double kR0 = kD0 / kD2, kR1 = kD1 / kD2, kR3 = kD3 / kD2, kR4 = kD4 / kD2;
 
-// Reciprocal: hardware estimate plus two Newton steps (error within a couple of ulp;
-// the argument is a positive normal number wherever it is used).
+// Reciprocal of a positive normal number: the hardware estimate (24 bits) and one
+// third-order step, r (1 + e + e^2) with e = 1 - x r, whose remainder e^3 is below 2^-69:
+// one instruction less than two Newton steps, error within an ulp.
 __device__ __forceinline__ double recip_nr(double x)
 {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-x, r, 1.0);
-    return fma(r, e, r);
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 }
 
 // Square root of a positive normal number: reciprocal-square-root estimate refined
@@ -218,14 +219,28 @@ __device__ __forceinline__ double sqrt_nr(double x)
     return fma(d, h, g);
 }
 
-// K consecutive faces from K+7 points s[0..K+6] (face j uses s[j..j+7]).  The forward
-// differences, the scaled first differences, the squared second differences and the
-// squared third differences (with eps added) are formed once per point and shared by the
-// K faces.  The linear weights and the 1/12 of the candidates are folded into the
-// candidate coefficients, and the weighted sums are evaluated in Horner form over the
-// prefix products of (eps + S_k).  The candidates are taken relative to the face's base
-// point w3 and written in Newton form over the shared forward differences, so they cost
-// three FMAs each; face j's value is base[j] + num[j] / den[j].
+// K consecutive faces from K+7 points s[0..K+6] (face j uses s[j..j+7]); face j's value is
+// (base[j] + num[j] / den[j]) / kFace.  The forward differences up to the fourth and the
+// squared third differences (eps added) are formed once per point and shared by the K faces.
+//
+// Everything that differs between two neighbouring candidates at a face is a multiple of
+// one fourth difference D4_k of the window (points k .. k+4), so each candidate is the
+// central one plus one or two fourth differences.  With A = the first-derivative term,
+// b = the second-derivative term, q = the candidate value, of candidates 0..4 (unscaled):
+//   a1 = a2 + D4_1,  a0 = a1 - 2 D4_0,  a3 = a2 + 2 D4_2,  a4 = a3 + 11 D4_3
+//   b1 = D2_2,  b2 = D2_3,  b0 = b1 - D4_0,  b3 = b1 - D4_2,  b4 = b3 - 2 D4_3
+//   12 (q1 - q2) = D4_1,  12 (q0 - q2) = D4_1 - 3 D4_0
+//   12 (q3 - q2) = D4_2,  12 (q4 - q2) = D4_2 - 3 D4_3
+//   a2 = 6 D1_2 + 3 D2_2 - D3_2,  12 q2 = 12 w3 + a2 + D2_2
+// With d_k the linear weights over the central one, e_k = eps + S_k and P = e0 e1 e2 e3 e4,
+// D = sum d_k P / e_k and N = sum 12 d_k (q_k - q2) P / e_k (the central candidate drops out)
+// are formed in pairs (0, 1) and (3, 4): D01 = d0 e1 + d1 e0, N01 = D4_1 D01 - 3 D4_0 d0 e1.
+// Bound by FP64 VALU issue (one instruction per four cycles), so the count is what matters:
+// 62 instructions per face and side with K = 2 against 86 with every candidate built from
+// its own differences (a whole RHS of 600x256x128 2.57 -> 2.23 ms on one box, an RK3 step of
+// 600x128x128 4.49 -> 3.94 ms).
+constexpr double kFace = 12.0;
+
 template <bool REV, int K, typename Load>
 __device__ __forceinline__ void weno_k(Load ld, double (&num)[K], double (&den)[K], double (&base)[K])
 {
@@ -237,69 +252,55 @@ __device__ __forceinline__ void weno_k(Load ld, double (&num)[K], double (&den)[
     double s[NP];
 #pragma unroll
     for (int i = 0; i < NP; ++i) s[i] = ld(i);
-    double D1[NP - 1], D2[NP - 2], D3[NP - 3], G1[NP - 1], C3[NP - 3], B2[NP - 2];
+    double D1[NP - 1], D2[NP - 2], D3[NP - 3], D4[NP - 4], C3[NP - 3], B[K + 1], T[NP - 4];
 #pragma unroll
-    for (int i = 0; i < NP - 1; ++i) { D1[i] = s[i + 1] - s[i]; G1[i] = (6.0 * kA39) * D1[i]; }
+    for (int i = 0; i < NP - 1; ++i) D1[i] = s[i + 1] - s[i];
 #pragma unroll
-    for (int i = 0; i < NP - 2; ++i) { D2[i] = D1[i + 1] - D1[i]; B2[i] = D2[i] * D2[i]; }
+    for (int i = 0; i < NP - 2; ++i) D2[i] = D1[i + 1] - D1[i];
 #pragma unroll
-    for (int i = 0; i < NP - 3; ++i) { D3[i] = D2[i + 1] - D2[i]; C3[i] = fma(kC39 * D3[i], D3[i], kEps39); }
+    for (int i = 0; i < NP - 3; ++i) { D3[i] = D2[i + 1] - D2[i]; C3[i] = fma(D3[i], D3[i], kEpsS); }
+#pragma unroll
+    for (int i = 0; i < NP - 4; ++i) { D4[i] = D3[i + 1] - D3[i]; T[i] = 3.0 * D4[i]; }
+    // the scaled second differences centred on the two points beside each face
+#pragma unroll
+    for (int i = 0; i < K + 1; ++i) B[i] = kBS * D2[i + 2];
 #pragma unroll
     for (int j = 0; j < K; ++j) {
-        // window point k of this face, and the anchors of candidate k's differences
-        auto w = [&](int k) { return REV ? s[j + 7 - k] : s[j + k]; };
-        auto i1 = [&](int k) { return REV ? j + 6 - k : j + k; };
-        auto i2 = [&](int k) { return REV ? j + 5 - k : j + k; };
-        auto i3 = [&](int k) { return REV ? j + 4 - k : j + k; };
-        const double sb = REV ? -kA39 : kA39;
-        // first-derivative terms over sqrt(39) (the sign of a term is irrelevant: it is squared)
-        const double a0 = fma(11.0 * kA39, D3[i3(0)], fma(sb * 15.0, D2[i2(0)], G1[i1(0)]));
-        const double a1 = fma(2.0 * kA39, D3[i3(1)], fma(sb * 9.0, D2[i2(1)], G1[i1(1)]));
-        const double a2 = fma(-1.0 * kA39, D3[i3(2)], fma(sb * 3.0, D2[i2(2)], G1[i1(2)]));
-        const double a3 = fma(2.0 * kA39, D3[i3(3)], fma(sb * -3.0, D2[i2(3)], G1[i1(3)]));
-        const double a4 = fma(11.0 * kA39, D3[i3(4)], fma(sb * -9.0, D2[i2(4)], G1[i1(4)]));
-        // second-derivative terms of candidates 0, 3, 4 (1 and 2 are plain second differences)
-        const double b0 = REV ? fma(-2.0, D3[j + 4], D2[j + 5]) : fma(2.0, D3[j], D2[j]);
-        const double b3 = REV ? D2[j + 2] + D3[j + 1] : D2[j + 3] - D3[j + 3];
-        const double b4 = REV ? fma(2.0, D3[j], D2[j + 1]) : fma(-2.0, D3[j + 4], D2[j + 4]);
-        const double bb1 = REV ? B2[j + 3] : B2[j + 2];
-        const double bb2 = REV ? B2[j + 2] : B2[j + 3];
+        // differences of the window as the rule sees it (reversed for REV: odd ones change sign)
+        auto d4 = [&](int k) { return D4[REV ? j + 3 - k : j + k]; };
+        auto c3 = [&](int k) { return C3[REV ? j + 4 - k : j + k]; };
+        const double d2c = D2[REV ? j + 3 : j + 2];
+        const double a2u = REV ? fma(-6.0, D1[j + 4], fma(3.0, d2c, D3[j + 2]))
+                               : fma(6.0, D1[j + 2], fma(3.0, d2c, -D3[j + 2]));
+        const double a2 = kAS * a2u;
+        const double a1 = fma(kAS, d4(1), a2);
+        const double a0 = fma(-2.0 * kAS, d4(0), a1);
+        const double a3 = fma(2.0 * kAS, d4(2), a2);
+        const double a4 = fma(11.0 * kAS, d4(3), a3);
+        const double b1 = B[REV ? j + 1 : j], b2 = B[REV ? j : j + 1];
+        const double b0 = fma(-kBS, d4(0), b1);
+        const double b3 = fma(-kBS, d4(2), b1);
+        const double b4 = fma(-2.0 * kBS, d4(3), b3);
         // e_k = eps + S_k (eps rides in C3)
-        const double e0 = fma(a0, a0, fma(b0, b0, C3[i3(0)]));
-        const double e1 = fma(a1, a1, bb1 + C3[i3(1)]);
-        const double e2 = fma(a2, a2, bb2 + C3[i3(2)]);
-        const double e3 = fma(a3, a3, fma(b3, b3, C3[i3(3)]));
-        double e4 = fma(a4, a4, fma(b4, b4, C3[i3(4)]));
+        const double e0 = fma(a0, a0, fma(b0, b0, c3(0)));
+        const double e1 = fma(a1, a1, fma(b1, b1, c3(1)));
+        const double e2 = fma(a2, a2, fma(b2, b2, c3(2)));
+        const double e3 = fma(a3, a3, fma(b3, b3, c3(3)));
+        double e4 = fma(a4, a4, fma(b4, b4, c3(4)));
         e4 = fmax(fmax(fmax(e0, e1), fmax(e2, e3)), e4);
-        // candidates relative to the base point w(3), in Newton form over the forward
-        // differences at each candidate's first point (linear weights folded in): each
-        // candidate's coefficients sum to 12, so the base drops out
-        const double sd = REV ? -1.0 : 1.0;   // sign of odd differences of the reversed window
-        auto d1 = [&](int k) { return D1[REV ? j + 6 - k : j + k]; };
-        auto d2 = [&](int k) { return D2[REV ? j + 5 - k : j + k]; };
-        auto d3 = [&](int k) { return D3[REV ? j + 4 - k : j + k]; };
-        const double c0 = fma(sd * kD0 * (13.0 / 12.0), d3(0), fma(kD0 * (4.0 / 3.0), d2(0), (sd * kD0 * 0.5) * d1(0)));
-        const double c1 = fma(sd * kD1 * (1.0 / 4.0), d3(1), fma(kD1 * (5.0 / 6.0), d2(1), (sd * kD1 * 0.5) * d1(1)));
-        const double c2 = fma(sd * kD2 * (-1.0 / 12.0), d3(2), fma(kD2 * (1.0 / 3.0), d2(2), (sd * kD2 * 0.5) * d1(2)));
-        const double c3 = fma(sd * kD3 * (1.0 / 12.0), d3(3), fma(kD3 * (-1.0 / 6.0), d2(3), (sd * kD3 * 0.5) * d1(3)));
-        const double c4 = fma(sd * kD4 * (-1.0 / 4.0), d3(4), fma(kD4 * (1.0 / 3.0), d2(4),
-                              fma(sd * kD4 * -0.5, d1(4), (sd * kD4) * d1(3))));
-        base[j] = w(3);
-        const double p01 = e0 * e1;
-        double N = fma(c0, e1, c1 * e0);
-        double D = fma(kD0, e1, kD1 * e0);
-        N = fma(N, e2, c2 * p01);
-        D = fma(D, e2, kD2 * p01);
-        const double p012 = p01 * e2;
-        N = fma(N, e3, c3 * p012);
-        D = fma(D, e3, kD3 * p012);
-        const double p0123 = p012 * e3;
-        num[j] = fma(N, e4, c4 * p0123);
-        den[j] = fma(D, e4, kD4 * p0123);
+        base[j] = fma(kFace, s[REV ? j + 4 : j + 3], a2u + d2c);
+        const double t0 = kR0 * e1, t4 = kR4 * e3;
+        const double D01 = fma(kR1, e0, t0), D34 = fma(kR3, e4, t4);
+        const double N01 = fma(d4(1), D01, -(T[REV ? j + 3 : j] * t0));
+        const double N34 = fma(d4(2), D34, -(T[REV ? j : j + 3] * t4));
+        const double p01 = e0 * e1, p34 = e3 * e4;
+        const double q01 = e2 * p34, q34 = e2 * p01;
+        num[j] = fma(N01, q01, N34 * q34);
+        den[j] = fma(p34, fma(e2, D01, p01), q34 * D34);
     }
 }
 
-// One face of weno_k from the 8-point window q[0..7]: base + num / den is the face value.
+// One face of weno_k from the 8-point window q[0..7]: (base + num / den) / kFace is its value.
 template <bool REV>
 __device__ __forceinline__ void face64(const double *q, double &num, double &den, double &base)
 {
