@@ -33,6 +33,8 @@ KParams make_kparams(const ws_config &c)
     k.c1 = 2.0 * (c.gamma - 1.0);                          // OCFD_init.cpp:385
     k.c3 = (3.0 - c.gamma) / (2.0 * (c.gamma - 1.0));      // OCFD_init.cpp:386
     k.half_rcp_gamma = 0.5 / c.gamma;
+    k.quarter_rcp_gamma = 0.25 / c.gamma;
+    k.c3h = 0.5 + k.c3;
     k.gm1 = c.gamma - 1.0;
     k.eps2 = c.epsl_sw * c.epsl_sw;
     k.ama = c.ama; k.rcp_ama = 1.0 / c.ama;
@@ -44,6 +46,7 @@ KParams make_kparams(const ws_config &c)
         const double a1 = c.metric[3 * dir], a2 = c.metric[3 * dir + 1], a3 = c.metric[3 * dir + 2];
         const double sn = std::sqrt(a1 * a1 + a2 * a2 + a3 * a3);
         k.Anorm[dir] = sn;
+        k.Arnorm[dir] = 1.0 / sn;
         k.Ak[3 * dir] = a1 / sn; k.Ak[3 * dir + 1] = a2 / sn; k.Ak[3 * dir + 2] = a3 / sn;
     }
     k.ajac = c.metric[9];

@@ -219,6 +219,27 @@ __device__ __forceinline__ double sqrt_nr(double x)
     return fma(d, h, g);
 }
 
+// Square root of a positive normal number and its reciprocal: the reciprocal-square-root
+// estimate y (24 bits) and one third-order step, with e = 1 - x y^2: sqrt(x) = x y (1 + e/2 +
+// 3/8 e^2), 1/sqrt(x) = y (1 + e/2 + 3/8 e^2); the remainder 5/16 e^3 is below 2^-70.  Two
+// instructions fewer than sqrt_nr; error within an ulp.
+__device__ __forceinline__ double sqrt_h(double x)
+{
+#pragma clang fp contract(off)
+    const double y = __builtin_amdgcn_rsq(x), g = x * y;
+    const double e = fma(-g, y, 1.0);
+    return fma(g * e, fma(0.375, e, 0.5), g);
+}
+
+__device__ __forceinline__ void sqrt_rsqrt_h(double x, double &root, double &rcp)
+{
+#pragma clang fp contract(off)
+    const double y = __builtin_amdgcn_rsq(x), g = x * y;
+    const double e = fma(-g, y, 1.0), p = fma(0.375, e, 0.5);
+    root = fma(g * e, p, g);
+    rcp = fma(y * e, p, y);
+}
+
 // K consecutive faces from K+7 points s[0..K+6] (face j uses s[j..j+7]); face j's value is
 // (base[j] + num[j] / den[j]) / kFace.  The forward differences up to the fourth and the
 // squared third differences (eps added) are formed once per point and shared by the K faces.
@@ -598,9 +619,56 @@ __device__ __forceinline__ bool closure_m(Cell cell, int n, int f, bool lo, int 
     return false;
 }
 
-// Steger-Warming split in the form the tiled kernels use: A1..A3 the metric terms,
-// sn = |A|, k1..k3 = A/|A| supplied by the caller (constants when metrics are uniform).
+// Steger-Warming split in the form the tiled FP64 kernels use: A1..A3 the metric terms, sn = |A|
+// and rsn = 1/|A| supplied by the caller (constants when metrics are uniform).  With vs = A.u,
+// cs = c |A|, P_i twice the smoothed positive eigenvalues of vs, vs - cs, vs + cs and
+// s = P_2 + P_3, d = P_3 - P_2, the mass flux is f0 = t (c1 P_1 + s), the momentum flux f0 u_i +
+// t c/|A| d A_i and the energy flux t (P_1 vv + s (|u|^2/2 + c^2/2 + W2) + d c vs/|A|); the
+// negative part takes 2 vs - P_1, 4 vs - s and 4 cs - d.  71 FP64 instructions against the 108
+// of split_mixed (whose shifted velocities u -+ c k are spelled out); a tile splits 25-31 %
+// more points than it owns.
 __device__ __forceinline__ void split_fast(const KParams &k, double d, double u, double v, double w,
+                                           double cc, double A1, double A2, double A3, double sn,
+                                           double rsn, double fp[5], double fm[5])
+{
+    // contraction off: a point split by two tiles must come out the same in both
+#pragma clang fp contract(off)
+    const double vs = fma(A3, w, fma(A2, v, A1 * u));
+    const double cs = cc * sn;
+    const double E2 = vs - cs, E3 = vs + cs;
+    // eps2 > 0 keeps the radicands positive and normal
+    const double P1 = vs + sqrt_h(fma(vs, vs, k.eps2));
+    const double P2 = E2 + sqrt_h(fma(E2, E2, k.eps2));
+    const double P3 = E3 + sqrt_h(fma(E3, E3, k.eps2));
+    const double t = d * k.quarter_rcp_gamma;
+    const double cr = cc * rsn, cv = cr * vs, tc = t * cr;
+    const double q = fma(w, w, fma(v, v, u * u));
+    const double vv = k.gm1 * q, H = fma(0.5, q, k.c3h * (cc * cc));
+    const double sP = P2 + P3, dP = P3 - P2;
+    {
+        const double g = tc * dP;
+        fp[0] = t * fma(k.c1, P1, sP);
+        fp[1] = fma(g, A1, fp[0] * u);
+        fp[2] = fma(g, A2, fp[0] * v);
+        fp[3] = fma(g, A3, fp[0] * w);
+        fp[4] = t * fma(P1, vv, fma(sP, H, dP * cv));
+    }
+    {
+        const double M1 = fma(2.0, vs, -P1), sM = fma(4.0, vs, -sP), dM = fma(4.0, cs, -dP);
+        const double g = tc * dM;
+        fm[0] = t * fma(k.c1, M1, sM);
+        fm[1] = fma(g, A1, fm[0] * u);
+        fm[2] = fma(g, A2, fm[0] * v);
+        fm[3] = fma(g, A3, fm[0] * w);
+        fm[4] = t * fma(M1, vv, fma(sM, H, dM * cv));
+    }
+}
+
+// Steger-Warming split of the mixed-precision kernels: k1..k3 = A/|A|.  The mixed
+// reconstruction rounds first differences of these values to FP32, where a last-bit change
+// of a value can flip a rounding a hundred million times its size, so this form keeps its
+// arithmetic.
+__device__ __forceinline__ void split_mixed(const KParams &k, double d, double u, double v, double w,
                                            double cc, double A1, double A2, double A3, double sn,
                                            double k1, double k2, double k3, double fp[5], double fm[5])
 {

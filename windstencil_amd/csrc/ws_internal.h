@@ -19,6 +19,8 @@ struct KParams {
     double c1;                 // 2(gamma-1)
     double c3;                 // (3-gamma)/(2(gamma-1))
     double half_rcp_gamma;     // 0.5/gamma
+    double quarter_rcp_gamma;  // 0.25/gamma
+    double c3h;                // 0.5 + c3
     double gm1;                // gamma-1
     double eps2;               // epsl_sw^2
     double ama, rcp_ama;
@@ -27,7 +29,7 @@ struct KParams {
     double rh[3];              // 1/h
     // constant metrics: direction d uses A[3d..3d+2]; their norm and unit vector
     double A[9];
-    double Anorm[3];
+    double Anorm[3], Arnorm[3];   // Arnorm: 1/Anorm
     double Ak[9];
     double ajac;
     // one-sided closures of the inviscid scheme at the domain faces (x-, x+, y-, y+, z-, z+:
