@@ -338,8 +338,8 @@ int ws_ana_state_noalloc(ws_ctx *ctx, const ws_state *st, const ws_metric_fields
  * src/kernels/commen_kernel.cpp:123-141), central-difference gradients of u, v, w, T, the
  * stress and heat flux of each direction, their periodic exchange and central derivative,
  * du += Ajac * that.  u, v, w, T must have their periodic ghosts filled; cfg.viscous gives
- * the order (6 or 8).  Uses a device scratch of 12 ghosted fields owned by the context,
- * allocated at the first call. */
+ * the order (6 or 8).  The anchor kernel family uses a device scratch of 12 ghosted fields
+ * owned by the context, allocated at its first call; the tiled family none. */
 int ws_viscous_rhs(ws_ctx *ctx, ws_field u, ws_field v, ws_field w, ws_field T, const ws_metric_fields *metrics,
                    ws_soa du, hipStream_t stream);
 

@@ -231,3 +231,65 @@ def test_viscous_terms_with_closed_faces(orc, ws, faces, order, kernel):
         assert np.array_equal(dg, full)
     else:
         assert err <= 1e-12
+
+
+@pytest.mark.parametrize("pads", [(0, 0), (3, 0), (0, 5)])
+@pytest.mark.parametrize("order", [6, 8])
+@pytest.mark.parametrize("faces", [((1, 1, 1), (0, 0, 0, 0, 0, 0))] + CLOSED)
+def test_fused_viscous_terms_over_metric_fields_layouts_and_chunks(orc, ws, faces, order, pads):
+    """The fused kernel with metric fields, every closure combination, tiles and z chunks with
+    remainders (each extent one past a multiple of the tile of one order), fields that share a
+    pitch (one 32-bit offset) and, by a padded T or a padded metric term, fields that do not.
+    Within 1e-13 of the oracle alone, as for constant metrics."""
+    import torch
+    from tests.test_gpu_rhs import _wavy_metrics
+    periodic, bnd = faces
+    nx, ny, nz = 53, 25, 31
+    prims = random_state(nx, ny, nz, 19, "vortex")
+    p = orc.params(nx, ny, nz, periodic=periodic, d0_bound=bnd)
+    g = [ghosted(a) for a in prims]
+    met = [ghosted(a) for a in _wavy_metrics(nx, ny, nz)]
+    for a in g + met:
+        orc.ghost_fill_periodic(p, a)
+    ref = orc.viscous_rhs(p, g[1], g[2], g[3], g[4], RE, PR, TREF, order, metrics=met[:9], ajac=met[9])
+
+    def padded(a, pad):
+        t = W.ghosted_tensor(nx, ny, nz, pad)
+        t[:, :, :nx + 8] = torch.from_numpy(a)
+        return t
+    fields = [padded(g[q], pads[0] if q == 4 else 0) for q in (1, 2, 3, 4)]
+    terms = [padded(a, pads[1] if q == 7 else 0) for q, a in enumerate(met)]
+    mf = W.WsMetricFields()
+    for q in range(9):
+        mf.A[q] = W.field_of(terms[q])
+    mf.ajac = W.field_of(terms[9])
+    ctx = make_ctx(nx, ny, nz, periodic=periodic, d0_bound=bnd, **_vis_cfg(order))
+    du = W.soa_tensor(nx, ny, nz)
+    W.check(W.lib().ws_viscous_rhs(ctx.handle, *[W.field_of(t) for t in fields], ctypes.byref(mf), W.soa_of(du),
+                                   W.stream_handle()))
+    torch.cuda.synchronize()
+    err = rel_l2(du.cpu().numpy(), ref)
+    log(f"fused viscous {faces} order {order} pads {pads}: rel L2 {err:.3e}")
+    assert err <= 1e-13
+
+
+@pytest.mark.parametrize("shape", [(4, 4, 4), (5, 4, 9), (26, 10, 7), (27, 11, 130), (25, 9, 65)])
+@pytest.mark.parametrize("order", [6, 8])
+def test_fused_viscous_terms_at_tile_edges(orc, ws, shape, order):
+    """Extents of one tile, one past it, and below the stencil's reach (the halo wraps more
+    than once), periodic: within 1e-13 of the oracle alone."""
+    import torch
+    nx, ny, nz = shape
+    prims = random_state(nx, ny, nz, 23, "blobs")
+    p = orc.params(nx, ny, nz)
+    g = [ghosted(a) for a in prims]
+    for a in g:
+        orc.ghost_fill_periodic(p, a)
+    ref = orc.viscous_rhs(p, g[1], g[2], g[3], g[4], RE, PR, TREF, order)
+    ctx = make_ctx(nx, ny, nz, **_vis_cfg(order))
+    st = upload_state(prims)
+    W.check(W.lib().ws_viscous_rhs(ctx.handle, st.ws.u, st.ws.v, st.ws.w, st.ws.T, None, st.ws.du, W.stream_handle()))
+    torch.cuda.synchronize()
+    err = rel_l2(st.interior("du").cpu().numpy(), ref)
+    log(f"fused viscous {shape} order {order}: rel L2 {err:.3e}")
+    assert err <= 1e-13

@@ -467,6 +467,11 @@ int ws_ctx_create(const ws_config *cfg, ws_ctx **out)
     }
     hipError_t e = hipGetDevice(&c->device);
     if (e != hipSuccess) { delete c; return hip_error(e, "hipGetDevice"); }
+    if (hipDeviceGetAttribute(&c->compute_units, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess ||
+        c->compute_units <= 0) {
+        (void)hipGetLastError();
+        c->compute_units = 256;
+    }
     c->cfl_blocks = 1024;
     e = hipMalloc(&c->cfl_partial, sizeof(double) * c->cfl_blocks);
     if (e != hipSuccess) { delete c; return hip_error(e, "CFL scratch allocation"); }

@@ -1,8 +1,8 @@
 // k_viscous.hip -- viscous terms of the RHS (the reference's du_vis_Jacobian3d path).
 //
-// The tiled kernel family with constant metrics runs one fused kernel, k_vis_fused (below),
-// whose fluxes never leave the chip.  The anchor family and per-cell metric fields run two
-// kernels around a ghost fill, each marching column tiles along z:
+// The tiled kernel family runs one fused kernel, k_vis_fused (below), whose fluxes never
+// leave the chip.  The anchor family runs two kernels around a ghost fill, each marching
+// column tiles along z:
 //   k_vis_flux: per interior cell, Sutherland viscosity, the twelve central-difference
 //               gradients (u, v, w, T along x, y, z), the stress tensor and heat flux, and
 //               the four viscous fluxes of each of the three directions (twelve ghosted
@@ -15,12 +15,10 @@
 // fluxes' derivatives round-tripping through HBM; here the gradients never leave
 // registers.
 //
-// EXACT kernels evaluate every expression in the reference's order with contraction off
+// The two kernels evaluate every expression in the reference's order with contraction off
 // and divide as the reference does ((stencil / 60) / h): bit-identical to the CPU
-// restatement; they serve the anchor kernel family.  The fast kernels (the tiled family)
-// multiply the stencil sum by 1 / (60 h) (1 / (840 h) for the eighth order): two correctly
-// rounded divisions per derivative become one multiplication, which moves a derivative by
-// a few units in the last place.
+// restatement.  The fused kernel weights the differences f(c + q) - f(c - q) instead, which
+// moves a derivative by a few units in the last place.
 #include <hip/hip_runtime.h>
 
 #include "ws_device.h"
@@ -40,8 +38,6 @@ constexpr int ZC = 32;
 struct VisParams {
     int nx, ny, nz, nyg;
     double h[3];
-    double rh[3];            // 1 / h
-    double rch[3];           // 1 / (60 h) or 1 / (840 h): the fast kernels' derivative scale
     double amu_c0, tsb, vis_c;
     double metric[10];       // constant Akx..Asz, Ajac
     int bnd[6];              // closed faces (D0_bound): x-, x+, y-, y+, z-, z+
@@ -66,27 +62,13 @@ __device__ __forceinline__ double cd_stencil8(const double *s)
     return (672.0 * (s[5] - s[3]) - 168.0 * (s[6] - s[2]) + 32.0 * (s[7] - s[1]) - 3.0 * (s[8] - s[0])) / 840.0;
 }
 
-__device__ __forceinline__ double cd_sum6(const double *s)
-{
-    return 45.0 * (s[4] - s[2]) - 9.0 * (s[5] - s[1]) + (s[6] - s[0]);
-}
-
-__device__ __forceinline__ double cd_sum8(const double *s)
-{
-    return 672.0 * (s[5] - s[3]) - 168.0 * (s[6] - s[2]) + 32.0 * (s[7] - s[1]) - 3.0 * (s[8] - s[0]);
-}
-
 // central derivative along direction d of the stencil values s[0 .. ORDER]
-template <int ORDER, bool EXACT>
+template <int ORDER>
 __device__ __forceinline__ double cd_dir(const double *s, const VisParams &p, int d)
 {
-    if constexpr (EXACT) {
 #pragma clang fp contract(off)
-        const double tmp = ORDER == 8 ? cd_stencil8(s) : cd_stencil6(s);
-        return tmp / p.h[d];
-    } else {
-        return (ORDER == 8 ? cd_sum8(s) : cd_sum6(s)) * p.rch[d];
-    }
+    const double tmp = ORDER == 8 ? cd_stencil8(s) : cd_stencil6(s);
+    return tmp / p.h[d];
 }
 
 // The forms of the four cells next to a closed face (the reference's D0_bound,
@@ -119,24 +101,17 @@ __device__ __forceinline__ bool cd_closure(const double *s0, int c, int n, bool 
 }
 
 // Derivative along direction d at interior index c: a closure form next to a closed face
-// (BND), else the central form.  The exact kernels divide the form by h as the reference
-// does (put_d0_kernel), the fast ones multiply by 1/h.
-template <int ORDER, bool EXACT, bool BND>
+// (BND), else the central form; either is divided by h as the reference does (put_d0_kernel).
+template <int ORDER, bool BND>
 __device__ __forceinline__ double cd_at(const double *s, const VisParams &p, int d, int c)
 {
+#pragma clang fp contract(off)
     if constexpr (BND) {
         const int n = d == 0 ? p.nx : d == 1 ? p.ny : p.nz;
         double tmp;
-        if (cd_closure<ORDER / 2>(s, c, n, p.bnd[2 * d] != 0, p.bnd[2 * d + 1] != 0, tmp)) {
-            if constexpr (EXACT) {
-#pragma clang fp contract(off)
-                return tmp / p.h[d];
-            } else {
-                return tmp * p.rh[d];
-            }
-        }
+        if (cd_closure<ORDER / 2>(s, c, n, p.bnd[2 * d] != 0, p.bnd[2 * d + 1] != 0, tmp)) return tmp / p.h[d];
     }
-    return cd_dir<ORDER, EXACT>(s, p, d);
+    return cd_dir<ORDER>(s, p, d);
 }
 
 // Plane tile with an R-deep halo in x and y (no corners): tile coordinates (px, py),
@@ -236,7 +211,7 @@ __device__ __forceinline__ Col column(const double *ptr, uint32_t pitch, int nyg
     return Col{ptr + fidx(pitch, nyg, x, y, 0), (size_t)pitch * (size_t)nyg};
 }
 
-template <int ORDER, bool FIELDS, bool EXACT, bool BND>
+template <int ORDER, bool FIELDS, bool BND>
 __global__ void __launch_bounds__(NT) k_vis_flux(VisParams p, ws_field u, ws_field v, ws_field w, ws_field T,
                                                  ws_metric_fields mf, EvFields ev)
 {
@@ -303,18 +278,18 @@ __global__ void __launch_bounds__(NT) k_vis_flux(VisParams p, ws_field u, ws_fie
                 double s[Q];
 #pragma unroll
                 for (int q = 0; q < Q; ++q) s[q] = lds[b][f][R + t.ty][t.tx + q];
-                return cd_at<ORDER, EXACT, BND>(s, p, 0, cx);
+                return cd_at<ORDER, BND>(s, p, 0, cx);
             };
             auto dy = [&](int f) {
                 double s[Q];
 #pragma unroll
                 for (int q = 0; q < Q; ++q) s[q] = lds[b][f][t.ty + q][R + t.tx];
-                return cd_at<ORDER, EXACT, BND>(s, p, 1, cy);
+                return cd_at<ORDER, BND>(s, p, 1, cy);
             };
             const double uk = dx(0), vk = dx(1), wk = dx(2), Tk = dx(3);
             const double ui = dy(0), vi = dy(1), wi = dy(2), Ti = dy(3);
-            const double us = cd_at<ORDER, EXACT, BND>(c[0], p, 2, cz), vs = cd_at<ORDER, EXACT, BND>(c[1], p, 2, cz);
-            const double ws = cd_at<ORDER, EXACT, BND>(c[2], p, 2, cz), Ts = cd_at<ORDER, EXACT, BND>(c[3], p, 2, cz);
+            const double us = cd_at<ORDER, BND>(c[0], p, 2, cz), vs = cd_at<ORDER, BND>(c[1], p, 2, cz);
+            const double ws = cd_at<ORDER, BND>(c[2], p, 2, cz), Ts = cd_at<ORDER, BND>(c[3], p, 2, cz);
             const double Akx = met(0), Aky = met(1), Akz = met(2), Aix = met(3), Aiy = met(4), Aiz = met(5);
             const double Asx = met(6), Asy = met(7), Asz = met(8), aj1 = met(9);
             // viscosity (get_Amu_kernal) and the stress tensor (vis_flux_ker)
@@ -356,7 +331,7 @@ __global__ void __launch_bounds__(NT) k_vis_flux(VisParams p, ws_field u, ws_fie
     }
 }
 
-template <int ORDER, bool FIELDS, bool EXACT, bool BND>
+template <int ORDER, bool FIELDS, bool BND>
 __global__ void __launch_bounds__(NT) k_vis_div(VisParams p, EvFields ev, ws_field ajac, ws_soa du)
 {
 #pragma clang fp contract(off)
@@ -436,17 +411,17 @@ __global__ void __launch_bounds__(NT) k_vis_div(VisParams p, EvFields ev, ws_fie
                 double s[Q];
 #pragma unroll
                 for (int q = 0; q < Q; ++q) s[q] = lx[b][m][t.ty][t.tx + q];
-                acc[m] = acc[m] + aj * cd_at<ORDER, EXACT, BND>(s, p, 0, cx);
+                acc[m] = acc[m] + aj * cd_at<ORDER, BND>(s, p, 0, cx);
             }
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
                 double s[Q];
 #pragma unroll
                 for (int q = 0; q < Q; ++q) s[q] = ly[b][m][t.ty + q][t.tx];
-                acc[m] = acc[m] + aj * cd_at<ORDER, EXACT, BND>(s, p, 1, cy);
+                acc[m] = acc[m] + aj * cd_at<ORDER, BND>(s, p, 1, cy);
             }
 #pragma unroll
-            for (int m = 0; m < 4; ++m) acc[m] = acc[m] + aj * cd_at<ORDER, EXACT, BND>(cz[m], p, 2, ck);
+            for (int m = 0; m < 4; ++m) acc[m] = acc[m] + aj * cd_at<ORDER, BND>(cz[m], p, 2, ck);
 #pragma unroll
             for (int m = 0; m < 4; ++m) dp[(m + 1) * vstride] = acc[m];
         }
@@ -457,28 +432,69 @@ __global__ void __launch_bounds__(NT) k_vis_div(VisParams p, EvFields ev, ws_fie
     }
 }
 
-// ---- fused form (fast family, constant metrics) ------------------------------------------
+// ---- fused form (fast family) ------------------------------------------------------------
 //
 // One kernel for the whole viscous update: no flux field goes through memory.  A work-group
 // of FX x FY = 32 x 16 threads owns the flux points of a (FX - 2R) x (FY - 2R) cell tile plus
 // an R-deep ring around it and marches a chunk of planes along z.  At each flux plane every
 // thread computes the twelve gradients at its point (x and y stencils from an LDS copy of
 // the plane with a further R-deep border, the z stencil from its column's register window)
-// and the fluxes its point contributes: x fluxes on the tile's rows, y fluxes on its
-// columns, all twelve inside the tile.  The x and y fluxes go to LDS and the tile's threads
-// take their derivatives at once; the z fluxes stay in a register ring, so a cell's update
-// completes R planes later: du += Ajac * (dx F_x + dy F_y) + Ajac * dz F_z.  Data points are
-// addressed in interior coordinates: a periodic direction wraps them onto the interior (the
-// flux at a point past the face is the one of its periodic image, bit for bit), a closed one
-// clamps them (the closure forms read no point past the face), so neither the fields' ghost
-// layers nor any scratch is touched.  Algorithmic traffic 96 B per cell: u, v, w, T in and
-// du[1..4] read and written.
+// and the fluxes its point contributes: x fluxes on the tile's rows, y fluxes on its columns,
+// z fluxes inside the tile.  The x and y fluxes go to LDS and are differentiated one plane
+// later; a z flux is added at once, weighted, to the 2R cells of its column whose derivative
+// it enters (register accumulators of the cells zf - R .. zf + R), so a cell is complete R
+// planes after its own flux plane.
+//
+// Both LDS arrays are double-buffered: a step computes plane zf's fluxes from one copy,
+// writes the copy of plane zf + 1, and differentiates the fluxes of plane zf - 1, with one
+// barrier between steps; the loads of the next step are issued at its top.  The window and
+// the accumulators turn by one slot per plane, so the loop is unrolled over one turn (2R + 1
+// steps) and no slot is ever moved.
+//
+// Data points are addressed in interior coordinates: a periodic direction wraps them onto the
+// interior (the flux at a point past the face is the one of its periodic image, bit for bit),
+// so neither the fields' ghost layers nor any scratch is touched.  At a closed face the
+// derivative forms (cd_closure) are all weights on f(c + q) - f(c - q), q <= 3, if the points
+// past the face repeat the face cell's value: the first-order one-sided difference is q = 1
+// with weight 1.  Points past the face therefore are the face point itself (its data, its
+// flux), the weights come from a table by the distance to the face, and a difference whose
+// weight is zero reads the cell itself on both sides.
+//
+// MODE: constant metrics without off-diagonal terms (a Cartesian box; the weights carry the
+// metric terms), constant metrics, or metric fields read per flux point.  FAST: the fields
+// share one pitch and a plane of them fits 32-bit byte offsets (the launcher checks), so one
+// offset per thread addresses them all; otherwise each field is addressed by itself.
+//
+// Algorithmic traffic 96 B per cell (constant metrics): u, v, w, T in and du[1..4] read and
+// written.  512 threads of up to 256 VGPRs: one work-group per compute unit.
+//
+// What bounds it: a step moves 84 values per thread through LDS at 128 B per cycle (3,100 of
+// about 5,300 cycles), and the eight wavefronts read LDS and compute in the same phases, so
+// the two add up; issuing each stage's reads under the stage before it, and letting half the
+// wavefronts run half a step behind, were tried and measured no faster.  Before this form (z
+// fluxes and xy sums in LDS rings, closure forms branched per derivative, fixed 64-plane
+// chunks) and now, alone: 600x128x128 sixth order 638 -> 515 us, eighth 942 -> 734;
+// 157x111x75 193 -> 83 and 227 -> 133; x faces closed 211x93x67 461 -> 96 and 458 -> 180, all
+// faces closed 520 -> 164 and 522 -> 203; metric fields 256x160x96 (two kernels around a ghost
+// fill of twelve flux fields before) 445 -> 321 and 450 -> 387.
 constexpr int FX = 32, FY = 16, FNT = FX * FY;
+enum { VM_DIAG, VM_CONST, VM_FIELDS };
+enum { VC_NONE, VC_XY, VC_ALL };
+
+// Weights of the differences f(c + q) - f(c - q), q = 1..4 at index q - 1.
+struct VisWeights {
+    double g[3][4];          // gradient along d: coefficient / h_d (VM_DIAG: times A_dd)
+    double f[3][4];          // flux derivative along d: coefficient / h_d times the Jacobian factors
+    double row[5][4];        // coefficients at distance 0..3 from a closed face, and the central ones
+    double rg[5][4], rf[5][4];   // the same times gs[2] and fs[2]
+    double gs[3], fs[3];     // what g and f multiply the central coefficients by
+};
 
 template <int R>
 struct Fused {
     static constexpr int TX = FX - 2 * R, TY = FY - 2 * R;     // cells of the tile
     static constexpr int PX = FX + 2 * R, PY = FY + 2 * R;     // plane copy: flux points + border
+    static constexpr int PN = PX * PY;
     static constexpr int NBX = 2 * R * FY;                     // border points left and right
     static constexpr int NB = NBX + 2 * R * FX;                // and below and above (no corners)
     static_assert(NB <= FNT, "one border point per thread");
@@ -508,23 +524,64 @@ __device__ __forceinline__ int wrap_coord(int c, int n, bool periodic)
     return c < 0 ? 0 : (c >= n ? n - 1 : c);
 }
 
-// DIAG: the constant metrics have zero off-diagonal terms (a Cartesian box), so each metric
-// product keeps only its diagonal term; the values are the general form's (a zero product
-// adds nothing to a sum or an FMA), with about 10 % fewer instructions.
-template <int ORDER, bool BND, bool DIAG>
-__global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, ws_field u, ws_field v, ws_field w, ws_field T,
-                                                   ws_soa du, int zc)
+// Byte offsets of consecutive planes of a ghosted field (uniform across the work-group):
+// wrap_coord of planes z, z + 1, ...; PER: every direction is periodic
+template <bool PER>
+struct PlaneWalk {
+    int raw, n;              // periodic: the wrapped plane
+    bool periodic;
+    size_t bytes, off;       // bytes per plane; offset of the current plane
+    __device__ PlaneWalk(int z, int n_, bool per, size_t bytes_) : n(n_), periodic(PER || per), bytes(bytes_)
+    {
+        const int at = wrap_coord(z, n, periodic);
+        raw = periodic ? at : z;
+        off = bytes * (size_t)(at + LAP);
+    }
+    __device__ int plane() const { return periodic ? raw : min(max(raw, 0), n - 1); }
+    __device__ void next()
+    {
+        ++raw;
+        if (PER || periodic) {
+            const bool turn = raw == n;
+            off = turn ? bytes * LAP : off + bytes;
+            raw = turn ? 0 : raw;
+        } else {
+            off = raw > 0 && raw < n ? off + bytes : off;
+        }
+    }
+};
+
+// row of VisWeights::row of cell c, and how many differences that row has
+__device__ __forceinline__ int closure_row(int c, int n, bool lo, bool hi)
+{
+    return lo && c <= 3 ? c : hi && c >= n - 4 ? n - 1 - c : 4;
+}
+
+template <int R>
+__device__ __forceinline__ int closure_reach(int row)
+{
+    return row == 0 ? 1 : row == 4 ? R : row;
+}
+
+template <int P>
+struct Phase {
+    static constexpr int value = P;
+};
+
+template <int ORDER, int MODE, int CLOSED, bool FAST>
+__global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, ws_field u, ws_field v, ws_field w,
+                                                   ws_field T, ws_metric_fields mf, ws_soa du, int zc)
 {
     // contraction stays on here (the fast family's arithmetic need not follow the reference's
     // order): every thread runs the same instructions for its flux point, so the flux at a
     // point past a periodic face still equals the one at its image bit for bit
     constexpr int R = ORDER / 2, Q = 2 * R + 1;
     using FZ = Fused<R>;
-    __shared__ double pl[4][FZ::PY][FZ::PX];      // u, v, w, T of the plane: flux points and border
-    __shared__ double fxa[4][FZ::TY][FX];          // x fluxes on the tile's rows
-    __shared__ double fya[4][FY][FZ::TX];          // y fluxes on the tile's columns
-    __shared__ double fzr[Q][4][FZ::TY * FZ::TX];  // z fluxes of the tile, ring of Q planes
-    __shared__ double rpl[R + 1][4][FZ::TY * FZ::TX];   // Ajac (dx F_x + dy F_y), ring of R + 1 planes
+    constexpr int PX = FZ::PX, PN = FZ::PN, XN = FZ::TY * FX, YN = FY * PX;
+    constexpr bool FLD = MODE == VM_FIELDS, BND = CLOSED != VC_NONE, BNDZ = CLOSED == VC_ALL;
+    __shared__ double pl[2][4][PN];      // u, v, w, T of a plane: flux points and border
+    __shared__ double fxa[2][4][XN];     // x fluxes on the tile's rows (rows of FX)
+    __shared__ double fya[2][4][YN];     // y fluxes on the tile's columns (rows of PX, as the plane copy)
     const int gx = (p.nx + FZ::TX - 1) / FZ::TX, gy = (p.ny + FZ::TY - 1) / FZ::TY, gz = (p.nz + zc - 1) / zc;
     const int ntiles = gx * gy * gz;
     const int per = (ntiles + 7) / 8;
@@ -532,7 +589,11 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, ws_field u, ws_f
     if (tile >= ntiles) return;
     const int x0 = (tile % gx) * FZ::TX, y0 = ((tile / gx) % gy) * FZ::TY;
     const int z0 = (tile / (gx * gy)) * zc, z1 = min(z0 + zc, p.nz);
-    const int tx = (int)threadIdx.x % FX, ty = (int)threadIdx.x / FX;
+    // the tile's rows go to the first wavefronts, the ring's to the last ones, which then have
+    // no flux derivatives to take
+    constexpr int TY = FZ::TY;
+    const int tx = (int)threadIdx.x % FX, ti = (int)threadIdx.x / FX;
+    const int ty = ti < TY ? ti + R : ti < TY + R ? ti - TY : ti;
     const bool perx = p.per[0] != 0, pery = p.per[1] != 0, perz = p.per[2] != 0;
     // this thread's flux point and (inside the tile) cell
     const int fx = x0 - R + tx, fy = y0 - R + ty;
@@ -540,215 +601,398 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, ws_field u, ws_f
     const bool cell = xrow && ycol && fx < p.nx && fy < p.ny;
     const int nyg = p.nyg;
     const ws_field fl[4] = {u, v, w, T};
-    auto at = [&](const ws_field &f, int x, int y, int z) {
-        return f.ptr[fidx(f.pitch, nyg, x + LAP, y + LAP, z + LAP)];
-    };
-    // the column of this flux point, and this thread's border point of the plane copy
+    // the column of this flux point, and this thread's border point of the plane copy (threads
+    // without one load their own point again)
     const int cxw = wrap_coord(fx, p.nx, perx), cyw = wrap_coord(fy, p.ny, pery);
-    int bpx = 0, bpy = 0, bxw = 0, byw = 0;
-    const bool bord = (int)threadIdx.x < FZ::NB;
+    const int bi = FNT - 1 - (int)threadIdx.x;     // the last threads first: ring wavefronts
+    const bool bord = bi < FZ::NB;
+    int bpx = 0, bpy = 0, bxw = cxw, byw = cyw;
     if (bord) {
-        FZ::border((int)threadIdx.x, bpx, bpy);
+        FZ::border(bi, bpx, bpy);
         bxw = wrap_coord(x0 - 2 * R + bpx, p.nx, perx);
         byw = wrap_coord(y0 - 2 * R + bpy, p.ny, pery);
     }
+    // FAST: byte offsets within a plane of the fields (they share u's pitch) and of du (threads
+    // without a cell point at its first)
+    uint32_t off = 8u * ((uint32_t)(cxw + LAP) + u.pitch * (uint32_t)(cyw + LAP));
+    uint32_t boff = 8u * ((uint32_t)(bxw + LAP) + u.pitch * (uint32_t)(byw + LAP));
+    uint32_t doff = cell ? 8u * ((uint32_t)fx + du.pitch * (uint32_t)fy) : 0u;
+    const size_t vstride = (size_t)du.pitch * p.ny * p.nz, dplane = 8 * (size_t)du.pitch * p.ny;
+    const size_t fplane = 8 * (size_t)u.pitch * nyg;          // FAST: bytes of a field's plane
+    // element of field f at this thread's point of the plane a walk stands on
+    auto at = [&](const ws_field &f, const PlaneWalk<!BNDZ> &z) -> double {
+        if constexpr (FAST) return *(const double *)((const char *)f.ptr + z.off + off);
+        else return f.ptr[fidx(f.pitch, nyg, cxw + LAP, cyw + LAP, z.plane() + LAP)];
+    };
+    auto at_border = [&](const ws_field &f, const PlaneWalk<!BNDZ> &z) -> double {
+        if constexpr (FAST) return *(const double *)((const char *)f.ptr + z.off + boff);
+        else return f.ptr[fidx(f.pitch, nyg, bxw + LAP, byw + LAP, z.plane() + LAP)];
+    };
+    double *const dm[4] = {du.ptr + vstride, du.ptr + 2 * vstride, du.ptr + 3 * vstride, du.ptr + 4 * vstride};
+    // du[m + 1] of this thread's cell at plane offset z (bytes)
+    auto du_at = [&](int m, size_t z) -> double & {
+        if constexpr (FAST) return *(double *)((char *)dm[m] + z + doff);
+        else return *(double *)((char *)dm[m] + z + 8 * (cell ? (size_t)fx + (size_t)du.pitch * fy : 0));
+    };
+    // where this thread reads the plane copy; past a closed face the face point (BND), with the
+    // weights and the reach (0 where the weight is) of the differences along x and y
+    int own = (ty + R) * PX + tx + R;
+    const int mine = own;
+    __shared__ double wxl[BND ? R : 1][FX], wyl[BND ? R : 1][FY];
+    int ox[BND ? R : 1], oy[BND ? R : 1];
+    const bool zlo = BNDZ && p.bnd[4], zhi = BNDZ && p.bnd[5];
+    if constexpr (BND) {
+        const int px = perx ? fx : cxw, py = pery ? fy : cyw;
+        own = (py - (y0 - 2 * R)) * PX + px - (x0 - 2 * R);
+        const int rx = closure_row(cxw, p.nx, p.bnd[0] != 0, p.bnd[1] != 0);
+        const int ry = closure_row(cyw, p.ny, p.bnd[2] != 0, p.bnd[3] != 0);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            if (ty == 0) wxl[q][tx] = wt.row[rx][q];
+            if (tx == 0) wyl[q][ty] = wt.row[ry][q];
+            ox[q] = q < closure_reach<R>(rx) ? q + 1 : 0;
+            oy[q] = (q < closure_reach<R>(ry) ? q + 1 : 0) * PX;
+        }
+    }
+    // derivatives along x and y (rows of PX) at element e of an LDS array
+    int wtx = tx, wty = ty;
+    auto ddx = [&](const double *e, const double *wgt, double scale) {
+        double t = 0.0;
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const double d = BND ? e[ox[q]] - e[-ox[q]] : e[q + 1] - e[-q - 1], a = BND ? wxl[q][wtx] : wgt[q];
+            t = q == 0 ? a * d : fma(a, d, t);
+        }
+        return BND ? t * scale : t;
+    };
+    auto ddy = [&](const double *e, const double *wgt, double scale) {
+        double t = 0.0;
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const double d = BND ? e[oy[q]] - e[-oy[q]] : e[(q + 1) * PX] - e[-(q + 1) * PX];
+            const double a = BND ? wyl[q][wty] : wgt[q];
+            t = q == 0 ? a * d : fma(a, d, t);
+        }
+        return BND ? t * scale : t;
+    };
     // flux planes zf0 .. zf1 - 1 produce the chunk's cells z0 .. z1 - 1
     const int zf0 = z0 - R, zf1 = z1 + R;
-    double c[4][Q];                 // the column's u, v, w, T at planes zf - R .. zf + R
+    // slot (P + R + k) % Q at the step of phase P: plane zf + k of the column (c), and the
+    // derivative sum of cell zf + k (acc)
+    double c[4][Q], acc[4][Q];
+    // loaded for the coming step: the newest column plane, the border of the plane after its
+    // flux plane, du of the cell it writes, and with metric fields that cell's Jacobian
+    double nq[4], hb[4], dn[4], jn = 0.0;
+    size_t dz = dplane * (size_t)z0;               // du plane of the cell the coming step writes
+    PlaneWalk<!BNDZ> wq(zf0 - R, p.nz, perz, fplane), wb(zf0, p.nz, perz, fplane), wm(zf0, p.nz, perz, fplane),
+        wj(z0, p.nz, perz, fplane);
 #pragma unroll
-    for (int f = 0; f < 4; ++f)
+    for (int q = 0; q < Q - 1; ++q, wq.next())
 #pragma unroll
-        for (int q = 0; q < Q - 1; ++q) c[f][q] = at(fl[f], cxw, cyw, wrap_coord(zf0 - R + q, p.nz, perz));
-    double nq[4], hb[4];            // next column slot, border point of the next plane
-    auto fetch = [&](int zf) {
-        const int zc_ = wrap_coord(zf + R, p.nz, perz), zb = wrap_coord(zf, p.nz, perz);
+        for (int f = 0; f < 4; ++f) c[f][q] = at(fl[f], wq);
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) acc[f][q] = 0.0;
+        pl[0][f][mine] = c[f][R];
+        hb[f] = at_border(fl[f], wb);
+        dn[f] = 0.0;
+    }
+    wb.next();
+    if (bord)
+#pragma unroll
+        for (int f = 0; f < 4; ++f) pl[0][f][bpy * PX + bpx] = hb[f];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        nq[f] = at(fl[f], wq);
+        hb[f] = at_border(fl[f], wb);
+    }
+    wq.next();
+    wb.next();
+    __syncthreads();
+    int zf = zf0, cur = 0;
+    // one step; false when the march is complete
+    auto step = [&](auto phase) __attribute__((always_inline)) -> bool {
+        constexpr int P = decltype(phase)::value;
+        auto slot = [](int k) constexpr { return (P + R + k + 2 * Q) % Q; };
+        const int nxt = cur ^ 1;
+        // keeps the plane offsets scalar: the loads take them as their scalar base
+        asm volatile("" : "+v"(off), "+v"(boff), "+v"(doff));
+        // the cell that the last step completed (its slot is the coming cell's)
+        if (cell && zf - R - 1 >= z0)
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                du_at(m, dz) = FLD ? fma(jn, acc[m][slot(-R - 1)], dn[m]) : dn[m] + acc[m][slot(-R - 1)];
+        if (zf == zf1) return false;
+        // the newest plane of the column, and the copy of the next plane
 #pragma unroll
         for (int f = 0; f < 4; ++f) {
-            nq[f] = at(fl[f], cxw, cyw, zc_);
-            hb[f] = bord ? at(fl[f], bxw, byw, zb) : 0.0;
+            c[f][slot(R)] = nq[f];
+            pl[nxt][f][mine] = c[f][slot(1)];
         }
-    };
-    const size_t vstride = (size_t)du.pitch * p.ny * p.nz;
-    auto du_at = [&](int z) { return du.ptr + (size_t)fx + (size_t)du.pitch * ((size_t)fy + (size_t)p.ny * (size_t)z); };
-    fetch(zf0);
-    // flux plane zf keeps its z fluxes in slot (zf - zf0) % Q of fzr and Ajac (dx F_x + dy F_y)
-    // in slot (zf - zf0) % (R + 1) of rpl
-    const int ci = (ty - R) * FZ::TX + (tx - R);   // this cell's index in the rings (tile threads)
-    const double aj = p.metric[9];
-    const double Akx = p.metric[0], Aky = p.metric[1], Akz = p.metric[2], Aix = p.metric[3], Aiy = p.metric[4];
-    const double Aiz = p.metric[5], Asx = p.metric[6], Asy = p.metric[7], Asz = p.metric[8];
-    // One barrier after the plane copy is written and one after the fluxes are: every read of
-    // the plane copy precedes the second, every read of the flux arrays the next first one.
-    for (int zf = zf0; zf < zf1; ++zf) {
+        if (bord)
+#pragma unroll
+            for (int f = 0; f < 4; ++f) pl[nxt][f][bpy * PX + bpx] = hb[f];
+        // the loads of the coming step
 #pragma unroll
         for (int f = 0; f < 4; ++f) {
-            c[f][Q - 1] = nq[f];
-            pl[f][ty + R][tx + R] = c[f][R];
-            if (bord) pl[f][bpy][bpx] = hb[f];
+            nq[f] = at(fl[f], wq);
+            hb[f] = at_border(fl[f], wb);
         }
-        // du of the cell this step completes (plane zf - R), used after the second barrier
-        const int zo = zf - R;
-        const bool out = cell && zo >= z0;
-        double duo[4];
+        wq.next();
+        wb.next();
+        __builtin_amdgcn_sched_barrier(0);
+        // Gradients and fluxes at this thread's flux point of plane zf; with a closed z face there
+        // are no fluxes past it.
+        const bool zin = !BNDZ || perz || (zf >= 0 && zf < p.nz);
+        if (BND) asm volatile("" : "+v"(wtx), "+v"(wty));    // the weights are read where they are used
+        const double *pc = &pl[cur][0][own];
+        double gk[4], gi[4], gs[4], met[FLD ? 10 : 1];
 #pragma unroll
-        for (int m = 0; m < 4; ++m) duo[m] = out ? du_at(zo)[(m + 1) * vstride] : 0.0;
-        if (zf + 1 < zf1) fetch(zf + 1);
-        __syncthreads();
-        // gradients and fluxes at this thread's flux point of plane zf
-        {
-            auto dx = [&](int f) {
-                double s[Q];
+        for (int f = 0; f < 4; ++f) {
+            if constexpr (FLD) {
+                // this plane's metric terms, used once the gradients are complete
+                if (f == 2) {
 #pragma unroll
-                for (int q = 0; q < Q; ++q) s[q] = pl[f][ty + R][tx + q];
-                return cd_at<ORDER, false, BND>(s, p, 0, fx);
-            };
-            auto dy = [&](int f) {
-                double s[Q];
-#pragma unroll
-                for (int q = 0; q < Q; ++q) s[q] = pl[f][ty + q][tx + R];
-                return cd_at<ORDER, false, BND>(s, p, 1, fy);
-            };
-            const double uk = dx(0), vk = dx(1), wk = dx(2), Tk = dx(3);
-            const double ui = dy(0), vi = dy(1), wi = dy(2), Ti = dy(3);
-            const double us = cd_at<ORDER, false, BND>(c[0], p, 2, zf), vs = cd_at<ORDER, false, BND>(c[1], p, 2, zf);
-            const double ws = cd_at<ORDER, false, BND>(c[2], p, 2, zf), Ts = cd_at<ORDER, false, BND>(c[3], p, 2, zf);
-            const double tc = c[3][R];
-            const double amu = p.amu_c0 * sqrt_nr(tc * tc * tc) * recip_nr(p.tsb + tc);
-            // physical derivatives from the computational ones (k, i, s)
-            auto gx = [&](double gk, double gi, double gs) { return DIAG ? gk * Akx : gk * Akx + gi * Aix + gs * Asx; };
-            auto gy = [&](double gk, double gi, double gs) { return DIAG ? gi * Aiy : gk * Aky + gi * Aiy + gs * Asy; };
-            auto gz = [&](double gk, double gi, double gs) { return DIAG ? gs * Asz : gk * Akz + gi * Aiz + gs * Asz; };
-            const double ux = gx(uk, ui, us), vx = gx(vk, vi, vs), wx = gx(wk, wi, ws);
-            const double uy = gy(uk, ui, us), vy = gy(vk, vi, vs), wy = gy(wk, wi, ws);
-            const double uz = gz(uk, ui, us), vz = gz(vk, vi, vs), wz = gz(wk, wi, ws);
-            const double div = ux + vy + wz;
-            const double s11 = (2.0 * ux - 2.0 / 3.0 * div) * amu;
-            const double s22 = (2.0 * vy - 2.0 / 3.0 * div) * amu;
-            const double s33 = (2.0 * wz - 2.0 / 3.0 * div) * amu;
-            const double s12 = (uy + vx) * amu, s13 = (uz + wx) * amu, s23 = (vz + wy) * amu;
-            const double amuk = amu * p.vis_c;
-            const double Tx = gx(Tk, Ti, Ts), Ty = gy(Tk, Ti, Ts), Tz = gz(Tk, Ti, Ts);
-            const double uc = c[0][R], vc = c[1][R], wc = c[2][R];
-            const double E1 = uc * s11 + vc * s12 + wc * s13 + amuk * Tx;
-            const double E2 = uc * s12 + vc * s22 + wc * s23 + amuk * Ty;
-            const double E3 = uc * s13 + vc * s23 + wc * s33 + amuk * Tz;
-            auto flux = [&](int d, double out[4]) {
-                if constexpr (DIAG) {
-                    // row d of the metrics keeps its diagonal term A[4d] only
-                    const double a = p.metric[4 * d] * aj;
-                    out[0] = a * (d == 0 ? s11 : d == 1 ? s12 : s13);
-                    out[1] = a * (d == 0 ? s12 : d == 1 ? s22 : s23);
-                    out[2] = a * (d == 0 ? s13 : d == 1 ? s23 : s33);
-                    out[3] = a * (d == 0 ? E1 : d == 1 ? E2 : E3);
-                } else {
-                    const double akx = p.metric[3 * d] * aj, aky = p.metric[3 * d + 1] * aj;
-                    const double akz = p.metric[3 * d + 2] * aj;
-                    out[0] = akx * s11 + aky * s12 + akz * s13;
-                    out[1] = akx * s12 + aky * s22 + akz * s23;
-                    out[2] = akx * s13 + aky * s23 + akz * s33;
-                    out[3] = akx * E1 + aky * E2 + akz * E3;
+                    for (int q = 0; q < 10; ++q) met[q] = at(q < 9 ? mf.A[q] : mf.ajac, wm);
+                    wm.next();
                 }
-            };
-            double F[4];
-            if (xrow) {
-                flux(0, F);
-#pragma unroll
-                for (int m = 0; m < 4; ++m) fxa[m][ty - R][tx] = F[m];
             }
-            if (ycol) {
-                flux(1, F);
+            gk[f] = ddx(pc + f * PN, wt.g[0], wt.gs[0]);
+            gi[f] = ddy(pc + f * PN, wt.g[1], wt.gs[1]);
+            if constexpr (!BNDZ) {
+                gs[f] = wt.g[2][0] * (c[f][slot(1)] - c[f][slot(-1)]);
 #pragma unroll
-                for (int m = 0; m < 4; ++m) fya[m][ty][tx - R] = F[m];
+                for (int q = 2; q <= R; ++q) gs[f] = fma(wt.g[2][q - 1], c[f][slot(q)] - c[f][slot(-q)], gs[f]);
             }
-            if (xrow && ycol) {
-                flux(2, F);
-                const int slot = (zf - zf0) % Q;
-#pragma unroll
-                for (int m = 0; m < 4; ++m) fzr[slot][m][ci] = F[m];
-            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __syncthreads();
-        if (xrow && ycol) {
-            // x and y derivatives of the plane's fluxes at this cell
-            const int ps = (zf - zf0) % (R + 1);
+        if constexpr (BNDZ) {
+            // selects and not branches: the arrays stay in registers without copies at joins
+            const int row = closure_row(min(max(zf, 0), p.nz - 1), p.nz, zlo, zhi), reach = closure_reach<R>(row);
 #pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                double s[Q];
+            for (int q = 1; q <= R; ++q)
 #pragma unroll
-                for (int q = 0; q < Q; ++q) s[q] = fxa[m][ty - R][tx - R + q];
-                const double ddx = cd_at<ORDER, false, BND>(s, p, 0, fx);
-#pragma unroll
-                for (int q = 0; q < Q; ++q) s[q] = fya[m][ty - R + q][tx - R];
-                const double ddy = cd_at<ORDER, false, BND>(s, p, 1, fy);
-                rpl[ps][m][ci] = aj * ddx + aj * ddy;
+                for (int f = 0; f < 4; ++f) {
+                    const double d = q <= reach ? c[f][slot(q)] - c[f][slot(-q)] : 0.0;
+                    gs[f] = q == 1 ? wt.rg[row][0] * d : fma(wt.rg[row][q - 1], d, gs[f]);
+                }
+        }
+        const double uc = c[0][slot(0)], vc = c[1][slot(0)], wc = c[2][slot(0)], tc = c[3][slot(0)];
+        const double amu = p.amu_c0 * sqrt_h(tc * tc * tc) * recip_nr(p.tsb + tc);
+        auto A = [&](int q) {
+            if constexpr (FLD) return met[q];
+            else return p.metric[q];
+        };
+        // physical derivatives from the computational ones (VM_DIAG: the weights carry A_dd)
+        auto px = [&](int f) { return MODE == VM_DIAG ? gk[f] : gk[f] * A(0) + gi[f] * A(3) + gs[f] * A(6); };
+        auto py = [&](int f) { return MODE == VM_DIAG ? gi[f] : gk[f] * A(1) + gi[f] * A(4) + gs[f] * A(7); };
+        auto pz = [&](int f) { return MODE == VM_DIAG ? gs[f] : gk[f] * A(2) + gi[f] * A(5) + gs[f] * A(8); };
+        const double ux = px(0), vx = px(1), wx_ = px(2), Tx = px(3);
+        const double uy = py(0), vy = py(1), wy_ = py(2), Ty = py(3);
+        const double uz = pz(0), vz = pz(1), wz = pz(2), Tz = pz(3);
+        const double div = ux + vy + wz;
+        const double s11 = (2.0 * ux - 2.0 / 3.0 * div) * amu;
+        const double s22 = (2.0 * vy - 2.0 / 3.0 * div) * amu;
+        const double s33 = (2.0 * wz - 2.0 / 3.0 * div) * amu;
+        const double s12 = (uy + vx) * amu, s13 = (uz + wx_) * amu, s23 = (vz + wy_) * amu;
+        const double amuk = amu * p.vis_c;
+        const double E1 = uc * s11 + vc * s12 + wc * s13 + amuk * Tx;
+        const double E2 = uc * s12 + vc * s22 + wc * s23 + amuk * Ty;
+        const double E3 = uc * s13 + vc * s23 + wc * s33 + amuk * Tz;
+        // flux of direction d (the weights of its derivative carry the constant factors)
+        auto flux = [&](int d, double out[4]) {
+            if constexpr (MODE == VM_DIAG) {
+                out[0] = d == 0 ? s11 : d == 1 ? s12 : s13;
+                out[1] = d == 0 ? s12 : d == 1 ? s22 : s23;
+                out[2] = d == 0 ? s13 : d == 1 ? s23 : s33;
+                out[3] = d == 0 ? E1 : d == 1 ? E2 : E3;
+            } else {
+                double a1 = A(3 * d), a2 = A(3 * d + 1), a3 = A(3 * d + 2);
+                if constexpr (FLD) { a1 *= met[9]; a2 *= met[9]; a3 *= met[9]; }
+                out[0] = a1 * s11 + a2 * s12 + a3 * s13;
+                out[1] = a1 * s12 + a2 * s22 + a3 * s23;
+                out[2] = a1 * s13 + a2 * s23 + a3 * s33;
+                out[3] = a1 * E1 + a2 * E2 + a3 * E3;
             }
-            // the cell of plane zf - R is complete: its z fluxes span planes zf - 2R .. zf (the
-            // ring slots the thread wrote itself, so no barrier is needed for them)
-            if (out) {
-                double *dp = du_at(zo);
-                const int s0 = (zf - zf0 + 1) % Q;      // slot of flux plane zf - 2R
-                const int po = (zf - zf0 + 1) % (R + 1);  // slot of plane zf - R
+        };
+        double F[4];
+        if (xrow) {
+            flux(0, F);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) fxa[cur][m][(ty - R) * FX + tx] = F[m];
+        }
+        if (ycol) {
+            flux(1, F);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) fya[cur][m][ty * PX + tx] = F[m];
+        }
+        flux(2, F);
+        if constexpr (BNDZ) {
+#pragma unroll
+            for (int q = 1; q <= R; ++q) {
+                const int zl = zf - q, zh = zf + q;
+                const int lo = closure_row(min(max(zl, 0), p.nz - 1), p.nz, zlo, zhi);
+                const int hi = closure_row(min(max(zh, 0), p.nz - 1), p.nz, zlo, zhi);
+                const bool ul = zin && (perz || zl >= 0) && q <= closure_reach<R>(lo);
+                const bool uh = zin && (perz || zh < p.nz) && q <= closure_reach<R>(hi);
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
-                    double sz[Q];
-#pragma unroll
-                    for (int q = 0; q < Q; ++q) {
-                        const int sl = s0 + q;
-                        sz[q] = fzr[sl >= Q ? sl - Q : sl][m][ci];
-                    }
-                    const double ddz = cd_at<ORDER, false, BND>(sz, p, 2, zo);
-                    dp[(m + 1) * vstride] = (duo[m] + rpl[po][m][ci]) + aj * ddz;
+                    const double Fl = ul ? F[m] : 0.0, Fh = uh ? F[m] : 0.0;
+                    acc[m][slot(-q)] = fma(wt.rf[lo][q - 1], Fl, acc[m][slot(-q)]);
+                    acc[m][slot(q)] = q == R ? -wt.rf[hi][q - 1] * Fh : fma(-wt.rf[hi][q - 1], Fh, acc[m][slot(q)]);
                 }
             }
+            // the face cells' one-sided differences take the face point's flux on both sides
+            const bool first = zlo && zf == 0, last = zhi && zf == p.nz - 1;
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                acc[m][slot(0)] = fma(wt.rf[0][0], last ? F[m] : first ? -F[m] : 0.0, acc[m][slot(0)]);
+        } else {
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int q = 1; q <= R; ++q) {
+                    acc[m][slot(-q)] = fma(wt.f[2][q - 1], F[m], acc[m][slot(-q)]);
+                    acc[m][slot(q)] = q == R ? -wt.f[2][q - 1] * F[m] : fma(-wt.f[2][q - 1], F[m], acc[m][slot(q)]);
+                }
+        }
+        // du of the cell the coming step writes: here rather than with the other loads, whose
+        // registers the gradients need
+        if (zf - R > z0) {
+            dz += dplane;
+            if constexpr (FLD) wj.next();
         }
 #pragma unroll
-        for (int f = 0; f < 4; ++f)
+        for (int m = 0; m < 4; ++m) dn[m] = du_at(m, dz);
+        if constexpr (FLD) jn = at(mf.ajac, wj);
+        __builtin_amdgcn_sched_barrier(0);
+        // x and y derivatives of the previous plane's fluxes
+        if (cell)
 #pragma unroll
-            for (int q = 0; q < Q - 1; ++q) c[f][q] = c[f][q + 1];
+            for (int m = 0; m < 4; ++m) {
+                acc[m][slot(-1)] += ddx(&fxa[nxt][m][(ty - R) * FX + tx], wt.f[0], wt.fs[0]) +
+                                    ddy(&fya[nxt][m][ty * PX + tx], wt.f[1], wt.fs[1]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        // the sums are formed here: used only where a cell is written, they would otherwise be
+        // sunk there, with every flux of the last 2R planes kept alive for them
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int q = -R; q <= R; ++q) asm volatile("" : "+v"(acc[m][slot(q)]));
+        ++zf;
+        __syncthreads();
+        cur = nxt;
+        return true;
+    };
+    auto turn = [&](auto... phase) __attribute__((always_inline)) { return (step(phase) && ...); };
+    if constexpr (Q == 7) {
+        while (turn(Phase<0>{}, Phase<1>{}, Phase<2>{}, Phase<3>{}, Phase<4>{}, Phase<5>{}, Phase<6>{})) {}
+    } else {
+        while (turn(Phase<0>{}, Phase<1>{}, Phase<2>{}, Phase<3>{}, Phase<4>{}, Phase<5>{}, Phase<6>{}, Phase<7>{},
+                    Phase<8>{})) {}
     }
 }
 
-inline unsigned fused_blocks(int nx, int ny, int nz, int order, int zc)
+// Planes per work-group of the fused form: its work-groups hold a compute unit each, so a
+// launch takes about (rounds of work-groups) x (planes each marches, the 2R of its halo
+// included) plane steps; the chunk count with the smallest product is taken.
+inline int fused_chunk(long columns, int nz, int R, int cus)
 {
-    const int R = order / 2;
-    const long ntiles = (long)((nx + FX - 2 * R - 1) / (FX - 2 * R)) * ((ny + FY - 2 * R - 1) / (FY - 2 * R)) *
-                        ((nz + zc - 1) / zc);
-    return (unsigned)(8 * ((ntiles + 7) / 8));
+    int best = nz;
+    long cost = 0;
+    for (int n = 1; n <= nz; ++n) {
+        const int zc = (nz + n - 1) / n;
+        const long groups = columns * ((nz + zc - 1) / zc);
+        const long t = (groups + cus - 1) / cus * (zc + 2 * R);
+        if (n == 1 || t < cost) { cost = t; best = zc; }
+    }
+    return best;
 }
 
-template <int ORDER, bool FIELDS, bool EXACT, bool BND>
+template <int ORDER, int MODE>
+void launch_fused(const VisParams &vp, ws_field u, ws_field v, ws_field w, ws_field T, const ws_metric_fields &mf,
+                  ws_soa du, int cus, hipStream_t s)
+{
+    constexpr int R = ORDER / 2;
+    using FZ = Fused<R>;
+    const double coef[2][4] = {{45.0 / 60.0, -9.0 / 60.0, 1.0 / 60.0, 0.0},
+                               {672.0 / 840.0, -168.0 / 840.0, 32.0 / 840.0, -3.0 / 840.0}};
+    const double rows[4][4] = {{1.0, 0.0, 0.0, 0.0}, {0.5, 0.0, 0.0, 0.0}, {8.0 / 12.0, -1.0 / 12.0, 0.0, 0.0},
+                               {45.0 / 60.0, -9.0 / 60.0, 1.0 / 60.0, 0.0}};
+    VisWeights wt{};
+    const double aj = vp.metric[9];
+    for (int d = 0; d < 3; ++d) {
+        const double A = MODE == VM_DIAG ? vp.metric[4 * d] : 1.0;
+        wt.gs[d] = A / vp.h[d];
+        wt.fs[d] = MODE == VM_FIELDS ? 1.0 / vp.h[d] : aj * (A * aj) / vp.h[d];
+        for (int q = 0; q < 4; ++q) {
+            wt.g[d][q] = coef[ORDER == 8][q] * wt.gs[d];
+            wt.f[d][q] = coef[ORDER == 8][q] * wt.fs[d];
+        }
+    }
+    for (int q = 0; q < 4; ++q) {
+        for (int r = 0; r < 4; ++r) wt.row[r][q] = rows[r][q];
+        wt.row[4][q] = coef[ORDER == 8][q];
+        for (int r = 0; r < 5; ++r) {
+            wt.rg[r][q] = wt.row[r][q] * wt.gs[2];
+            wt.rf[r][q] = wt.row[r][q] * wt.fs[2];
+        }
+    }
+    const bool bnd_xy = vp.bnd[0] || vp.bnd[1] || vp.bnd[2] || vp.bnd[3], bnd_z = vp.bnd[4] || vp.bnd[5];
+    // one offset for every field: shared pitch, planes of fewer than 2^32 bytes
+    bool fast = v.pitch == u.pitch && w.pitch == u.pitch && T.pitch == u.pitch &&
+                (uint64_t)u.pitch * (uint64_t)vp.nyg < (1ull << 29) && (uint64_t)du.pitch * (uint64_t)vp.ny < (1ull << 29);
+    if (MODE == VM_FIELDS) {
+        for (int q = 0; q < 9; ++q) fast = fast && mf.A[q].pitch == u.pitch;
+        fast = fast && mf.ajac.pitch == u.pitch;
+    }
+    const long columns = (long)((vp.nx + FZ::TX - 1) / FZ::TX) * ((vp.ny + FZ::TY - 1) / FZ::TY);
+    const int zc = fused_chunk(columns, vp.nz, R, cus);
+    const long ntiles = columns * ((vp.nz + zc - 1) / zc);
+    const dim3 g((unsigned)(8 * ((ntiles + 7) / 8)));
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, g, dim3(FNT), 0, s, vp, wt, u, v, w, T, mf, du, zc); };
+    // the closure form's table holds the central weights too: it also serves the rare layouts
+    if (!fast) go(k_vis_fused<ORDER, MODE, VC_ALL, false>);
+    else if (bnd_z) go(k_vis_fused<ORDER, MODE, VC_ALL, true>);
+    else if (bnd_xy) go(k_vis_fused<ORDER, MODE, VC_XY, true>);
+    else go(k_vis_fused<ORDER, MODE, VC_NONE, true>);
+}
+
+template <int ORDER, bool FIELDS, bool BND>
 void launch_order_b(const VisParams &vp, ws_field u, ws_field v, ws_field w, ws_field T, const ws_metric_fields &mf,
                     const EvFields &ev, ws_soa du, const Ctx &c, hipStream_t s, int &r)
 {
     const unsigned g = march_blocks(vp.nx, vp.ny, vp.nz);
-    hipLaunchKernelGGL((k_vis_flux<ORDER, FIELDS, EXACT, BND>), dim3(g), dim3(NT), 0, s, vp, u, v, w, T, mf, ev);
+    hipLaunchKernelGGL((k_vis_flux<ORDER, FIELDS, BND>), dim3(g), dim3(NT), 0, s, vp, u, v, w, T, mf, ev);
     // periodic directions only: the closure forms read no flux past a closed face
     ws_field fl[12];
     for (int q = 0; q < 12; ++q) fl[q] = ws_field{ev.f[q], ev.pitch, 0};
     if ((r = launch_ghost_fill(c, fl, 12, s))) return;
-    hipLaunchKernelGGL((k_vis_div<ORDER, FIELDS, EXACT, BND>), dim3(g), dim3(NT), 0, s, vp, ev, mf.ajac, du);
+    hipLaunchKernelGGL((k_vis_div<ORDER, FIELDS, BND>), dim3(g), dim3(NT), 0, s, vp, ev, mf.ajac, du);
 }
 
-template <int ORDER, bool FIELDS, bool EXACT>
+template <int ORDER, bool FIELDS>
 void launch_order(const VisParams &vp, ws_field u, ws_field v, ws_field w, ws_field T, const ws_metric_fields &mf,
                   const EvFields &ev, ws_soa du, const Ctx &c, hipStream_t s, int &r)
 {
     bool bnd = false;
     for (int q = 0; q < 6; ++q) bnd = bnd || vp.bnd[q];
-    if (bnd) launch_order_b<ORDER, FIELDS, EXACT, true>(vp, u, v, w, T, mf, ev, du, c, s, r);
-    else launch_order_b<ORDER, FIELDS, EXACT, false>(vp, u, v, w, T, mf, ev, du, c, s, r);
+    if (bnd) launch_order_b<ORDER, FIELDS, true>(vp, u, v, w, T, mf, ev, du, c, s, r);
+    else launch_order_b<ORDER, FIELDS, false>(vp, u, v, w, T, mf, ev, du, c, s, r);
 }
 
-template <int ORDER, bool EXACT>
+template <int ORDER>
 void launch_fields(const VisParams &vp, ws_field u, ws_field v, ws_field w, ws_field T, const ws_metric_fields *m,
                    const EvFields &ev, ws_soa du, const Ctx &c, hipStream_t s, int &r)
 {
     ws_metric_fields mf{};
     if (m) {
         mf = *m;
-        launch_order<ORDER, true, EXACT>(vp, u, v, w, T, mf, ev, du, c, s, r);
+        launch_order<ORDER, true>(vp, u, v, w, T, mf, ev, du, c, s, r);
     } else {
-        launch_order<ORDER, false, EXACT>(vp, u, v, w, T, mf, ev, du, c, s, r);
+        launch_order<ORDER, false>(vp, u, v, w, T, mf, ev, du, c, s, r);
     }
 }
 
@@ -762,11 +1006,6 @@ int launch_viscous(Ctx &c, ws_field u, ws_field v, ws_field w, ws_field T, const
     VisParams vp{};
     vp.nx = cfg.nx; vp.ny = cfg.ny; vp.nz = cfg.nz; vp.nyg = cfg.ny + 2 * LAP;
     vp.h[0] = cfg.hx; vp.h[1] = cfg.hy; vp.h[2] = cfg.hz;
-    const double den = cfg.viscous == 8 ? 840.0 : 60.0;
-    for (int d = 0; d < 3; ++d) {
-        vp.rch[d] = 1.0 / (den * vp.h[d]);
-        vp.rh[d] = 1.0 / vp.h[d];
-    }
     for (int q = 0; q < 6; ++q) vp.bnd[q] = cfg.d0_bound[q] ? 1 : 0;
     for (int q = 0; q < 3; ++q) vp.per[q] = cfg.periodic[q] ? 1 : 0;
     // constants as the reference's opencfd_para_init forms them (src/runtime/OCFD_init.cpp:379-396)
@@ -777,25 +1016,23 @@ int launch_viscous(Ctx &c, ws_field u, ws_field v, ws_field w, ws_field T, const
     for (int q = 0; q < 10; ++q) vp.metric[q] = cfg.metric[q];
     // the anchor kernel family keeps the reference's arithmetic bit for bit
     const bool exact = cfg.kernel == WS_KERNEL_ANCHOR;
-    bool bnd = false;
-    for (int q = 0; q < 6; ++q) bnd = bnd || vp.bnd[q];
-    if (!exact && !m) {
-        // the fast family with constant metrics: one fused kernel, no scratch
-        const int zc = c.vis_zchunk;
-        const unsigned g = fused_blocks(cfg.nx, cfg.ny, cfg.nz, cfg.viscous, zc);
+    if (!exact) {
+        // the fast family: one fused kernel, no scratch
         const double *A = cfg.metric;
         const bool diag = A[1] == 0.0 && A[2] == 0.0 && A[3] == 0.0 && A[5] == 0.0 && A[6] == 0.0 && A[7] == 0.0;
-        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(g), dim3(FNT), 0, s, vp, u, v, w, T, du, zc); };
-        const int sel = (cfg.viscous == 8 ? 4 : 0) + (bnd ? 2 : 0) + (diag ? 1 : 0);
-        switch (sel) {
-        case 0: go(k_vis_fused<6, false, false>); break;
-        case 1: go(k_vis_fused<6, false, true>); break;
-        case 2: go(k_vis_fused<6, true, false>); break;
-        case 3: go(k_vis_fused<6, true, true>); break;
-        case 4: go(k_vis_fused<8, false, false>); break;
-        case 5: go(k_vis_fused<8, false, true>); break;
-        case 6: go(k_vis_fused<8, true, false>); break;
-        default: go(k_vis_fused<8, true, true>); break;
+        const ws_metric_fields mf = m ? *m : ws_metric_fields{};
+        const int mode = m ? VM_FIELDS : diag ? VM_DIAG : VM_CONST;
+        auto go = [&](auto launch) { launch(vp, u, v, w, T, mf, du, c.compute_units, s); };
+        if (cfg.viscous == 8) {
+            // no VM_DIAG form: with the eighth order's longer windows its instance spills (the
+            // general one keeps fewer values across the flux stage and does not), which costs
+            // more than the general metric products (157x111x75: 190 us against 133)
+            if (mode == VM_FIELDS) go(launch_fused<8, VM_FIELDS>);
+            else go(launch_fused<8, VM_CONST>);
+        } else {
+            if (mode == VM_FIELDS) go(launch_fused<6, VM_FIELDS>);
+            else if (mode == VM_DIAG) go(launch_fused<6, VM_DIAG>);
+            else go(launch_fused<6, VM_CONST>);
         }
         hipError_t e = hipGetLastError();
         return e == hipSuccess ? WS_OK : hip_error(e, "fused viscous launch");
@@ -816,11 +1053,9 @@ int launch_viscous(Ctx &c, ws_field u, ws_field v, ws_field w, ws_field T, const
     ev.pitch = pitch;
     int r = WS_OK;
     if (cfg.viscous == 8) {
-        if (exact) launch_fields<8, true>(vp, u, v, w, T, m, ev, du, c, s, r);
-        else launch_fields<8, false>(vp, u, v, w, T, m, ev, du, c, s, r);
+        launch_fields<8>(vp, u, v, w, T, m, ev, du, c, s, r);
     } else {
-        if (exact) launch_fields<6, true>(vp, u, v, w, T, m, ev, du, c, s, r);
-        else launch_fields<6, false>(vp, u, v, w, T, m, ev, du, c, s, r);
+        launch_fields<6>(vp, u, v, w, T, m, ev, du, c, s, r);
     }
     if (r) return r;
     hipError_t e = hipGetLastError();

@@ -83,6 +83,7 @@ struct Ctx {
     ws_config cfg;
     KParams kp;
     int device;
+    int compute_units = 256;
     // CFL scratch: per-block maxima
     double *cfl_partial = nullptr;
     int cfl_blocks = 0;
@@ -104,11 +105,10 @@ struct Ctx {
     // also derive the primitives of stages 1 and 2 (2), and within ws_rk3_run those of
     // stage 3 too, alternating the primitive sets from step to step (3)
     int fuse_stage = 3;
-    // viscous terms of the two-kernel form (anchor family, metric fields): twelve ghosted
-    // flux fields, allocated at the first use; planes per work-group of the fused form
+    // viscous terms of the two-kernel form (anchor family): twelve ghosted flux fields,
+    // allocated at the first use
     double *vis_scratch = nullptr;
     size_t vis_scratch_elems = 0;
-    int vis_zchunk = 64;
     // second set of ghosted primitive fields (d, u, v, w, T, cc) that RK3 stages 1 and 2
     // write their primitives to, allocated at the first eager RK3 step that can use it
     double *prim_scratch = nullptr;
