@@ -413,3 +413,51 @@ def test_anchor_contexts_on_two_streams_run_concurrently(orc, ws):
     for _, st, ref, _ in runs:
         du = st.interior("du").cpu().numpy()
         assert np.array_equal(du, ref), f"rel L2 {rel_l2(du, ref)}"
+
+
+@pytest.mark.parametrize("precision", [W.WS_PREC_FP64, W.WS_PREC_MIXED])
+def test_planes_beyond_the_tiles_32_bit_offsets(ws, precision):
+    """Rows so long that a ghosted plane holds more elements than the tiles' 32-bit offsets
+    reach (13.1 million): the 64-bit kernels give the RHS of the short rows bit for bit, in
+    every tile shape and schedule asked for, alone, in two RK3 steps (no stage fusion there)
+    and as a block of a batch."""
+    import torch
+    nx, ny, nz = 9, 5, 6
+    prims = random_state(nx, ny, nz, 29, "blobs")
+    L = W.lib()
+    sh = W.stream_handle()
+    got = {}
+    for pad in (0, 1_100_000):
+        st = upload_state(prims, pad=pad)
+        assert (st.ws.d.pitch * (ny + 8) >= (1 << 29) // 41) == (pad > 0)
+        out = []
+        for tile, sched in ((W.WS_TILE_30x16_K2, W.WS_SCHED_GRID), (W.WS_TILE_126x2_K2, W.WS_SCHED_PREFETCH)):
+            ctx = make_ctx(nx, ny, nz, precision=precision)
+            ctx.set_tile_shape(tile)
+            ctx.set_schedule(sched)
+            out.append(gpu_du_comput(ctx, st))
+        ctx = make_ctx(nx, ny, nz, precision=precision)
+        W.check(L.ws_pri_to_cons(ctx.handle, st.ws.f, st.ws.d, st.ws.u, st.ws.v, st.ws.w, st.ws.T,
+                                 W.job((0, 0, 0), (nx, ny, nz)), sh))
+        b = W.Batch(W.default_config(8, 8, 8, precision=precision), [(nx, ny, nz)], [st])
+        W.check(L.ws_batch_set_schedule(b.handle, W.WS_SCHED_GRID))
+        W.check(L.ws_batch_du_comput(b.handle, sh))
+        torch.cuda.synchronize()
+        out.append(st.interior("du").cpu().numpy())
+        W.check(L.ws_batch_rk3_run(b.handle, 2, 0.5, 0, sh))
+        b.sync_states()
+        out.append(st.interior("f").cpu().numpy())
+        W.check(L.ws_rk3_run(ctx.handle, ctypes.byref(st.ws), 2, 0.5, 1, sh))
+        st.sync_from_ws()
+        out.append(st.interior("f").cpu().numpy())
+        got[pad] = out
+        b.close()
+        del b, st
+        torch.cuda.empty_cache()
+    short, long_ = got[0], got[1_100_000]
+    assert np.array_equal(long_[0], short[0])
+    tol = 1e-13 if precision == W.WS_PREC_FP64 else 1e-9
+    for a, b in zip(long_[1:], short[1:]):
+        err = rel_l2(a, b)
+        log(f"  long rows against short ones: {err:.3e}")
+        assert err <= tol

@@ -34,9 +34,9 @@ struct ws_batch {
     int stage_order = WS_ORDER_XYZ;
     // and its tile shape (-1: tile_shape)
     int stage_shape = -1;
-    // KParams::off32 for the RHS inputs of d_blocks (every block's own fields) and of
-    // d_blocks2 (the second primitive sets): every block's five fields pass prim_off32
-    int off32_own = 0, off32_second = 0;
+    // KParams::same_pitch for the RHS inputs of d_blocks (every block's own fields) and of
+    // d_blocks2 (the second primitive sets), and KParams::big over every block's fields
+    int same_own = 0, same_second = 0, big = 0;
     std::vector<ws_ctx *> ctx;
     std::vector<ws_state> st;
     BatchBlock *d_blocks = nullptr;
@@ -98,7 +98,7 @@ int stage_shape_of(const ws_batch *b) { return b->stage_shape >= 0 ? b->stage_sh
 BatchTiles tiles_of(const ws_batch *b, bool stage = false)
 {
     BatchTiles t;
-    t.shape = stage ? stage_shape_of(b) : b->tile_shape;
+    t.shape = b->big ? WS_TILE_30x16_K2 : stage ? stage_shape_of(b) : b->tile_shape;
     t.schedule = b->schedule;
     t.blocks = b->d_blocks;
     t.stage = nullptr;
@@ -121,7 +121,8 @@ int batch_rhs(ws_batch *b, hipStream_t s, const BatchStage *stage = nullptr, con
         return WS_OK;
     }
     KParams k = b->ctx[0]->kp;   // physics constants and metrics are the batch's
-    k.off32 = table && table == b->d_blocks2 ? b->off32_second : b->off32_own;
+    k.same_pitch = table && table == b->d_blocks2 ? b->same_second : b->same_own;
+    k.big = b->big;
     BatchTiles t = tiles_of(b, stage != nullptr);
     t.stage = stage;
     if (table) t.blocks = table;
@@ -138,11 +139,11 @@ bool prim_tables(ws_batch *b, hipStream_t s)
     if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return false;
     const size_t n = b->host_blocks.size();
     std::vector<BatchBlock> a = b->host_blocks, c = b->host_blocks;
-    int second32 = 1;
+    int same = 1;
     for (size_t i = 0; i < n; ++i) {
         ws_field sec[6];
         if (!prim_set(b->ctx[i], s, sec)) return false;
-        if (!prim_off32(b->ctx[i]->kp, sec[0], sec[1], sec[2], sec[3], sec[5])) second32 = 0;
+        if (!same_pitch(sec[0], sec[1], sec[2], sec[3], sec[5])) same = 0;
         const ws_state &st = b->st[i];
         a[i].od = sec[0]; a[i].ou = sec[1]; a[i].ov = sec[2]; a[i].ow = sec[3]; a[i].oT = sec[4]; a[i].occ = sec[5];
         c[i].d = sec[0]; c[i].u = sec[1]; c[i].v = sec[2]; c[i].w = sec[3]; c[i].cc = sec[5];
@@ -158,7 +159,7 @@ bool prim_tables(ws_batch *b, hipStream_t s)
     }
     b->host_blocks = a;
     b->d_blocks2 = d2;
-    b->off32_second = second32;
+    b->same_second = same;
     return true;
 }
 
@@ -273,10 +274,11 @@ int ws_batch_create(const ws_config *base, int32_t nblocks, const int32_t *exten
         h.rh[0] = 1.0 / cfg.hx; h.rh[1] = 1.0 / cfg.hy; h.rh[2] = 1.0 / cfg.hz;
         b->cells += (long long)cfg.nx * cfg.ny * cfg.nz;
     }
-    b->off32_own = 1;
+    b->same_own = 1;
     for (int i = 0; i < nblocks; ++i) {
         const ws_state &st = states[i];
-        if (!prim_off32(b->ctx[i]->kp, st.d, st.u, st.v, st.w, st.cc)) b->off32_own = 0;
+        if (!same_pitch(st.d, st.u, st.v, st.w, st.cc)) b->same_own = 0;
+        if (!rel_state(b->ctx[i]->kp, st)) b->big = 1;
     }
     hipError_t e = hipMalloc(&b->d_blocks, sizeof(BatchBlock) * nblocks);
     if (e != hipSuccess) return fail(b, set_error(WS_ERR_NOMEM, "batch block table"));
@@ -486,7 +488,7 @@ static int batch_step(ws_batch *b, const double *dt_dev, hipStream_t s, bool cfl
     // block's f and fn as created, and whether they are exchanged now is the same for all
     // blocks (they swap together).
     bool fuse = b->kernel == WS_KERNEL_TILED && !b->base.viscous && b->schedule == WS_SCHED_GRID &&
-                b->ctx[0]->fuse_stage;
+                !b->big && b->ctx[0]->fuse_stage;
     const int swapped = b->st[0].f.ptr == b->fb0 ? 1 : 0;
     for (size_t i = 0; i < b->st.size() && fuse; ++i)
         fuse = b->st[i].f.ptr == (swapped ? b->fbs[i] : b->fas[i]);
@@ -586,7 +588,7 @@ int ws_batch_rk3_step(ws_batch *b, const double *dt_dev, hipStream_t s)
 static bool batch_alternating(ws_batch *b, hipStream_t s, bool cfl)
 {
     if (b->kernel != WS_KERNEL_TILED || b->base.viscous || b->schedule != WS_SCHED_GRID ||
-        b->ctx[0]->fuse_stage < 3)
+        b->big || b->ctx[0]->fuse_stage < 3)
         return false;
     if (!prim_tables(b, s) || !aux_table(b, s) || !b->aux_second) return false;
     if (!cfl || b->d_cfl_tiles) return true;
@@ -794,7 +796,7 @@ int ws_batch_autotune(ws_batch *b, int32_t reps, float *times_ms, hipStream_t s)
             if (times_ms) times_ms[shape * WS_SCHED_COUNT + sched] = ms;
             if (ms < best_ms) { best_ms = ms; best_shape = shape; best_sched = sched; }
         }
-    if (!r && best_sched == WS_SCHED_GRID && !b->base.viscous && b->ctx[0]->fuse_stage) {
+    if (!r && best_sched == WS_SCHED_GRID && !b->base.viscous && !b->big && b->ctx[0]->fuse_stage) {
         b->tile_shape = best_shape;
         b->schedule = best_sched;
         // the stage candidates differ by 1-3 %: three times the repetitions

@@ -286,18 +286,18 @@ double *cfl_stage_buffer(ws_ctx *c)
     return c->cfl_stage;
 }
 
-bool fused_stage_ok(const ws_ctx *c)
+bool fused_stage_ok(const ws_ctx *c, const ws_state *st)
 {
     const bool closures = c->kp.bnd_any[0] || c->kp.bnd_any[1] || c->kp.bnd_any[2];
     return c->fuse_stage && c->cfg.kernel == WS_KERNEL_TILED && !c->cfg.viscous && c->schedule == WS_SCHED_GRID &&
-           !closures;
+           !closures && rel_state(c->kp, *st);
 }
 
-bool alternating_steps(ws_ctx *c, hipStream_t s, bool cfl)
+bool alternating_steps(ws_ctx *c, const ws_state *st, hipStream_t s, bool cfl)
 {
     const bool periodic = c->cfg.periodic[0] && c->cfg.periodic[1] && c->cfg.periodic[2];
     ws_field second[6];
-    if (c->fuse_stage < 3 || !fused_stage_ok(c) || !periodic || !prim_set(c, s, second)) return false;
+    if (c->fuse_stage < 3 || !fused_stage_ok(c, st) || !periodic || !prim_set(c, s, second)) return false;
     if (!cfl) return true;
     // room for either producer's count (tiles of the stage launch; stage-kernel work-groups)
     const long tiles = stage_launch_tiles(*c), blocks = stage_blocks(*c);
@@ -336,7 +336,7 @@ int rk3_step_fused(ws_ctx *c, ws_state *st, const double *dt_dev, hipStream_t s,
     std::swap(st->f, st->fn);
     const ws_soa nolap{};
     const bool periodic = c->cfg.periodic[0] && c->cfg.periodic[1] && c->cfg.periodic[2];
-    const bool fuse = fused_stage_ok(c);
+    const bool fuse = fused_stage_ok(c, st);
     ws_field second[6];
     const bool prims = fuse && periodic && c->fuse_stage > 1 && prim_set(c, s, second);
     const ws_field g[6] = {st->d, st->u, st->v, st->w, st->T, st->cc};
@@ -804,7 +804,7 @@ int ws_rk3_run(ws_ctx *c, ws_state *st, int32_t nsteps, double cfl, int32_t use_
     // stage fusion 3 the steps alternate the primitive sets (rk3_step_fused), the
     // stage-applying launch of each step but the last leaves the maxima per tile in
     // c->cfl_tiles, and the last step ends in the state's fields.
-    const bool alt = nsteps > 1 && alternating_steps(c, s, dt_dev != nullptr);
+    const bool alt = nsteps > 1 && alternating_steps(c, st, s, dt_dev != nullptr);
     double *cfl_next = !dt_dev ? nullptr : alt ? c->cfl_tiles : cfl_stage_buffer(c);
     const int cfl_n = alt ? (int)stage_launch_tiles(*c) : (int)c->cfl_stage_n;
     auto mode_of = [&](int n) {

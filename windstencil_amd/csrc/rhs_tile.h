@@ -103,35 +103,71 @@ __device__ __forceinline__ TileGeo tile_geo(const Box &box, int bx, int by, int 
     return g;
 }
 
-// The primitive values (rho, u, v, w, c) of this thread's phase-1 points.
-template <int DIR, int L, int W, int K>
-struct TileLoads {
-    double v[Tile<DIR, L, W, K>::ROUNDS][5];
-};
+// Addresses are a uniform base (the tile's first point or cell, a 64-bit scalar) plus a
+// lane's byte offset within the tile: 32 bits, formed with one 24-bit multiply-add and
+// taken as such by the memory instructions, so an access costs no vector address
+// arithmetic of its own and five fields of one pitch share one offset.  That holds while
+// the planes of every field a launch touches are below kTilePlane elements (rel_planes); BIG
+// kernels keep 64-bit lane offsets for larger ones.  Against 64-bit addresses per access: the
+// FP64 RHS of 256x160x96 392 -> 383 us, over metric fields 535 -> 507 us, of 600x256x128
+// 1850 -> 1822 us.  The mixed kernels, which wait on memory rather than on issue, load their
+// primitives by 64-bit offsets: 600x256x128 takes 1902 us so, 1963 us with 32-bit ones, whose
+// loads leave in denser bursts (1918 us with 64-bit addresses throughout).
+template <bool BIG> struct LaneOff { using type = uint32_t; };
+template <> struct LaneOff<true> { using type = size_t; };
 
-// point pt of the tile: line l, point p (x fastest in memory for every direction)
-template <int DIR, int L, int W, int K>
-__device__ __forceinline__ void tile_point_at(int pt, int &l, int &p)
+// byte offset of point p of line l from the tile's first point, in a field of `rows` rows per
+// plane
+template <int DIR, bool BIG>
+__device__ __forceinline__ typename LaneOff<BIG>::type lane_off(uint32_t pitch, int rows, int l, int p)
 {
-    using TL = Tile<DIR, L, W, K>;
-    if (DIR == 0) { p = pt % TL::NL; l = pt / TL::NL; }
-    else          { l = pt % W;      p = pt / W; }
+    const int a = DIR == 0 ? l : p, b = DIR == 0 ? p : l;      // steps of the line/plane stride, and of 1
+    if constexpr (BIG) {
+        const size_t stride = DIR == 2 ? (size_t)pitch * (size_t)rows : (size_t)pitch;
+        return 8 * ((size_t)a * stride + (size_t)b);
+    } else {
+        const uint32_t stride = DIR == 2 ? pitch * (uint32_t)rows : pitch;
+        return 8u * (__umul24((uint32_t)a, stride) + (uint32_t)b);
+    }
 }
 
-// point r of this thread
+template <typename Off>
+__device__ __forceinline__ double &elem(double *base, Off off)
+{
+    return *(double *)((char *)base + off);
+}
+
+// element index of point (x, y, z), which may lie before the first one (aligned tiles)
+__device__ __forceinline__ long origin(uint32_t pitch, int rows, int x, int y, int z)
+{
+    return (long)x + (long)pitch * ((long)y + (long)rows * (long)z);
+}
+
+// The primitive values (rho, u, v, w, c) of this thread's phase-1 points, with metric fields
+// also the direction's three metric terms.
+template <int DIR, int L, int W, int K, bool FIELDS>
+struct TileLoads {
+    double v[Tile<DIR, L, W, K>::ROUNDS][FIELDS ? 8 : 5];
+};
+
+// line l and point p (0 .. NL-1, or past it in the last round) of this thread's round r; x is
+// fastest in memory for every direction.  A y/z work-group holds whole rows of W lines, so
+// its threads keep their line and step T points per round.
 template <int DIR, int L, int W, int K>
 __device__ __forceinline__ void tile_point(int r, int &l, int &p)
 {
-    tile_point_at<DIR, L, W, K>((int)threadIdx.x + r * Tile<DIR, L, W, K>::NT, l, p);
+    using TL = Tile<DIR, L, W, K>;
+    const int t = threadIdx.x;
+    if (DIR == 0) { const int pt = t + r * TL::NT; p = pt % TL::NL; l = pt / TL::NL; }
+    else          { l = t % W; p = t / W + r * TL::T; }
 }
 
 template <int DIR, int L, int W, int K>
-__device__ __forceinline__ bool tile_point_ok(const TileGeo &g, int r, int l, int p)
+__device__ __forceinline__ bool tile_point_ok(const TileGeo &g, int l, int p)
 {
     using TL = Tile<DIR, L, W, K>;
     // a line needs points -LAP .. lim_line+LAP-1 of lines lo_across .. lim_across-1
-    return (int)threadIdx.x + r * TL::NT < TL::NPTS && l >= g.lo_across && l < g.lim_across &&
-           p < g.lim_line + 2 * LAP;
+    return (DIR == 0 ? l < W : p < TL::NL) && l >= g.lo_across && l < g.lim_across && p < g.lim_line + 2 * LAP;
 }
 
 template <int DIR>
@@ -142,21 +178,24 @@ __device__ __forceinline__ void tile_point_xyz(const TileGeo &g, int l, int p, i
     else               { x = g.x0 + l; y = g.y0; z = g.z0 - LAP + p; }
 }
 
-// Cell coordinates of phase-3 cell c (0 .. W*L-1 in the tile's cell order) for loads that
-// every lane issues: clamped to the tile's last cell and, across and along the line, to
-// its cells inside the box (the values of a clamped lane are never used).
+// line l and cell i of this thread's phase-3 cell of round r (i >= L or l >= W: none)
 template <int DIR, int L, int W, int K>
-__device__ __forceinline__ void tile_cell_clamped(const TileGeo &g, int c, int &cx, int &cy, int &cz)
+__device__ __forceinline__ void tile_cell(int r, int &l, int &i)
 {
-    c = min(c, W * L - 1);
-    int l, i;
-    if (DIR == 0) { i = c % L; l = c / L; }
-    else          { l = c % W; i = c / W; }
+    using TL = Tile<DIR, L, W, K>;
+    const int t = threadIdx.x;
+    if (DIR == 0) { const int c = t + r * TL::NT; i = c % L; l = c / L; }
+    else          { l = t % W; i = t / W + r * TL::T; }
+}
+
+// tile_cell for loads that every lane issues: clamped to the tile's cells inside the box
+// (the values of a clamped lane are never used)
+template <int DIR, int L, int W, int K>
+__device__ __forceinline__ void tile_cell_clamped(const TileGeo &g, int r, int &l, int &i)
+{
+    tile_cell<DIR, L, W, K>(r, l, i);
     l = min(max(l, g.lo_across), min(g.lim_across, W) - 1);
     i = min(i, min(g.lim_line, L) - 1);
-    if (DIR == 0)      { cx = g.x0 + i; cy = g.y0 + l; cz = g.z0; }
-    else if (DIR == 1) { cx = g.x0 + l; cy = g.y0 + i; cz = g.z0; }
-    else               { cx = g.x0 + l; cy = g.y0; cz = g.z0 + i; }
 }
 
 // Phase 1a: issue the loads of this thread's points (nothing waits on them here).  Every
@@ -165,47 +204,56 @@ __device__ __forceinline__ void tile_cell_clamped(const TileGeo &g, int c, int &
 // used).  With no lane-dependent branch around them the number of loads in flight is the
 // same on every path, so the split of round r waits for its own loads only while the
 // later rounds' (and an accumulating launch's du) loads are still in flight.
-template <int DIR, int L, int W, int K>
+template <int DIR, int L, int W, int K, bool BIG = false, bool FIELDS = false>
 __device__ __forceinline__ void tile_load(int nyg, const ws_field &d, const ws_field &u, const ws_field &v,
-                                          const ws_field &w, const ws_field &cc, const TileGeo &g,
-                                          TileLoads<DIR, L, W, K> &ld, int off32)
+                                          const ws_field &w, const ws_field &cc, const ws_metric_fields *mf,
+                                          const TileGeo &g, TileLoads<DIR, L, W, K, FIELDS> &ld, int same_pitch)
 {
     using TL = Tile<DIR, L, W, K>;
     const int lhi = min(g.lim_across, W) - 1, phi = min(g.lim_line + 2 * LAP, TL::NL) - 1;
-    if (off32) {
-        // one 32-bit offset for the five fields (KParams::off32: a uniform branch)
-#pragma unroll
-        for (int r = 0; r < TL::ROUNDS; ++r) {
-            int l, p, x, y, z;
-            tile_point_at<DIR, L, W, K>(min((int)threadIdx.x + r * TL::NT, TL::NPTS - 1), l, p);
-            l = min(max(l, g.lo_across), lhi);
-            p = min(p, phi);
-            tile_point_xyz<DIR>(g, l, p, x, y, z);
-            const unsigned o = (unsigned)x + __umul24(d.pitch, (unsigned)y + __umul24((unsigned)nyg, (unsigned)z));
-            ld.v[r][0] = d.ptr[o];
-            ld.v[r][1] = u.ptr[o];
-            ld.v[r][2] = v.ptr[o];
-            ld.v[r][3] = w.ptr[o];
-            ld.v[r][4] = cc.ptr[o];
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        return;
-    }
-#pragma unroll
-    for (int r = 0; r < TL::ROUNDS; ++r) {
-        int l, p, x, y, z;
-        tile_point_at<DIR, L, W, K>(min((int)threadIdx.x + r * TL::NT, TL::NPTS - 1), l, p);
+    int x0, y0, z0;
+    tile_point_xyz<DIR>(g, 0, 0, x0, y0, z0);
+    const ws_field in[5] = {d, u, v, w, cc};
+    auto base = [&](const ws_field &f) { return f.ptr + origin(f.pitch, nyg, x0, y0, z0); };
+    auto point = [&](int r, int &l, int &p) {
+        tile_point<DIR, L, W, K>(r, l, p);
         l = min(max(l, g.lo_across), lhi);
         p = min(p, phi);
-        tile_point_xyz<DIR>(g, l, p, x, y, z);
-        ld.v[r][0] = d.ptr[fidx(d.pitch, nyg, x, y, z)];
-        ld.v[r][1] = u.ptr[fidx(u.pitch, nyg, x, y, z)];
-        ld.v[r][2] = v.ptr[fidx(v.pitch, nyg, x, y, z)];
-        ld.v[r][3] = w.ptr[fidx(w.pitch, nyg, x, y, z)];
-        ld.v[r][4] = cc.ptr[fidx(cc.pitch, nyg, x, y, z)];
-        // rounds go out in order (the scheduler would otherwise issue them in any order,
-        // and the wait for round 0 would then cover whatever went out before it)
-        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (same_pitch) {
+        // one offset for the five fields (KParams::same_pitch: a uniform branch)
+#pragma unroll
+        for (int r = 0; r < TL::ROUNDS; ++r) {
+            int l, p;
+            point(r, l, p);
+            const auto o = lane_off<DIR, BIG>(d.pitch, nyg, l, p);
+#pragma unroll
+            for (int q = 0; q < 5; ++q) ld.v[r][q] = elem(base(in[q]), o);
+            // rounds go out in order (the scheduler would otherwise issue them in any order,
+            // and the wait for round 0 would then cover whatever went out before it)
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < TL::ROUNDS; ++r) {
+            int l, p;
+            point(r, l, p);
+#pragma unroll
+            for (int q = 0; q < 5; ++q) ld.v[r][q] = elem(base(in[q]), lane_off<DIR, BIG>(in[q].pitch, nyg, l, p));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    if constexpr (FIELDS) {
+#pragma unroll
+        for (int r = 0; r < TL::ROUNDS; ++r) {
+            int l, p;
+            point(r, l, p);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const ws_field &f = mf->A[3 * DIR + q];
+                ld.v[r][5 + q] = elem(base(f), lane_off<DIR, BIG>(f.pitch, nyg, l, p));
+            }
+        }
     }
 }
 
@@ -217,9 +265,9 @@ __device__ __forceinline__ void tile_load(int nyg, const ws_field &d, const ws_f
 // cells: f = stage(fn, f, du + this direction's terms), du itself is not written.
 // Returns, when the launch applies a stage with sa.cfl_part set, the maximum CFL speed of
 // this thread's cells (0 otherwise).
-template <int DIR, int L, int W, int K, bool FIELDS, bool ACC, bool MIX, bool BND, bool STG, typename Next>
+template <int DIR, int L, int W, int K, bool FIELDS, bool ACC, bool MIX, bool BND, bool STG, bool BIG, typename Next>
 __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric_fields &mf, const ws_soa &du,
-                                               const TileGeo &g, TileLoads<DIR, L, W, K> &ld, double *sp,
+                                               const TileGeo &g, TileLoads<DIR, L, W, K, FIELDS> &ld, double *sp,
                                                const StageArgs &sa, Next next)
 {
     static_assert(!(STG && (BND || !ACC)), "the stage is applied by an accumulating launch without closures");
@@ -234,18 +282,20 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
     // wait the compiler places before the reconstruction exposes their whole latency)
     constexpr int CPT = (W * L + TL::NT - 1) / TL::NT;    // cells per thread (upper bound)
     const size_t vstride = (size_t)du.pitch * k.ny * k.nz;
+    // the tile's first cell in an interior state
+    auto cell0 = [&](const ws_soa &f) { return f.ptr + origin(f.pitch, k.ny, g.x0 - LAP, g.y0 - LAP, g.z0 - LAP); };
+    double *const dbase = cell0(du);
     double duo[ACC ? CPT : 1][5];
     if (ACC) {
         // issued by every lane, like the primitive loads, so that the split does not wait
         // for them
 #pragma unroll
         for (int r = 0; r < CPT; ++r) {
-            int cx, cy, cz;
-            tile_cell_clamped<DIR, L, W, K>(g, t + r * TL::NT, cx, cy, cz);
-            const double *dp = du.ptr + (size_t)(cx - LAP) +
-                               (size_t)du.pitch * ((size_t)(cy - LAP) + (size_t)k.ny * (size_t)(cz - LAP));
+            int l, i;
+            tile_cell_clamped<DIR, L, W, K>(g, r, l, i);
+            const auto o = lane_off<DIR, BIG>(du.pitch, k.ny, l, i);
 #pragma unroll
-            for (int m = 0; m < 5; ++m) duo[r][m] = dp[m * vstride];
+            for (int m = 0; m < 5; ++m) duo[r][m] = elem(dbase + m * vstride, o);
         }
     }
 
@@ -254,17 +304,11 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
     for (int r = 0; r < TL::ROUNDS; ++r) {
         int l, p;
         tile_point<DIR, L, W, K>(r, l, p);
-        if (!tile_point_ok<DIR, L, W, K>(g, r, l, p)) continue;
+        if (!tile_point_ok<DIR, L, W, K>(g, l, p)) continue;
         const double dd = ld.v[r][0], uu = ld.v[r][1], vv = ld.v[r][2], ww = ld.v[r][3], c = ld.v[r][4];
         double fp[5], fm[5];
         if (FIELDS) {
-            int x, y, z;
-            tile_point_xyz<DIR>(g, l, p, x, y, z);
-            const int nyg = k.nyg;
-            const ws_field &f1 = mf.A[3 * DIR + 0], &f2 = mf.A[3 * DIR + 1], &f3 = mf.A[3 * DIR + 2];
-            const double A1 = f1.ptr[fidx(f1.pitch, nyg, x, y, z)];
-            const double A2 = f2.ptr[fidx(f2.pitch, nyg, x, y, z)];
-            const double A3 = f3.ptr[fidx(f3.pitch, nyg, x, y, z)];
+            const double A1 = ld.v[r][FIELDS ? 5 : 0], A2 = ld.v[r][FIELDS ? 6 : 0], A3 = ld.v[r][FIELDS ? 7 : 0];
             if (MIX) {
                 const double sn = sqrt(fma(A3, A3, fma(A2, A2, A1 * A1)));
                 const double rs = 1.0 / sn;
@@ -400,18 +444,18 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
     double fnv[STG ? CPT : 1][5], fvv[STG ? CPT : 1][5];
     if (STG) {
         const size_t nstride = (size_t)sa.fn.pitch * k.ny * k.nz, fstride = (size_t)sa.f.pitch * k.ny * k.nz;
+        double *const nbase = cell0(sa.fn), *const fbase = cell0(sa.f);
 #pragma unroll
         for (int r = 0; r < CPT; ++r) {
-            int cx, cy, cz;
-            tile_cell_clamped<DIR, L, W, K>(g, t + r * TL::NT, cx, cy, cz);   // every lane loads
-            const size_t cell = (size_t)(cy - LAP) + (size_t)k.ny * (size_t)(cz - LAP);
-            const double *np = sa.fn.ptr + (size_t)(cx - LAP) + (size_t)sa.fn.pitch * cell;
-            const double *fp = sa.f.ptr + (size_t)(cx - LAP) + (size_t)sa.f.pitch * cell;
+            int l, i;
+            tile_cell_clamped<DIR, L, W, K>(g, r, l, i);   // every lane loads
+            const auto no = lane_off<DIR, BIG>(sa.fn.pitch, k.ny, l, i);
+            const auto fo = lane_off<DIR, BIG>(sa.f.pitch, k.ny, l, i);
 #pragma unroll
-            for (int m = 0; m < 5; ++m) fnv[r][m] = np[m * nstride];
+            for (int m = 0; m < 5; ++m) fnv[r][m] = elem(nbase + m * nstride, no);
             if (sa.krk != 1)
 #pragma unroll
-                for (int m = 0; m < 5; ++m) fvv[r][m] = fp[m * fstride];
+                for (int m = 0; m < 5; ++m) fvv[r][m] = elem(fbase + m * fstride, fo);
         }
     }
     // face fluxes reuse the split buffer (its first 5*W*F entries; the M split values, from
@@ -436,20 +480,21 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
     double cfl_max = 0.0;
 #pragma unroll
     for (int r = 0; r < CPT; ++r) {
-        const int c = t + r * TL::NT;
-        if (c >= W * L) break;
         int l, i;
-        if (DIR == 0) { i = c % L; l = c / L; }
-        else          { l = c % W; i = c / W; }
+        tile_cell<DIR, L, W, K>(r, l, i);
+        if (DIR == 0 ? l >= W : i >= L) break;
         if (l < g.lo_across || l >= g.lim_across || i >= g.lim_line) continue;
         int cx, cy, cz;
         if (DIR == 0)      { cx = g.x0 + i; cy = g.y0 + l; cz = g.z0; }
         else if (DIR == 1) { cx = g.x0 + l; cy = g.y0 + i; cz = g.z0; }
         else               { cx = g.x0 + l; cy = g.y0; cz = g.z0 + i; }
-        const double aj = FIELDS ? mf.ajac.ptr[fidx(mf.ajac.pitch, k.nyg, cx, cy, cz)] : k.ajac;
+        // a ghosted field at this cell
+        auto ghosted = [&](const ws_field &f) -> double & {
+            return elem(f.ptr + origin(f.pitch, k.nyg, g.x0, g.y0, g.z0), lane_off<DIR, BIG>(f.pitch, k.nyg, l, i));
+        };
+        const double aj = FIELDS ? ghosted(mf.ajac) : k.ajac;
         const double scale = aj * scale0;
-        double *dp = du.ptr + (size_t)(cx - LAP) +
-                     (size_t)du.pitch * ((size_t)(cy - LAP) + (size_t)k.ny * (size_t)(cz - LAP));
+        const auto dofs = lane_off<DIR, BIG>(du.pitch, k.ny, l, i);
         const int fl = TL::fidx(l, i), fr = TL::fidx(l, i + 1);
         // non-reflecting flags: the first cell takes only the M pass, the last only the P pass
         const bool first_only_m = BND && nr_lo && gl0 + i == 0;
@@ -470,9 +515,9 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
             if (STG) {
                 rv[m] = acc_sum(duo[r][m], val);   // the complete RHS, staged below
             } else if (ACC) {
-                dp[m * vstride] = acc_sum(duo[r][m], val);
+                elem(dbase + m * vstride, dofs) = acc_sum(duo[r][m], val);
             } else {
-                dp[m * vstride] = val;
+                elem(dbase + m * vstride, dofs) = val;
             }
         }
         if (STG) {
@@ -489,15 +534,15 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
             // the new f's primitives for the next stage's RHS (and OCFD_bc on the planes)
             if (sa.pd.ptr) {
                 const CellPrims p = cell_primitives(rv, k.cv);
-                sa.pd.ptr[fidx(sa.pd.pitch, k.nyg, cx, cy, cz)] = p.d;
-                sa.pu.ptr[fidx(sa.pu.pitch, k.nyg, cx, cy, cz)] = p.u;
-                sa.pv.ptr[fidx(sa.pv.pitch, k.nyg, cx, cy, cz)] = p.v;
-                sa.pw.ptr[fidx(sa.pw.pitch, k.nyg, cx, cy, cz)] = p.w;
-                sa.pT.ptr[fidx(sa.pT.pitch, k.nyg, cx, cy, cz)] = p.T;
+                ghosted(sa.pd) = p.d;
+                ghosted(sa.pu) = p.u;
+                ghosted(sa.pv) = p.v;
+                ghosted(sa.pw) = p.w;
+                ghosted(sa.pT) = p.T;
                 // the stage kernel's expressions for the sound speed, pressure and CFL speed
                 const double c = sqrt(p.T) / k.ama;
-                if (sa.pcc.ptr) sa.pcc.ptr[fidx(sa.pcc.pitch, k.nyg, cx, cy, cz)] = c;
-                if (sa.pP.ptr) sa.pP.ptr[fidx(sa.pP.pitch, k.nyg, cx, cy, cz)] = p.e / p.d * (k.gamma - 1.0);
+                if (sa.pcc.ptr) ghosted(sa.pcc) = c;
+                if (sa.pP.ptr) ghosted(sa.pP) = p.e / p.d * (k.gamma - 1.0);
                 if (sa.cfl_part) cfl_max = fmax(cfl_max, fmax(fabs(p.u) + c, fmax(fabs(p.v) + c, fabs(p.w) + c)));
                 const int ix = cx - LAP, iy = cy - LAP, iz = cz - LAP;
                 if (sa.halo) {
@@ -523,11 +568,11 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
                 if (sa.planes && (ix == 0 || ix == k.nx - 1 || iy == 0 || iy == k.ny - 1 || iz == 0 || iz == k.nz - 1))
                     plane_conserved(p, k.cv, rv);
             }
-            const size_t fo = (size_t)(cx - LAP) +
-                              (size_t)sa.f.pitch * ((size_t)(cy - LAP) + (size_t)k.ny * (size_t)(cz - LAP));
+            const auto fo = lane_off<DIR, BIG>(sa.f.pitch, k.ny, l, i);
             const size_t fstride = (size_t)sa.f.pitch * k.ny * k.nz;
+            double *const fbase = cell0(sa.f);
 #pragma unroll
-            for (int m = 0; m < 5; ++m) sa.f.ptr[fo + m * fstride] = rv[m];
+            for (int m = 0; m < 5; ++m) elem(fbase + m * fstride, fo) = rv[m];
         }
     }
     return cfl_max;
@@ -558,7 +603,7 @@ __device__ __forceinline__ void tile_wg_max(double v, double *red, double *out)
 // dispatch of work-groups to the eight XCDs each XCD gets a contiguous range of tiles, so
 // neighbouring tiles, which share halo lines and the cache lines of their edge columns,
 // meet in the same L2.
-template <int DIR, int L, int W, int K, bool FIELDS, bool ACC, bool MIX, bool BND, bool STG = false>
+template <int DIR, int L, int W, int K, bool FIELDS, bool ACC, bool MIX, bool BND, bool STG = false, bool BIG = false>
 __global__ void __launch_bounds__(320)
 k_rhs_tile(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc, ws_metric_fields mf,
            ws_soa du, Box box, int gx, int gy, int ntiles, StageArgs sa)
@@ -570,9 +615,9 @@ k_rhs_tile(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field c
     if (tile >= ntiles) return;
     const int r = tile / gx;
     const TileGeo g = tile_geo<DIR, L, W, K>(box, tile - r * gx, r % gy, r / gy);
-    TileLoads<DIR, L, W, K> ld;
-    tile_load<DIR, L, W, K>(k.nyg, d, u, v, w, cc, g, ld, k.off32);
-    const double cmax = tile_compute<DIR, L, W, K, FIELDS, ACC, MIX, BND, STG>(k, mf, du, g, ld, sp, sa, [] {});
+    TileLoads<DIR, L, W, K, FIELDS> ld;
+    tile_load<DIR, L, W, K, BIG || MIX, FIELDS>(k.nyg, d, u, v, w, cc, &mf, g, ld, k.same_pitch);
+    const double cmax = tile_compute<DIR, L, W, K, FIELDS, ACC, MIX, BND, STG, BIG>(k, mf, du, g, ld, sp, sa, [] {});
     if (STG && sa.cfl_part) {
         __syncthreads();   // phase 3 has read its faces from sp
         tile_wg_max<TL::NT>(cmax, sp, sa.cfl_part + tile);
@@ -598,17 +643,17 @@ k_rhs_persist(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_fiel
         const int r = i / gx;
         return tile_geo<DIR, L, W, K>(box, i - r * gx, r % gy, r / gy);
     };
-    TileLoads<DIR, L, W, K> ld;
+    TileLoads<DIR, L, W, K, false> ld;
     TileGeo g = geo(first);
-    if (PREFETCH) tile_load<DIR, L, W, K>(k.nyg, d, u, v, w, cc, g, ld, k.off32);
+    if (PREFETCH) tile_load<DIR, L, W, K, MIX>(k.nyg, d, u, v, w, cc, nullptr, g, ld, k.same_pitch);
     for (int i = first; i < last; ++i) {
-        if (!PREFETCH) tile_load<DIR, L, W, K>(k.nyg, d, u, v, w, cc, g, ld, k.off32);
+        if (!PREFETCH) tile_load<DIR, L, W, K, MIX>(k.nyg, d, u, v, w, cc, nullptr, g, ld, k.same_pitch);
         const bool more = i + 1 < last;
         const TileGeo gn = more ? geo(i + 1) : g;
         auto next = [&] {
-            if (PREFETCH && more) tile_load<DIR, L, W, K>(k.nyg, d, u, v, w, cc, gn, ld, k.off32);
+            if (PREFETCH && more) tile_load<DIR, L, W, K, MIX>(k.nyg, d, u, v, w, cc, nullptr, gn, ld, k.same_pitch);
         };
-        tile_compute<DIR, L, W, K, false, ACC, MIX, false, false>(k, nomf, du, g, ld, sp, StageArgs{}, next);
+        tile_compute<DIR, L, W, K, false, ACC, MIX, false, false, false>(k, nomf, du, g, ld, sp, StageArgs{}, next);
         __syncthreads();   // the next tile reuses the LDS buffer
         g = gn;
     }
@@ -642,12 +687,12 @@ k_rhs_batch(KParams k, const BatchBlock *blocks, const int4 *tiles, int ntiles, 
         return make_int4(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y),
                          __builtin_amdgcn_readfirstlane(v.z), __builtin_amdgcn_readfirstlane(v.w));
     };
-    TileLoads<DIR, L, W, K> ld;
+    TileLoads<DIR, L, W, K, false> ld;
     int4 tl = tile_at(first);
     TileGeo g = tile_geo<DIR, L, W, K>(box_of(blocks[tl.x]), tl.y, tl.z, tl.w);
     if (PREFETCH) {
         const BatchBlock &b = blocks[tl.x];
-        tile_load<DIR, L, W, K>(b.n[1] + 2 * LAP, b.d, b.u, b.v, b.w, b.cc, g, ld, k.off32);
+        tile_load<DIR, L, W, K, MIX>(b.n[1] + 2 * LAP, b.d, b.u, b.v, b.w, b.cc, nullptr, g, ld, k.same_pitch);
     }
     for (int i = first; i < last; ++i) {
         const BatchBlock &b = blocks[tl.x];
@@ -655,7 +700,7 @@ k_rhs_batch(KParams k, const BatchBlock *blocks, const int4 *tiles, int ntiles, 
         kb.nx = b.n[0]; kb.ny = b.n[1]; kb.nz = b.n[2];
         kb.nyg = b.n[1] + 2 * LAP; kb.nzg = b.n[2] + 2 * LAP;
         kb.rh[DIR] = b.rh[DIR];
-        if (!PREFETCH) tile_load<DIR, L, W, K>(kb.nyg, b.d, b.u, b.v, b.w, b.cc, g, ld, k.off32);
+        if (!PREFETCH) tile_load<DIR, L, W, K, MIX>(kb.nyg, b.d, b.u, b.v, b.w, b.cc, nullptr, g, ld, k.same_pitch);
         const bool more = i + 1 < last;
         const int4 tn = more ? tile_at(i + 1) : tl;
         const TileGeo gn = tile_geo<DIR, L, W, K>(box_of(blocks[tn.x]), tn.y, tn.z, tn.w);
@@ -664,10 +709,11 @@ k_rhs_batch(KParams k, const BatchBlock *blocks, const int4 *tiles, int ntiles, 
         auto next = [&] {
             if (PREFETCH && more) {
                 const BatchBlock &bn = blocks[tn.x];
-                tile_load<DIR, L, W, K>(bn.n[1] + 2 * LAP, bn.d, bn.u, bn.v, bn.w, bn.cc, gn, ld, k.off32);
+                tile_load<DIR, L, W, K, MIX>(bn.n[1] + 2 * LAP, bn.d, bn.u, bn.v, bn.w, bn.cc, nullptr, gn, ld,
+                                        k.same_pitch);
             }
         };
-        tile_compute<DIR, L, W, K, false, ACC, MIX, false, false>(kb, nomf, b.du, g, ld, sp, StageArgs{}, next);
+        tile_compute<DIR, L, W, K, false, ACC, MIX, false, false, false>(kb, nomf, b.du, g, ld, sp, StageArgs{}, next);
         __syncthreads();   // the next tile reuses the LDS buffer
         tl = tn;
         g = gn;
@@ -676,7 +722,7 @@ k_rhs_batch(KParams k, const BatchBlock *blocks, const int4 *tiles, int ntiles, 
 
 // Batched form with one tile per work-group (grid = tile count): no loop-carried
 // state, so it needs no more registers than the single-box kernel.
-template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool STG = false>
+template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool STG = false, bool BIG = false>
 __global__ void __launch_bounds__(320)
 k_rhs_batch_grid(KParams k, const BatchBlock *blocks, const int4 *tiles, int ntiles, BatchStage bs)
 {
@@ -696,8 +742,8 @@ k_rhs_batch_grid(KParams k, const BatchBlock *blocks, const int4 *tiles, int nti
     box.s[0] = box.s[1] = box.s[2] = LAP;
     box.e[0] = b.n[0] + LAP; box.e[1] = b.n[1] + LAP; box.e[2] = b.n[2] + LAP;
     const TileGeo g = tile_geo<DIR, L, W, K>(box, tl.y, tl.z, tl.w);
-    TileLoads<DIR, L, W, K> ld;
-    tile_load<DIR, L, W, K>(kb.nyg, b.d, b.u, b.v, b.w, b.cc, g, ld, k.off32);
+    TileLoads<DIR, L, W, K, false> ld;
+    tile_load<DIR, L, W, K, BIG || MIX>(kb.nyg, b.d, b.u, b.v, b.w, b.cc, nullptr, g, ld, k.same_pitch);
     const ws_metric_fields nomf{};
     StageArgs sa{};
     if (STG) {
@@ -711,7 +757,7 @@ k_rhs_batch_grid(KParams k, const BatchBlock *blocks, const int4 *tiles, int nti
             sa.halo = bs.halo;
         }
     }
-    const double cmax = tile_compute<DIR, L, W, K, false, ACC, MIX, false, STG>(kb, nomf, b.du, g, ld, sp, sa, [] {});
+    const double cmax = tile_compute<DIR, L, W, K, false, ACC, MIX, false, STG, BIG>(kb, nomf, b.du, g, ld, sp, sa, [] {});
     if (STG && sa.cfl_part) {
         __syncthreads();   // phase 3 has read its faces from sp
         tile_wg_max<TL::NT>(cmax, sp, sa.cfl_part + tile);
@@ -745,7 +791,7 @@ void launch_persist(const KParams &k, ws_field d, ws_field u, ws_field v, ws_fie
                        cc, du, box, gx, gy, n, chunk);
 }
 
-template <int DIR, int L, int W, int K, bool FIELDS, bool ACC, bool MIX>
+template <int DIR, int L, int W, int K, bool FIELDS, bool ACC, bool MIX, bool BIG>
 void launch_dir(const KParams &k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc,
                 const ws_metric_fields &mf, ws_soa du, const Box &box, int sched, hipStream_t s)
 {
@@ -761,10 +807,10 @@ void launch_dir(const KParams &k, ws_field d, ws_field u, ws_field v, ws_field w
     const dim3 grid1(8 * ((ntiles + 7) / 8));
     if (k.bnd_any[DIR]) {
         // one-sided closures in this direction: the grid schedule with the closure code
-        hipLaunchKernelGGL((k_rhs_tile<DIR, L, W, K, FIELDS, ACC, MIX, true>), grid1, dim3(TL::NT), 0, s, k, d, u, v,
+        hipLaunchKernelGGL((k_rhs_tile<DIR, L, W, K, FIELDS, ACC, MIX, true, false, BIG>), grid1, dim3(TL::NT), 0, s, k, d, u, v,
                            w, cc, mf, du, box, (int)grid.x, (int)grid.y, ntiles, StageArgs{});
-    } else if (FIELDS || sched == WS_SCHED_GRID) {
-        hipLaunchKernelGGL((k_rhs_tile<DIR, L, W, K, FIELDS, ACC, MIX, false>), grid1, dim3(TL::NT), 0, s, k, d, u,
+    } else if (FIELDS || BIG || sched == WS_SCHED_GRID) {
+        hipLaunchKernelGGL((k_rhs_tile<DIR, L, W, K, FIELDS, ACC, MIX, false, false, BIG>), grid1, dim3(TL::NT), 0, s, k, d, u,
                            v, w, cc, mf, du, box, (int)grid.x, (int)grid.y, ntiles, StageArgs{});
     } else if (sched == WS_SCHED_PREFETCH) {
         launch_persist<DIR, L, W, K, ACC, MIX, true>(k, d, u, v, w, cc, du, box, grid.x, grid.y, grid.z, s);
@@ -803,43 +849,43 @@ void launch_dir_stage(const KParams &k, ws_field d, ws_field u, ws_field v, ws_f
 // read-modify-write it.  Which direction pays for that read shifts the time differently
 // per precision, so the order is a tuning choice (WS_ORDER_*).  With a stage (sa) the last
 // launch applies it instead of writing du.
-template <int L0, int W0, int L1, int W1, int L2, int W2, int K, bool FIELDS, bool MIX>
+template <int L0, int W0, int L1, int W1, int L2, int W2, int K, bool FIELDS, bool MIX, bool BIG>
 void launch_all(const KParams &k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc,
                 const ws_metric_fields &mf, ws_soa du, const Box &box, int accumulate, int sched, int order,
                 const StageArgs *sa, hipStream_t s)
 {
     if (order == WS_ORDER_ZYX) {
-        if (accumulate) launch_dir<2, L2, W2, K, FIELDS, true, MIX>(k, d, u, v, w, cc, mf, du, box, sched, s);
-        else launch_dir<2, L2, W2, K, FIELDS, false, MIX>(k, d, u, v, w, cc, mf, du, box, sched, s);
-        launch_dir<1, L1, W1, K, FIELDS, true, MIX>(k, d, u, v, w, cc, mf, du, box, sched, s);
+        if (accumulate) launch_dir<2, L2, W2, K, FIELDS, true, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
+        else launch_dir<2, L2, W2, K, FIELDS, false, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
+        launch_dir<1, L1, W1, K, FIELDS, true, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
         if constexpr (!FIELDS) {
             if (sa) {
                 launch_dir_stage<0, L0, W0, K, MIX>(k, d, u, v, w, cc, du, box, *sa, s);
                 return;
             }
         }
-        launch_dir<0, L0, W0, K, FIELDS, true, MIX>(k, d, u, v, w, cc, mf, du, box, sched, s);
+        launch_dir<0, L0, W0, K, FIELDS, true, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
         return;
     }
-    if (accumulate) launch_dir<0, L0, W0, K, FIELDS, true, MIX>(k, d, u, v, w, cc, mf, du, box, sched, s);
-    else launch_dir<0, L0, W0, K, FIELDS, false, MIX>(k, d, u, v, w, cc, mf, du, box, sched, s);
-    launch_dir<1, L1, W1, K, FIELDS, true, MIX>(k, d, u, v, w, cc, mf, du, box, sched, s);
+    if (accumulate) launch_dir<0, L0, W0, K, FIELDS, true, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
+    else launch_dir<0, L0, W0, K, FIELDS, false, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
+    launch_dir<1, L1, W1, K, FIELDS, true, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
     if constexpr (!FIELDS) {
         if (sa) {
             launch_dir_stage<2, L2, W2, K, MIX>(k, d, u, v, w, cc, du, box, *sa, s);
             return;
         }
     }
-    launch_dir<2, L2, W2, K, FIELDS, true, MIX>(k, d, u, v, w, cc, mf, du, box, sched, s);
+    launch_dir<2, L2, W2, K, FIELDS, true, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
 }
 
-template <int S, bool FIELDS, bool MIX>
+template <int S, bool FIELDS, bool MIX, bool BIG = false>
 void launch_shape_n(const KParams &k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc,
                     const ws_metric_fields &mf, ws_soa du, const Box &box, int acc, int sched, int order,
                     const StageArgs *sa, hipStream_t s)
 {
     constexpr TileShapeDef D = kTileShapes[S];
-    launch_all<D.L0, D.W0, D.L1, D.W1, D.L2, D.W2, D.K, FIELDS, MIX>(k, d, u, v, w, cc, mf, du, box, acc, sched,
+    launch_all<D.L0, D.W0, D.L1, D.W1, D.L2, D.W2, D.K, FIELDS, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, acc, sched,
                                                                     order, sa, s);
 }
 
@@ -848,6 +894,11 @@ void launch_shape(int shape, const KParams &k, ws_field d, ws_field u, ws_field 
                   const ws_metric_fields &mf, ws_soa du, const Box &box, int acc, int sched, int order,
                   const StageArgs *sa, hipStream_t s)
 {
+    if (k.big) {
+        // planes beyond 32-bit tile offsets: one shape serves them (and no stage is fused)
+        launch_shape_n<WS_TILE_30x16_K2, FIELDS, MIX, true>(k, d, u, v, w, cc, mf, du, box, acc, sched, order, sa, s);
+        return;
+    }
     switch (shape) {
     case 0: launch_shape_n<0, FIELDS, MIX>(k, d, u, v, w, cc, mf, du, box, acc, sched, order, sa, s); break;
     case 1: launch_shape_n<1, FIELDS, MIX>(k, d, u, v, w, cc, mf, du, box, acc, sched, order, sa, s); break;
@@ -896,12 +947,12 @@ void launch_batch_dir(const KParams &k, const BatchTiles &bt, hipStream_t s)
 
 // one tile per work-group over direction DIR's tile list (the grid schedule), STG: this
 // launch applies the RK3 stage bt.stage
-template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool STG>
+template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool STG, bool BIG = false>
 void launch_batch_grid(const KParams &k, const BatchTiles &bt, hipStream_t s)
 {
     const int n = bt.ntiles[DIR];
     if (n <= 0) return;
-    hipLaunchKernelGGL((k_rhs_batch_grid<DIR, L, W, K, ACC, MIX, STG>), dim3(8 * ((n + 7) / 8)),
+    hipLaunchKernelGGL((k_rhs_batch_grid<DIR, L, W, K, ACC, MIX, STG, BIG>), dim3(8 * ((n + 7) / 8)),
                        dim3(Tile<DIR, L, W, K>::NT), 0, s, k, bt.blocks, bt.tiles[DIR], n,
                        STG ? *bt.stage : BatchStage{});
 }
@@ -910,6 +961,16 @@ template <int S, bool MIX, bool PF>
 void launch_batch_shape_n(const KParams &k, const BatchTiles &bt, hipStream_t s)
 {
     constexpr TileShapeDef D = kTileShapes[S];
+    if (k.big) {
+        // planes beyond 32-bit tile offsets: the grid schedule in this one shape (the caller
+        // passes its tile lists)
+        if constexpr (S == WS_TILE_30x16_K2 && !PF) {
+            launch_batch_grid<0, D.L0, D.W0, D.K, false, MIX, false, true>(k, bt, s);
+            launch_batch_grid<1, D.L1, D.W1, D.K, true, MIX, false, true>(k, bt, s);
+            launch_batch_grid<2, D.L2, D.W2, D.K, true, MIX, false, true>(k, bt, s);
+        }
+        return;
+    }
     if (bt.stage && bt.stage_order == WS_ORDER_ZYX) {
         // z writes du, y accumulates, x adds its terms and applies the stage
         launch_batch_grid<2, D.L2, D.W2, D.K, false, MIX, false>(k, bt, s);
@@ -946,7 +1007,8 @@ int launch_rhs_tile(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w
     const int shape = sa && c.stage_shape >= 0 ? c.stage_shape : c.tile_shape;
     const int order = sa ? c.stage_order : c.dir_order;
     KParams k = c.kp;
-    k.off32 = prim_off32(k, d, u, v, w, cc) ? 1 : 0;
+    k.same_pitch = same_pitch(d, u, v, w, cc) ? 1 : 0;
+    k.big = rel_planes(k, {d, u, v, w, cc}, {du}) && (!m || rel_planes(k, *m)) ? 0 : 1;
     if (m) {
         mf = *m;
         launch_shape<true, MIX>(shape, k, d, u, v, w, cc, mf, du, box, accumulate, c.schedule, order, nullptr, s);
@@ -961,7 +1023,7 @@ int launch_rhs_tile(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w
 template <bool MIX>
 int launch_rhs_batch_tile(const KParams &k, const BatchTiles &bt, hipStream_t s)
 {
-    if (bt.schedule == WS_SCHED_PREFETCH) launch_batch_pf<MIX, true>(k, bt, s);
+    if (bt.schedule == WS_SCHED_PREFETCH && !k.big) launch_batch_pf<MIX, true>(k, bt, s);
     else launch_batch_pf<MIX, false>(k, bt, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_error(e, MIX ? "batched mixed-precision RHS launch" : "batched RHS launch");

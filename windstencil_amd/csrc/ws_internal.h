@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <initializer_list>
 #include <string>
 
 #include "windstencil_amd.h"
@@ -39,20 +40,49 @@ struct KParams {
     int bnd[6];
     int nonref[6];
     int bnd_any[3];
-    // set per launch: the RHS inputs d, u, v, w, cc share d's pitch and every offset into
-    // them is below 2^31 with pitch and nyg*nzg below 2^24, so one 32-bit offset with
-    // 24-bit products addresses all five (prim_off32)
-    int off32 = 0;
+    // set per launch: the RHS inputs d, u, v, w, cc share d's pitch, so one offset addresses
+    // all five; big: a field of the launch has planes of kTilePlane elements or more
+    int same_pitch = 0;
+    int big = 0;
 };
 
-// whether the five RHS input fields of a box of these extents can be addressed with one
-// 32-bit offset (KParams::off32)
-inline bool prim_off32(const KParams &k, const ws_field &d, const ws_field &u, const ws_field &v,
-                       const ws_field &w, const ws_field &cc)
+inline bool same_pitch(const ws_field &d, const ws_field &u, const ws_field &v, const ws_field &w, const ws_field &cc)
 {
-    const unsigned long long p = d.pitch, plane = (unsigned long long)k.nyg * (unsigned long long)k.nzg;
-    return u.pitch == d.pitch && v.pitch == d.pitch && w.pitch == d.pitch && cc.pitch == d.pitch &&
-           p < (1ull << 24) && plane < (1ull << 24) && p * plane < (1ull << 31);
+    return u.pitch == d.pitch && v.pitch == d.pitch && w.pitch == d.pitch && cc.pitch == d.pitch;
+}
+
+// The tiled kernels address a tile's points by 32-bit byte offsets from its first one, formed
+// with 24-bit products.  The longest reach is that of z tiles: at most 40 planes (L + 2 LAP
+// with L = 32) and one row, so planes below (2^32 / 8) / 41 elements, about 13.1 million, keep
+// every offset below 2^32 and every stride below 2^24.  x tiles reach 16 rows, y tiles 40, both
+// within a plane's rows or (few rows per plane) below 40 pitches.
+constexpr unsigned long long kTilePlane = (1ull << 29) / 41;
+
+inline bool rel_field(const ws_field &f, int rows)
+{
+    return !f.ptr || (unsigned long long)f.pitch * (unsigned long long)rows < kTilePlane;
+}
+
+inline bool rel_soa(const ws_soa &f, int rows)
+{
+    return !f.ptr || (unsigned long long)f.pitch * (unsigned long long)rows < kTilePlane;
+}
+
+// whether every field given has planes the tiles' 32-bit offsets reach
+inline bool rel_planes(const KParams &k, std::initializer_list<ws_field> fields, std::initializer_list<ws_soa> states)
+{
+    for (const ws_field &f : fields)
+        if (!rel_field(f, k.nyg)) return false;
+    for (const ws_soa &f : states)
+        if (!rel_soa(f, k.ny)) return false;
+    return true;
+}
+
+inline bool rel_planes(const KParams &k, const ws_metric_fields &m)
+{
+    for (const ws_field &f : m.A)
+        if (!rel_field(f, k.nyg)) return false;
+    return rel_field(m.ajac, k.nyg);
 }
 
 // The SSP-RK3 stage the last directional RHS launch applies to its cells itself (f from fn,
@@ -78,6 +108,13 @@ struct StageArgs {
     int halo = 0;
 };
 
+// whether the tiles' 32-bit offsets reach all of a state and the context's second primitive
+// set (its pitch: nx + 2 LAP rounded to 32)
+inline bool rel_state(const KParams &k, const ws_state &st)
+{
+    const ws_field second{st.d.ptr, (uint32_t)((k.nx + 2 * LAP + 31) / 32 * 32), 0};
+    return rel_planes(k, {st.d, st.u, st.v, st.w, st.T, st.P, st.cc, second}, {st.f, st.fn, st.du});
+}
 
 struct Ctx {
     ws_config cfg;
@@ -249,8 +286,8 @@ int rhs_for_ctx(ws_ctx *c, const ws_state *st, hipStream_t s);
 // RHS, plus the viscous terms when the configuration has them
 int du_from_prepared(ws_ctx *c, const ws_state *st, hipStream_t s);
 // whether RK3 steps can let the last RHS launch apply the stage (stage fusion on, tiled
-// kernels, grid schedule, no closures, no viscous terms)
-bool fused_stage_ok(const ws_ctx *c);
+// kernels, grid schedule, no closures, no viscous terms, planes the tiles' offsets reach)
+bool fused_stage_ok(const ws_ctx *c, const ws_state *st);
 // How a step of stage fusion 3 treats the primitive sets (rk3_step_fused): STEP_PLAIN starts
 // and ends with the primitives in the state's fields (every level); STEP_FROM_STATE and
 // STEP_FROM_SECOND start from the state's fields or the context's second set, prepared, and
@@ -265,7 +302,7 @@ int rk3_step_fused(ws_ctx *c, ws_state *st, const double *dt_dev, hipStream_t s,
                    StepMode mode = STEP_PLAIN, bool prepare = true);
 // whether ws_rk3_run can alternate the primitive sets (stage fusion 3 and every condition of
 // the primitives-deriving fusion), allocating what that needs (outside a stream capture)
-bool alternating_steps(ws_ctx *c, hipStream_t s, bool cfl);
+bool alternating_steps(ws_ctx *c, const ws_state *st, hipStream_t s, bool cfl);
 // the context's second set of ghosted primitive fields (d, u, v, w, T, cc), allocated at
 // the first call outside a stream capture; 0 if it is not available
 int prim_set(ws_ctx *c, hipStream_t s, ws_field out[6]);
