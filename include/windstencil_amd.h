@@ -178,6 +178,9 @@ int ws_ctx_destroy(ws_ctx *ctx);
 int ws_ctx_get_config(const ws_ctx *ctx, ws_config *out);
 int ws_ctx_set_precision(ws_ctx *ctx, int32_t precision);
 int ws_ctx_set_kernel(ws_ctx *ctx, int32_t kernel);
+/* WS_TILE_*.  Until a tile shape, a stage shape or a schedule is set, RHS calls on small jobs
+ * (at most 1200 cells per compute unit, no closures) run one launch over cubes of 4^3 cells
+ * instead of the directional tiles, with the same bits. */
 int ws_ctx_set_tile_shape(ws_ctx *ctx, int32_t shape);
 int ws_ctx_get_tile_shape(const ws_ctx *ctx, int32_t *shape);
 /* WS_SCHED_*; the persistent schedules apply without metric fields (with them the
@@ -294,7 +297,8 @@ int ws_cfl_dt(ws_ctx *ctx, const ws_state *st, double cfl, double *dt_dev, hipSt
  * launch (ws_ctx_set_stage_fusion), the stage order and tile shape are then timed the same
  * way (every shape in both orders, 3 * reps launches each): the RHS of an RK3 stage 2 whose last launch writes the
  * new f, primitives, sound speed and halo into scratch the call allocates and frees (the
- * state's f is read, not written).  times_ms
+ * state's f is read, not written).  On a small grid the one-launch kernel
+ * (ws_ctx_set_tile_shape) is timed last and kept when it is the fastest.  times_ms
  * (WS_TILE_COUNT * WS_SCHED_COUNT entries, shape-major, each the faster of the two orders)
  * may be NULL.  Overwrites st->du; synchronises the stream.  No counterpart in the
  * reference. */

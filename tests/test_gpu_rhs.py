@@ -461,3 +461,61 @@ def test_planes_beyond_the_tiles_32_bit_offsets(ws, precision):
         err = rel_l2(a, b)
         log(f"  long rows against short ones: {err:.3e}")
         assert err <= tol
+
+
+@pytest.mark.parametrize("precision", [W.WS_PREC_FP64, W.WS_PREC_MIXED])
+@pytest.mark.parametrize("shape", [(4, 4, 4), (5, 7, 6), (8, 4, 9), (13, 11, 5), (67, 68, 67)])
+def test_one_launch_rhs_of_small_jobs(ws, shape, precision):
+    """The one-launch kernel against the directional tiles (a context with a tile shape set),
+    bit for bit: whole cubes, remainders in every direction and 4913 cubes on a chip that
+    holds 768 at once, on a blast whose FP32 weights overflow; both direction orders, inputs
+    of one pitch and of two, metric fields, a sub-box, accumulation, three RK3 steps (a stage per
+    launch, periodic halo, CFL maxima) and the same steps with a closure, which keep the tiles."""
+    import torch
+    from windstencil_amd import initial as I
+    nx, ny, nz = shape
+    L = W.lib()
+    sh = W.stream_handle()
+    prims = I.blast(nx, ny, nz, 5, 1e8) if precision == W.WS_PREC_MIXED else random_state(nx, ny, nz, 31, "shock")
+    rng = np.random.default_rng(41)
+    tens = [torch.from_numpy(0.7 + 0.6 * rng.random((nz + 8, ny + 8, nx + 8))).cuda() for _ in range(10)]
+    mf = W.WsMetricFields()
+    for i in range(9):
+        mf.A[i] = W.field_of(tens[i])
+    mf.ajac = W.field_of(tens[9])
+    inner = W.job((4 + 1, 4 + 2, 4 + 1), (4 + nx, 4 + ny - 1, 4 + nz))
+
+    def results(tiles):
+        out = []
+        for order in W.ORDERS:
+            ctx = make_ctx(nx, ny, nz, precision=precision)
+            ctx.set_direction_order(order)
+            ctx.set_stage_order(order)
+            if tiles:
+                ctx.set_tile_shape(W.WS_TILE_30x16_K2)
+            st = upload_state(prims)
+            out.append(gpu_du_comput(ctx, st).copy())
+            out.append(gpu_du_comput(ctx, st, accumulate=True).copy())
+            st.t["du"].fill_(7.0)
+            out.append(gpu_du_comput(ctx, st, job=inner).copy())
+            out.append(gpu_du_comput(ctx, st, metrics=mf).copy())
+            st.t["cc"] = W.ghosted_tensor(nx, ny, nz, pad=5)
+            st.refresh()
+            out.append(gpu_du_comput(ctx, st).copy())
+            for closed in (False, True):
+                kw = dict(periodic=(0, 1, 1), d0_bound=(1, 1, 0, 0, 0, 0)) if closed and nx >= 8 else {}
+                rk = make_ctx(nx, ny, nz, precision=precision, **kw)
+                rk.set_stage_order(order)
+                rk.set_direction_order(order)
+                if tiles:
+                    rk.set_tile_shape(W.WS_TILE_30x16_K2)
+                st = upload_state(random_state(nx, ny, nz, 31, "blobs"))
+                W.check(L.ws_pri_to_cons(rk.handle, st.ws.f, st.ws.d, st.ws.u, st.ws.v, st.ws.w, st.ws.T,
+                                         W.job((0, 0, 0), shape), sh))
+                W.check(L.ws_rk3_run(rk.handle, ctypes.byref(st.ws), 3, 0.5, 1, sh))
+                st.sync_from_ws()
+                out += [st.interior(q).cpu().numpy().copy() for q in ("f", "d", "u", "v", "w", "T")]
+        return out
+
+    for i, (a, b) in enumerate(zip(results(False), results(True))):
+        assert np.array_equal(a, b, equal_nan=True), i

@@ -23,7 +23,7 @@ namespace {
 
 std::mutex g_mu;
 struct Choice {
-    int shape, schedule, order, stage_order, stage_shape;
+    int shape, schedule, order, stage_order, stage_shape, box;
 };
 // (nx, ny, nz, precision) -> choice
 std::map<std::tuple<int, int, int, int>, Choice> g_best;
@@ -131,7 +131,7 @@ bool tune_stage(ws_ctx *c, const ws_state *st, const ws_job &job, int reps, hipE
 namespace ws {
 
 bool remembered_choice(int nx, int ny, int nz, int precision, int *shape, int *schedule, int *order,
-                       int *stage_order, int *stage_shape)
+                       int *stage_order, int *stage_shape, int *box)
 {
     std::lock_guard<std::mutex> lk(g_mu);
     auto it = g_best.find(std::make_tuple(nx, ny, nz, precision));
@@ -141,6 +141,7 @@ bool remembered_choice(int nx, int ny, int nz, int precision, int *shape, int *s
     *order = it->second.order;
     *stage_order = it->second.stage_order;
     *stage_shape = it->second.stage_shape;
+    *box = it->second.box;
     return true;
 }
 
@@ -157,11 +158,12 @@ extern "C" int ws_autotune(ws_ctx *c, const ws_state *st, int32_t reps, float *t
     if (e != hipSuccess) return hip_error(e, "autotune event");
     e = hipEventCreate(&e1);
     if (e != hipSuccess) { hipEventDestroy(e0); return hip_error(e, "autotune event"); }
-    const Choice saved{c->tile_shape, c->schedule, c->dir_order, c->stage_order, c->stage_shape};
+    const Choice saved{c->tile_shape, c->schedule, c->dir_order, c->stage_order, c->stage_shape, c->box};
     Choice best = saved;
     int r = WS_OK;
     float best_ms = 1e30f;
     auto rhs = [&]() { return launch(*c, st, job, s); };
+    c->box = 0;
     for (int shape = 0; shape < WS_TILE_COUNT && !r; ++shape)
         for (int sched = 0; sched < WS_SCHED_COUNT && !r; ++sched) {
             float pair_ms = 1e30f;
@@ -174,7 +176,7 @@ extern "C" int ws_autotune(ws_ctx *c, const ws_state *st, int32_t reps, float *t
                 if (ms < pair_ms) pair_ms = ms;
                 if (ms < best_ms) {
                     best_ms = ms;
-                    best = Choice{shape, sched, order, saved.stage_order, saved.stage_shape};
+                    best = Choice{shape, sched, order, saved.stage_order, saved.stage_shape, 0};
                 }
             }
             if (times_ms) times_ms[shape * WS_SCHED_COUNT + sched] = pair_ms;
@@ -190,6 +192,16 @@ extern "C" int ws_autotune(ws_ctx *c, const ws_state *st, int32_t reps, float *t
             best.stage_order = o;
         }
     }
+    if (!r) {
+        // the one-launch kernel, where the job is small enough for it (elsewhere it stays
+        // allowed for smaller jobs of the context)
+        c->box = 1;
+        if (box_serves(*c, job)) {
+            const float ms = time_launches(rhs, reps, e0, e1, s, r);
+            c->box = !r && ms < best_ms;
+        }
+        best.box = c->box;
+    }
     hipEventDestroy(e0);
     hipEventDestroy(e1);
     const Choice &use = r ? saved : best;
@@ -198,6 +210,7 @@ extern "C" int ws_autotune(ws_ctx *c, const ws_state *st, int32_t reps, float *t
     c->dir_order = use.order;
     c->stage_order = use.stage_order;
     c->stage_shape = use.stage_shape;
+    c->box = use.box;
     if (!r) {
         std::lock_guard<std::mutex> lk(g_mu);
         g_best[std::make_tuple(c->cfg.nx, c->cfg.ny, c->cfg.nz, c->cfg.precision)] = best;

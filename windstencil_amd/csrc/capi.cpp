@@ -100,14 +100,6 @@ int check_metrics(const ws_ctx *c, const ws_metric_fields *m)
     return check_field(c, m->ajac, "ajac");
 }
 
-ws_job interior_job(const ws_ctx *c)
-{
-    ws_job j;
-    j.start = {(uint32_t)LAP, (uint32_t)LAP, (uint32_t)LAP};
-    j.end = {(uint32_t)(c->cfg.nx + LAP), (uint32_t)(c->cfg.ny + LAP), (uint32_t)(c->cfg.nz + LAP)};
-    return j;
-}
-
 ws_job ghosted_job(const ws_ctx *c)
 {
     ws_job j;
@@ -289,8 +281,8 @@ double *cfl_stage_buffer(ws_ctx *c)
 bool fused_stage_ok(const ws_ctx *c, const ws_state *st)
 {
     const bool closures = c->kp.bnd_any[0] || c->kp.bnd_any[1] || c->kp.bnd_any[2];
-    return c->fuse_stage && c->cfg.kernel == WS_KERNEL_TILED && !c->cfg.viscous && c->schedule == WS_SCHED_GRID &&
-           !closures && rel_state(c->kp, *st);
+    return c->fuse_stage && c->cfg.kernel == WS_KERNEL_TILED && !c->cfg.viscous &&
+           (c->schedule == WS_SCHED_GRID || box_serves(*c, interior_job(c))) && !closures && rel_state(c->kp, *st);
 }
 
 bool alternating_steps(ws_ctx *c, const ws_state *st, hipStream_t s, bool cfl)
@@ -456,14 +448,15 @@ int ws_ctx_create(const ws_config *cfg, ws_ctx **out)
     if (!c) return set_error(WS_ERR_NOMEM, "host allocation failed");
     c->cfg = *cfg;
     c->kp = make_kparams(*cfg);
-    int shape, sched, order, stage_order, stage_shape;
+    int shape, sched, order, stage_order, stage_shape, box;
     if (remembered_choice(cfg->nx, cfg->ny, cfg->nz, cfg->precision, &shape, &sched, &order, &stage_order,
-                          &stage_shape)) {
+                          &stage_shape, &box)) {
         c->tile_shape = shape;
         c->schedule = sched;
         c->dir_order = order;
         c->stage_order = stage_order;
         c->stage_shape = stage_shape;
+        c->box = box;
     }
     hipError_t e = hipGetDevice(&c->device);
     if (e != hipSuccess) { delete c; return hip_error(e, "hipGetDevice"); }
@@ -509,14 +502,15 @@ int ws_ctx_set_precision(ws_ctx *c, int32_t precision)
     if (!c) return set_error(WS_ERR_INVALID, "null context");
     if (precision != WS_PREC_FP64 && precision != WS_PREC_MIXED) return set_error(WS_ERR_INVALID, "unknown precision");
     c->cfg.precision = precision;
-    int shape, sched, order, stage_order, stage_shape;
+    int shape, sched, order, stage_order, stage_shape, box;
     if (remembered_choice(c->cfg.nx, c->cfg.ny, c->cfg.nz, precision, &shape, &sched, &order, &stage_order,
-                          &stage_shape)) {
+                          &stage_shape, &box)) {
         c->tile_shape = shape;
         c->schedule = sched;
         c->dir_order = order;
         c->stage_order = stage_order;
         c->stage_shape = stage_shape;
+        c->box = box;
     }
     return WS_OK;
 }
@@ -534,6 +528,7 @@ int ws_ctx_set_tile_shape(ws_ctx *c, int32_t shape)
     if (!c) return set_error(WS_ERR_INVALID, "null context");
     if (shape < 0 || shape >= WS_TILE_COUNT) return set_error(WS_ERR_INVALID, "unknown tile shape");
     c->tile_shape = shape;
+    c->box = 0;
     return WS_OK;
 }
 
@@ -542,6 +537,7 @@ int ws_ctx_set_schedule(ws_ctx *c, int32_t schedule)
     if (!c) return set_error(WS_ERR_INVALID, "null context");
     if (schedule < 0 || schedule >= WS_SCHED_COUNT) return set_error(WS_ERR_INVALID, "unknown schedule");
     c->schedule = schedule;
+    c->box = 0;
     return WS_OK;
 }
 
@@ -587,6 +583,7 @@ int ws_ctx_set_stage_shape(ws_ctx *c, int32_t shape)
     if (!c) return set_error(WS_ERR_INVALID, "null context");
     if (shape < -1 || shape >= WS_TILE_COUNT) return set_error(WS_ERR_INVALID, "unknown tile shape");
     c->stage_shape = shape;
+    c->box = 0;
     return WS_OK;
 }
 

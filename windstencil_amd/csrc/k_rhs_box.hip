@@ -1,0 +1,297 @@
+// k_rhs_box.hip -- LDS-tiled inviscid RHS of small jobs, FP64 and mixed: one launch for all
+// three directions.
+//
+// The directional launches of rhs_tile.h want some thousand tiles in flight: a grid of
+// 64x32x16 cells gives each of them about 100 work-groups for 256 compute units, so a launch
+// takes as long as one work-group does and the three follow one another.  Here a work-group
+// owns a cube of 4^3 cells and does the three directions together, so a small grid spreads
+// over the chip, every cell's flux differences meet in registers, and du is written once (or
+// the RK3 stage applied at once).
+// Faces and cells are computed by the expressions of rhs_tile.h and summed in the same order
+// (dir_order), so du has the bits of the directional launches.
+#include "rhs_tile.h"
+
+namespace ws {
+
+namespace {
+
+constexpr int B = 4;                           // edge of the cube
+constexpr int BOX_NT = 256;
+constexpr int BOX_NL = B + 2 * LAP;            // points per line
+constexpr int BOX_F = B + 1;                   // faces per line
+constexpr int BOX_LINES = B * B;               // lines per direction
+constexpr int BOX_LT = 3 * BOX_LINES;          // lines of the three directions
+constexpr int BOX_CELLS = B * B * B;
+constexpr int BOX_DPTS = BOX_LINES * BOX_NL;   // points per direction
+constexpr int BOX_NPTS = 3 * BOX_DPTS;
+constexpr int BOX_ROUNDS = (BOX_NPTS + BOX_NT - 1) / BOX_NT;
+static_assert(BOX_DPTS % 64 == 0, "a wavefront's points lie in one direction");
+static_assert(BOX_LT * 5 <= BOX_NT && BOX_CELLS <= BOX_NT, "a thread per line and variable, and per cell");
+
+// LDS index of quantity q (P 0..4, M 5..9) at point p of line l (directions one after the
+// other): consecutive lines are consecutive doubles, which the threads of a wavefront read
+// and, in y and z, write together
+__device__ constexpr int box_pidx(int q, int p, int l) { return (q * BOX_NL + p) * BOX_LT + l; }
+// the face fluxes reuse the buffer, line-major: with an odd number of faces per line both the
+// writes (consecutive lines) and the reads (consecutive cells) spread over the banks
+__device__ constexpr int box_fidx(int m, int l, int f) { return (m * BOX_LT + l) * BOX_F + f; }
+
+// this thread's point of round r: direction (the same for a whole wavefront), line and point;
+// false: none (a valid point all the same).  Along x consecutive threads take 4 points of 16
+// lines: loads of 32-byte runs, LDS writes two to a bank.
+__device__ __forceinline__ bool box_point(int r, int &dir, int &l, int &p)
+{
+    const int g = (int)threadIdx.x + r * BOX_NT;
+    const bool in = g < BOX_NPTS;
+    int q = min(g, BOX_NPTS - 1);
+    dir = __builtin_amdgcn_readfirstlane(q / BOX_DPTS);
+    q -= dir * BOX_DPTS;
+    if (dir == 0) { p = (q & 3) + q / (4 * BOX_LINES) * 4; l = (q >> 2) % BOX_LINES; }
+    else          { l = q % BOX_LINES; p = q / BOX_LINES; }
+    return in;
+}
+
+// What bounds it: on a small grid the chain load - split - reconstruct - store of one cube,
+// with one to three cubes per compute unit to overlap it; on a larger one the FP64 issue.
+// Both want few operations, so one thread reconstructs all five faces of one line and
+// variable, which share the window's differences: 128 FP64 operations per face against 190 with
+// a thread per face (64x32x16 9.5 us so, 100x60x40 52).  Cubes of 8^3 cells through the three
+// directions in turn took 19-23 us on a grid of any small size.
+// FP64 RHS, the directional launches before and this kernel: 64x32x16 23.1 -> 8.8 us,
+// 48x48x48 35.1 -> 20.8 us; an RK3 step of 64x32x16 85 -> 47 us.
+template <bool FIELDS, bool MIX, bool STG>
+__global__ void __launch_bounds__(BOX_NT, 3)
+k_rhs_box(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc, ws_metric_fields mf, ws_soa du,
+          Box box, int gx, int gy, int ntiles, int order, int accumulate, StageArgs sa)
+{
+    constexpr int K = BOX_F;
+    __shared__ double sp[10 * BOX_NPTS];
+    // cubes in x-fastest order, a contiguous range of them per XCD (as k_rhs_tile)
+    const int per = (ntiles + 7) / 8;
+    const int tile = ((int)blockIdx.x % 8) * per + (int)blockIdx.x / 8;
+    if (tile >= ntiles) return;
+    const int trow = tile / gx;
+    const int x0 = box.s[0] + (tile - trow * gx) * B, y0 = box.s[1] + trow % gy * B, z0 = box.s[2] + trow / gy * B;
+    // cells of the cube inside the box
+    const int lx = min(B, box.e[0] - x0), ly = min(B, box.e[1] - y0), lz = min(B, box.e[2] - z0);
+    const int t = threadIdx.x;
+
+    // ---- loads: primitives (and metric terms) of this thread's points; points that no face
+    // inside the box reaches repeat one that does (their values go to no stored face)
+    double ld[BOX_ROUNDS][FIELDS ? 8 : 5];
+#pragma unroll
+    for (int r = 0; r < BOX_ROUNDS; ++r) {
+        int dir, l, p;
+        box_point(r, dir, l, p);
+        const int a = min(l % B, (dir == 0 ? ly : lx) - 1), b = min(l / B, (dir == 2 ? ly : lz) - 1);
+        const int c = min(p, (dir == 0 ? lx : dir == 1 ? ly : lz) + 2 * LAP - 1);
+        // from the first point of the direction's lines
+        const int bx = x0 - (dir == 0 ? LAP : 0), by = y0 - (dir == 1 ? LAP : 0), bz = z0 - (dir == 2 ? LAP : 0);
+        const uint32_t px = dir == 0 ? c : a, py = dir == 1 ? c : dir == 0 ? a : b, pz = dir == 2 ? c : b;
+        auto off = [&](const ws_field &f) { return 8u * (px + f.pitch * (py + (uint32_t)k.nyg * pz)); };
+        auto base = [&](const ws_field &f) { return f.ptr + origin(f.pitch, k.nyg, bx, by, bz); };
+        const ws_field in[5] = {d, u, v, w, cc};
+        if (k.same_pitch) {
+            const uint32_t o = off(d);
+#pragma unroll
+            for (int q = 0; q < 5; ++q) ld[r][q] = elem(base(in[q]), o);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 5; ++q) ld[r][q] = elem(base(in[q]), off(in[q]));
+        }
+        if constexpr (FIELDS) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) ld[r][5 + q] = elem(base(mf.A[3 * dir + q]), off(mf.A[3 * dir + q]));
+        }
+    }
+
+    // this thread's cell (threads past the last cell, and cells past the box: none)
+    const int ix = t % B, iy = t / B % B, iz = t / (B * B);
+    const bool cell = t < BOX_CELLS && ix < lx && iy < ly && iz < lz;
+    auto ghosted = [&](const ws_field &f) -> double & {
+        return elem(f.ptr + origin(f.pitch, k.nyg, x0, y0, z0),
+                    8u * ((uint32_t)ix + f.pitch * ((uint32_t)iy + (uint32_t)k.nyg * (uint32_t)iz)));
+    };
+    auto state = [&](const ws_soa &f, int m) -> double & {
+        return elem(f.ptr + (size_t)m * f.pitch * k.ny * k.nz + origin(f.pitch, k.ny, x0 - LAP, y0 - LAP, z0 - LAP),
+                    8u * ((uint32_t)ix + f.pitch * ((uint32_t)iy + (uint32_t)k.ny * (uint32_t)iz)));
+    };
+    double acc[5] = {}, fnv[5] = {}, fvv[5] = {};
+    double aj = k.ajac;
+    if (cell) {
+        if (FIELDS) aj = ghosted(mf.ajac);
+        if (STG) {
+#pragma unroll
+            for (int m = 0; m < 5; ++m) fnv[m] = state(sa.fn, m);
+            if (sa.krk != 1)
+#pragma unroll
+                for (int m = 0; m < 5; ++m) fvv[m] = state(sa.f, m);
+        } else if (accumulate) {
+#pragma unroll
+            for (int m = 0; m < 5; ++m) acc[m] = state(du, m);
+        }
+    }
+
+    // ---- split every point into LDS ----------------------------------------------------------
+#pragma unroll
+    for (int r = 0; r < BOX_ROUNDS; ++r) {
+        int dir, l, p;
+        if (!box_point(r, dir, l, p)) continue;
+        const double dd = ld[r][0], uu = ld[r][1], vv = ld[r][2], ww = ld[r][3], c = ld[r][4];
+        double fp[5], fm[5];
+        if (FIELDS) {
+            const double A1 = ld[r][FIELDS ? 5 : 0], A2 = ld[r][FIELDS ? 6 : 0], A3 = ld[r][FIELDS ? 7 : 0];
+            if (MIX) {
+                const double sn = sqrt(fma(A3, A3, fma(A2, A2, A1 * A1)));
+                const double rs = 1.0 / sn;
+                split_mixed(k, dd, uu, vv, ww, c, A1, A2, A3, sn, A1 * rs, A2 * rs, A3 * rs, fp, fm);
+            } else {
+                double sn, rs;
+                sqrt_rsqrt_h(fma(A3, A3, fma(A2, A2, A1 * A1)), sn, rs);
+                split_fast(k, dd, uu, vv, ww, c, A1, A2, A3, sn, rs, fp, fm);
+            }
+        } else {
+            const double A1 = k.A[3 * dir], A2 = k.A[3 * dir + 1], A3 = k.A[3 * dir + 2];
+            if (MIX)
+                split_mixed(k, dd, uu, vv, ww, c, A1, A2, A3, k.Anorm[dir], k.Ak[3 * dir], k.Ak[3 * dir + 1],
+                            k.Ak[3 * dir + 2], fp, fm);
+            else
+                split_fast(k, dd, uu, vv, ww, c, A1, A2, A3, k.Anorm[dir], k.Arnorm[dir], fp, fm);
+        }
+#pragma unroll
+        for (int m = 0; m < 5; ++m) {
+            sp[box_pidx(m, p, dir * BOX_LINES + l)] = fp[m];
+            sp[box_pidx(5 + m, p, dir * BOX_LINES + l)] = fm[m];
+        }
+    }
+    __syncthreads();
+
+    // ---- reconstruct: the faces of line tl, variable m ------------------------------------------
+    const int tl = t % BOX_LT, var = t / BOX_LT;
+    double Fv[K];
+    if (var < 5) {
+        const double *qp = sp + box_pidx(var, 0, tl), *qm = sp + box_pidx(5 + var, 0, tl);
+        if (MIX) {
+            double bP[K], bM[K];
+            float cP[K], cM[K];
+            unsigned badP, badM;
+            weno_k_mixed<false, K>([&](int j) { return qp[j * BOX_LT]; }, bP, cP, badP);
+            weno_k_mixed<true, K>([&](int j) { return qm[j * BOX_LT]; }, bM, cM, badM);
+#pragma unroll
+            for (int j = 0; j < K; ++j) Fv[j] = (bP[j] + bM[j]) + (double)(cP[j] + cM[j]);
+            // FP32 weights out of FP32's range: both halves again in FP64 (as in rhs_tile.h)
+            const unsigned bad = badP | badM;
+            if (bad) {
+#pragma unroll 1
+                for (int j = 0; j < K; ++j) {
+                    if (!((bad >> j) & 1u)) continue;
+                    double nP[1], dP[1], cP1[1], nM[1], dM[1], cM1[1];
+                    weno_k<false, 1>([&](int i) { return qp[(i + j) * BOX_LT]; }, nP, dP, cP1);
+                    weno_k<true, 1>([&](int i) { return qm[(i + j) * BOX_LT]; }, nM, dM, cM1);
+                    const double val = fma(fma(nP[0], dM[0], nM[0] * dP[0]), recip_nr(dP[0] * dM[0]), cP1[0] + cM1[0]) / kFace;
+#pragma unroll
+                    for (int q = 0; q < K; ++q)
+                        if (q == j) Fv[q] = val;
+                }
+            }
+        } else {
+            double nP[K], dP[K], nM[K], dM[K], bP[K], bM[K];
+            weno_k<false, K>([&](int j) { return qp[j * BOX_LT]; }, nP, dP, bP);
+            weno_k<true, K>([&](int j) { return qm[j * BOX_LT]; }, nM, dM, bM);
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                const double den = dP[j] * dM[j];
+                Fv[j] = fma(fma(nP[j], dM[j], nM[j] * dP[j]), recip_nr(den), bP[j] + bM[j]);
+            }
+        }
+        // finished here (the compiler would otherwise carry the parts to the store below)
+#pragma unroll
+        for (int j = 0; j < K; ++j) asm volatile("" : "+v"(Fv[j]));
+    }
+    __syncthreads();
+    if (var < 5)
+#pragma unroll
+        for (int j = 0; j < K; ++j) sp[box_fidx(var, tl, j)] = Fv[j];
+    __syncthreads();
+
+    // ---- flux differences of this thread's cell, summed in the order of the directional launches
+    double cmax = 0.0;
+    if (cell) {
+        constexpr double FS = MIX ? 1.0 : kFace;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const int dir = order == WS_ORDER_ZYX ? 2 - q : q;
+            const int i = dir == 0 ? ix : dir == 1 ? iy : iz;
+            const int line = dir * BOX_LINES + (dir == 0 ? iy : ix) + B * (dir == 2 ? iy : iz);
+            const double scale = aj * (-k.rh[dir] / FS);
+#pragma unroll
+            for (int m = 0; m < 5; ++m) {
+                const double val = scale * (sp[box_fidx(m, line, i + 1)] - sp[box_fidx(m, line, i)]);
+                acc[m] = q == 0 && !accumulate ? val : acc_sum(acc[m], val);
+            }
+        }
+        if (STG)
+            cmax = stage_cell(k, sa, x0 + ix, y0 + iy, z0 + iz, ghosted, fnv, fvv, sa.dt_dev ? *sa.dt_dev : sa.dt, acc);
+        const ws_soa &out = STG ? sa.f : du;
+#pragma unroll
+        for (int m = 0; m < 5; ++m) state(out, m) = acc[m];
+    }
+    if (STG && sa.cfl_part) {
+        // the cells are the first wavefront's, so its lanes hold every maximum
+        if (t < 64) {
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) cmax = fmax(cmax, __shfl_xor(cmax, o));
+            if (t == 0) sa.cfl_part[tile] = cmax;
+        }
+    }
+}
+
+dim3 box_grid(const Box &box)
+{
+    return dim3((box.e[0] - box.s[0] + B - 1) / B, (box.e[1] - box.s[1] + B - 1) / B, (box.e[2] - box.s[2] + B - 1) / B);
+}
+
+}  // namespace
+
+bool box_serves(const Ctx &c, const ws_job &job)
+{
+    if (!c.box || c.kp.bnd_any[0] || c.kp.bnd_any[1] || c.kp.bnd_any[2]) return false;
+    const long n = (long)(job.end.x - job.start.x) * (long)(job.end.y - job.start.y) * (long)(job.end.z - job.start.z);
+    // 1200 cells per compute unit, 307 thousand on 256: at 48x48x48 the directional tiles take
+    // 35.1 us (FP64; mixed 37.5) and this kernel 20.8 (21.4), at 100x60x40 51.6 (54.0) and 38.0
+    // (41.1), at 96x96x64, 393 thousand cells, 79.0 (81.8) and 84.7 (94.7): there the tiles
+    // fill the chip, and split 1.27 points per cell and direction where a cube splits 3
+    return n <= 1200l * c.compute_units;
+}
+
+long box_launch_tiles(const ws_job &job)
+{
+    const dim3 g = box_grid(job_box(job));
+    return (long)g.x * g.y * g.z;
+}
+
+void launch_rhs_box(bool mixed, const KParams &k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc,
+                    const ws_metric_fields *m, ws_soa du, const ws_job &job, int order, int accumulate,
+                    const StageArgs *sa, hipStream_t s)
+{
+    const Box box = job_box(job);
+    const dim3 g = box_grid(box);
+    const int n = (int)(g.x * g.y * g.z);
+    if (n <= 0) return;
+    const ws_metric_fields mf = m ? *m : ws_metric_fields{};
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(8 * ((n + 7) / 8)), dim3(BOX_NT), 0, s, k, d, u, v, w, cc, mf, du, box, (int)g.x,
+                           (int)g.y, n, order, accumulate, sa ? *sa : StageArgs{});
+    };
+    if (mixed) {
+        if (sa) go(k_rhs_box<false, true, true>);
+        else if (m) go(k_rhs_box<true, true, false>);
+        else go(k_rhs_box<false, true, false>);
+    } else {
+        if (sa) go(k_rhs_box<false, false, true>);
+        else if (m) go(k_rhs_box<true, false, false>);
+        else go(k_rhs_box<false, false, false>);
+    }
+}
+
+}  // namespace ws

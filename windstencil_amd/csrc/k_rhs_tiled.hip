@@ -18,9 +18,9 @@ int launch_rhs_tiled_stage(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_
 
 long stage_launch_tiles(const Ctx &c)
 {
-    Box box;
-    for (int d = 0; d < 3; ++d) box.s[d] = LAP;
-    box.e[0] = c.kp.nx + LAP; box.e[1] = c.kp.ny + LAP; box.e[2] = c.kp.nz + LAP;
+    const ws_job job = interior_job(&c);
+    if (box_serves(c, job)) return box_launch_tiles(job);
+    const Box box = job_box(job);
     switch (c.stage_shape >= 0 ? c.stage_shape : c.tile_shape) {
     case 0: return stage_tiles_n<0>(box, c.stage_order);
     case 1: return stage_tiles_n<1>(box, c.stage_order);

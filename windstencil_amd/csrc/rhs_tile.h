@@ -33,6 +33,11 @@ struct Box {
     int e[3];   // end
 };
 
+Box job_box(const ws_job &job)
+{
+    return {{(int)job.start.x, (int)job.start.y, (int)job.start.z}, {(int)job.end.x, (int)job.end.y, (int)job.end.z}};
+}
+
 template <int DIR, int L, int W, int K>
 struct Tile {
     static constexpr int NL = L + 2 * LAP;                // points per line
@@ -255,6 +260,66 @@ __device__ __forceinline__ void tile_load(int nyg, const ws_field &d, const ws_f
             }
         }
     }
+}
+
+// The RK3 stage of one cell (ghosted coordinates cx, cy, cz): rv, its complete RHS, becomes
+// the new f (which the caller writes); the primitives and their halo copies go to the fields
+// of sa.  ghosted(field): the cell's element of a ghosted field.  Returns the cell's CFL
+// speed when sa.cfl_part is set, else 0.
+template <typename Ghosted>
+__device__ __forceinline__ double stage_cell(const KParams &k, const StageArgs &sa, int cx, int cy, int cz,
+                                             Ghosted ghosted, const double (&fnv)[5], const double (&fvv)[5],
+                                             double sdt, double (&rv)[5])
+{
+    double speed = 0.0;
+    if (sa.krk == 1) {
+#pragma unroll
+        for (int m = 0; m < 5; ++m) rv[m] = rk3_stage_value<1>(fnv[m], 0.0, rv[m], sdt);
+    } else if (sa.krk == 2) {
+#pragma unroll
+        for (int m = 0; m < 5; ++m) rv[m] = rk3_stage_value<2>(fnv[m], fvv[m], rv[m], sdt);
+    } else {
+#pragma unroll
+        for (int m = 0; m < 5; ++m) rv[m] = rk3_stage_value<3>(fnv[m], fvv[m], rv[m], sdt);
+    }
+    // the new f's primitives for the next stage's RHS (and OCFD_bc on the planes)
+    if (sa.pd.ptr) {
+        const CellPrims p = cell_primitives(rv, k.cv);
+        ghosted(sa.pd) = p.d;
+        ghosted(sa.pu) = p.u;
+        ghosted(sa.pv) = p.v;
+        ghosted(sa.pw) = p.w;
+        ghosted(sa.pT) = p.T;
+        // the stage kernel's expressions for the sound speed, pressure and CFL speed
+        const double c = sqrt(p.T) / k.ama;
+        if (sa.pcc.ptr) ghosted(sa.pcc) = c;
+        if (sa.pP.ptr) ghosted(sa.pP) = p.e / p.d * (k.gamma - 1.0);
+        if (sa.cfl_part) speed = fmax(fabs(p.u) + c, fmax(fabs(p.v) + c, fabs(p.w) + c));
+        const int ix = cx - LAP, iy = cy - LAP, iz = cz - LAP;
+        if (sa.halo) {
+            // the ghost fill's copies of this cell: ghost g < LAP of a direction holds
+            // interior n + g, ghost n + LAP + g holds interior LAP + g (ghosted
+            // coordinates), one direction at a time (faces only); with n < 2 LAP a
+            // cell feeds both sides
+            auto put = [&](int gx, int gy, int gz) {
+                sa.pd.ptr[fidx(sa.pd.pitch, k.nyg, gx, gy, gz)] = p.d;
+                sa.pu.ptr[fidx(sa.pu.pitch, k.nyg, gx, gy, gz)] = p.u;
+                sa.pv.ptr[fidx(sa.pv.pitch, k.nyg, gx, gy, gz)] = p.v;
+                sa.pw.ptr[fidx(sa.pw.pitch, k.nyg, gx, gy, gz)] = p.w;
+                sa.pT.ptr[fidx(sa.pT.pitch, k.nyg, gx, gy, gz)] = p.T;
+                if (sa.pcc.ptr) sa.pcc.ptr[fidx(sa.pcc.pitch, k.nyg, gx, gy, gz)] = c;
+            };
+            if (ix < LAP) put(cx + k.nx, cy, cz);
+            if (ix >= k.nx - LAP) put(cx - k.nx, cy, cz);
+            if (iy < LAP) put(cx, cy + k.ny, cz);
+            if (iy >= k.ny - LAP) put(cx, cy - k.ny, cz);
+            if (iz < LAP) put(cx, cy, cz + k.nz);
+            if (iz >= k.nz - LAP) put(cx, cy, cz - k.nz);
+        }
+        if (sa.planes && (ix == 0 || ix == k.nx - 1 || iy == 0 || iy == k.ny - 1 || iz == 0 || iz == k.nz - 1))
+            plane_conserved(p, k.cv, rv);
+    }
+    return speed;
 }
 
 // Phases 1b-3 of one tile with the block's LDS buffer sp (10 * QS + PAD doubles):
@@ -521,53 +586,7 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
             }
         }
         if (STG) {
-            if (sa.krk == 1) {
-#pragma unroll
-                for (int m = 0; m < 5; ++m) rv[m] = rk3_stage_value<1>(fnv[r][m], 0.0, rv[m], sdt);
-            } else if (sa.krk == 2) {
-#pragma unroll
-                for (int m = 0; m < 5; ++m) rv[m] = rk3_stage_value<2>(fnv[r][m], fvv[r][m], rv[m], sdt);
-            } else {
-#pragma unroll
-                for (int m = 0; m < 5; ++m) rv[m] = rk3_stage_value<3>(fnv[r][m], fvv[r][m], rv[m], sdt);
-            }
-            // the new f's primitives for the next stage's RHS (and OCFD_bc on the planes)
-            if (sa.pd.ptr) {
-                const CellPrims p = cell_primitives(rv, k.cv);
-                ghosted(sa.pd) = p.d;
-                ghosted(sa.pu) = p.u;
-                ghosted(sa.pv) = p.v;
-                ghosted(sa.pw) = p.w;
-                ghosted(sa.pT) = p.T;
-                // the stage kernel's expressions for the sound speed, pressure and CFL speed
-                const double c = sqrt(p.T) / k.ama;
-                if (sa.pcc.ptr) ghosted(sa.pcc) = c;
-                if (sa.pP.ptr) ghosted(sa.pP) = p.e / p.d * (k.gamma - 1.0);
-                if (sa.cfl_part) cfl_max = fmax(cfl_max, fmax(fabs(p.u) + c, fmax(fabs(p.v) + c, fabs(p.w) + c)));
-                const int ix = cx - LAP, iy = cy - LAP, iz = cz - LAP;
-                if (sa.halo) {
-                    // the ghost fill's copies of this cell: ghost g < LAP of a direction holds
-                    // interior n + g, ghost n + LAP + g holds interior LAP + g (ghosted
-                    // coordinates), one direction at a time (faces only); with n < 2 LAP a
-                    // cell feeds both sides
-                    auto put = [&](int gx, int gy, int gz) {
-                        sa.pd.ptr[fidx(sa.pd.pitch, k.nyg, gx, gy, gz)] = p.d;
-                        sa.pu.ptr[fidx(sa.pu.pitch, k.nyg, gx, gy, gz)] = p.u;
-                        sa.pv.ptr[fidx(sa.pv.pitch, k.nyg, gx, gy, gz)] = p.v;
-                        sa.pw.ptr[fidx(sa.pw.pitch, k.nyg, gx, gy, gz)] = p.w;
-                        sa.pT.ptr[fidx(sa.pT.pitch, k.nyg, gx, gy, gz)] = p.T;
-                        if (sa.pcc.ptr) sa.pcc.ptr[fidx(sa.pcc.pitch, k.nyg, gx, gy, gz)] = c;
-                    };
-                    if (ix < LAP) put(cx + k.nx, cy, cz);
-                    if (ix >= k.nx - LAP) put(cx - k.nx, cy, cz);
-                    if (iy < LAP) put(cx, cy + k.ny, cz);
-                    if (iy >= k.ny - LAP) put(cx, cy - k.ny, cz);
-                    if (iz < LAP) put(cx, cy, cz + k.nz);
-                    if (iz >= k.nz - LAP) put(cx, cy, cz - k.nz);
-                }
-                if (sa.planes && (ix == 0 || ix == k.nx - 1 || iy == 0 || iy == k.ny - 1 || iz == 0 || iz == k.nz - 1))
-                    plane_conserved(p, k.cv, rv);
-            }
+            cfl_max = fmax(cfl_max, stage_cell(k, sa, cx, cy, cz, ghosted, fnv[r], fvv[r], sdt, rv));
             const auto fo = lane_off<DIR, BIG>(sa.f.pitch, k.ny, l, i);
             const size_t fstride = (size_t)sa.f.pitch * k.ny * k.nz;
             double *const fbase = cell0(sa.f);
@@ -1000,16 +1019,16 @@ int launch_rhs_tile(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w
                     const ws_metric_fields *m, ws_soa du, ws_job job, int accumulate, hipStream_t s,
                     const StageArgs *sa = nullptr)
 {
-    Box box;
-    box.s[0] = (int)job.start.x; box.s[1] = (int)job.start.y; box.s[2] = (int)job.start.z;
-    box.e[0] = (int)job.end.x; box.e[1] = (int)job.end.y; box.e[2] = (int)job.end.z;
+    const Box box = job_box(job);
     ws_metric_fields mf{};
     const int shape = sa && c.stage_shape >= 0 ? c.stage_shape : c.tile_shape;
     const int order = sa ? c.stage_order : c.dir_order;
     KParams k = c.kp;
     k.same_pitch = same_pitch(d, u, v, w, cc) ? 1 : 0;
     k.big = rel_planes(k, {d, u, v, w, cc}, {du}) && (!m || rel_planes(k, *m)) ? 0 : 1;
-    if (m) {
+    if (!k.big && box_serves(c, job)) {
+        launch_rhs_box(MIX, k, d, u, v, w, cc, m, du, job, order, accumulate, sa, s);
+    } else if (m) {
         mf = *m;
         launch_shape<true, MIX>(shape, k, d, u, v, w, cc, mf, du, box, accumulate, c.schedule, order, nullptr, s);
     } else {

@@ -138,6 +138,9 @@ struct Ctx {
     int stage_order = WS_ORDER_XYZ;
     // tile shape of those stage-applying launches (-1: the context's tile_shape)
     int stage_shape = -1;
+    // jobs small enough may take the one-launch kernel of k_rhs_box.hip (box_serves); off once
+    // the caller chooses a tile shape or schedule, or autotuning finds the tiles faster
+    int box = 1;
     // RK3 steps apply each stage's update in the last RHS launch where they can (1), there
     // also derive the primitives of stages 1 and 2 (2), and within ws_rk3_run those of
     // stage 3 too, alternating the primitive sets from step to step (3)
@@ -164,6 +167,15 @@ struct Ctx {
 };
 
 KParams make_kparams(const ws_config &cfg);
+
+// the interior of the context's grid
+inline ws_job interior_job(const Ctx *c)
+{
+    ws_job j;
+    j.start = {(uint32_t)LAP, (uint32_t)LAP, (uint32_t)LAP};
+    j.end = {(uint32_t)(c->cfg.nx + LAP), (uint32_t)(c->cfg.ny + LAP), (uint32_t)(c->cfg.nz + LAP)};
+    return j;
+}
 
 // One block of a batch, as the batched RHS kernels see it.
 struct BatchBlock {
@@ -249,7 +261,7 @@ int launch_cfl_batch(const AuxBlock *tab, int nb, const double *cfl_part, double
 // (tile shape, schedule, direction order, stage order and shape) the autotuner found best for these
 // extents and precision; false if none
 bool remembered_choice(int nx, int ny, int nz, int precision, int *shape, int *schedule, int *order,
-                       int *stage_order, int *stage_shape);
+                       int *stage_order, int *stage_shape, int *box);
 
 // error reporting (thread-local message)
 int set_error(int code, const std::string &msg);
@@ -262,12 +274,20 @@ int launch_rhs_tiled(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field 
                      const ws_metric_fields *m, ws_soa du, ws_job job, int accumulate, hipStream_t s);
 int launch_rhs_mixed(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc,
                      const ws_metric_fields *m, ws_soa du, ws_job job, int accumulate, hipStream_t s);
-// tiles of the context's launch that applies an RK3 stage (the last direction of its order,
-// in its tile shape): the entries that launch writes to StageArgs::cfl_part
+// The one-launch RHS of small jobs (k_rhs_box.hip): whether it serves a job (otherwise the
+// directional tiles do: a larger job, closures, or turned off).
+bool box_serves(const Ctx &c, const ws_job &job);
+// its work-groups over the job (with a stage, the entries written to StageArgs::cfl_part)
+long box_launch_tiles(const ws_job &job);
+void launch_rhs_box(bool mixed, const KParams &k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc,
+                    const ws_metric_fields *m, ws_soa du, const ws_job &job, int order, int accumulate,
+                    const StageArgs *sa, hipStream_t s);
+// work-groups of the context's launch that applies an RK3 stage (the last direction of its
+// order, in its tile shape, or the one-launch kernel): the entries that launch writes to StageArgs::cfl_part
 long stage_launch_tiles(const Ctx &c);
 // the RHS with the RK3 stage `sa` applied by its last launch (grid schedule; the caller
 // checks that the configuration allows it: tiled kernels, constant metrics, no closures,
-// no viscous terms); du holds partial sums afterwards
+// no viscous terms); du holds partial sums afterwards, or what it held (one-launch kernel)
 int launch_rhs_tiled_stage(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc, ws_soa du,
                            ws_job job, const StageArgs &sa, hipStream_t s);
 int launch_rhs_mixed_stage(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc, ws_soa du,
@@ -286,7 +306,7 @@ int rhs_for_ctx(ws_ctx *c, const ws_state *st, hipStream_t s);
 // RHS, plus the viscous terms when the configuration has them
 int du_from_prepared(ws_ctx *c, const ws_state *st, hipStream_t s);
 // whether RK3 steps can let the last RHS launch apply the stage (stage fusion on, tiled
-// kernels, grid schedule, no closures, no viscous terms, planes the tiles' offsets reach)
+// kernels, grid schedule or one-launch kernel, no closures, no viscous terms, planes the tiles' offsets reach)
 bool fused_stage_ok(const ws_ctx *c, const ws_state *st);
 // How a step of stage fusion 3 treats the primitive sets (rk3_step_fused): STEP_PLAIN starts
 // and ends with the primitives in the state's fields (every level); STEP_FROM_STATE and
