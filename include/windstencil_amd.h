@@ -325,8 +325,8 @@ int ws_ana_state(ws_ctx *ctx, const ws_state *st, const ws_metric_fields *metric
 
 /* ws_ana_state without any device allocation: the partial records live in a fixed device
  * array of the library (513 records, about 37 KB per GPU, held until the process ends), so
- * the call makes no hipMalloc or hipFree (ws_ana_state allocates and frees its records, and
- * the free waits for the device).  The array's size does not depend on the box (the pass is
+ * the call never makes a hipMalloc or hipFree (ws_ana_state has a second such array and
+ * allocates records only for a call that overlaps another on its GPU).  The array's size does not depend on the box (the pass is
  * grid-strided), so no box is too large for it; boxes beyond 2^40 ghosted cells are refused
  * as by ws_ana_state.  Every call on one GPU uses that GPU's array: calls that overlap on
  * one GPU (two host threads, or two streams) race and must be serialised by the caller.

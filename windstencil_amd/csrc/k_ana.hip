@@ -19,6 +19,7 @@ namespace {
 
 constexpr int AT = 256;
 constexpr int ABLOCKS = 512;
+constexpr int AU = 4;           // points in flight per thread
 constexpr long long NONE = 0x7fffffffffffffffLL;
 
 // per-quantity count and first offending ghosted index
@@ -59,25 +60,50 @@ __global__ void __launch_bounds__(AT) k_ana_partial(KParams k, ws_field d, ws_fi
     r.smax = 0.0;
     const int nxg = k.nx + 2 * LAP;
     const long long total = (long long)nxg * k.nyg * k.nzg;
-    for (long long i = (long long)blockIdx.x * AT + threadIdx.x; i < total; i += (long long)gridDim.x * AT) {
-        const int x = (int)(i % nxg), y = (int)((i / nxg) % k.nyg), z = (int)(i / ((long long)nxg * k.nyg));
-        const double tv = T.ptr[fidx(T.pitch, k.nyg, x, y, z)];
-        const double dv = d.ptr[fidx(d.pitch, k.nyg, x, y, z)];
-        const double jv = ajac.ptr ? ajac.ptr[fidx(ajac.pitch, k.nyg, x, y, z)] : k.ajac;
-        const bool bad[4] = {isnan(tv), tv < 0.0, dv < 0.0, jv < 0.0};
+    const long long stride = (long long)gridDim.x * AT;
+    for (long long i0 = (long long)blockIdx.x * AT + threadIdx.x; i0 < total; i0 += AU * stride) {
+        // the loads of AU points go out together; points past the end repeat the last one and
+        // are not counted, and ghost points read the velocities of the nearest interior cell,
+        // which are not used
+        double tv[AU], dv[AU], jv[AU], uv[AU], vv[AU], wv[AU];
+        bool interior[AU];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (bad[q]) {
-                ++r.count[q];
-                r.first[q] = min(r.first[q], i);
+        for (int q = 0; q < AU; ++q) {
+            const long long i = min(i0 + q * stride, total - 1);
+            int x, y, z;
+            if (total <= 0xffffffffLL) {   // a 32-bit division costs a tenth of a 64-bit one
+                const uint32_t row = (uint32_t)i / (uint32_t)nxg;
+                x = (int)((uint32_t)i - row * (uint32_t)nxg);
+                z = (int)(row / (uint32_t)k.nyg);
+                y = (int)(row - (uint32_t)z * (uint32_t)k.nyg);
+            } else {
+                x = (int)(i % nxg); y = (int)((i / nxg) % k.nyg); z = (int)(i / ((long long)nxg * k.nyg));
             }
-        const bool interior = x >= LAP && x < LAP + k.nx && y >= LAP && y < LAP + k.ny && z >= LAP && z < LAP + k.nz;
-        if (interior && tv >= 0.0) {
-            const double c = sqrt(tv) / k.ama;
-            const double a = fmax(fabs(u.ptr[fidx(u.pitch, k.nyg, x, y, z)]),
-                                  fmax(fabs(v.ptr[fidx(v.pitch, k.nyg, x, y, z)]),
-                                       fabs(w.ptr[fidx(w.pitch, k.nyg, x, y, z)])));
-            r.smax = fmax(r.smax, a + c);
+            tv[q] = T.ptr[fidx(T.pitch, k.nyg, x, y, z)];
+            dv[q] = d.ptr[fidx(d.pitch, k.nyg, x, y, z)];
+            jv[q] = ajac.ptr ? ajac.ptr[fidx(ajac.pitch, k.nyg, x, y, z)] : k.ajac;
+            const int cx = min(max(x, LAP), LAP + k.nx - 1), cy = min(max(y, LAP), LAP + k.ny - 1),
+                      cz = min(max(z, LAP), LAP + k.nz - 1);
+            interior[q] = cx == x && cy == y && cz == z;
+            uv[q] = u.ptr[fidx(u.pitch, k.nyg, cx, cy, cz)];
+            vv[q] = v.ptr[fidx(v.pitch, k.nyg, cx, cy, cz)];
+            wv[q] = w.ptr[fidx(w.pitch, k.nyg, cx, cy, cz)];
+        }
+#pragma unroll
+        for (int q = 0; q < AU; ++q) {
+            const long long i = i0 + q * stride;
+            if (i >= total) break;
+            const bool bad[4] = {isnan(tv[q]), tv[q] < 0.0, dv[q] < 0.0, jv[q] < 0.0};
+#pragma unroll
+            for (int n = 0; n < 4; ++n)
+                if (bad[n]) {
+                    ++r.count[n];
+                    r.first[n] = min(r.first[n], i);
+                }
+            if (interior[q] && tv[q] >= 0.0) {
+                const double c = sqrt(tv[q]) / k.ama;
+                r.smax = fmax(r.smax, fmax(fabs(uv[q]), fmax(fabs(vv[q]), fabs(wv[q]))) + c);
+            }
         }
     }
     rec_reduce(r, red);
@@ -104,26 +130,31 @@ __global__ void __launch_bounds__(AT) k_ana_final(const AnaRec *partial, int n, 
 // device (ana_scratch_ptr), never `scratch` itself.
 constexpr int ANA_SCRATCH_RECS = ABLOCKS + 1;
 static __device__ __align__(256) AnaRec scratch[ANA_SCRATCH_RECS];
+// The same for ws_ana_state, one call per device at a time (held under g_ana_busy until the
+// call's last work has ended; a call that finds it taken allocates its own): an allocation
+// and a free on every call cost more than the pass over a middling box.
+static __device__ __align__(256) AnaRec scratch_state[ANA_SCRATCH_RECS];
 
 constexpr int ANA_MAX_DEVICES = 64;
 std::mutex g_ana_mutex;
-AnaRec *g_ana_scratch[ANA_MAX_DEVICES] = {};
+AnaRec *g_ana_scratch[ANA_MAX_DEVICES][2] = {};
+std::mutex g_ana_busy[ANA_MAX_DEVICES];
 
-// The device address of `scratch` on the current device, looked up once per device.
-int ana_scratch_ptr(AnaRec **out)
+// The device address of `scratch` (which 0) or `scratch_state` (which 1) on the current device
+// `dev`, looked up once per device.
+int ana_scratch_ptr(int dev, int which, AnaRec **out)
 {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return hip_error(e, "hipGetDevice");
     if (dev < 0 || dev >= ANA_MAX_DEVICES) return set_error(WS_ERR_UNSUPPORTED, "device index beyond 64");
     std::lock_guard<std::mutex> lock(g_ana_mutex);
-    if (!g_ana_scratch[dev]) {
+    AnaRec *&at = g_ana_scratch[dev][which];
+    if (!at) {
         void *ptr = nullptr;
-        e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
+        hipError_t e = which ? hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch_state))
+                             : hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
         if (e != hipSuccess || !ptr) return hip_error(e, "analysis scratch: hipGetSymbolAddress");
-        g_ana_scratch[dev] = static_cast<AnaRec *>(ptr);
+        at = static_cast<AnaRec *>(ptr);
     }
-    *out = g_ana_scratch[dev];
+    *out = at;
     return WS_OK;
 }
 
@@ -184,7 +215,16 @@ extern "C" int ws_ana_state(ws_ctx *c, const ws_state *st, const ws_metric_field
 {
     int r = ana_check(c, st, metrics, rep);
     if (r) return r;
+    int dev = 0;
     AnaRec *buf = nullptr;
+    if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < ANA_MAX_DEVICES) {
+        std::unique_lock<std::mutex> busy(g_ana_busy[dev], std::try_to_lock);
+        if (busy.owns_lock() && ana_scratch_ptr(dev, 1, &buf) == WS_OK) {
+            r = ana_run(c, st, metrics, dt, rep, s, buf);
+            if (r) (void)hipStreamSynchronize(s);   // nothing of a failed call still writes it
+            return r;
+        }
+    }
     hipError_t e = hipMalloc(&buf, sizeof(AnaRec) * ANA_SCRATCH_RECS);
     if (e != hipSuccess) return hip_error(e, "analysis scratch");
     r = ana_run(c, st, metrics, dt, rep, s, buf);
@@ -198,6 +238,9 @@ extern "C" int ws_ana_state_noalloc(ws_ctx *c, const ws_state *st, const ws_metr
     int r = ana_check(c, st, metrics, rep);
     if (r) return r;
     AnaRec *buf = nullptr;
-    if ((r = ana_scratch_ptr(&buf))) return r;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return hip_error(e, "hipGetDevice");
+    if ((r = ana_scratch_ptr(dev, 0, &buf))) return r;
     return ana_run(c, st, metrics, dt, rep, s, buf);
 }

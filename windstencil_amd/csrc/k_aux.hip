@@ -16,6 +16,23 @@ struct FieldList {
     ws_field f[8];
 };
 
+// Cell i of nx x ny x nz cells, x fastest.  A 64-bit division by a run-time extent costs an
+// order more instructions than a 32-bit one, enough to keep these kernels from the memory's
+// rate, and only a box past 2^32 cells needs it (a uniform branch on `total`, its cells).
+__device__ __forceinline__ void cell_xyz(long i, long total, int nx, int ny, int &x, int &y, int &z)
+{
+    if (total <= 0xffffffffL) {
+        const uint32_t q = (uint32_t)i / (uint32_t)nx;
+        x = (int)((uint32_t)i - q * (uint32_t)nx);
+        z = (int)(q / (uint32_t)ny);
+        y = (int)(q - (uint32_t)z * (uint32_t)ny);
+    } else {
+        x = (int)(i % nx);
+        y = (int)((i / nx) % ny);
+        z = (int)(i / ((long)nx * ny));
+    }
+}
+
 // Periodic LAP-deep face halo of the periodic directions.  Linear index over the face
 // slabs of one field:
 // x slabs (2*LAP*ny*nz), y slabs (2*LAP*nx*nz), z slabs (2*LAP*nx*ny).
@@ -26,25 +43,23 @@ __device__ __forceinline__ void ghost_point(const ws_field &f, int nx, int ny, i
     // slabs of non-periodic directions are left to the caller
     const long nxs = px ? 2L * LAP * ny * nz : 0, nys = py ? 2L * LAP * nx * nz : 0;
     const long nzs = pz ? 2L * LAP * nx * ny : 0;
+    const long total = nxs + nys + nzs;
     int dx, dy, dz, sx, sy, sz;
     if (i < nxs) {
-        const int g = (int)(i % (2 * LAP));            // 0..3 left ghosts, 4..7 right ghosts
-        const int y = (int)((i / (2 * LAP)) % ny);
-        const int z = (int)(i / (2L * LAP * ny));
+        int g, y, z;
+        cell_xyz(i, total, 2 * LAP, ny, g, y, z);      // g: 0..3 left ghosts, 4..7 right ghosts
         dy = sy = y + LAP; dz = sz = z + LAP;
         if (g < LAP) { dx = g;                sx = nx + g; }           // [0,4) <- [nx, nx+4)
         else         { dx = nx + LAP + g - LAP; sx = g; }               // [nx+4, nx+8) <- [4, 8)
     } else if ((i -= nxs) < nys) {
-        const int x = (int)(i % nx);
-        const int g = (int)((i / nx) % (2 * LAP));
-        const int z = (int)(i / (2L * LAP * nx));
+        int x, g, z;
+        cell_xyz(i, total, nx, 2 * LAP, x, g, z);
         dx = sx = x + LAP; dz = sz = z + LAP;
         if (g < LAP) { dy = g;                sy = ny + g; }
         else         { dy = ny + g;           sy = g; }
     } else if ((i -= nys) < nzs) {
-        const int x = (int)(i % nx);
-        const int y = (int)((i / nx) % ny);
-        const int g = (int)(i / ((long)nx * ny));
+        int x, y, g;
+        cell_xyz(i, total, nx, ny, x, y, g);
         dx = sx = x + LAP; dy = sy = y + LAP;
         if (g < LAP) { dz = g;                sz = nz + g; }
         else         { dz = nz + g;           sz = g; }
@@ -67,7 +82,7 @@ __global__ void __launch_bounds__(NT) k_copy_fields(FieldList from, FieldList to
 {
     const long i = (long)blockIdx.x * NT + threadIdx.x;
     if (i >= (long)nxg * rows) return;
-    const long row = i / nxg;
+    const long row = (long)nxg * rows <= 0xffffffffL ? (long)((uint32_t)i / (uint32_t)nxg) : i / nxg;
     const int x = (int)(i - row * nxg);
     const ws_field &a = from.f[blockIdx.y], &b = to.f[blockIdx.y];
     b.ptr[(size_t)x + (size_t)b.pitch * (size_t)row] = a.ptr[(size_t)x + (size_t)a.pitch * (size_t)row];
@@ -80,9 +95,9 @@ __global__ void __launch_bounds__(NT) k_sound_speed(ws_field T, ws_field cc, int
     const long total = (long)nx * ny * nz;
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= total) return;
-    const int x = sx + (int)(i % nx);
-    const int y = sy + (int)((i / nx) % ny);
-    const int z = sz + (int)(i / ((long)nx * ny));
+    int x, y, z;
+    cell_xyz(i, total, nx, ny, x, y, z);
+    x += sx; y += sy; z += sz;
     cc.ptr[fidx(cc.pitch, nyg, x, y, z)] = sqrt(T.ptr[fidx(T.pitch, nyg, x, y, z)]) / ama;
 }
 
@@ -104,9 +119,8 @@ __global__ void __launch_bounds__(NT) k_cons_to_pri(KParams k, ws_soa f, ws_fiel
     const long total = (long)k.nx * k.ny * k.nz;
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= total) return;
-    const int x = (int)(i % k.nx);
-    const int y = (int)((i / k.nx) % k.ny);
-    const int z = (int)(i / ((long)k.nx * k.ny));
+    int x, y, z;
+    cell_xyz(i, total, k.nx, k.ny, x, y, z);
     const double d1 = f.ptr[sidx(f.pitch, k.ny, k.nz, x, y, z, 0)];
     const double u1 = f.ptr[sidx(f.pitch, k.ny, k.nz, x, y, z, 1)] / d1;
     const double v1 = f.ptr[sidx(f.pitch, k.ny, k.nz, x, y, z, 2)] / d1;
@@ -133,9 +147,9 @@ __global__ void __launch_bounds__(NT) k_pri_to_cons(KParams k, ws_soa f, ws_fiel
     const long total = (long)bx * by * bz;
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= total) return;
-    const int x = sx + (int)(i % bx);
-    const int y = sy + (int)((i / bx) % by);
-    const int z = sz + (int)(i / ((long)bx * by));
+    int x, y, z;
+    cell_xyz(i, total, bx, by, x, y, z);
+    x += sx; y += sy; z += sz;
     const int gx = x + LAP, gy = y + LAP, gz = z + LAP;
     const double dd = d.ptr[fidx(d.pitch, k.nyg, gx, gy, gz)];
     const double uu = u.ptr[fidx(u.pitch, k.nyg, gx, gy, gz)];
@@ -158,9 +172,8 @@ __global__ void __launch_bounds__(NT) k_time_advance(KParams k, ws_soa f, ws_soa
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= total) return;
     const double dt = dt_dev ? *dt_dev : dt_val;
-    const int x = (int)(i % k.nx);
-    const int y = (int)((i / k.nx) % k.ny);
-    const int z = (int)(i / ((long)k.nx * k.ny));
+    int x, y, z;
+    cell_xyz(i, total, k.nx, k.ny, x, y, z);
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
         const size_t a = sidx(f.pitch, k.ny, k.nz, x, y, z, m);
@@ -191,9 +204,9 @@ __device__ __forceinline__ double stage_cell(const KParams &k, ws_soa f, ws_soa 
 {
 #pragma clang fp contract(off)
     const double dt = (KRK != 0 && dt_dev) ? *dt_dev : dt_val;
-    const int x = (int)(i % k.nx);
-    const int y = (int)((i / k.nx) % k.ny);
-    const int z = (int)(i / ((long)k.nx * k.ny));
+    const long total = (long)k.nx * k.ny * k.nz;
+    int x, y, z;
+    cell_xyz(i, total, k.nx, k.ny, x, y, z);
     double r[5];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
@@ -275,15 +288,26 @@ __global__ void __launch_bounds__(NT) k_cfl_partial(KParams k, ws_field u, ws_fi
     __shared__ double red[NT];
     const long total = (long)k.nx * k.ny * k.nz;
     double mx = 0.0;
-    for (long i = (long)blockIdx.x * NT + threadIdx.x; i < total; i += (long)gridDim.x * NT) {
-        const int x = (int)(i % k.nx) + LAP;
-        const int y = (int)((i / k.nx) % k.ny) + LAP;
-        const int z = (int)(i / ((long)k.nx * k.ny)) + LAP;
-        const double c = sqrt(T.ptr[fidx(T.pitch, k.nyg, x, y, z)]) / k.ama;
-        const double a = fabs(u.ptr[fidx(u.pitch, k.nyg, x, y, z)]) + c;
-        const double b = fabs(v.ptr[fidx(v.pitch, k.nyg, x, y, z)]) + c;
-        const double e = fabs(w.ptr[fidx(w.pitch, k.nyg, x, y, z)]) + c;
-        mx = fmax(mx, fmax(a, fmax(b, e)));
+    // four cells at a time, all their loads in flight (cells past the end repeat the last one,
+    // which changes no maximum)
+    const long stride = (long)gridDim.x * NT;
+    for (long i0 = (long)blockIdx.x * NT + threadIdx.x; i0 < total; i0 += 4 * stride) {
+        double q4[4][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            int x, y, z;
+            cell_xyz(min(i0 + q * stride, total - 1), total, k.nx, k.ny, x, y, z);
+            x += LAP; y += LAP; z += LAP;
+            q4[q][0] = T.ptr[fidx(T.pitch, k.nyg, x, y, z)];
+            q4[q][1] = u.ptr[fidx(u.pitch, k.nyg, x, y, z)];
+            q4[q][2] = v.ptr[fidx(v.pitch, k.nyg, x, y, z)];
+            q4[q][3] = w.ptr[fidx(w.pitch, k.nyg, x, y, z)];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const double c = sqrt(q4[q][0]) / k.ama;
+            mx = fmax(mx, fmax(fabs(q4[q][1]) + c, fmax(fabs(q4[q][2]) + c, fabs(q4[q][3]) + c)));
+        }
     }
     red[threadIdx.x] = mx;
     __syncthreads();
@@ -358,8 +382,11 @@ __global__ void __launch_bounds__(NT) k_sound_batch(const AuxBlock *tab, int nb,
     const AuxBlock &b = aux_block<false>(tab, nb, wg);
     const int nx = b.n[0], ny = b.n[1];
     const long i = (wg - b.cell_wg0) * NT + threadIdx.x;
-    if (i >= (long)nx * ny * b.n[2]) return;
-    const int x = (int)(i % nx) + LAP, y = (int)((i / nx) % ny) + LAP, z = (int)(i / ((long)nx * ny)) + LAP;
+    const long total = (long)nx * ny * b.n[2];
+    if (i >= total) return;
+    int x, y, z;
+    cell_xyz(i, total, nx, ny, x, y, z);
+    x += LAP; y += LAP; z += LAP;
     const ws_field &T = b.g[0][4], &cc = b.g[0][5];
     cc.ptr[fidx(cc.pitch, b.nyg, x, y, z)] = sqrt(T.ptr[fidx(T.pitch, b.nyg, x, y, z)]) / ama;
 }
