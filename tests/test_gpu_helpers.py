@@ -1,0 +1,75 @@
+"""The memory-bound kernels around the RHS at the edges of their index arithmetic."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import windstencil_amd as W
+from tests.gpu_util import make_ctx, upload_state
+from tests.helpers import random_state
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("periodic", [(1, 1, 1), (0, 1, 1), (1, 0, 0), (0, 0, 0)])
+@pytest.mark.parametrize("shape", [(4, 4, 4), (9, 6, 5), (70, 65, 66)])
+def test_rhs_inputs_in_one_launch(ws, shape, periodic):
+    """ws_du_comput's inputs (one launch, one point per thread up to 2^18 ghosted points, two
+    above) against a ghost fill and a pass over T: every point of the ghosted box bit for bit,
+    the caller's ghost layers and corners included, with a sound speed of another pitch."""
+    import torch
+    nx, ny, nz = shape
+    L, sh = W.lib(), W.stream_handle()
+    ctx = make_ctx(nx, ny, nz, periodic=periodic)
+    states = []
+    for _ in range(2):
+        st = upload_state(random_state(nx, ny, nz, 3, "blobs"))
+        st.t["cc"] = W.ghosted_tensor(nx, ny, nz, pad=3)
+        st.refresh()
+        gen = torch.Generator(device="cuda").manual_seed(7)
+        for k in ("d", "u", "v", "w", "T"):
+            inner = st.interior(k).clone()
+            st.t[k].copy_(1.0 + 0.2 * torch.rand(st.t[k].shape, dtype=torch.float64, device="cuda", generator=gen))
+            st.interior(k).copy_(inner)
+        states.append(st)
+    a, b = states
+    W.check(L.ws_du_comput(ctx.handle, ctypes.byref(a.ws), None, sh))
+    fl = (W.WsField * 5)(b.ws.d, b.ws.u, b.ws.v, b.ws.w, b.ws.T)
+    W.check(L.ws_ghost_fill_periodic(ctx.handle, fl, 5, sh))
+    W.check(L.ws_sound_speed(ctx.handle, b.ws.T, b.ws.cc, W.job((0, 0, 0), (nx + 8, ny + 8, nz + 8)), sh))
+    for k in ("d", "u", "v", "w", "T", "cc"):
+        assert torch.equal(a.t[k][..., :nx + 8], b.t[k][..., :nx + 8]), k
+
+
+@pytest.mark.parametrize("shape", [(4, 4, 4), (33, 17, 9), (129, 127, 131)])
+def test_reductions_over_ragged_boxes(ws, shape):
+    """The CFL step and the state analysis take four points per thread and round: the largest
+    speed and each bad cell count wherever they lie, the last cell and the ends of a round
+    included, and points past the end are not counted twice."""
+    import torch
+    nx, ny, nz = shape
+    L, sh = W.lib(), W.stream_handle()
+    ctx = make_ctx(nx, ny, nz)
+    dt = torch.zeros(1, dtype=torch.float64, device="cuda")
+    hmin = min(ctx.cfg.hx, ctx.cfg.hy, ctx.cfg.hz)
+    n = nx * ny * nz
+    for at in sorted({0, n - 1, n // 2, min(n - 1, 4 * 1024 * 256), min(n - 1, 1024 * 256 - 1)}):
+        st = upload_state(random_state(nx, ny, nz, 3, "blobs"))
+        z, y, x = np.unravel_index(at, (nz, ny, nx))
+        st.interior("v")[z, y, x] = -50.0
+        W.check(L.ws_cfl_dt(ctx.handle, ctypes.byref(st.ws), 0.5, dt.data_ptr(), sh))
+        c = np.sqrt(st.interior("T")[z, y, x].item()) / ctx.cfg.ama
+        want = 0.5 * hmin / (50.0 + c)
+        assert abs(dt.item() - want) <= 4 * np.finfo(float).eps * want
+        for k in ("d", "u", "v", "w", "T"):
+            full = st.t[k]
+            inner = st.interior(k).clone()
+            full.fill_(1.0)
+            st.interior(k).copy_(inner)
+        st.interior("T")[z, y, x] = float("nan")
+        st.t["d"][-1, -1, nx + 7] = -1.0      # the last ghosted point
+        rep = W.WsAnaReport()
+        W.check(L.ws_ana_state(ctx.handle, ctypes.byref(st.ws), None, 0.1, ctypes.byref(rep), sh))
+        assert (rep.nan_T, rep.neg_T, rep.neg_d, rep.neg_jac) == (1, 0, 1, 0)
+        assert tuple(rep.first_nan_T) == (x, y, z)
+        assert tuple(rep.first_neg_d) == (nx + 3, ny + 3, nz + 3)

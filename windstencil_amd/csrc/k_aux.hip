@@ -37,43 +37,107 @@ __device__ __forceinline__ void cell_xyz(long i, long total, int nx, int ny, int
 // slabs of one field:
 // x slabs (2*LAP*ny*nz), y slabs (2*LAP*nx*nz), z slabs (2*LAP*nx*ny).
 // Ghost points read only interior points, so the three directions need no ordering.
-__device__ __forceinline__ void ghost_point(const ws_field &f, int nx, int ny, int nz, int nyg, bool px, bool py,
-                                            bool pz, long i)
+// The ghost point dst of index i and the interior point src it copies; false: none.
+struct GhostPoint {
+    int dx, dy, dz, sx, sy, sz;
+};
+
+__device__ __forceinline__ bool ghost_point(int nx, int ny, int nz, bool px, bool py, bool pz, long i, GhostPoint &q)
 {
     // slabs of non-periodic directions are left to the caller
     const long nxs = px ? 2L * LAP * ny * nz : 0, nys = py ? 2L * LAP * nx * nz : 0;
     const long nzs = pz ? 2L * LAP * nx * ny : 0;
     const long total = nxs + nys + nzs;
-    int dx, dy, dz, sx, sy, sz;
     if (i < nxs) {
         int g, y, z;
         cell_xyz(i, total, 2 * LAP, ny, g, y, z);      // g: 0..3 left ghosts, 4..7 right ghosts
-        dy = sy = y + LAP; dz = sz = z + LAP;
-        if (g < LAP) { dx = g;                sx = nx + g; }           // [0,4) <- [nx, nx+4)
-        else         { dx = nx + LAP + g - LAP; sx = g; }               // [nx+4, nx+8) <- [4, 8)
+        q.dy = q.sy = y + LAP; q.dz = q.sz = z + LAP;
+        if (g < LAP) { q.dx = g;                q.sx = nx + g; }           // [0,4) <- [nx, nx+4)
+        else         { q.dx = nx + LAP + g - LAP; q.sx = g; }               // [nx+4, nx+8) <- [4, 8)
     } else if ((i -= nxs) < nys) {
         int x, g, z;
         cell_xyz(i, total, nx, 2 * LAP, x, g, z);
-        dx = sx = x + LAP; dz = sz = z + LAP;
-        if (g < LAP) { dy = g;                sy = ny + g; }
-        else         { dy = ny + g;           sy = g; }
+        q.dx = q.sx = x + LAP; q.dz = q.sz = z + LAP;
+        if (g < LAP) { q.dy = g;                q.sy = ny + g; }
+        else         { q.dy = ny + g;           q.sy = g; }
     } else if ((i -= nys) < nzs) {
         int x, y, g;
         cell_xyz(i, total, nx, ny, x, y, g);
-        dx = sx = x + LAP; dy = sy = y + LAP;
-        if (g < LAP) { dz = g;                sz = nz + g; }
-        else         { dz = nz + g;           sz = g; }
+        q.dx = q.sx = x + LAP; q.dy = q.sy = y + LAP;
+        if (g < LAP) { q.dz = g;                q.sz = nz + g; }
+        else         { q.dz = nz + g;           q.sz = g; }
     } else {
-        return;
+        return false;
     }
-    f.ptr[fidx(f.pitch, nyg, dx, dy, dz)] = f.ptr[fidx(f.pitch, nyg, sx, sy, sz)];
+    return true;
 }
 
-__global__ void __launch_bounds__(NT) k_ghost_fill(FieldList fl, int nx, int ny, int nz, int nyg, int px, int py,
+// The ghost point of n fields (at most NF): every field's load goes out before the first store.
+template <int NF>
+__device__ __forceinline__ void ghost_copy(const ws_field *f, int n, int nyg, const GhostPoint &q, double (&val)[NF])
+{
+#pragma unroll
+    for (int j = 0; j < NF; ++j)
+        if (j < n) val[j] = f[j].ptr[fidx(f[j].pitch, nyg, q.sx, q.sy, q.sz)];
+#pragma unroll
+    for (int j = 0; j < NF; ++j)
+        if (j < n) f[j].ptr[fidx(f[j].pitch, nyg, q.dx, q.dy, q.dz)] = val[j];
+}
+
+__global__ void __launch_bounds__(NT) k_ghost_fill(FieldList fl, int n, int nx, int ny, int nz, int nyg, int px, int py,
                                                    int pz)
 {
-    ghost_point(fl.f[blockIdx.y], nx, ny, nz, nyg, px != 0, py != 0, pz != 0,
-                (long)blockIdx.x * blockDim.x + threadIdx.x);
+    GhostPoint q;
+    double val[8];
+    if (ghost_point(nx, ny, nz, px != 0, py != 0, pz != 0, (long)blockIdx.x * NT + threadIdx.x, q))
+        ghost_copy<8>(fl.f, n, nyg, q, val);
+}
+
+// The RHS's inputs from the interior primitives, PER points of the ghosted box per thread:
+// beside a periodic face the ghost point of d, u, v, w and T (as k_ghost_fill), and
+// everywhere the sound speed of the T that the point then holds (as k_sound_speed).  Writes no
+// point it reads, so one launch does what a ghost fill and a pass over T did.
+// Bound by memory and, on a small grid, by its launch; against the two launches: 64x32x16 5.3 ->
+// 3.9 us, 157x111x75 8.5 -> 5.5, 600x256x128 105 -> 97.  Two points per thread keep more loads
+// in flight on a large box (600x256x128: one point 116 us, four 101); a box of up to 2^18
+// points spreads wider with one (64x32x16: two points 4.4 us).
+template <int PER>
+__global__ void __launch_bounds__(NT) k_prepare(FieldList fl, ws_field cc, int nx, int ny, int nz, int px, int py,
+                                                int pz, double ama)
+{
+#pragma clang fp contract(off)
+    const int nxg = nx + 2 * LAP, nyg = ny + 2 * LAP;
+    const long total = (long)nxg * nyg * (nz + 2 * LAP);
+    const long i0 = (long)blockIdx.x * (PER * NT) + threadIdx.x;
+    const ws_field &fT = fl.f[4];
+    GhostPoint q[PER];
+    bool ghost[PER];
+    double T[PER];
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+        // past the end: the last point again, not written
+        GhostPoint &p = q[r];
+        cell_xyz(min(i0 + r * NT, total - 1), total, nxg, nyg, p.dx, p.dy, p.dz);
+        const bool ox = p.dx < LAP || p.dx >= nx + LAP, oy = p.dy < LAP || p.dy >= ny + LAP,
+                   oz = p.dz < LAP || p.dz >= nz + LAP;
+        ghost[r] = ox + oy + oz == 1 && (ox ? px : oy ? py : pz);
+        // ghost g < LAP holds interior n + g, ghost n + LAP + g holds interior LAP + g
+        p.sx = p.dx + (!ghost[r] || !ox ? 0 : p.dx < LAP ? nx : -nx);
+        p.sy = p.dy + (!ghost[r] || !oy ? 0 : p.dy < LAP ? ny : -ny);
+        p.sz = p.dz + (!ghost[r] || !oz ? 0 : p.dz < LAP ? nz : -nz);
+        T[r] = fT.ptr[fidx(fT.pitch, nyg, p.sx, p.sy, p.sz)];
+    }
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+        if (i0 + r * NT >= total) break;
+        const GhostPoint &p = q[r];
+        if (ghost[r]) {
+            double val[4];
+            ghost_copy<4>(fl.f, 4, nyg, p, val);
+            fT.ptr[fidx(fT.pitch, nyg, p.dx, p.dy, p.dz)] = T[r];
+        }
+        cc.ptr[fidx(cc.pitch, nyg, p.dx, p.dy, p.dz)] = sqrt(T[r]) / ama;
+    }
 }
 
 // to = from over a ghosted box of nxg x rows points (rows = nyg * nzg), one field per
@@ -99,17 +163,6 @@ __global__ void __launch_bounds__(NT) k_sound_speed(ws_field T, ws_field cc, int
     cell_xyz(i, total, nx, ny, x, y, z);
     x += sx; y += sy; z += sz;
     cc.ptr[fidx(cc.pitch, nyg, x, y, z)] = sqrt(T.ptr[fidx(T.pitch, nyg, x, y, z)]) / ama;
-}
-
-// Sound speed over a whole ghosted field treated as one flat array (pitch padding
-// included, which no kernel reads): cc = sqrt(T)/Ma, two points per thread.
-__global__ void __launch_bounds__(NT) k_sound_flat(const double2 *T, double2 *cc, long n2, double ama)
-{
-#pragma clang fp contract(off)
-    const long i = (long)blockIdx.x * NT + threadIdx.x;
-    if (i >= n2) return;
-    const double2 t = T[i];
-    cc[i] = make_double2(sqrt(t.x) / ama, sqrt(t.y) / ama);
 }
 
 __global__ void __launch_bounds__(NT) k_cons_to_pri(KParams k, ws_soa f, ws_field d, ws_field u, ws_field v,
@@ -370,14 +423,28 @@ __global__ void __launch_bounds__(NT) k_ghost_fill_batch(const AuxBlock *tab, in
 {
     const long wg = blockIdx.x;
     const AuxBlock &b = aux_block<true>(tab, nb, wg);
-    ghost_point(b.g[set][blockIdx.y], b.n[0], b.n[1], b.n[2], b.nyg, true, true, true,
-                (wg - b.ghost_wg0) * NT + threadIdx.x);
+    GhostPoint q;
+    double val[6];
+    if (ghost_point(b.n[0], b.n[1], b.n[2], true, true, true, (wg - b.ghost_wg0) * NT + threadIdx.x, q))
+        ghost_copy<6>(b.g[set], 6, b.nyg, q, val);
 }
 
-// the sound speed of every block's interior (k_sound_flat's expression)
-__global__ void __launch_bounds__(NT) k_sound_batch(const AuxBlock *tab, int nb, double ama)
+// The sound speed of every block's interior (k_sound_speed's expression) by the first
+// cell_wgs work-groups, and by the others the ghost points of d, u, v, w, T and of the sound
+// speed, which is that of the interior T copied (what a fill after the first part would copy).
+__global__ void __launch_bounds__(NT) k_prepare_batch(const AuxBlock *tab, int nb, long cell_wgs, double ama)
 {
 #pragma clang fp contract(off)
+    if (blockIdx.x >= cell_wgs) {
+        const long wg = blockIdx.x - cell_wgs;
+        const AuxBlock &b = aux_block<true>(tab, nb, wg);
+        GhostPoint q;
+        double val[5];
+        if (!ghost_point(b.n[0], b.n[1], b.n[2], true, true, true, (wg - b.ghost_wg0) * NT + threadIdx.x, q)) return;
+        ghost_copy<5>(b.g[0], 5, b.nyg, q, val);
+        b.g[0][5].ptr[fidx(b.g[0][5].pitch, b.nyg, q.dx, q.dy, q.dz)] = sqrt(val[4]) / ama;
+        return;
+    }
     const long wg = blockIdx.x;
     const AuxBlock &b = aux_block<false>(tab, nb, wg);
     const int nx = b.n[0], ny = b.n[1];
@@ -447,8 +514,8 @@ int launch_ghost_fill(const Ctx &c, const ws_field *f, int n, hipStream_t s)
         FieldList fl{};
         const int cnt = n - base < 8 ? n - base : 8;
         for (int i = 0; i < cnt; ++i) fl.f[i] = f[base + i];
-        hipLaunchKernelGGL(k_ghost_fill, dim3(blocks_for(per), cnt), dim3(NT), 0, s, fl, k.nx, k.ny, k.nz, k.nyg,
-                           px, py, pz);
+        hipLaunchKernelGGL(k_ghost_fill, dim3(blocks_for(per)), dim3(NT), 0, s, fl, cnt, k.nx, k.ny, k.nz, k.nyg, px, py,
+                           pz);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? WS_OK : hip_error(e, "ghost fill launch");
@@ -476,18 +543,16 @@ int launch_prepare(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w,
                    hipStream_t s)
 {
     const KParams &k = c.kp;
-    const ws_field g[5] = {d, u, v, w, T};
-    int r = launch_ghost_fill(c, g, 5, s);
-    if (r) return r;
-    const ws_job box{{0, 0, 0}, {(uint32_t)(k.nx + 2 * LAP), (uint32_t)(k.ny + 2 * LAP), (uint32_t)(k.nz + 2 * LAP)}};
-    const long n = (long)T.pitch * (k.ny + 2 * LAP) * (k.nz + 2 * LAP);
-    // the flat form needs one layout and 16-byte alignment; otherwise the box kernel
-    if (T.pitch != cc.pitch || n % 2 || ((uintptr_t)T.ptr | (uintptr_t)cc.ptr) % 16)
-        return launch_sound_speed(c, T, cc, box, s);
-    hipLaunchKernelGGL(k_sound_flat, dim3(blocks_for(n / 2)), dim3(NT), 0, s, (const double2 *)T.ptr,
-                       (double2 *)cc.ptr, n / 2, k.ama);
+    const FieldList fl{{d, u, v, w, T}};
+    const long n = (long)(k.nx + 2 * LAP) * k.nyg * k.nzg;
+    auto go = [&](auto kern, int per) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)((n + per * NT - 1) / (per * NT))), dim3(NT), 0, s, fl, cc, k.nx, k.ny,
+                           k.nz, c.cfg.periodic[0], c.cfg.periodic[1], c.cfg.periodic[2], k.ama);
+    };
+    if (n <= 1l << 18) go(k_prepare<1>, 1);
+    else go(k_prepare<2>, 2);
     hipError_t e = hipGetLastError();
-    return e == hipSuccess ? WS_OK : hip_error(e, "sound speed launch");
+    return e == hipSuccess ? WS_OK : hip_error(e, "RHS input launch");
 }
 
 int launch_sound_speed(const Ctx &c, ws_field T, ws_field cc, ws_job job, hipStream_t s)
@@ -623,7 +688,7 @@ int launch_ghost_fill_batch(const AuxBlock *tab, int nb, long ghost_wgs, int set
 {
     if (set < 0 || set > 1) return set_error(WS_ERR_INVALID, "field set must be 0 or 1");
     if (ghost_wgs <= 0 || nb <= 0) return WS_OK;
-    hipLaunchKernelGGL(k_ghost_fill_batch, dim3((unsigned)ghost_wgs, 6), dim3(NT), 0, s, tab, nb, set);
+    hipLaunchKernelGGL(k_ghost_fill_batch, dim3((unsigned)ghost_wgs), dim3(NT), 0, s, tab, nb, set);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? WS_OK : hip_error(e, "batched ghost fill launch");
 }
@@ -632,10 +697,9 @@ int launch_prepare_batch(const KParams &k, const AuxBlock *tab, int nb, long gho
                          hipStream_t s)
 {
     if (nb <= 0 || cell_wgs <= 0) return WS_OK;
-    hipLaunchKernelGGL(k_sound_batch, dim3((unsigned)cell_wgs), dim3(NT), 0, s, tab, nb, k.ama);
+    hipLaunchKernelGGL(k_prepare_batch, dim3((unsigned)(cell_wgs + ghost_wgs)), dim3(NT), 0, s, tab, nb, cell_wgs, k.ama);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return hip_error(e, "batched sound speed launch");
-    return launch_ghost_fill_batch(tab, nb, ghost_wgs, 0, s);
+    return e == hipSuccess ? WS_OK : hip_error(e, "batched RHS input launch");
 }
 
 int launch_stage_batch(const KParams &k, const AuxBlock *tab, int nb, long cell_wgs, int swapped, bool planes,
