@@ -357,8 +357,9 @@ int ws_viscous_rhs(ws_ctx *ctx, ws_field u, ws_field v, ws_field w, ws_field T, 
 int ws_rk3_step(ws_ctx *ctx, ws_state *st, const double *dt_dev, hipStream_t stream);
 
 /* nsteps RK3 steps.  cfl > 0: dt recomputed on the device at the start of every step
- * with ws_cfl_dt; cfl <= 0: cfg.dt.  use_graph = 1 captures one step in a hipGraph
- * and replays it.  Synchronises the stream before returning.  After the first step the
+ * with ws_cfl_dt; cfl <= 0: cfg.dt.  use_graph = 1 captures two steps in a hipGraph
+ * and replays it for each pair of steps after the first (with at least two pairs; the
+ * other steps run eagerly).  Synchronises the stream before returning.  After the first step the
  * CFL maxima come from the stage kernel that ends the previous step (same dt bits as a
  * ws_cfl_dt pass; the context keeps one double per 256 cells for them). */
 int ws_rk3_run(ws_ctx *ctx, ws_state *st, int32_t nsteps, double cfl, int32_t use_graph,
@@ -468,7 +469,7 @@ int ws_batch_cfl_dt(ws_batch *batch, double cfl, double *dt_dev, hipStream_t str
 /* One SSP-RK3 step of every block (as ws_rk3_step). */
 int ws_batch_rk3_step(ws_batch *batch, const double *dt_dev, hipStream_t stream);
 /* nsteps batch RK3 steps, dt from the CFL reduction (cfl > 0) or cfg.dt; use_graph = 1
- * captures a whole step (CFL included) in one hipGraph and replays it. */
+ * captures two whole steps (CFL included) in one hipGraph and replays it as ws_rk3_run does. */
 int ws_batch_rk3_run(ws_batch *batch, int32_t nsteps, double cfl, int32_t use_graph, hipStream_t stream);
 /* Time every (tile shape, schedule) pair of the batched RHS and keep the fastest (as
  * ws_autotune); with the grid schedule and stage fusion on, then the stage shape and order, timed on

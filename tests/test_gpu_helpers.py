@@ -73,3 +73,31 @@ def test_reductions_over_ragged_boxes(ws, shape):
         assert (rep.nan_T, rep.neg_T, rep.neg_d, rep.neg_jac) == (1, 0, 1, 0)
         assert tuple(rep.first_nan_T) == (x, y, z)
         assert tuple(rep.first_neg_d) == (nx + 3, ny + 3, nz + 3)
+
+
+@pytest.mark.parametrize("viscous", [0, 6])
+@pytest.mark.parametrize("steps", [1, 2, 4, 5, 6, 8])
+def test_runs_replaying_pairs_of_steps(ws, steps, viscous):
+    """ws_rk3_run and ws_batch_rk3_run replay a graph of two steps where there are at least two
+    pairs after the first step: any number of steps gives the eager run bit for bit."""
+    n = (20, 13, 11)
+    L, sh = W.lib(), W.stream_handle()
+    got = []
+    for graph in (0, 1):
+        out = []
+        for batch in (False, True):
+            st = upload_state(random_state(*n, 3, "blobs"))
+            ctx = make_ctx(*n, viscous=viscous)
+            W.check(L.ws_pri_to_cons(ctx.handle, st.ws.f, st.ws.d, st.ws.u, st.ws.v, st.ws.w, st.ws.T,
+                                     W.job((0, 0, 0), n), sh))
+            if batch:
+                b = W.Batch(W.default_config(8, 8, 8, viscous=viscous), [n], [st])
+                W.check(L.ws_batch_rk3_run(b.handle, steps, 0.5, graph, sh))
+                b.sync_states()
+            else:
+                W.check(L.ws_rk3_run(ctx.handle, ctypes.byref(st.ws), steps, 0.5, graph, sh))
+                st.sync_from_ws()
+            out += [st.interior(k).cpu().numpy().copy() for k in ("f", "d", "u", "v", "w", "T")]
+        got.append(out)
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)

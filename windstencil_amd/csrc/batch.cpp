@@ -461,6 +461,13 @@ int ws_batch_du_comput(ws_batch *b, hipStream_t s)
 int ws_batch_cfl_dt(ws_batch *b, double cfl, double *dt_dev, hipStream_t s)
 {
     if (!b || !dt_dev || !(cfl > 0.0)) return set_error(WS_ERR_INVALID, "bad CFL request");
+    const int nb = (int)b->ctx.size();
+    if (aux_table(b, s)) {
+        // three launches for all blocks: with two per block, which each of twelve blocks of 24 to
+        // 112 cells a side is too small for, a run of three steps took 80 us longer (of 5.9 ms)
+        int r = launch_cfl_partial_batch(b->ctx[0]->kp, b->d_aux, nb, b->cell_wgs, b->d_cfl_part, s);
+        return r ? r : launch_cfl_batch(b->d_aux, nb, b->d_cfl_part, cfl, b->d_dts, dt_dev, s);
+    }
     for (size_t i = 0; i < b->ctx.size(); ++i) {
         int r = launch_cfl(*b->ctx[i], b->st[i], cfl, b->d_dts + i, s);
         if (r) return r;
@@ -649,41 +656,40 @@ int ws_batch_rk3_run(ws_batch *b, int32_t nsteps, double cfl, int32_t use_graph,
     if (!use_graph) {
         for (int n = 0; n < nsteps && !r; ++n) r = step(n, s);
     } else {
-        // one captured graph per parity of the f/fn swap (a step ends with them exchanged,
-        // and, alternating, with the primitives in the other set); step 0 runs eagerly, and
-        // so does an alternating run's last step, which ends differently
-        hipGraphExec_t exec[2] = {nullptr, nullptr};
+        // one captured graph of two steps, after which f and fn (and, alternating, the primitive
+        // sets) have their old roles again, for every pair after step 0, as in ws_rk3_run; the
+        // steps outside a pair, and all of them with no second pair, run eagerly
         const int replayed = alt ? nsteps - 1 : nsteps;
-        for (int n = 0; n < replayed && !r; ++n) {
-            if (n == 0) {
-                r = step(0, s);
+        const int pairs = (replayed - 1) / 2;
+        hipGraphExec_t exec = nullptr;
+        for (int n = 0; n < nsteps && !r;) {
+            if (n == 0 || pairs < 2 || n > 2 * pairs) {
+                r = step(n++, s);
                 continue;
             }
-            const int p = n & 1;
-            if (!exec[p]) {
+            if (!exec) {
                 const std::vector<ws_state> saved = b->st;
                 hipGraph_t g = nullptr;
                 hipError_t e = hipStreamBeginCapture(b->capture_stream, hipStreamCaptureModeThreadLocal);
                 if (e != hipSuccess) { r = hip_error(e, "begin capture"); break; }
                 r = step(n, b->capture_stream);
+                if (!r) r = step(n + 1, b->capture_stream);
                 e = hipStreamEndCapture(b->capture_stream, &g);
-                b->st = saved;   // capture recorded the step; the swap happens at replay
+                b->st = saved;   // capture recorded the steps; nothing ran yet
                 if (r) { if (g) hipGraphDestroy(g); break; }
                 if (e != hipSuccess) { r = hip_error(e, "end capture"); break; }
-                e = hipGraphInstantiate(&exec[p], g, nullptr, nullptr, 0);
+                e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
                 hipGraphDestroy(g);
                 if (e != hipSuccess) { r = hip_error(e, "graph instantiate"); break; }
             }
-            hipError_t e = hipGraphLaunch(exec[p], s);
+            hipError_t e = hipGraphLaunch(exec, s);
             if (e != hipSuccess) { r = hip_error(e, "graph launch"); break; }
-            for (ws_state &st : b->st) std::swap(st.f, st.fn);
+            n += 2;
         }
-        if (!r && alt) r = step(nsteps - 1, s);
-        for (int p = 0; p < 2; ++p)
-            if (exec[p]) {
-                hipStreamSynchronize(s);
-                hipGraphExecDestroy(exec[p]);
-            }
+        if (exec) {
+            hipStreamSynchronize(s);
+            hipGraphExecDestroy(exec);
+        }
     }
     hipError_t e = hipStreamSynchronize(s);
     if (!r && e != hipSuccess) r = hip_error(e, "batch RK3 run");

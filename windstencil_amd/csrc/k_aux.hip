@@ -479,6 +479,23 @@ __global__ void __launch_bounds__(NT) k_stage_batch(KParams k, const AuxBlock *t
     if (CFLP) wg_max(mx, cfl_part + wg);
 }
 
+// k_cfl_partial's maxima of every block, one per work-group of the cell grid
+__global__ void __launch_bounds__(NT) k_cfl_partial_batch(const AuxBlock *tab, int nb, double ama, double *cfl_part)
+{
+    const long wg = blockIdx.x;
+    const AuxBlock &b = aux_block<false>(tab, nb, wg);
+    const long total = (long)b.n[0] * b.n[1] * b.n[2];
+    // past the end: the last cell again, which changes no maximum
+    const long i = min((wg - b.cell_wg0) * NT + threadIdx.x, total - 1);
+    int x, y, z;
+    cell_xyz(i, total, b.n[0], b.n[1], x, y, z);
+    x += LAP; y += LAP; z += LAP;
+    auto at = [&](const ws_field &f) { return f.ptr[fidx(f.pitch, b.nyg, x, y, z)]; };
+    const double T = at(b.g[0][4]), u = at(b.g[0][1]), v = at(b.g[0][2]), w = at(b.g[0][3]);
+    const double c = sqrt(T) / ama;
+    wg_max(fmax(0.0, fmax(fabs(u) + c, fmax(fabs(v) + c, fabs(w) + c))), cfl_part + wg);
+}
+
 // one work-group per block: k_cfl_final over the block's partials
 __global__ void __launch_bounds__(NT) k_cfl_final_batch(const AuxBlock *tab, const double *part, double cfl,
                                                         double *dts, const int2 *ranges)
@@ -652,11 +669,6 @@ int launch_fill(double value, double *ptr, uint32_t pitch, uint32_t sx, uint32_t
 int launch_cfl(Ctx &c, const ws_state &st, double cfl, double *dt_dev, hipStream_t s)
 {
     const KParams &k = c.kp;
-    if (!c.cfl_partial) {
-        c.cfl_blocks = 1024;
-        hipError_t e = hipMalloc(&c.cfl_partial, sizeof(double) * c.cfl_blocks);
-        if (e != hipSuccess) return hip_error(e, "cfl scratch allocation");
-    }
     const double hmin = fmin(k.h[0], fmin(k.h[1], k.h[2]));
     hipLaunchKernelGGL(k_cfl_partial, dim3(c.cfl_blocks), dim3(NT), 0, s, k, st.u, st.v, st.w, st.T, c.cfl_partial);
     hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(NT), 0, s, (const double *)c.cfl_partial, c.cfl_blocks, cfl, hmin,
@@ -721,6 +733,14 @@ int launch_stage_batch(const KParams &k, const AuxBlock *tab, int nb, long cell_
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? WS_OK : hip_error(e, "batched stage launch");
+}
+
+int launch_cfl_partial_batch(const KParams &k, const AuxBlock *tab, int nb, long cell_wgs, double *cfl_part, hipStream_t s)
+{
+    if (nb <= 0 || cell_wgs <= 0) return WS_OK;
+    hipLaunchKernelGGL(k_cfl_partial_batch, dim3((unsigned)cell_wgs), dim3(NT), 0, s, tab, nb, k.ama, cfl_part);
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? WS_OK : hip_error(e, "batched cfl launch");
 }
 
 int launch_cfl_batch(const AuxBlock *tab, int nb, const double *cfl_part, double cfl, double *dts, double *dt_dev,

@@ -121,7 +121,7 @@ struct Ctx {
     KParams kp;
     int device;
     int compute_units = 256;
-    // CFL scratch: per-block maxima
+    // CFL scratch: per-block maxima, and behind them the dt of a ws_rk3_run
     double *cfl_partial = nullptr;
     int cfl_blocks = 0;
     // private stream for graph capture (the caller's stream may be the legacy
@@ -252,6 +252,8 @@ int launch_prepare_batch(const KParams &k, const AuxBlock *tab, int nb, long gho
 // CFL maximum of each work-group.
 int launch_stage_batch(const KParams &k, const AuxBlock *tab, int nb, long cell_wgs, int swapped, bool planes,
                        bool sound, double *cfl_part, hipStream_t s);
+// the CFL maximum of each work-group's cells from set 0's u, v, w and T (cell_wgs entries)
+int launch_cfl_partial_batch(const KParams &k, const AuxBlock *tab, int nb, long cell_wgs, double *cfl_part, hipStream_t s);
 // dts[b] = cfl * hmin / (maximum of block b's CFL partials), then *dt_dev = min over b.
 // Block b's partials are cfl_part[ranges[b].x .. ranges[b].y) when ranges is set (the tiles
 // of a stage-applying launch), else those of its stage-kernel work-groups.
