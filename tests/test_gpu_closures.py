@@ -112,3 +112,27 @@ def test_closure_configuration_errors(ws):
     assert L.ws_ctx_create(ctypes.byref(cfg), ctypes.byref(h)) == W.WS_ERR_INVALID   # too few cells
     cfg = W.default_config(16, 16, 16, periodic=(0, 1, 1), viscous=6)
     assert L.ws_ctx_create(ctypes.byref(cfg), ctypes.byref(h)) == W.WS_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("precision", [W.WS_PREC_FP64, W.WS_PREC_MIXED])
+@pytest.mark.parametrize("n", [8, 9, 15, 30, 32, 33, 37])
+def test_closed_faces_at_tile_edges(orc, ws, n, precision):
+    """The faces beside a closed face are shared out over the work-group: extents that put both
+    closed ends in one tile, the high end's faces on either side of a tile edge, and a last
+    tile of a cell or two, for every tile shape, in each direction in turn, with non-reflecting
+    flags on both passes and the high face in the rim kernel's form where it may be."""
+    for d in range(3):
+        ext = [10, 11, 9]
+        ext[d] = n
+        prims = random_state(*ext, 14, "shock")
+        periodic = tuple(int(q != d) for q in range(3))
+        d0 = tuple(0 if q // 2 != d else (2 if q % 2 else 1) for q in range(6))
+        nr = tuple(int(q // 2 == d) for q in range(6))
+        g = _ghosted_state(orc, prims, periodic, 3)
+        kw = dict(periodic=periodic, d0_bound=d0, non_ref=nr)
+        ref = _oracle(orc, g, **kw)
+        for tile in W.TILE_SHAPES:
+            ctx = make_ctx(*ext, precision=precision, **kw)
+            ctx.set_tile_shape(tile)
+            err = rel_l2(gpu_du_comput(ctx, _upload(g)), ref)
+            assert err <= (1e-12 if precision == W.WS_PREC_FP64 else 1e-6), (d, tile, err)

@@ -412,32 +412,17 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
     const bool lo = BND && k.bnd[2 * DIR];
     const int hi = BND ? k.bnd[2 * DIR + 1] : 0;     // the high face's closure form (0: none)
     const bool nr_lo = lo && k.nonref[2 * DIR], nr_hi = hi && k.nonref[2 * DIR + 1];
-    double nfix[BND ? 5 : 1];       // P(n) - P(n-1) of the line's last cell (non-reflecting M)
+    // faces 0..3 beside a closed low face and n-3..n beside a high one take their closure's value
+    // (at n-3 of the M half only)
+    auto covered = [&](int fg) { return BND && ((lo && fg <= 3) || (hi && fg >= n_dom - 3)); };
     // MIX: bit m*K + j set when face j of variable m had FP32 weights out of FP32's range
     unsigned bad_mix = 0;
     if (active) {
         const int base = TL::pidx(line, f0);
-        const bool near = BND && ((lo && gl0 + f0 <= 3) || (hi && gl0 + f0 + K - 1 >= n_dom - 3));
 #pragma unroll 1
         for (int m = 0; m < 5; ++m) {
             const double *qp = sp + m * TL::QS + base;
             const double *qm = sp + (5 + m) * TL::QS + base;
-            auto cellP = [&](int cg) { return sp[m * TL::QS + TL::pidx(line, cg - gl0 + LAP)]; };
-            auto cellM = [&](int cg) { return sp[(5 + m) * TL::QS + TL::pidx(line, cg - gl0 + LAP)]; };
-            // faces covered by a closure: P + M with either side replaced (FP64 closures)
-            auto closed = [&](int j, auto wenoP, auto wenoM) {
-                const int fg = gl0 + f0 + j;
-                double pv, mv;
-                const bool cp = closure_p(cellP, n_dom, fg, lo, hi, pv);
-                const bool cm = closure_m(cellM, n_dom, fg, lo, hi, mv);
-                if (cp || cm) Fv[m][j] = FS * ((cp ? pv : wenoP()) + (cm ? mv : wenoM()));
-                if (BND && nr_hi && fg == n_dom) {
-                    double a = 0.0, b = 0.0;
-                    closure_p(cellP, n_dom, n_dom - 1, lo, hi, a);
-                    closure_p(cellP, n_dom, n_dom, lo, hi, b);
-                    nfix[m] = FS * (b - a);
-                }
-            };
             // a stored face f (f <= lim_line) reads only points f..f+7, all written in
             // phase 1; faces past lim_line read stale LDS and are not stored
             if (MIX) {
@@ -450,10 +435,6 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
 #pragma unroll
                 for (int j = 0; j < K; ++j) Fv[m][j] = (bP[j] + bM[j]) + (double)(cP[j] + cM[j]);
                 bad_mix |= (badP | badM) << (m * K);
-                if (near)
-#pragma unroll
-                    for (int j = 0; j < K; ++j)
-                        closed(j, [&] { return bP[j] + (double)cP[j]; }, [&] { return bM[j] + (double)cM[j]; });
             } else {
                 double nP[K], dP[K], nM[K], dM[K], bP[K], bM[K];
                 weno_k<false, K>([&](int j) { return qp[j]; }, nP, dP, bP);
@@ -463,15 +444,11 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
                     const double den = dP[j] * dM[j];
                     Fv[m][j] = fma(fma(nP[j], dM[j], nM[j] * dP[j]), recip_nr(den), bP[j] + bM[j]);
                 }
-                if (near)
-#pragma unroll
-                    for (int j = 0; j < K; ++j)
-                        closed(j, [&] { return (bP[j] + nP[j] / dP[j]) / kFace; }, [&] { return (bM[j] + nM[j] / dM[j]) / kFace; });
             }
         }
         // Faces whose FP32 weights left FP32's range (strong discontinuities of the split
         // flux): both halves again in FP64 from the split values still in LDS, merged as the
-        // FP64 kernel merges them (a half a closure covers keeps its closure value).  Done
+        // FP64 kernel merges them (faces beside a closed one are handled below).  Done
         // after the variable loop, when the FP32 registers are dead, and skipped by every
         // wave without such a face.
         if (MIX && bad_mix) {
@@ -481,23 +458,60 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
                 for (int j = 0; j < K; ++j) {
                     if (!((bad_mix >> (m * K + j)) & 1u)) continue;
                     const double *qp = sp + m * TL::QS + base, *qm = sp + (5 + m) * TL::QS + base;
-                    double nP, dP, nM, dM, bP, bM, val;
-                    const int fg = gl0 + f0 + j;
-                    if (BND && ((lo && fg <= 3) || (hi && fg >= n_dom - 3))) {
-                        auto cellP = [&](int cg) { return sp[m * TL::QS + TL::pidx(line, cg - gl0 + LAP)]; };
-                        auto cellM = [&](int cg) { return sp[(5 + m) * TL::QS + TL::pidx(line, cg - gl0 + LAP)]; };
-                        double pv, mv;
-                        if (!closure_p(cellP, n_dom, fg, lo, hi, pv)) { face64<false>(qp + j, nP, dP, bP); pv = (bP + nP / dP) / kFace; }
-                        if (!closure_m(cellM, n_dom, fg, lo, hi, mv)) { face64<true>(qm + j, nM, dM, bM); mv = (bM + nM / dM) / kFace; }
-                        val = pv + mv;
-                    } else {
-                        face64<false>(qp + j, nP, dP, bP);
-                        face64<true>(qm + j, nM, dM, bM);
-                        val = fma(fma(nP, dM, nM * dP), recip_nr(dP * dM), bP + bM) / kFace;
-                    }
+                    if (covered(gl0 + f0 + j)) continue;
+                    double nP, dP, nM, dM, bP, bM;
+                    face64<false>(qp + j, nP, dP, bP);
+                    face64<true>(qm + j, nM, dM, bM);
+                    const double val = fma(fma(nP, dM, nM * dP), recip_nr(dP * dM), bP + bM) / kFace;
 #pragma unroll
                     for (int q = 0; q < 5; ++q)
                         if (q == m) Fv[q][j] = val;
+                }
+            }
+        }
+    }
+    // The faces beside a closed face, one (face, variable, line) per thread with the lines
+    // fastest, so that a wavefront evaluates one or two of the closures: by the face's own thread,
+    // each wavefront of the tile went through all of them, for every variable (the x launch of
+    // 211x93x67 with x closed 109 -> 63 us; 54 for the y launch, which has no closures).
+    constexpr int CI = BND ? (8 * 5 * W + TL::NT - 1) / TL::NT : 1;
+    double cval[CI], cfix[CI];      // the face's value; P(n) - P(n-1) of the last cell (non-reflecting M)
+    int cat[CI];                    // its place in the face buffer (-1: none)
+    if (BND) {
+#pragma unroll
+        for (int r = 0; r < CI; ++r) cat[r] = -1;
+        if ((lo && gl0 <= 3) || (hi && gl0 + g.lim_line >= n_dom - 3)) {
+#pragma unroll
+            for (int r = 0; r < CI; ++r) {
+                const int it = t + r * TL::NT, l = it % W, m = it / W % 5, q = it / (5 * W);
+                const int fg = q < 4 ? q : n_dom - 7 + q, f = fg - gl0;
+                if (q >= 8 || !(q < 4 ? lo : hi != 0) || f < 0 || f > g.lim_line || f >= TL::F || l < g.lo_across ||
+                    l >= g.lim_across)
+                    continue;
+                const double *qp = sp + m * TL::QS + TL::pidx(l, f), *qm = qp + 5 * TL::QS;
+                auto cellP = [&](int cg) { return qp[cg - fg + LAP]; };
+                auto cellM = [&](int cg) { return qm[cg - fg + LAP]; };
+                double pv, mv;
+                closure_m(cellM, n_dom, fg, lo, hi, mv);
+                if (!closure_p(cellP, n_dom, fg, lo, hi, pv)) {
+                    double nP, dP, bP;
+                    face64<false>(qp, nP, dP, bP);
+                    pv = (bP + nP / dP) / kFace;
+                    if (MIX) {
+                        double bp[1], bm[1];
+                        float cp[1], cm[1];
+                        unsigned badP, badM;
+                        weno_k_mixed<false, 1>([&](int i) { return qp[i]; }, bp, cp, badP);
+                        weno_k_mixed<true, 1>([&](int i) { return qm[i]; }, bm, cm, badM);
+                        if (!(badP | badM)) pv = bp[0] + (double)cp[0];
+                    }
+                }
+                cval[r] = FS * (pv + mv);
+                cat[r] = m * W * TL::F + TL::fidx(l, f);
+                if (nr_hi && fg == n_dom) {
+                    double a = 0.0;
+                    closure_p(cellP, n_dom, n_dom - 1, lo, hi, a);
+                    cfix[r] = FS * (pv - a);
                 }
             }
         }
@@ -530,11 +544,18 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
 #pragma unroll
         for (int j = 0; j < K; ++j) {
             if (f0 + j > g.lim_line || f0 + j >= TL::F) break;
+            if (covered(gl0 + f0 + j)) continue;
 #pragma unroll
             for (int m = 0; m < 5; ++m) sp[m * W * TL::F + TL::fidx(line, f0 + j)] = Fv[m][j];
-            if (BND && nr_hi && gl0 + f0 + j == n_dom)
+        }
+    }
+    if (BND) {
 #pragma unroll
-                for (int m = 0; m < 5; ++m) nfix_lds[line * 5 + m] = nfix[m];
+        for (int r = 0; r < CI; ++r) {
+            if (cat[r] < 0) continue;
+            sp[cat[r]] = cval[r];
+            const int it = t + r * TL::NT;
+            if (nr_hi && it / (5 * W) == 7) nfix_lds[it % W * 5 + it / W % 5] = cfix[r];
         }
     }
     __syncthreads();
