@@ -11,18 +11,27 @@ from tests.helpers import random_state
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("precision", [W.WS_PREC_FP64, W.WS_PREC_MIXED])
 @pytest.mark.parametrize("periodic", [(1, 1, 1), (0, 1, 1), (1, 0, 0), (0, 0, 0)])
 @pytest.mark.parametrize("shape", [(4, 4, 4), (9, 6, 5), (70, 65, 66)])
-def test_rhs_inputs_in_one_launch(ws, shape, periodic):
-    """ws_du_comput's inputs (one launch, one point per thread up to 2^18 ghosted points, two
-    above) against a ghost fill and a pass over T: every point of the ghosted box bit for bit,
-    the caller's ghost layers and corners included, with a sound speed of another pitch."""
+def test_rhs_inputs_in_one_launch(ws, shape, periodic, precision):
+    """The RHS's inputs, prepared alone (one point per thread up to 2^18 ghosted points, two
+    above) and by a small grid's du_comput in the launch that computes the RHS, against a
+    ghost fill, a pass over T and the RHS: every point of the ghosted box and du bit for bit, the
+    caller's ghost layers and corners included, with a sound speed of another pitch and with
+    metric fields."""
     import torch
     nx, ny, nz = shape
     L, sh = W.lib(), W.stream_handle()
-    ctx = make_ctx(nx, ny, nz, periodic=periodic)
+    ctx = make_ctx(nx, ny, nz, periodic=periodic, precision=precision)
+    rng = np.random.default_rng(41)
+    tens = [torch.from_numpy(0.7 + 0.6 * rng.random((nz + 8, ny + 8, nx + 8))).cuda() for _ in range(10)]
+    mf = W.WsMetricFields()
+    for i in range(9):
+        mf.A[i] = W.field_of(tens[i])
+    mf.ajac = W.field_of(tens[9])
     states = []
-    for _ in range(2):
+    for _ in range(4):
         st = upload_state(random_state(nx, ny, nz, 3, "blobs"))
         st.t["cc"] = W.ghosted_tensor(nx, ny, nz, pad=3)
         st.refresh()
@@ -32,13 +41,20 @@ def test_rhs_inputs_in_one_launch(ws, shape, periodic):
             st.t[k].copy_(1.0 + 0.2 * torch.rand(st.t[k].shape, dtype=torch.float64, device="cuda", generator=gen))
             st.interior(k).copy_(inner)
         states.append(st)
-    a, b = states
+    a, am, p, b = states
     W.check(L.ws_du_comput(ctx.handle, ctypes.byref(a.ws), None, sh))
+    W.check(L.ws_du_comput(ctx.handle, ctypes.byref(am.ws), ctypes.byref(mf), sh))
+    W.check(L.ws_prepare_rhs_inputs(ctx.handle, ctypes.byref(p.ws), sh))
     fl = (W.WsField * 5)(b.ws.d, b.ws.u, b.ws.v, b.ws.w, b.ws.T)
     W.check(L.ws_ghost_fill_periodic(ctx.handle, fl, 5, sh))
     W.check(L.ws_sound_speed(ctx.handle, b.ws.T, b.ws.cc, W.job((0, 0, 0), (nx + 8, ny + 8, nz + 8)), sh))
     for k in ("d", "u", "v", "w", "T", "cc"):
-        assert torch.equal(a.t[k][..., :nx + 8], b.t[k][..., :nx + 8]), k
+        for st in (a, am, p):
+            assert torch.equal(st.t[k][..., :nx + 8], b.t[k][..., :nx + 8]), k
+    job = W.interior_job(nx, ny, nz)
+    for st, m in ((a, None), (am, ctypes.byref(mf))):
+        W.check(L.ws_inviscid_rhs(ctx.handle, b.ws.d, b.ws.u, b.ws.v, b.ws.w, b.ws.cc, m, b.ws.du, job, 0, sh))
+        assert torch.equal(st.interior("du"), b.interior("du"))
 
 
 @pytest.mark.parametrize("shape", [(4, 4, 4), (33, 17, 9), (129, 127, 131)])

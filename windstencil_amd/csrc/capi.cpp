@@ -692,8 +692,13 @@ int ws_du_comput(ws_ctx *c, const ws_state *st, const ws_metric_fields *metrics,
 {
     if (!c || !st) return set_error(WS_ERR_INVALID, "null argument");
     int r;
-    if ((r = ws_prepare_rhs_inputs(c, st, s))) return r;
-    if ((r = ws_inviscid_rhs(c, st->d, st->u, st->v, st->w, st->cc, metrics, st->du, interior_job(c), 0, s))) return r;
+    bool done = false;
+    if ((r = check_prims(c, st)) || (r = check_soa(c, st->du, "du")) || (r = check_metrics(c, metrics))) return r;
+    if ((r = launch_prepared_rhs(*c, *st, metrics, &done, s))) return r;
+    if (!done) {
+        if ((r = ws_prepare_rhs_inputs(c, st, s))) return r;
+        if ((r = ws_inviscid_rhs(c, st->d, st->u, st->v, st->w, st->cc, metrics, st->du, interior_job(c), 0, s))) return r;
+    }
     if (c->cfg.viscous) return launch_viscous(*c, st->u, st->v, st->w, st->T, metrics, st->du, s);
     return WS_OK;
 }

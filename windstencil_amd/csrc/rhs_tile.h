@@ -1048,7 +1048,7 @@ int launch_rhs_tile(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w
     k.same_pitch = same_pitch(d, u, v, w, cc) ? 1 : 0;
     k.big = rel_planes(k, {d, u, v, w, cc}, {du}) && (!m || rel_planes(k, *m)) ? 0 : 1;
     if (!k.big && box_serves(c, job)) {
-        launch_rhs_box(MIX, k, d, u, v, w, cc, m, du, job, order, accumulate, sa, s);
+        launch_rhs_box(MIX, k, d, u, v, w, cc, m, du, job, order, accumulate, sa, nullptr, s);
     } else if (m) {
         mf = *m;
         launch_shape<true, MIX>(shape, k, d, u, v, w, cc, mf, du, box, accumulate, c.schedule, order, nullptr, s);

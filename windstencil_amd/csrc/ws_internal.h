@@ -274,8 +274,18 @@ int launch_rhs_anchor(Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w, ws
                       const ws_metric_fields *m, ws_soa du, ws_job job, int accumulate, hipStream_t s);
 int launch_rhs_tiled(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc,
                      const ws_metric_fields *m, ws_soa du, ws_job job, int accumulate, hipStream_t s);
+// launch_prepare and the interior's RHS in one launch, where the one-launch RHS serves it
+// (otherwise nothing happens and *done is false)
+int launch_prepared_rhs(const Ctx &c, const ws_state &st, const ws_metric_fields *m, bool *done, hipStream_t s);
 int launch_rhs_mixed(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc,
                      const ws_metric_fields *m, ws_soa du, ws_job job, int accumulate, hipStream_t s);
+// With it the one-launch RHS also does what launch_prepare does (over the interior only): the T
+// whose ghost points and sound speed it writes, and the periodic directions.
+struct BoxPrep {
+    ws_field T;
+    int per[3];
+};
+
 // The one-launch RHS of small jobs (k_rhs_box.hip): whether it serves a job (otherwise the
 // directional tiles do: a larger job, closures, or turned off).
 bool box_serves(const Ctx &c, const ws_job &job);
@@ -283,7 +293,7 @@ bool box_serves(const Ctx &c, const ws_job &job);
 long box_launch_tiles(const ws_job &job);
 void launch_rhs_box(bool mixed, const KParams &k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc,
                     const ws_metric_fields *m, ws_soa du, const ws_job &job, int order, int accumulate,
-                    const StageArgs *sa, hipStream_t s);
+                    const StageArgs *sa, const BoxPrep *prep, hipStream_t s);
 // work-groups of the context's launch that applies an RK3 stage (the last direction of its
 // order, in its tile shape, or the one-launch kernel): the entries that launch writes to StageArgs::cfl_part
 long stage_launch_tiles(const Ctx &c);
