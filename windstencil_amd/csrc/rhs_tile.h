@@ -338,6 +338,12 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
     static_assert(!(STG && (BND || !ACC)), "the stage is applied by an accumulating launch without closures");
     using TL = Tile<DIR, L, W, K>;
     const int t = threadIdx.x;
+    // FP64: a wavefront that loads, splits or stores goes ahead of those that reconstruct, which
+    // have instructions to spare for the wait (256x160x96 over metric fields 538 -> 523 us,
+    // 600x256x128 1950 -> 1927); the mixed kernels and those that apply a stage gain nothing (1929
+    // -> 1985 us, 3925 -> 3938 per RK3 step of 600x128x128)
+    constexpr bool AHEAD = !MIX && !STG;
+    if (AHEAD) __builtin_amdgcn_s_setprio(2);
     const double cA1 = k.A[3 * DIR + 0], cA2 = k.A[3 * DIR + 1], cA3 = k.A[3 * DIR + 2];
     const double cSn = k.Anorm[DIR], cRs = k.Arnorm[DIR];
     const double cK1 = k.Ak[3 * DIR + 0], cK2 = k.Ak[3 * DIR + 1], cK3 = k.Ak[3 * DIR + 2];
@@ -398,6 +404,7 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
     next();
     __syncthreads();
 
+    if (AHEAD) __builtin_amdgcn_s_setprio(0);
     // ---- phase 2: K faces of one line per thread, all five variables --------------------
     const int line = t / TL::T, seg = t % TL::T;
     const int f0 = seg * K;                               // first face of this thread
@@ -537,6 +544,7 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
                 for (int m = 0; m < 5; ++m) fvv[r][m] = elem(fbase + m * fstride, fo);
         }
     }
+    if (AHEAD) __builtin_amdgcn_s_setprio(2);
     // face fluxes reuse the split buffer (its first 5*W*F entries; the M split values, from
     // 5*QS on, stay intact for the non-reflecting fix of phase 3)
     double *nfix_lds = sp + 5 * W * TL::F;        // [W][5], free space below 5*QS
