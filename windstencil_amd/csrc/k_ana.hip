@@ -20,6 +20,7 @@ namespace {
 constexpr int AT = 256;
 constexpr int ABLOCKS = 512;
 constexpr int AU = 4;           // points in flight per thread
+constexpr int FT = 512;         // threads of the final reduction
 constexpr long long NONE = 0x7fffffffffffffffLL;
 
 // per-quantity count and first offending ghosted index
@@ -39,21 +40,36 @@ __device__ __forceinline__ void rec_merge(AnaRec &a, const AnaRec &b)
     a.smax = fmax(a.smax, b.smax);
 }
 
-__device__ __forceinline__ void rec_reduce(AnaRec &r, AnaRec *red)
+// r of thread 0: the work-group's NTH records merged (every thread calls it), within each
+// wavefront by lane exchanges, then over the wavefronts
+template <int NTH>
+__device__ __forceinline__ void rec_reduce(AnaRec &r)
 {
-    red[threadIdx.x] = r;
+    __shared__ AnaRec wave[NTH / 64];
+    auto fold = [&](int o) {
+        AnaRec b;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            b.count[q] = __shfl_xor(r.count[q], o);
+            b.first[q] = __shfl_xor(r.first[q], o);
+        }
+        b.smax = __shfl_xor(r.smax, o);
+        rec_merge(r, b);
+    };
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) fold(o);
+    if ((threadIdx.x & 63) == 0) wave[threadIdx.x >> 6] = r;
     __syncthreads();
-    for (int s = AT / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) rec_merge(red[threadIdx.x], red[threadIdx.x + s]);
-        __syncthreads();
+    if (threadIdx.x < 64) {
+        r = wave[threadIdx.x & (NTH / 64 - 1)];
+#pragma unroll
+        for (int o = NTH / 128; o > 0; o >>= 1) fold(o);
     }
-    r = red[0];
 }
 
 __global__ void __launch_bounds__(AT) k_ana_partial(KParams k, ws_field d, ws_field u, ws_field v, ws_field w,
                                                     ws_field T, ws_field ajac, AnaRec *partial)
 {
-    __shared__ AnaRec red[AT];
     AnaRec r;
 #pragma unroll
     for (int q = 0; q < 4; ++q) { r.count[q] = 0; r.first[q] = NONE; }
@@ -106,19 +122,18 @@ __global__ void __launch_bounds__(AT) k_ana_partial(KParams k, ws_field d, ws_fi
             }
         }
     }
-    rec_reduce(r, red);
+    rec_reduce<AT>(r);
     if (threadIdx.x == 0) partial[blockIdx.x] = r;
 }
 
-__global__ void __launch_bounds__(AT) k_ana_final(const AnaRec *partial, int n, AnaRec *out)
+__global__ void __launch_bounds__(FT) k_ana_final(const AnaRec *partial, int n, AnaRec *out)
 {
-    __shared__ AnaRec red[AT];
     AnaRec r;
 #pragma unroll
     for (int q = 0; q < 4; ++q) { r.count[q] = 0; r.first[q] = NONE; }
     r.smax = 0.0;
-    for (int i = threadIdx.x; i < n; i += AT) rec_merge(r, partial[i]);
-    rec_reduce(r, red);
+    for (int i = threadIdx.x; i < n; i += FT) rec_merge(r, partial[i]);
+    rec_reduce<FT>(r);
     if (threadIdx.x == 0) *out = r;
 }
 
@@ -139,6 +154,7 @@ constexpr int ANA_MAX_DEVICES = 64;
 std::mutex g_ana_mutex;
 AnaRec *g_ana_scratch[ANA_MAX_DEVICES][2] = {};
 std::mutex g_ana_busy[ANA_MAX_DEVICES];
+AnaRec *g_ana_host[ANA_MAX_DEVICES] = {};    // pinned result of ws_ana_state, under g_ana_busy
 
 // The device address of `scratch` (which 0) or `scratch_state` (which 1) on the current device
 // `dev`, looked up once per device.
@@ -159,19 +175,21 @@ int ana_scratch_ptr(int dev, int which, AnaRec **out)
 }
 
 // The pass and its report; buf holds ABLOCKS + 1 records of device memory.  Every record
-// is written before it is read, so buf needs no clearing between calls.
+// is written before it is read, so buf needs no clearing between calls.  host: pinned memory
+// the result is written to by the kernel itself (null: a copy from buf's last record).
 int ana_run(ws_ctx *c, const ws_state *st, const ws_metric_fields *metrics, double dt, ws_ana_report *rep,
-            hipStream_t s, AnaRec *buf)
+            hipStream_t s, AnaRec *buf, AnaRec *host = nullptr)
 {
     const KParams &k = c->kp;
     const ws_field aj = metrics ? metrics->ajac : ws_field{};
     hipLaunchKernelGGL(k_ana_partial, dim3(ABLOCKS), dim3(AT), 0, s, k, st->d, st->u, st->v, st->w, st->T, aj, buf);
-    hipLaunchKernelGGL(k_ana_final, dim3(1), dim3(AT), 0, s, (const AnaRec *)buf, ABLOCKS, buf + ABLOCKS);
+    hipLaunchKernelGGL(k_ana_final, dim3(1), dim3(FT), 0, s, (const AnaRec *)buf, ABLOCKS, host ? host : buf + ABLOCKS);
     AnaRec r{};
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(&r, buf + ABLOCKS, sizeof(AnaRec), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess && !host) e = hipMemcpyAsync(&r, buf + ABLOCKS, sizeof(AnaRec), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return hip_error(e, "state analysis");
+    if (host) r = *host;
     const long long nxg = k.nx + 2 * LAP, nyg = k.nyg;
     int64_t *cnt[4] = {&rep->nan_T, &rep->neg_T, &rep->neg_d, &rep->neg_jac};
     int32_t *first[4] = {rep->first_nan_T, rep->first_neg_T, rep->first_neg_d, rep->first_neg_jac};
@@ -220,7 +238,12 @@ extern "C" int ws_ana_state(ws_ctx *c, const ws_state *st, const ws_metric_field
     if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < ANA_MAX_DEVICES) {
         std::unique_lock<std::mutex> busy(g_ana_busy[dev], std::try_to_lock);
         if (busy.owns_lock() && ana_scratch_ptr(dev, 1, &buf) == WS_OK) {
-            r = ana_run(c, st, metrics, dt, rep, s, buf);
+            AnaRec *&host = g_ana_host[dev];
+            if (!host && hipHostMalloc((void **)&host, sizeof(AnaRec), hipHostMallocDefault) != hipSuccess) {
+                host = nullptr;
+                (void)hipGetLastError();
+            }
+            r = ana_run(c, st, metrics, dt, rep, s, buf, host);
             if (r) (void)hipStreamSynchronize(s);   // nothing of a failed call still writes it
             return r;
         }

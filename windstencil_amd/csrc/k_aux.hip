@@ -265,21 +265,25 @@ __global__ void __launch_bounds__(NT) k_cfl_partial(KParams k, ws_field u, ws_fi
     if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-__global__ void __launch_bounds__(NT) k_cfl_final(const double *partial, int n, double cfl, double hmin,
-                                                  double *dt_out)
+constexpr int CFT = 1024;        // threads of k_cfl_final
+
+__global__ void __launch_bounds__(CFT) k_cfl_final(const double *partial, int n, double cfl, double hmin,
+                                                   double *dt_out)
 {
 #pragma clang fp contract(off)
-    __shared__ double red[NT];
+    __shared__ double red[CFT / 64];
     double mx = 0.0;
 #pragma unroll 8
-    for (int i = threadIdx.x; i < n; i += NT) mx = fmax(mx, partial[i]);
-    red[threadIdx.x] = mx;
+    for (int i = threadIdx.x; i < n; i += CFT) mx = fmax(mx, partial[i]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
     __syncthreads();
-    for (int s = NT / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + s]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *dt_out = cfl * hmin / red[0];
+    if (threadIdx.x >= 64) return;
+    mx = red[threadIdx.x % (CFT / 64)];
+#pragma unroll
+    for (int o = CFT / 128; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+    if (threadIdx.x == 0) *dt_out = cfl * hmin / mx;
 }
 
 __global__ void __launch_bounds__(NT) k_min_reduce(const double *v, int n, double *out)
@@ -565,7 +569,7 @@ int launch_cfl(Ctx &c, const ws_state &st, double cfl, double *dt_dev, hipStream
     const KParams &k = c.kp;
     const double hmin = fmin(k.h[0], fmin(k.h[1], k.h[2]));
     hipLaunchKernelGGL(k_cfl_partial, dim3(c.cfl_blocks), dim3(NT), 0, s, k, st.u, st.v, st.w, st.T, c.cfl_partial);
-    hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(NT), 0, s, (const double *)c.cfl_partial, c.cfl_blocks, cfl, hmin,
+    hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(CFT), 0, s, (const double *)c.cfl_partial, c.cfl_blocks, cfl, hmin,
                        dt_dev);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? WS_OK : hip_error(e, "cfl launch");
@@ -575,7 +579,7 @@ int launch_cfl_final(const Ctx &c, const double *partial, int n, double cfl, dou
 {
     const KParams &k = c.kp;
     const double hmin = fmin(k.h[0], fmin(k.h[1], k.h[2]));
-    hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(NT), 0, s, partial, n, cfl, hmin, dt_dev);
+    hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(CFT), 0, s, partial, n, cfl, hmin, dt_dev);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? WS_OK : hip_error(e, "cfl launch");
 }
