@@ -32,6 +32,7 @@ KParams make_kparams(const ws_config &c)
     k.gamma = c.gamma;
     k.c1 = 2.0 * (c.gamma - 1.0);                          // OCFD_init.cpp:385
     k.c3 = (3.0 - c.gamma) / (2.0 * (c.gamma - 1.0));      // OCFD_init.cpp:386
+    k.half_rcp_gamma = 0.5 / c.gamma;
     k.quarter_rcp_gamma = 0.25 / c.gamma;
     k.c3h = 0.5 + k.c3;
     k.gm1 = c.gamma - 1.0;
@@ -46,6 +47,7 @@ KParams make_kparams(const ws_config &c)
         const double sn = std::sqrt(a1 * a1 + a2 * a2 + a3 * a3);
         k.Anorm[dir] = sn;
         k.Arnorm[dir] = 1.0 / sn;
+        k.Ak[3 * dir] = a1 / sn; k.Ak[3 * dir + 1] = a2 / sn; k.Ak[3 * dir + 2] = a3 / sn;
     }
     k.ajac = c.metric[9];
     // bnd: the closure form of each face (0 none, 1 D0_bound, 2 the rim kernel's high face)

@@ -170,12 +170,22 @@ k_rhs_box(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc
         double fp[5], fm[5];
         if (FIELDS) {
             const double A1 = ld[r][FIELDS ? 5 : 0], A2 = ld[r][FIELDS ? 6 : 0], A3 = ld[r][FIELDS ? 7 : 0];
-            double sn, rs;
-            sqrt_rsqrt_h(fma(A3, A3, fma(A2, A2, A1 * A1)), sn, rs);
-            split_fast(k, dd, uu, vv, ww, c, A1, A2, A3, sn, rs, fp, fm);
+            if (MIX) {
+                const double sn = sqrt(fma(A3, A3, fma(A2, A2, A1 * A1)));
+                const double rs = 1.0 / sn;
+                split_mixed(k, dd, uu, vv, ww, c, A1, A2, A3, sn, A1 * rs, A2 * rs, A3 * rs, fp, fm);
+            } else {
+                double sn, rs;
+                sqrt_rsqrt_h(fma(A3, A3, fma(A2, A2, A1 * A1)), sn, rs);
+                split_fast(k, dd, uu, vv, ww, c, A1, A2, A3, sn, rs, fp, fm);
+            }
         } else {
-            split_fast(k, dd, uu, vv, ww, c, k.A[3 * dir], k.A[3 * dir + 1], k.A[3 * dir + 2], k.Anorm[dir],
-                       k.Arnorm[dir], fp, fm);
+            const double A1 = k.A[3 * dir], A2 = k.A[3 * dir + 1], A3 = k.A[3 * dir + 2];
+            if (MIX)
+                split_mixed(k, dd, uu, vv, ww, c, A1, A2, A3, k.Anorm[dir], k.Ak[3 * dir], k.Ak[3 * dir + 1],
+                            k.Ak[3 * dir + 2], fp, fm);
+            else
+                split_fast(k, dd, uu, vv, ww, c, A1, A2, A3, k.Anorm[dir], k.Arnorm[dir], fp, fm);
         }
 #pragma unroll
         for (int m = 0; m < 5; ++m) {

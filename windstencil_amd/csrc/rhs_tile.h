@@ -346,6 +346,7 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
     if (AHEAD) __builtin_amdgcn_s_setprio(2);
     const double cA1 = k.A[3 * DIR + 0], cA2 = k.A[3 * DIR + 1], cA3 = k.A[3 * DIR + 2];
     const double cSn = k.Anorm[DIR], cRs = k.Arnorm[DIR];
+    const double cK1 = k.Ak[3 * DIR + 0], cK2 = k.Ak[3 * DIR + 1], cK3 = k.Ak[3 * DIR + 2];
 
     // ---- phase 3 prologue: accumulating launches read du; those loads go out with the
     // tile's primitive loads, so one wait at the split covers both (issued later, the
@@ -379,9 +380,17 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
         double fp[5], fm[5];
         if (FIELDS) {
             const double A1 = ld.v[r][FIELDS ? 5 : 0], A2 = ld.v[r][FIELDS ? 6 : 0], A3 = ld.v[r][FIELDS ? 7 : 0];
-            double sn, rs;
-            sqrt_rsqrt_h(fma(A3, A3, fma(A2, A2, A1 * A1)), sn, rs);
-            split_fast(k, dd, uu, vv, ww, c, A1, A2, A3, sn, rs, fp, fm);
+            if (MIX) {
+                const double sn = sqrt(fma(A3, A3, fma(A2, A2, A1 * A1)));
+                const double rs = 1.0 / sn;
+                split_mixed(k, dd, uu, vv, ww, c, A1, A2, A3, sn, A1 * rs, A2 * rs, A3 * rs, fp, fm);
+            } else {
+                double sn, rs;
+                sqrt_rsqrt_h(fma(A3, A3, fma(A2, A2, A1 * A1)), sn, rs);
+                split_fast(k, dd, uu, vv, ww, c, A1, A2, A3, sn, rs, fp, fm);
+            }
+        } else if (MIX) {
+            split_mixed(k, dd, uu, vv, ww, c, cA1, cA2, cA3, cSn, cK1, cK2, cK3, fp, fm);
         } else {
             split_fast(k, dd, uu, vv, ww, c, cA1, cA2, cA3, cSn, cRs, fp, fm);
         }

@@ -206,10 +206,23 @@ __device__ __forceinline__ double recip_nr(double x)
     return fma(r, fma(e, e, e), r);
 }
 
+// Square root of a positive normal number: reciprocal-square-root estimate refined
+// with one coupled Newton step on (sqrt, 1/(2 sqrt)) and a final residual correction.
+__device__ __forceinline__ double sqrt_nr(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-g, h, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    const double d = fma(-g, g, x);
+    return fma(d, h, g);
+}
+
 // Square root of a positive normal number and its reciprocal: the reciprocal-square-root
 // estimate y (24 bits) and one third-order step, with e = 1 - x y^2: sqrt(x) = x y (1 + e/2 +
 // 3/8 e^2), 1/sqrt(x) = y (1 + e/2 + 3/8 e^2); the remainder 5/16 e^3 is below 2^-70.  Two
-// instructions fewer than a Newton step with a residual correction; error within an ulp.
+// instructions fewer than sqrt_nr; error within an ulp.
 __device__ __forceinline__ double sqrt_h(double x)
 {
 #pragma clang fp contract(off)
@@ -606,15 +619,14 @@ __device__ __forceinline__ bool closure_m(Cell cell, int n, int f, bool lo, int 
     return false;
 }
 
-// Steger-Warming split of the tiled kernels: A1..A3 the metric terms, sn = |A|
+// Steger-Warming split in the form the tiled FP64 kernels use: A1..A3 the metric terms, sn = |A|
 // and rsn = 1/|A| supplied by the caller (constants when metrics are uniform).  With vs = A.u,
 // cs = c |A|, P_i twice the smoothed positive eigenvalues of vs, vs - cs, vs + cs and
 // s = P_2 + P_3, d = P_3 - P_2, the mass flux is f0 = t (c1 P_1 + s), the momentum flux f0 u_i +
 // t c/|A| d A_i and the energy flux t (P_1 vv + s (|u|^2/2 + c^2/2 + W2) + d c vs/|A|); the
-// negative part takes 2 vs - P_1, 4 vs - s and 4 cs - d.  71 FP64 instructions against 108
-// with the shifted velocities u -+ c k spelled out; a tile splits 25-31 % more points than it
-// owns.  RHS of 600x256x128: FP64 2155 -> 2080 us; mixed 2086 -> 2011 us, where a last bit of a
-// split value now and then flips the rounding of a difference to FP32 (6e-13 of du).
+// negative part takes 2 vs - P_1, 4 vs - s and 4 cs - d.  71 FP64 instructions against the 108
+// of split_mixed (whose shifted velocities u -+ c k are spelled out); a tile splits 25-31 %
+// more points than it owns.
 __device__ __forceinline__ void split_fast(const KParams &k, double d, double u, double v, double w,
                                            double cc, double A1, double A2, double A3, double sn,
                                            double rsn, double fp[5], double fm[5])
@@ -649,6 +661,50 @@ __device__ __forceinline__ void split_fast(const KParams &k, double d, double u,
         fm[2] = fma(g, A2, fm[0] * v);
         fm[3] = fma(g, A3, fm[0] * w);
         fm[4] = t * fma(M1, vv, fma(sM, H, dM * cv));
+    }
+}
+
+// Steger-Warming split of the mixed-precision kernels: k1..k3 = A/|A|.  The mixed
+// reconstruction rounds first differences of these values to FP32, where a last-bit change
+// of a value can flip a rounding a hundred million times its size, so this form keeps its
+// arithmetic.
+__device__ __forceinline__ void split_mixed(const KParams &k, double d, double u, double v, double w,
+                                           double cc, double A1, double A2, double A3, double sn,
+                                           double k1, double k2, double k3, double fp[5], double fm[5])
+{
+    const double vs = fma(A3, w, fma(A2, v, A1 * u));
+    const double cs = cc * sn;
+    const double E1 = vs, E2 = vs - cs, E3 = vs + cs;
+    // eps2 > 0 keeps the radicands positive and normal
+    const double E1P = 0.5 * (E1 + sqrt_nr(fma(E1, E1, k.eps2)));
+    const double E2P = 0.5 * (E2 + sqrt_nr(fma(E2, E2, k.eps2)));
+    const double E3P = 0.5 * (E3 + sqrt_nr(fma(E3, E3, k.eps2)));
+    const double E1M = E1 - E1P, E2M = E2 - E2P, E3M = E3 - E3P;
+    const double t0 = d * k.half_rcp_gamma;
+    const double ck1 = cc * k1, ck2 = cc * k2, ck3 = cc * k3;
+    const double uc1 = u - ck1, uc2 = u + ck1;
+    const double vc1 = v - ck2, vc2 = v + ck2;
+    const double wc1 = w - ck3, wc2 = w + ck3;
+    const double h1 = 0.5 * fma(wc1, wc1, fma(vc1, vc1, uc1 * uc1));
+    const double h2 = 0.5 * fma(wc2, wc2, fma(vc2, vc2, uc2 * uc2));
+    const double vv = k.gm1 * fma(w, w, fma(v, v, u * u));
+    const double W2 = k.c3 * cc * cc;
+    // positive part
+    {
+        const double a = t0 * (k.c1 * E1P), b = t0 * E2P, c = t0 * E3P;
+        fp[0] = a + b + c;
+        fp[1] = fma(c, uc2, fma(b, uc1, a * u));
+        fp[2] = fma(c, vc2, fma(b, vc1, a * v));
+        fp[3] = fma(c, wc2, fma(b, wc1, a * w));
+        fp[4] = t0 * fma(W2, E2P + E3P, fma(E3P, h2, fma(E2P, h1, E1P * vv)));
+    }
+    {
+        const double a = t0 * (k.c1 * E1M), b = t0 * E2M, c = t0 * E3M;
+        fm[0] = a + b + c;
+        fm[1] = fma(c, uc2, fma(b, uc1, a * u));
+        fm[2] = fma(c, vc2, fma(b, vc1, a * v));
+        fm[3] = fma(c, wc2, fma(b, wc1, a * w));
+        fm[4] = t0 * fma(W2, E2M + E3M, fma(E3M, h2, fma(E2M, h1, E1M * vv)));
     }
 }
 

@@ -19,6 +19,7 @@ struct KParams {
     double gamma;
     double c1;                 // 2(gamma-1)
     double c3;                 // (3-gamma)/(2(gamma-1))
+    double half_rcp_gamma;     // 0.5/gamma
     double quarter_rcp_gamma;  // 0.25/gamma
     double c3h;                // 0.5 + c3
     double gm1;                // gamma-1
@@ -27,9 +28,10 @@ struct KParams {
     double cv;                 // 1/(gamma (gamma-1) Ma^2)
     double h[3];               // grid spacings
     double rh[3];              // 1/h
-    // constant metrics: direction d uses A[3d..3d+2]; their norm
+    // constant metrics: direction d uses A[3d..3d+2]; their norm and unit vector
     double A[9];
     double Anorm[3], Arnorm[3];   // Arnorm: 1/Anorm
+    double Ak[9];
     double ajac;
     // one-sided closures of the inviscid scheme at the domain faces (x-, x+, y-, y+, z-, z+:
     // 0 none, 1 the reference's D0_bound, 2 on a high face the rim kernel's form) and the
