@@ -243,7 +243,7 @@ def bench_batched(args):
     """48 periodic blocks with extents drawn from U{32..256} (seed 1), each a freestream
     of Mach U[0.3, 3] in a seeded direction with Gaussian blobs.  A step is one RHS of
     every block (per-block ghost fill and sound speed, then the batched RHS launches, one
-    per direction); then RK3 steps of the whole batch replayed from one hipGraph per step."""
+    per direction); then RK3 steps of the whole batch replayed from a hipGraph of two steps."""
     import torch
     import windstencil_amd as W
     from windstencil_amd import initial as I
@@ -344,7 +344,7 @@ def _ctx_choice(ctx):
 
 
 def bench_rk3(args):
-    """SSP-RK3 steps of one periodic box, replayed from one hipGraph per step (dt from
+    """SSP-RK3 steps of one periodic box, replayed from a hipGraph of two steps (dt from
     the CFL reduction every step): the FP64 drop-in workload (600x128x128 vortex
     lattice, 100 steps) or, with --grid 1200x256x256, Mach 2 blobs with a Mach 2 planar
     shock (1000 steps)."""
@@ -398,7 +398,7 @@ def bench_rk3(args):
     out = _common(args, f"SSP-RK3 Mcell-updates/s (N x 3 stages x steps / time), {nx}x{ny}x{nz}",
                   N * 3 * nsteps / secs / 1e6, ms, "f64" if prec == W.WS_PREC_FP64 else "f64-state/mixed-rhs",
                   {"workload": f"{nsteps} SSP-RK3 steps of the {nx}x{ny}x{nz} periodic box ({what}), CFL 0.5, "
-                               "one hipGraph per step", "grid": [nx, ny, nz], "precision": args.precision,
+                               "a hipGraph of two steps", "grid": [nx, ny, nz], "precision": args.precision,
                    "cells": N},
                   roofline=roof, rk3_steps=nsteps, seconds=round(secs, 4), state_finite=finite,
                   mcell_steps_per_s=round(N * nsteps / secs / 1e6, 2),

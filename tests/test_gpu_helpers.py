@@ -117,3 +117,34 @@ def test_runs_replaying_pairs_of_steps(ws, steps, viscous):
         got.append(out)
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+def test_state_analyses_that_overlap(ws):
+    """ws_ana_state's fixed records serve one call per GPU at a time and a call that finds them
+    taken allocates its own: four threads on streams of their own each get their state's counts."""
+    import threading
+
+    import torch
+    L = W.lib()
+    n = (70, 33, 29)
+    bad = []
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            ctx = make_ctx(*n)
+            st = upload_state(random_state(*n, 3 + i, "blobs"))
+            st.interior("T")[:i + 1, 0, 0] = float("nan")
+            stream.synchronize()
+            rep = W.WsAnaReport()
+            for _ in range(20):
+                W.check(L.ws_ana_state(ctx.handle, ctypes.byref(st.ws), None, 0.1, ctypes.byref(rep), W.stream_handle(stream)))
+                if (rep.nan_T, tuple(rep.first_nan_T)) != (i + 1, (0, 0, 0)):
+                    bad.append((i, rep.nan_T))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad, bad
