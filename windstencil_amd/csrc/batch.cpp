@@ -542,7 +542,7 @@ static int batch_step(ws_batch *b, const double *dt_dev, hipStream_t s, bool cfl
     }
     // the blocks are periodic (ws_batch_create); stages 1 and 2 leave the next stage's
     // inputs prepared (the last launch or the stage kernel writing the sound speed, the halo
-    // by that launch itself or a ghost fill after the stage kernel)
+    // by the same kernel)
     for (int krk = 1; krk <= 3 && !r; ++krk) {
         if (krk == 1) {
             if (aux) r = launch_prepare_batch(b->ctx[0]->kp, b->d_aux, nb, b->ghost_wgs, b->cell_wgs, s);
@@ -567,7 +567,6 @@ static int batch_step(ws_batch *b, const double *dt_dev, hipStream_t s, bool cfl
             const bool last = cfl_next && krk == 3;
             if (!r) r = launch_stage_batch(b->ctx[0]->kp, b->d_aux, nb, b->cell_wgs, swapped, planes, krk < 3,
                                            last ? b->d_cfl_part : nullptr, s);
-            if (!r && krk < 3) r = launch_ghost_fill_batch(b->d_aux, nb, b->ghost_wgs, 0, s);
             if (!r && last) b->cfl_in_batch = true;
             continue;
         }
@@ -576,10 +575,6 @@ static int batch_step(ws_batch *b, const double *dt_dev, hipStream_t s, bool cfl
             const ws_state &st = b->st[i];
             r = launch_stage(*c, fuse ? 0 : krk, st, nolap, c->cfg.dt, dt_dev, c->cfg.bc_planes != 0, krk < 3, s,
                              cfl_next && krk == 3 ? c->cfl_stage : nullptr);
-            if (!r && krk < 3) {
-                const ws_field g[6] = {st.d, st.u, st.v, st.w, st.T, st.cc};
-                r = launch_ghost_fill(*c, g, 6, s);
-            }
         }
     }
     return r;

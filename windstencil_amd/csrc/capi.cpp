@@ -225,8 +225,8 @@ int du_from_prepared(ws_ctx *c, const ws_state *st, hipStream_t s)
     return r;
 }
 
-// The stage kernel of stages 1 and 2 also writes the interior sound speed, and one ghost
-// fill of the primitives and cc then prepares the next stage's RHS: the same values as the
+// The stage kernel of stages 1 and 2 also writes the interior sound speed and the periodic face
+// halo of the primitives and cc, which prepares the next stage's RHS: the same values as the
 // separate ghost fill and ghosted-box sound speed on the faces the RHS reads (ghost cells
 // copy interior cells, whose sound speed is computed by the same expression).  With a
 // non-periodic direction the caller's ghost layers of T feed the sound speed there, so
@@ -390,7 +390,6 @@ int rk3_step_fused(ws_ctx *c, ws_state *st, const double *dt_dev, hipStream_t s,
             if (!r) r = du_from_prepared(c, st, s);
             if (!r) r = launch_stage(*c, krk, *st, nolap, c->cfg.dt, dt_dev, planes, sound, s, krk == 3 ? cfl_next : nullptr);
         }
-        if (!r && sound) r = launch_ghost_fill(*c, g, 6, s);
     }
     return r;
 }

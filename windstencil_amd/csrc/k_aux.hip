@@ -137,7 +137,8 @@ __global__ void __launch_bounds__(NT) k_time_advance(KParams k, ws_soa f, ws_soa
 // One RK3 stage of a solver step, fused: the stage update of f (as k_time_advance), the
 // primitives of the new f (as k_cons_to_pri), with PLANES the re-derivation of f on the six
 // boundary planes from those primitives (as k_pri_to_cons over the planes), and with
-// SOUND the sound speed of the interior (as k_sound_speed; a ghost fill then copies it).
+// SOUND (every direction periodic) the sound speed of the interior (as k_sound_speed) and
+// the face halo of d, u, v, w, T and cc (as k_ghost_fill).
 // Same expressions with contraction off as the separate kernels, so the state is
 // bit-identical; f is read once and the primitives are not read back.  KRK = 0: the last
 // RHS launch already wrote the stage's f; this reads it, writes the primitives, and
@@ -178,7 +179,26 @@ __device__ __forceinline__ double stage_cell(const KParams &k, ws_soa f, ws_soa 
     T.ptr[fidx(T.pitch, k.nyg, gx, gy, gz)] = p.T;
     if (P.ptr) P.ptr[fidx(P.pitch, k.nyg, gx, gy, gz)] = p.e / p.d * (k.gamma - 1.0);
     const double c = sqrt(p.T) / k.ama;
-    if (SOUND) cc.ptr[fidx(cc.pitch, k.nyg, gx, gy, gz)] = c;
+    if (SOUND) {
+        cc.ptr[fidx(cc.pitch, k.nyg, gx, gy, gz)] = c;
+        // the periodic face halo of the six fields, each ghost point by the cell it copies (a
+        // ghost fill behind this kernel before: three steps with CD8 terms of 157x111x75 3028 ->
+        // 3000 us, of 48x48x48 674 -> 650)
+        auto put = [&](int hx, int hy, int hz) {
+            d.ptr[fidx(d.pitch, k.nyg, hx, hy, hz)] = p.d;
+            u.ptr[fidx(u.pitch, k.nyg, hx, hy, hz)] = p.u;
+            v.ptr[fidx(v.pitch, k.nyg, hx, hy, hz)] = p.v;
+            w.ptr[fidx(w.pitch, k.nyg, hx, hy, hz)] = p.w;
+            T.ptr[fidx(T.pitch, k.nyg, hx, hy, hz)] = p.T;
+            cc.ptr[fidx(cc.pitch, k.nyg, hx, hy, hz)] = c;
+        };
+        if (x < LAP) put(gx + k.nx, gy, gz);
+        if (x >= k.nx - LAP) put(gx - k.nx, gy, gz);
+        if (y < LAP) put(gx, gy + k.ny, gz);
+        if (y >= k.ny - LAP) put(gx, gy - k.ny, gz);
+        if (z < LAP) put(gx, gy, gz + k.nz);
+        if (z >= k.nz - LAP) put(gx, gy, gz - k.nz);
+    }
     const bool plane = PLANES && (x == 0 || x == k.nx - 1 || y == 0 || y == k.ny - 1 || z == 0 || z == k.nz - 1);
     if (plane) plane_conserved(p, k.cv, r);
     if (KRK != 0 || plane)
@@ -315,16 +335,6 @@ __device__ __forceinline__ const AuxBlock &aux_block(const AuxBlock *tab, int nb
         else hi = mid - 1;
     }
     return tab[lo];
-}
-
-__global__ void __launch_bounds__(NT) k_ghost_fill_batch(const AuxBlock *tab, int nb, int set)
-{
-    const long wg = blockIdx.x;
-    const AuxBlock &b = aux_block<true>(tab, nb, wg);
-    GhostPoint q;
-    double val[6];
-    if (ghost_point(b.n[0], b.n[1], b.n[2], true, true, true, (wg - b.ghost_wg0) * NT + threadIdx.x, q))
-        ghost_copy<6>(b.g[set], 6, b.nyg, q, val);
 }
 
 // The sound speed of every block's interior (k_sound_speed's expression) by the first
@@ -592,15 +602,6 @@ int launch_min_reduce(const double *v, int n, double *out, hipStream_t s)
     hipLaunchKernelGGL(k_min_reduce, dim3(1), dim3(NT), 0, s, v, n, out);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? WS_OK : hip_error(e, "min reduce launch");
-}
-
-int launch_ghost_fill_batch(const AuxBlock *tab, int nb, long ghost_wgs, int set, hipStream_t s)
-{
-    if (set < 0 || set > 1) return set_error(WS_ERR_INVALID, "field set must be 0 or 1");
-    if (ghost_wgs <= 0 || nb <= 0) return WS_OK;
-    hipLaunchKernelGGL(k_ghost_fill_batch, dim3((unsigned)ghost_wgs), dim3(NT), 0, s, tab, nb, set);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? WS_OK : hip_error(e, "batched ghost fill launch");
 }
 
 int launch_prepare_batch(const KParams &k, const AuxBlock *tab, int nb, long ghost_wgs, long cell_wgs,

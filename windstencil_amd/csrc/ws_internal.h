@@ -240,15 +240,14 @@ struct AuxBlock {
 
 // Batched helper launches over a device table of nb blocks (k_aux.hip).  ghost_wgs and
 // cell_wgs: the table's last ghost_wg1 and cell_wg1.
-// Periodic ghost fill of field set `set` (0 or 1) of every block.
-int launch_ghost_fill_batch(const AuxBlock *tab, int nb, long ghost_wgs, int set, hipStream_t s);
 // cc = sqrt(T) / Ma on every block's interior (set 0), then the ghost fill of set 0: the
 // inputs of a batched RHS, as prepare_rhs_inputs leaves them on the cells the RHS reads.
 int launch_prepare_batch(const KParams &k, const AuxBlock *tab, int nb, long ghost_wgs, long cell_wgs,
                          hipStream_t s);
 // The stage kernel with krk 0 over every block (the last RHS launch already applied the
 // stage to f = fb when swapped, else fa): primitives of set 0 and P, with planes the
-// boundary planes, with sound the interior sound speed; cfl_part (cell_wgs entries): the
+// boundary planes, with sound the interior sound speed and the periodic halo of set 0;
+// cfl_part (cell_wgs entries): the
 // CFL maximum of each work-group.
 int launch_stage_batch(const KParams &k, const AuxBlock *tab, int nb, long cell_wgs, int swapped, bool planes,
                        bool sound, double *cfl_part, hipStream_t s);
