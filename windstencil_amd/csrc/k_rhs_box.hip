@@ -217,7 +217,7 @@ k_rhs_box(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc
                     double nP[1], dP[1], cP1[1], nM[1], dM[1], cM1[1];
                     weno_k<false, 1>([&](int i) { return qp[(i + j) * BOX_LT]; }, nP, dP, cP1);
                     weno_k<true, 1>([&](int i) { return qm[(i + j) * BOX_LT]; }, nM, dM, cM1);
-                    const double val = fma(fma(nP[0], dM[0], nM[0] * dP[0]), recip_nr(dP[0] * dM[0]), cP1[0] + cM1[0]) / kFace;
+                    const double val = face_merge(nP[0], dP[0], cP1[0], nM[0], dM[0], cM1[0]);
 #pragma unroll
                     for (int q = 0; q < K; ++q)
                         if (q == j) Fv[q] = val;
@@ -228,10 +228,7 @@ k_rhs_box(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc
             weno_k<false, K>([&](int j) { return qp[j * BOX_LT]; }, nP, dP, bP);
             weno_k<true, K>([&](int j) { return qm[j * BOX_LT]; }, nM, dM, bM);
 #pragma unroll
-            for (int j = 0; j < K; ++j) {
-                const double den = dP[j] * dM[j];
-                Fv[j] = fma(fma(nP[j], dM[j], nM[j] * dP[j]), recip_nr(den), bP[j] + bM[j]);
-            }
+            for (int j = 0; j < K; ++j) Fv[j] = face_merge(nP[j], dP[j], bP[j], nM[j], dM[j], bM[j]);
         }
         // finished here (the compiler would otherwise carry the parts to the store below)
 #pragma unroll
@@ -246,13 +243,12 @@ k_rhs_box(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc
     // ---- flux differences of this thread's cell, summed in the order of the directional launches
     double cmax = 0.0;
     if (cell) {
-        constexpr double FS = MIX ? 1.0 : kFace;
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             const int dir = order == WS_ORDER_ZYX ? 2 - q : q;
             const int i = dir == 0 ? ix : dir == 1 ? iy : iz;
             const int line = dir * BOX_LINES + (dir == 0 ? iy : ix) + B * (dir == 2 ? iy : iz);
-            const double scale = aj * (-k.rh[dir] / FS);
+            const double scale = aj * -k.rh[dir];
 #pragma unroll
             for (int m = 0; m < 5; ++m) {
                 const double val = scale * (sp[box_fidx(m, line, i + 1)] - sp[box_fidx(m, line, i)]);

@@ -409,9 +409,6 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
     const int line = t / TL::T, seg = t % TL::T;
     const int f0 = seg * K;                               // first face of this thread
     const bool active = (t < TL::NT) && (line >= g.lo_across) && (line < g.lim_across) && (f0 <= g.lim_line);
-    // face fluxes: times FS in the FP64 form (weno_k leaves its values times kFace; the flux
-    // difference of phase 3 divides by it)
-    constexpr double FS = MIX ? 1.0 : kFace;
     double Fv[5][K];
     // one-sided closures (BND): global index of the tile's first cell along the line
     const int n_dom = DIR == 0 ? k.nx : DIR == 1 ? k.ny : k.nz;
@@ -445,12 +442,12 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
             } else {
                 double nP[K], dP[K], nM[K], dM[K], bP[K], bM[K];
                 weno_k<false, K>([&](int j) { return qp[j]; }, nP, dP, bP);
+                // one half after the other: interleaved they hold 170 VGPRs instead of 139 in the
+                // launches that apply a stage, one wavefront per SIMD fewer
+                __builtin_amdgcn_sched_barrier(0);
                 weno_k<true, K>([&](int j) { return qm[j]; }, nM, dM, bM);
 #pragma unroll
-                for (int j = 0; j < K; ++j) {
-                    const double den = dP[j] * dM[j];
-                    Fv[m][j] = fma(fma(nP[j], dM[j], nM[j] * dP[j]), recip_nr(den), bP[j] + bM[j]);
-                }
+                for (int j = 0; j < K; ++j) Fv[m][j] = face_merge(nP[j], dP[j], bP[j], nM[j], dM[j], bM[j]);
             }
         }
         // Faces whose FP32 weights left FP32's range (strong discontinuities of the split
@@ -469,7 +466,7 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
                     double nP, dP, nM, dM, bP, bM;
                     face64<false>(qp + j, nP, dP, bP);
                     face64<true>(qm + j, nM, dM, bM);
-                    const double val = fma(fma(nP, dM, nM * dP), recip_nr(dP * dM), bP + bM) / kFace;
+                    const double val = face_merge(nP, dP, bP, nM, dM, bM);
 #pragma unroll
                     for (int q = 0; q < 5; ++q)
                         if (q == m) Fv[q][j] = val;
@@ -503,7 +500,7 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
                 if (!closure_p(cellP, n_dom, fg, lo, hi, pv)) {
                     double nP, dP, bP;
                     face64<false>(qp, nP, dP, bP);
-                    pv = (bP + nP / dP) / kFace;
+                    pv = fma(kNum, nP / dP, bP);
                     if (MIX) {
                         double bp[1], bm[1];
                         float cp[1], cm[1];
@@ -513,12 +510,12 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
                         if (!(badP | badM)) pv = bp[0] + (double)cp[0];
                     }
                 }
-                cval[r] = FS * (pv + mv);
+                cval[r] = pv + mv;
                 cat[r] = m * W * TL::F + TL::fidx(l, f);
                 if (nr_hi && fg == n_dom) {
                     double a = 0.0;
                     closure_p(cellP, n_dom, n_dom - 1, lo, hi, a);
-                    cfix[r] = FS * (pv - a);
+                    cfix[r] = pv - a;
                 }
             }
         }
@@ -569,7 +566,7 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
     __syncthreads();
 
     // ---- phase 3: flux difference of each cell ---------------------------------------------
-    const double scale0 = -k.rh[DIR] / FS;
+    const double scale0 = -k.rh[DIR];
     const double sdt = STG ? (sa.dt_dev ? *sa.dt_dev : sa.dt) : 0.0;
     double cfl_max = 0.0;
 #pragma unroll
@@ -602,7 +599,7 @@ __device__ __forceinline__ double tile_compute(const KParams &k, const ws_metric
                 double a = 0.0, b = 0.0;
                 closure_m(cellM, n_dom, 0, lo, hi, a);
                 closure_m(cellM, n_dom, 1, lo, hi, b);
-                val = scale * (FS * (b - a));
+                val = scale * (b - a);
             } else if (last_only_p) {
                 val = scale * nfix_lds[l * 5 + m];
             }

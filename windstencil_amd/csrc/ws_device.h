@@ -241,26 +241,33 @@ __device__ __forceinline__ void sqrt_rsqrt_h(double x, double &root, double &rcp
 }
 
 // K consecutive faces from K+7 points s[0..K+6] (face j uses s[j..j+7]); face j's value is
-// (base[j] + num[j] / den[j]) / kFace.  The forward differences up to the fourth and the
-// squared third differences (eps added) are formed once per point and shared by the K faces.
+// base[j] + kNum num[j] / den[j].  The forward differences and the squared third differences
+// (eps added) are formed once per point and shared by the K faces.
 //
-// Everything that differs between two neighbouring candidates at a face is a multiple of
-// one fourth difference D4_k of the window (points k .. k+4), so each candidate is the
-// central one plus one or two fourth differences.  With A = the first-derivative term,
-// b = the second-derivative term, q = the candidate value, of candidates 0..4 (unscaled):
-//   a1 = a2 + D4_1,  a0 = a1 - 2 D4_0,  a3 = a2 + 2 D4_2,  a4 = a3 + 11 D4_3
-//   b1 = D2_2,  b2 = D2_3,  b0 = b1 - D4_0,  b3 = b1 - D4_2,  b4 = b3 - 2 D4_3
-//   12 (q1 - q2) = D4_1,  12 (q0 - q2) = D4_1 - 3 D4_0
-//   12 (q3 - q2) = D4_2,  12 (q4 - q2) = D4_2 - 3 D4_3
-//   a2 = 6 D1_2 + 3 D2_2 - D3_2,  12 q2 = 12 w3 + a2 + D2_2
+// Candidate k covers the window's points k .. k+3.  Its first-derivative term a_k, its
+// second-derivative term b_k and its value's distance from the base point w3, c_k = 12 (q_k -
+// w3), are (unscaled, D1_i, D2_i, D3_i, D4_i the forward differences from point i)
+//   a0 = 6 D1_2 + 3 D2_1 + 2 D3_0    b0 = D2_1 + D3_0    c0 = a0 + b0
+//   a1 = 6 D1_2 + 3 D2_2 - D3_1      b1 = D2_2           c1 = a1 + b1
+//   a2 = 6 D1_2 + 3 D2_2 - D3_2      b2 = D2_3           c2 = a2 + b1
+//   a3 = 6 D1_3 - 3 D2_3 + 2 D3_3    b3 = D2_3 - D3_3    c3 = a3 + b3
+//   a4 = a3 + 11 D4_3                b4 = b3 - 2 D4_3    c4 = c3 - 3 D4_3
+// Each of candidates 0 to 3 is built from differences of its own four points only, so beside
+// a jump the candidates that do not cross it hold no value of the jump's size, and the face
+// keeps an error of an ulp of the smooth side whatever the jump.  Candidate 4 goes over
+// candidate 3: a jump inside 3 and outside 4 lies between points 3 and 4, where the cap on
+// e4 leaves candidate 4 no more weight than the one with the largest indicator.  (Building all
+// candidates from the central one by D4_0 .. D4_3 takes seven instructions fewer per face and
+// side but cancels the jump: 3e-14 of the quiet side's value at a ratio of 1e2, 3e-12 at 1e4,
+// 3e-4 at 1e12, against 1.2e-16 at any ratio.)
 // With d_k the linear weights over the central one, e_k = eps + S_k and P = e0 e1 e2 e3 e4,
-// D = sum d_k P / e_k and N = sum 12 d_k (q_k - q2) P / e_k (the central candidate drops out)
-// are formed in pairs (0, 1) and (3, 4): D01 = d0 e1 + d1 e0, N01 = D4_1 D01 - 3 D4_0 d0 e1.
+// D = sum d_k P / e_k and N = sum d_k c_k P / e_k are formed in pairs (0, 1) and (3, 4).
 // Bound by FP64 VALU issue (one instruction per four cycles), so the count is what matters:
-// 62 instructions per face and side with K = 2 against 86 with every candidate built from
-// its own differences (a whole RHS of 600x256x128 2.57 -> 2.23 ms on one box, an RK3 step of
-// 600x128x128 4.49 -> 3.94 ms).
-constexpr double kFace = 12.0;
+// 68 instructions per face and side with K = 2, against 86 with every candidate built by itself
+// and 62 for the central form above (a whole RHS of 600x256x128 2.19 ms, by the central form
+// 2.09; an RK3 step of 600x128x128 3.89 ms, 3.76).
+constexpr double kRho = kAS / kBS;              // c_k from the scaled a_k and b_k
+constexpr double kNum = 1.0 / (12.0 * kAS);     // c_k are formed kAS times
 
 template <bool REV, int K, typename Load>
 __device__ __forceinline__ void weno_k(Load ld, double (&num)[K], double (&den)[K], double (&base)[K])
@@ -270,38 +277,43 @@ __device__ __forceinline__ void weno_k(Load ld, double (&num)[K], double (&den)[
     // (at a tile edge) must come out bit for bit the same in both.
 #pragma clang fp contract(off)
     constexpr int NP = K + 7;
+    constexpr double SD = REV ? -1.0 : 1.0;     // odd differences of the reversed window change sign
     double s[NP];
 #pragma unroll
     for (int i = 0; i < NP; ++i) s[i] = ld(i);
-    double D1[NP - 1], D2[NP - 2], D3[NP - 3], D4[NP - 4], C3[NP - 3], B[K + 1], T[NP - 4];
+    double D1[NP - 1], D2[NP - 2], D3[NP - 3], C3[NP - 3], G[K + 1], B[K + 2];
 #pragma unroll
     for (int i = 0; i < NP - 1; ++i) D1[i] = s[i + 1] - s[i];
 #pragma unroll
     for (int i = 0; i < NP - 2; ++i) D2[i] = D1[i + 1] - D1[i];
 #pragma unroll
     for (int i = 0; i < NP - 3; ++i) { D3[i] = D2[i + 1] - D2[i]; C3[i] = fma(D3[i], D3[i], kEpsS); }
+    // the scaled first differences before and after each base point, and the scaled second
+    // differences of the window's inner points
+    constexpr int G0 = REV ? 3 : 2, B0 = REV ? 2 : 1;
 #pragma unroll
-    for (int i = 0; i < NP - 4; ++i) { D4[i] = D3[i + 1] - D3[i]; T[i] = 3.0 * D4[i]; }
-    // the scaled second differences centred on the two points beside each face
+    for (int i = 0; i < K + 1; ++i) G[i] = (6.0 * SD * kAS) * D1[G0 + i];
 #pragma unroll
-    for (int i = 0; i < K + 1; ++i) B[i] = kBS * D2[i + 2];
+    for (int i = 0; i < K + 2; ++i) B[i] = kBS * D2[B0 + i];
 #pragma unroll
     for (int j = 0; j < K; ++j) {
-        // differences of the window as the rule sees it (reversed for REV: odd ones change sign)
-        auto d4 = [&](int k) { return D4[REV ? j + 3 - k : j + k]; };
+        // differences of the window as the rule sees it (odd ones without their sign)
+        auto g1 = [&](int k) { return G[(REV ? j + 6 - k : j + k) - G0]; };
+        auto d2 = [&](int k) { return D2[REV ? j + 5 - k : j + k]; };
+        auto b = [&](int k) { return B[(REV ? j + 5 - k : j + k) - B0]; };
+        auto d3 = [&](int k) { return D3[REV ? j + 4 - k : j + k]; };
         auto c3 = [&](int k) { return C3[REV ? j + 4 - k : j + k]; };
-        const double d2c = D2[REV ? j + 3 : j + 2];
-        const double a2u = REV ? fma(-6.0, D1[j + 4], fma(3.0, d2c, D3[j + 2]))
-                               : fma(6.0, D1[j + 2], fma(3.0, d2c, -D3[j + 2]));
-        const double a2 = kAS * a2u;
-        const double a1 = fma(kAS, d4(1), a2);
-        const double a0 = fma(-2.0 * kAS, d4(0), a1);
-        const double a3 = fma(2.0 * kAS, d4(2), a2);
-        const double a4 = fma(11.0 * kAS, d4(3), a3);
-        const double b1 = B[REV ? j + 1 : j], b2 = B[REV ? j : j + 1];
-        const double b0 = fma(-kBS, d4(0), b1);
-        const double b3 = fma(-kBS, d4(2), b1);
-        const double b4 = fma(-2.0 * kBS, d4(3), b3);
+        const double d4 = REV ? D3[j + 1] - D3[j] : D3[j + 4] - D3[j + 3];
+        const double g12 = fma(3.0 * kAS, d2(2), g1(2));
+        const double a0 = fma(2.0 * SD * kAS, d3(0), fma(3.0 * kAS, d2(1), g1(2)));
+        const double a1 = fma(-SD * kAS, d3(1), g12);
+        const double a2 = fma(-SD * kAS, d3(2), g12);
+        const double a3 = fma(2.0 * SD * kAS, d3(3), fma(-3.0 * kAS, d2(3), g1(3)));
+        const double a4 = fma(11.0 * kAS, d4, a3);
+        const double b1 = b(2), b2 = b(3);
+        const double b0 = fma(SD * kBS, d3(0), b(1));
+        const double b3 = fma(-SD * kBS, d3(3), b2);
+        const double b4 = fma(-2.0 * kBS, d4, b3);
         // e_k = eps + S_k (eps rides in C3)
         const double e0 = fma(a0, a0, fma(b0, b0, c3(0)));
         const double e1 = fma(a1, a1, fma(b1, b1, c3(1)));
@@ -309,19 +321,26 @@ __device__ __forceinline__ void weno_k(Load ld, double (&num)[K], double (&den)[
         const double e3 = fma(a3, a3, fma(b3, b3, c3(3)));
         double e4 = fma(a4, a4, fma(b4, b4, c3(4)));
         e4 = fmax(fmax(fmax(e0, e1), fmax(e2, e3)), e4);
-        base[j] = fma(kFace, s[REV ? j + 4 : j + 3], a2u + d2c);
-        const double t0 = kR0 * e1, t4 = kR4 * e3;
-        const double D01 = fma(kR1, e0, t0), D34 = fma(kR3, e4, t4);
-        const double N01 = fma(d4(1), D01, -(T[REV ? j + 3 : j] * t0));
-        const double N34 = fma(d4(2), D34, -(T[REV ? j : j + 3] * t4));
-        const double p01 = e0 * e1, p34 = e3 * e4;
-        const double q01 = e2 * p34, q34 = e2 * p01;
-        num[j] = fma(N01, q01, N34 * q34);
-        den[j] = fma(p34, fma(e2, D01, p01), q34 * D34);
+        const double q0 = fma(kRho, b0, a0), q1 = fma(kRho, b1, a1), q2 = fma(kRho, b1, a2);
+        const double q3 = fma(kRho, b3, a3), q4 = fma(-3.0 * kAS, d4, q3);
+        base[j] = s[REV ? j + 4 : j + 3];
+        const double t0 = kR0 * e1, t1 = kR1 * e0, t3 = kR3 * e4, t4 = kR4 * e3;
+        const double N01 = fma(q0, t0, q1 * t1), N34 = fma(q3, t3, q4 * t4);
+        const double p01 = e0 * e1, p34 = e3 * e4, q34 = e2 * p01;
+        num[j] = fma(p34, fma(e2, N01, q2 * p01), q34 * N34);
+        den[j] = fma(p34, fma(e2, t0 + t1, p01), q34 * (t3 + t4));
     }
 }
 
-// One face of weno_k from the 8-point window q[0..7]: (base + num / den) / kFace is its value.
+// The value of a face from its two halves (weno_k<false> and weno_k<true>), merged over one
+// reciprocal.
+__device__ __forceinline__ double face_merge(double nP, double dP, double bP, double nM, double dM, double bM)
+{
+#pragma clang fp contract(off)
+    return fma(fma(nP, dM, nM * dP), kNum * recip_nr(dP * dM), bP + bM);
+}
+
+// One face of weno_k from the 8-point window q[0..7]: base + kNum num / den is its value.
 template <bool REV>
 __device__ __forceinline__ void face64(const double *q, double &num, double &den, double &base)
 {
