@@ -257,7 +257,7 @@ __device__ __forceinline__ void sqrt_rsqrt_h(double x, double &root, double &rcp
 // keeps an error of an ulp of the smooth side whatever the jump.  Candidate 4 goes over
 // candidate 3: a jump inside 3 and outside 4 lies between points 3 and 4, where the cap on
 // e4 leaves candidate 4 no more weight than the one with the largest indicator.  (Building all
-// candidates from the central one by D4_0 .. D4_3 takes seven instructions fewer per face and
+// candidates from the central one by D4_0 .. D4_3 takes six instructions fewer per face and
 // side but cancels the jump: 3e-14 of the quiet side's value at a ratio of 1e2, 3e-12 at 1e4,
 // 3e-4 at 1e12, against 1.2e-16 at any ratio.)
 // With d_k the linear weights over the central one, e_k = eps + S_k and P = e0 e1 e2 e3 e4,
@@ -640,12 +640,16 @@ __device__ __forceinline__ bool closure_m(Cell cell, int n, int f, bool lo, int 
 
 // Steger-Warming split in the form the tiled FP64 kernels use: A1..A3 the metric terms, sn = |A|
 // and rsn = 1/|A| supplied by the caller (constants when metrics are uniform).  With vs = A.u,
-// cs = c |A|, P_i twice the smoothed positive eigenvalues of vs, vs - cs, vs + cs and
-// s = P_2 + P_3, d = P_3 - P_2, the mass flux is f0 = t (c1 P_1 + s), the momentum flux f0 u_i +
-// t c/|A| d A_i and the energy flux t (P_1 vv + s (|u|^2/2 + c^2/2 + W2) + d c vs/|A|); the
-// negative part takes 2 vs - P_1, 4 vs - s and 4 cs - d.  71 FP64 instructions against the 108
-// of split_mixed (whose shifted velocities u -+ c k are spelled out); a tile splits 25-31 %
-// more points than it owns.
+// cs = c |A|, P_i twice the smoothed positive (or negative) eigenvalues of vs, vs - cs and
+// vs + cs, the mass flux is f0 = t (c1 P_1 + P_2 + P_3), the momentum flux f0 u_i + t c/|A| (P_3 -
+// P_2) A_i and the energy flux t (P_1 vv + P_2 (H - c vs/|A|) + P_3 (H + c vs/|A|)) with H =
+// |u|^2/2 + c^2/2 + W2.  75 FP64 instructions against the 108 of split_mixed (whose shifted
+// velocities u -+ c k are spelled out); a tile splits 25-31 % more points than it owns.  Both
+// halves are formed from their own eigenvalues: against 113-bit arithmetic the rounding of the
+// ten fluxes is 0.87 to 0.98 of split_mixed's form's (seven flows, at rest to Mach 10).  With the
+// negative ones as 2 vs - P_1 and so on, four instructions fewer, it is 0.93 to 1.09, and three
+// times that of its own in a supersonic stream's negative half (the RHS of 600x256x128 takes
+// 0.7 % longer than so).
 __device__ __forceinline__ void split_fast(const KParams &k, double d, double u, double v, double w,
                                            double cc, double A1, double A2, double A3, double sn,
                                            double rsn, double fp[5], double fm[5])
@@ -656,31 +660,25 @@ __device__ __forceinline__ void split_fast(const KParams &k, double d, double u,
     const double cs = cc * sn;
     const double E2 = vs - cs, E3 = vs + cs;
     // eps2 > 0 keeps the radicands positive and normal
-    const double P1 = vs + sqrt_h(fma(vs, vs, k.eps2));
-    const double P2 = E2 + sqrt_h(fma(E2, E2, k.eps2));
-    const double P3 = E3 + sqrt_h(fma(E3, E3, k.eps2));
+    const double S1 = sqrt_h(fma(vs, vs, k.eps2));
+    const double S2 = sqrt_h(fma(E2, E2, k.eps2));
+    const double S3 = sqrt_h(fma(E3, E3, k.eps2));
     const double t = d * k.quarter_rcp_gamma;
     const double cr = cc * rsn, cv = cr * vs, tc = t * cr;
     const double q = fma(w, w, fma(v, v, u * u));
     const double vv = k.gm1 * q, H = fma(0.5, q, k.c3h * (cc * cc));
-    const double sP = P2 + P3, dP = P3 - P2;
-    {
-        const double g = tc * dP;
-        fp[0] = t * fma(k.c1, P1, sP);
-        fp[1] = fma(g, A1, fp[0] * u);
-        fp[2] = fma(g, A2, fp[0] * v);
-        fp[3] = fma(g, A3, fp[0] * w);
-        fp[4] = t * fma(P1, vv, fma(sP, H, dP * cv));
-    }
-    {
-        const double M1 = fma(2.0, vs, -P1), sM = fma(4.0, vs, -sP), dM = fma(4.0, cs, -dP);
-        const double g = tc * dM;
-        fm[0] = t * fma(k.c1, M1, sM);
-        fm[1] = fma(g, A1, fm[0] * u);
-        fm[2] = fma(g, A2, fm[0] * v);
-        fm[3] = fma(g, A3, fm[0] * w);
-        fm[4] = t * fma(M1, vv, fma(sM, H, dM * cv));
-    }
+    const double H2 = H - cv, H3 = H + cv;
+    auto half = [&](double P1, double P2, double P3, double f[5]) {
+#pragma clang fp contract(off)
+        const double g = tc * (P3 - P2);
+        f[0] = t * (fma(k.c1, P1, P2) + P3);
+        f[1] = fma(g, A1, f[0] * u);
+        f[2] = fma(g, A2, f[0] * v);
+        f[3] = fma(g, A3, f[0] * w);
+        f[4] = t * fma(P3, H3, fma(P2, H2, P1 * vv));
+    };
+    half(vs + S1, E2 + S2, E3 + S3, fp);
+    half(vs - S1, E2 - S2, E3 - S3, fm);
 }
 
 // Steger-Warming split of the mixed-precision kernels: k1..k3 = A/|A|.  The mixed
