@@ -50,3 +50,72 @@ def test_quiet_side_of_a_jump_keeps_its_own_accuracy(orc, ws, axis, ratio):
         err = np.abs(du - ref)[tuple(quiet)].max(axis=(1, 2, 3)) / scale
         log(f"  axis {axis} ratio {ratio:g} tile {tile}: {err / EPS} eps")
         assert (err <= 64 * EPS).all()
+
+
+VIS = dict(re=500.0, pr=0.72, ref_t=288.15)
+SHEARED = (1.0, 0.2, -0.1, 0.15, 0.9, 0.05, -0.05, 0.12, 1.1, 0.8)
+
+
+def _device(a):
+    """A ghosted device tensor holding the interior array `a` (ghost layers zero)."""
+    import torch
+    nz, ny, nx = a.shape
+    t = W.ghosted_tensor(nx, ny, nz, 0)
+    t[4:-4, 4:-4, 4:4 + nx] = torch.from_numpy(np.ascontiguousarray(a))
+    return t
+
+
+def _viscous(prims, order, metrics=None, **kw):
+    """ws_viscous_rhs alone into a zero du (numpy, interior); metrics: ten interior arrays."""
+    import ctypes
+
+    import torch
+    nz, ny, nx = prims[0].shape
+    ctx = make_ctx(nx, ny, nz, viscous=order, **VIS, **kw)
+    terms = [_device(a) for a in (*prims[1:], *(metrics or ()))]
+    f = [W.field_of(t) for t in terms]
+    fl = (W.WsField * len(f))(*f)
+    W.check(W.lib().ws_ghost_fill_periodic(ctx.handle, fl, len(f), W.stream_handle()))
+    mf = None
+    if metrics:
+        mf = W.WsMetricFields()
+        for q in range(9):
+            mf.A[q] = f[4 + q]
+        mf.ajac = f[13]
+    du = W.soa_tensor(nx, ny, nz)
+    W.check(W.lib().ws_viscous_rhs(ctx.handle, *f[:4], ctypes.byref(mf) if mf else None, W.soa_of(du),
+                                   W.stream_handle()))
+    torch.cuda.synchronize()
+    return du.cpu().numpy()
+
+
+@pytest.mark.parametrize("mode", ["cartesian", "sheared", "fields"])
+@pytest.mark.parametrize("closed", [False, True])
+@pytest.mark.parametrize("order", [6, 8])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_constant_stress_exerts_no_force(ws, axis, order, closed, mode):
+    """A velocity across `axis` that changes by the same power of two from cell to cell, at
+    constant T: every difference is exact, so the stress is the same number at each cell and its
+    derivative, a sum of differences, exactly zero; along z as along x and y."""
+    n, across, step = 64, 12, 2.0 ** -4
+    i = np.arange(n)
+    line = step * (i if closed else np.minimum(i, n - i))
+    cells = slice(12, 52) if closed else slice(10, 23)    # 2 R cells off the faces and the kinks
+    shape = [across] * 3
+    shape[2 - axis] = n
+    ix = [None] * 3
+    ix[2 - axis] = slice(None)
+    prims = [np.ones(shape)] + [np.zeros(shape) for _ in range(3)] + [np.ones(shape)]
+    prims[1 + (axis + 1) % 3] = np.broadcast_to(line[tuple(ix)], shape)
+    kw = dict(hx=1 / 32, hy=1 / 32, hz=1 / 32, periodic=[1 - int(closed and d == axis) for d in range(3)],
+              d0_bound=[int(closed and q // 2 == axis) for q in range(6)])
+    metrics = None
+    if mode == "sheared":
+        kw["metric"] = SHEARED
+    if mode == "fields":
+        metrics = [np.full(shape, a) for a in SHEARED]
+    du = _viscous(prims, order, metrics, **kw)
+    at = [slice(None)] * 4
+    at[3 - axis] = cells
+    assert np.abs(du[4]).max() > 0          # the work term does vary
+    assert not du[tuple(at)][1:4].any()

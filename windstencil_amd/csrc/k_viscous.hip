@@ -441,9 +441,13 @@ __global__ void __launch_bounds__(NT) k_vis_div(VisParams p, EvFields ev, ws_fie
 // the plane with a further R-deep border, the z stencil from its column's register window)
 // and the fluxes its point contributes: x fluxes on the tile's rows, y fluxes on its columns,
 // z fluxes inside the tile.  The x and y fluxes go to LDS and are differentiated one plane
-// later; a z flux is added at once, weighted, to the 2R cells of its column whose derivative
-// it enters (register accumulators of the cells zf - R .. zf + R), so a cell is complete R
-// planes after its own flux plane.
+// later; a z flux is added at once, by its increment over the plane before, to the 2R cells of
+// its column whose derivative the two enter on either side (register accumulators of the cells
+// zf - R .. zf + R - 1), so a cell is complete R planes after its own flux plane.  With W_j = the
+// sum of the coefficients c_q, q >= max(j, 1 - j),
+//   sum_q c_q (F(c + q) - F(c - q)) = sum_j W_j (F(c + j) - F(c + j - 1)),  j = 1 - R .. R:
+// differences of the flux as along x and y, so a flux that does not change along z adds
+// nothing (its weighted values one by one would leave their rounding).
 //
 // Both LDS arrays are double-buffered: a step computes plane zf's fluxes from one copy,
 // writes the copy of plane zf + 1, and differentiates the fluxes of plane zf - 1, with one
@@ -484,9 +488,10 @@ enum { VC_NONE, VC_XY, VC_ALL };
 // Weights of the differences f(c + q) - f(c - q), q = 1..4 at index q - 1.
 struct VisWeights {
     double g[3][4];          // gradient along d: coefficient / h_d (VM_DIAG: times A_dd)
-    double f[3][4];          // flux derivative along d: coefficient / h_d times the Jacobian factors
+    double f[2][4];          // flux derivative along x and y: coefficient / h_d times the Jacobian factors
     double row[5][4];        // coefficients at distance 0..3 from a closed face, and the central ones
-    double rg[5][4], rf[5][4];   // the same times gs[2] and fs[2]
+    double rg[5][4];         // the same times gs[2]
+    double z[4], rz[5][4];   // the W_j = W_(1-j), j = 1..4, of the central form and of each row, times fs[2]
     double gs[3], fs[3];     // what g and f multiply the central coefficients by
 };
 
@@ -680,6 +685,16 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
     // slot (P + R + k) % Q at the step of phase P: plane zf + k of the column (c), and the
     // derivative sum of cell zf + k (acc)
     double c[4][Q], acc[4][Q];
+    // the z flux of plane zf - 1: in registers, but where an eighth-order instance has none to
+    // spare in LDS, which costs less than the scratch they would take (x closed 211x93x67 198 ->
+    // 178 us, all faces 220 -> 200, metric fields 256x160x96 394 -> 388)
+    constexpr bool FZL = ORDER == 8 && (BND || FLD);
+    __shared__ double fzl[4][FZL ? FNT : 1];
+    double fzr[4];
+    auto last = [&](int m) -> double & {
+        if constexpr (FZL) return fzl[m][threadIdx.x];
+        else return fzr[m];
+    };
     // loaded for the coming step: the newest column plane, the border of the plane after its
     // flux plane, du of the cell it writes, and with metric fields that cell's Jacobian
     double nq[4], hb[4], dn[4], jn = 0.0;
@@ -696,7 +711,7 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
         for (int q = 0; q < Q; ++q) acc[f][q] = 0.0;
         pl[0][f][mine] = c[f][R];
         hb[f] = at_border(fl[f], wb);
-        dn[f] = 0.0;
+        dn[f] = last(f) = 0.0;    // the first increment reaches no cell of the chunk
     }
     wb.next();
     if (bord)
@@ -742,9 +757,7 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
         wq.next();
         wb.next();
         __builtin_amdgcn_sched_barrier(0);
-        // Gradients and fluxes at this thread's flux point of plane zf; with a closed z face there
-        // are no fluxes past it.
-        const bool zin = !BNDZ || perz || (zf >= 0 && zf < p.nz);
+        // gradients and fluxes at this thread's flux point of plane zf
         if (BND) asm volatile("" : "+v"(wtx), "+v"(wty));    // the weights are read where they are used
         const double *pc = &pl[cur][0][own];
         double gk[4], gi[4], gs[4], met[FLD ? 10 : 1];
@@ -828,33 +841,37 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
             for (int m = 0; m < 4; ++m) fya[cur][m][ty * PX + tx] = F[m];
         }
         flux(2, F);
+        double G[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            G[m] = F[m] - last(m);
+            last(m) = F[m];
+        }
         if constexpr (BNDZ) {
+            // no flux changes past a closed z face
+            const bool zin = perz || (zf > 0 && zf < p.nz);
 #pragma unroll
             for (int q = 1; q <= R; ++q) {
-                const int zl = zf - q, zh = zf + q;
+                const int zl = zf - q, zh = zf + q - 1;
                 const int lo = closure_row(min(max(zl, 0), p.nz - 1), p.nz, zlo, zhi);
                 const int hi = closure_row(min(max(zh, 0), p.nz - 1), p.nz, zlo, zhi);
                 const bool ul = zin && (perz || zl >= 0) && q <= closure_reach<R>(lo);
                 const bool uh = zin && (perz || zh < p.nz) && q <= closure_reach<R>(hi);
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
-                    const double Fl = ul ? F[m] : 0.0, Fh = uh ? F[m] : 0.0;
-                    acc[m][slot(-q)] = fma(wt.rf[lo][q - 1], Fl, acc[m][slot(-q)]);
-                    acc[m][slot(q)] = q == R ? -wt.rf[hi][q - 1] * Fh : fma(-wt.rf[hi][q - 1], Fh, acc[m][slot(q)]);
+                    const double Gl = ul ? G[m] : 0.0, Gh = uh ? G[m] : 0.0;
+                    acc[m][slot(-q)] = fma(wt.rz[lo][q - 1], Gl, acc[m][slot(-q)]);
+                    acc[m][slot(q - 1)] =
+                        q == R ? wt.rz[hi][q - 1] * Gh : fma(wt.rz[hi][q - 1], Gh, acc[m][slot(q - 1)]);
                 }
             }
-            // the face cells' one-sided differences take the face point's flux on both sides
-            const bool first = zlo && zf == 0, last = zhi && zf == p.nz - 1;
-#pragma unroll
-            for (int m = 0; m < 4; ++m)
-                acc[m][slot(0)] = fma(wt.rf[0][0], last ? F[m] : first ? -F[m] : 0.0, acc[m][slot(0)]);
         } else {
 #pragma unroll
             for (int m = 0; m < 4; ++m)
 #pragma unroll
                 for (int q = 1; q <= R; ++q) {
-                    acc[m][slot(-q)] = fma(wt.f[2][q - 1], F[m], acc[m][slot(-q)]);
-                    acc[m][slot(q)] = q == R ? -wt.f[2][q - 1] * F[m] : fma(-wt.f[2][q - 1], F[m], acc[m][slot(q)]);
+                    acc[m][slot(-q)] = fma(wt.z[q - 1], G[m], acc[m][slot(-q)]);
+                    acc[m][slot(q - 1)] = q == R ? wt.z[q - 1] * G[m] : fma(wt.z[q - 1], G[m], acc[m][slot(q - 1)]);
                 }
         }
         // du of the cell the coming step writes: here rather than with the other loads, whose
@@ -880,7 +897,7 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
 #pragma unroll
         for (int m = 0; m < 4; ++m)
 #pragma unroll
-            for (int q = -R; q <= R; ++q) asm volatile("" : "+v"(acc[m][slot(q)]));
+            for (int q = -R; q < R; ++q) asm volatile("" : "+v"(acc[m][slot(q)]));
         ++zf;
         __syncthreads();
         cur = nxt;
@@ -917,28 +934,31 @@ void launch_fused(const VisParams &vp, ws_field u, ws_field v, ws_field w, ws_fi
 {
     constexpr int R = ORDER / 2;
     using FZ = Fused<R>;
-    const double coef[2][4] = {{45.0 / 60.0, -9.0 / 60.0, 1.0 / 60.0, 0.0},
-                               {672.0 / 840.0, -168.0 / 840.0, 32.0 / 840.0, -3.0 / 840.0}};
-    const double rows[4][4] = {{1.0, 0.0, 0.0, 0.0}, {0.5, 0.0, 0.0, 0.0}, {8.0 / 12.0, -1.0 / 12.0, 0.0, 0.0},
-                               {45.0 / 60.0, -9.0 / 60.0, 1.0 / 60.0, 0.0}};
+    // coefficients over their denominators: the four rows beside a closed face, the central form
+    const double num[5][4] = {{1, 0, 0, 0}, {1, 0, 0, 0}, {8, -1, 0, 0}, {45, -9, 1, 0},
+                              {ORDER == 8 ? 672.0 : 45.0, ORDER == 8 ? -168.0 : -9.0, ORDER == 8 ? 32.0 : 1.0,
+                               ORDER == 8 ? -3.0 : 0.0}};
+    const double den[5] = {1, 2, 12, 60, ORDER == 8 ? 840.0 : 60.0};
     VisWeights wt{};
     const double aj = vp.metric[9];
     for (int d = 0; d < 3; ++d) {
         const double A = MODE == VM_DIAG ? vp.metric[4 * d] : 1.0;
         wt.gs[d] = A / vp.h[d];
         wt.fs[d] = MODE == VM_FIELDS ? 1.0 / vp.h[d] : aj * (A * aj) / vp.h[d];
-        for (int q = 0; q < 4; ++q) {
-            wt.g[d][q] = coef[ORDER == 8][q] * wt.gs[d];
-            wt.f[d][q] = coef[ORDER == 8][q] * wt.fs[d];
+    }
+    for (int r = 0; r < 5; ++r) {
+        double sum = 0.0;
+        for (int q = 3; q >= 0; --q) {
+            sum += num[r][q];
+            wt.row[r][q] = num[r][q] / den[r];
+            wt.rg[r][q] = wt.row[r][q] * wt.gs[2];
+            wt.rz[r][q] = sum / den[r] * wt.fs[2];
         }
     }
     for (int q = 0; q < 4; ++q) {
-        for (int r = 0; r < 4; ++r) wt.row[r][q] = rows[r][q];
-        wt.row[4][q] = coef[ORDER == 8][q];
-        for (int r = 0; r < 5; ++r) {
-            wt.rg[r][q] = wt.row[r][q] * wt.gs[2];
-            wt.rf[r][q] = wt.row[r][q] * wt.fs[2];
-        }
+        wt.z[q] = wt.rz[4][q];
+        for (int d = 0; d < 3; ++d) wt.g[d][q] = wt.row[4][q] * wt.gs[d];
+        for (int d = 0; d < 2; ++d) wt.f[d][q] = wt.row[4][q] * wt.fs[d];
     }
     const bool bnd_xy = vp.bnd[0] || vp.bnd[1] || vp.bnd[2] || vp.bnd[3], bnd_z = vp.bnd[4] || vp.bnd[5];
     // one offset for every field: shared pitch, planes of fewer than 2^32 bytes
