@@ -119,3 +119,23 @@ def test_constant_stress_exerts_no_force(ws, axis, order, closed, mode):
     at[3 - axis] = cells
     assert np.abs(du[4]).max() > 0          # the work term does vary
     assert not du[tuple(at)][1:4].any()
+
+
+@pytest.mark.parametrize("order", [6, 8])
+@pytest.mark.parametrize("fields", [False, True])
+def test_viscous_terms_do_not_depend_on_the_chunks(ws, order, fields):
+    """A flow of four equal periods along z, and one of them alone: the march starts its chunks
+    at other planes, and the terms keep their bits."""
+    from tests.helpers import random_state
+    nx, ny, nz, reps = 53, 25, 40, 4
+    prims = random_state(nx, ny, nz, 19, "rough")
+    metrics = None
+    if fields:
+        from tests.test_gpu_rhs import _wavy_metrics
+        metrics = list(_wavy_metrics(nx, ny, nz))
+    h = dict(hx=0.02, hy=0.03, hz=0.025)
+    one = _viscous(prims, order, metrics, **h)
+    rep = lambda arrays: [np.concatenate([a] * reps) for a in arrays]
+    four = _viscous(rep(prims), order, rep(metrics) if metrics else None, **h)
+    for k in range(reps):
+        assert np.array_equal(four[:, k * nz:(k + 1) * nz], one), k

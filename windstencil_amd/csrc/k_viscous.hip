@@ -577,9 +577,11 @@ template <int ORDER, int MODE, int CLOSED, bool FAST>
 __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, ws_field u, ws_field v, ws_field w,
                                                    ws_field T, ws_metric_fields mf, ws_soa du, int zc)
 {
-    // contraction stays on here (the fast family's arithmetic need not follow the reference's
-    // order): every thread runs the same instructions for its flux point, so the flux at a
-    // point past a periodic face still equals the one at its image bit for bit
+    // Every fused multiply-add is written out: the step is compiled 2R + 1 times, and left to the
+    // compiler each of them could fuse differently, so that a flux would depend on the plane its
+    // chunk starts at.  So the flux at a point past a periodic face equals the one at its image
+    // bit for bit, and neither the chunks nor the tile a cell falls in change its bits.
+#pragma clang fp contract(off)
     constexpr int R = ORDER / 2, Q = 2 * R + 1;
     using FZ = Fused<R>;
     constexpr int PX = FZ::PX, PN = FZ::PN, XN = FZ::TY * FX, YN = FY * PX;
@@ -798,21 +800,22 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
             else return p.metric[q];
         };
         // physical derivatives from the computational ones (VM_DIAG: the weights carry A_dd)
-        auto px = [&](int f) { return MODE == VM_DIAG ? gk[f] : gk[f] * A(0) + gi[f] * A(3) + gs[f] * A(6); };
-        auto py = [&](int f) { return MODE == VM_DIAG ? gi[f] : gk[f] * A(1) + gi[f] * A(4) + gs[f] * A(7); };
-        auto pz = [&](int f) { return MODE == VM_DIAG ? gs[f] : gk[f] * A(2) + gi[f] * A(5) + gs[f] * A(8); };
+        auto dot = [](double a, double x, double b, double y, double c, double z) { return fma(c, z, fma(b, y, a * x)); };
+        auto px = [&](int f) { return MODE == VM_DIAG ? gk[f] : dot(gk[f], A(0), gi[f], A(3), gs[f], A(6)); };
+        auto py = [&](int f) { return MODE == VM_DIAG ? gi[f] : dot(gk[f], A(1), gi[f], A(4), gs[f], A(7)); };
+        auto pz = [&](int f) { return MODE == VM_DIAG ? gs[f] : dot(gk[f], A(2), gi[f], A(5), gs[f], A(8)); };
         const double ux = px(0), vx = px(1), wx_ = px(2), Tx = px(3);
         const double uy = py(0), vy = py(1), wy_ = py(2), Ty = py(3);
         const double uz = pz(0), vz = pz(1), wz = pz(2), Tz = pz(3);
-        const double div = ux + vy + wz;
-        const double s11 = (2.0 * ux - 2.0 / 3.0 * div) * amu;
-        const double s22 = (2.0 * vy - 2.0 / 3.0 * div) * amu;
-        const double s33 = (2.0 * wz - 2.0 / 3.0 * div) * amu;
+        const double div23 = -2.0 / 3.0 * (ux + vy + wz);
+        const double s11 = fma(2.0, ux, div23) * amu;
+        const double s22 = fma(2.0, vy, div23) * amu;
+        const double s33 = fma(2.0, wz, div23) * amu;
         const double s12 = (uy + vx) * amu, s13 = (uz + wx_) * amu, s23 = (vz + wy_) * amu;
         const double amuk = amu * p.vis_c;
-        const double E1 = uc * s11 + vc * s12 + wc * s13 + amuk * Tx;
-        const double E2 = uc * s12 + vc * s22 + wc * s23 + amuk * Ty;
-        const double E3 = uc * s13 + vc * s23 + wc * s33 + amuk * Tz;
+        const double E1 = fma(amuk, Tx, dot(uc, s11, vc, s12, wc, s13));
+        const double E2 = fma(amuk, Ty, dot(uc, s12, vc, s22, wc, s23));
+        const double E3 = fma(amuk, Tz, dot(uc, s13, vc, s23, wc, s33));
         // flux of direction d (the weights of its derivative carry the constant factors)
         auto flux = [&](int d, double out[4]) {
             if constexpr (MODE == VM_DIAG) {
@@ -823,10 +826,10 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
             } else {
                 double a1 = A(3 * d), a2 = A(3 * d + 1), a3 = A(3 * d + 2);
                 if constexpr (FLD) { a1 *= met[9]; a2 *= met[9]; a3 *= met[9]; }
-                out[0] = a1 * s11 + a2 * s12 + a3 * s13;
-                out[1] = a1 * s12 + a2 * s22 + a3 * s23;
-                out[2] = a1 * s13 + a2 * s23 + a3 * s33;
-                out[3] = a1 * E1 + a2 * E2 + a3 * E3;
+                out[0] = dot(a1, s11, a2, s12, a3, s13);
+                out[1] = dot(a1, s12, a2, s22, a3, s23);
+                out[2] = dot(a1, s13, a2, s23, a3, s33);
+                out[3] = dot(a1, E1, a2, E2, a3, E3);
             }
         };
         double F[4];
