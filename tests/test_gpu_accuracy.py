@@ -139,3 +139,21 @@ def test_viscous_terms_do_not_depend_on_the_chunks(ws, order, fields):
     four = _viscous(rep(prims), order, rep(metrics) if metrics else None, **h)
     for k in range(reps):
         assert np.array_equal(four[:, k * nz:(k + 1) * nz], one), k
+
+
+@pytest.mark.parametrize("fields", [False, True])
+def test_viscous_terms_of_a_cell_without_temperature(ws, fields):
+    """T = 0 has no viscosity (Sutherland's law gives 0): the terms stay finite and agree with
+    the anchor kernels."""
+    from tests.helpers import random_state, rel_l2
+    nx, ny, nz = 30, 20, 16
+    prims = [a.copy() for a in random_state(nx, ny, nz, 4, "vortex")]
+    prims[4][7, 9, 11] = 0.0
+    metrics = None
+    if fields:
+        from tests.test_gpu_rhs import _wavy_metrics
+        metrics = list(_wavy_metrics(nx, ny, nz))
+    ref = _viscous(prims, 6, metrics, kernel=W.WS_KERNEL_ANCHOR)
+    du = _viscous(prims, 6, metrics)
+    assert np.isfinite(ref).all() and np.isfinite(du).all()
+    assert rel_l2(du, ref) <= 1e-13

@@ -794,7 +794,8 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
                 }
         }
         const double uc = c[0][slot(0)], vc = c[1][slot(0)], wc = c[2][slot(0)], tc = c[3][slot(0)];
-        const double amu = p.amu_c0 * sqrt_h(tc * tc * tc) * recip_nr(p.tsb + tc);
+        // T^3 with a summand below its last bit, except for T = 0, of which sqrt_h is not defined
+        const double amu = p.amu_c0 * sqrt_h(fma(tc * tc, tc, 0x1p-1000)) * recip_nr(p.tsb + tc);
         auto A = [&](int q) {
             if constexpr (FLD) return met[q];
             else return p.metric[q];
