@@ -465,9 +465,11 @@ __global__ void __launch_bounds__(NT) k_vis_div(VisParams p, EvFields ev, ws_fie
 // weight is zero reads the cell itself on both sides.
 //
 // MODE: constant metrics without off-diagonal terms (a Cartesian box; the weights carry the
-// metric terms), constant metrics, or metric fields read per flux point.  FAST: the fields
-// share one pitch and a plane of them fits 32-bit byte offsets (the launcher checks), so one
-// offset per thread addresses them all; otherwise each field is addressed by itself.
+// metric terms), constant metrics, or metric fields read per flux point.  LAYOUT (the
+// launcher chooses): with one pitch and planes within 32-bit byte offsets one offset per thread
+// addresses every field (VL_ONE); with several pitches (VL_PITCHES) each load forms its own
+// from the thread's column and row, two instructions, rather than hold up to eighteen of them;
+// planes of 4 GB and more (VL_BIG) take 64-bit addresses.
 //
 // Algorithmic traffic 96 B per cell (constant metrics): u, v, w, T in and du[1..4] read and
 // written.  512 threads of up to 256 VGPRs: one work-group per compute unit.
@@ -484,6 +486,7 @@ __global__ void __launch_bounds__(NT) k_vis_div(VisParams p, EvFields ev, ws_fie
 constexpr int FX = 32, FY = 16, FNT = FX * FY;
 enum { VM_DIAG, VM_CONST, VM_FIELDS };
 enum { VC_NONE, VC_XY, VC_ALL };
+enum { VL_ONE, VL_PITCHES, VL_BIG };
 
 // Weights of the differences f(c + q) - f(c - q), q = 1..4 at index q - 1.
 struct VisWeights {
@@ -573,7 +576,7 @@ struct Phase {
     static constexpr int value = P;
 };
 
-template <int ORDER, int MODE, int CLOSED, bool FAST>
+template <int ORDER, int MODE, int CLOSED, int LAYOUT>
 __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, ws_field u, ws_field v, ws_field w,
                                                    ws_field T, ws_metric_fields mf, ws_soa du, int zc)
 {
@@ -619,26 +622,33 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
         bxw = wrap_coord(x0 - 2 * R + bpx, p.nx, perx);
         byw = wrap_coord(y0 - 2 * R + bpy, p.ny, pery);
     }
-    // FAST: byte offsets within a plane of the fields (they share u's pitch) and of du (threads
-    // without a cell point at its first)
+    // VL_ONE: byte offsets within a plane of the fields (they share u's pitch); VL_PITCHES: the
+    // column and row they come from; of du (threads without a cell point at its first)
     uint32_t off = 8u * ((uint32_t)(cxw + LAP) + u.pitch * (uint32_t)(cyw + LAP));
     uint32_t boff = 8u * ((uint32_t)(bxw + LAP) + u.pitch * (uint32_t)(byw + LAP));
+    uint32_t cx = 8u * (uint32_t)(cxw + LAP), cy = (uint32_t)(cyw + LAP);
+    uint32_t bx = 8u * (uint32_t)(bxw + LAP), by = (uint32_t)(byw + LAP);
     uint32_t doff = cell ? 8u * ((uint32_t)fx + du.pitch * (uint32_t)fy) : 0u;
     const size_t vstride = (size_t)du.pitch * p.ny * p.nz, dplane = 8 * (size_t)du.pitch * p.ny;
-    const size_t fplane = 8 * (size_t)u.pitch * nyg;          // FAST: bytes of a field's plane
+    const size_t fplane = 8 * (size_t)u.pitch * nyg;          // VL_ONE: bytes of a field's plane
+    auto plane_of = [&](const ws_field &f, const PlaneWalk<!BNDZ> &z) {
+        return (const char *)f.ptr + 8 * (size_t)f.pitch * (size_t)nyg * (size_t)(z.plane() + LAP);
+    };
     // element of field f at this thread's point of the plane a walk stands on
     auto at = [&](const ws_field &f, const PlaneWalk<!BNDZ> &z) -> double {
-        if constexpr (FAST) return *(const double *)((const char *)f.ptr + z.off + off);
+        if constexpr (LAYOUT == VL_ONE) return *(const double *)((const char *)f.ptr + z.off + off);
+        else if constexpr (LAYOUT == VL_PITCHES) return *(const double *)(plane_of(f, z) + (cx + 8u * f.pitch * cy));
         else return f.ptr[fidx(f.pitch, nyg, cxw + LAP, cyw + LAP, z.plane() + LAP)];
     };
     auto at_border = [&](const ws_field &f, const PlaneWalk<!BNDZ> &z) -> double {
-        if constexpr (FAST) return *(const double *)((const char *)f.ptr + z.off + boff);
+        if constexpr (LAYOUT == VL_ONE) return *(const double *)((const char *)f.ptr + z.off + boff);
+        else if constexpr (LAYOUT == VL_PITCHES) return *(const double *)(plane_of(f, z) + (bx + 8u * f.pitch * by));
         else return f.ptr[fidx(f.pitch, nyg, bxw + LAP, byw + LAP, z.plane() + LAP)];
     };
     double *const dm[4] = {du.ptr + vstride, du.ptr + 2 * vstride, du.ptr + 3 * vstride, du.ptr + 4 * vstride};
     // du[m + 1] of this thread's cell at plane offset z (bytes)
     auto du_at = [&](int m, size_t z) -> double & {
-        if constexpr (FAST) return *(double *)((char *)dm[m] + z + doff);
+        if constexpr (LAYOUT != VL_BIG) return *(double *)((char *)dm[m] + z + doff);
         else return *(double *)((char *)dm[m] + z + 8 * (cell ? (size_t)fx + (size_t)du.pitch * fy : 0));
     };
     // where this thread reads the plane copy; past a closed face the face point (BND), with the
@@ -735,6 +745,8 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
         const int nxt = cur ^ 1;
         // keeps the plane offsets scalar: the loads take them as their scalar base
         asm volatile("" : "+v"(off), "+v"(boff), "+v"(doff));
+        // and the fields' own offsets from being formed once for all steps and kept
+        if constexpr (LAYOUT == VL_PITCHES) asm volatile("" : "+v"(cx), "+v"(cy), "+v"(bx), "+v"(by));
         // the cell that the last step completed (its slot is the coming cell's)
         if (cell && zf - R - 1 >= z0)
 #pragma unroll
@@ -965,23 +977,33 @@ void launch_fused(const VisParams &vp, ws_field u, ws_field v, ws_field w, ws_fi
         for (int d = 0; d < 2; ++d) wt.f[d][q] = wt.row[4][q] * wt.fs[d];
     }
     const bool bnd_xy = vp.bnd[0] || vp.bnd[1] || vp.bnd[2] || vp.bnd[3], bnd_z = vp.bnd[4] || vp.bnd[5];
-    // one offset for every field: shared pitch, planes of fewer than 2^32 bytes
-    bool fast = v.pitch == u.pitch && w.pitch == u.pitch && T.pitch == u.pitch &&
-                (uint64_t)u.pitch * (uint64_t)vp.nyg < (1ull << 29) && (uint64_t)du.pitch * (uint64_t)vp.ny < (1ull << 29);
+    // the layout: shared pitch, planes of fewer than 2^32 bytes
+    bool one = true, small = (uint64_t)du.pitch * (uint64_t)vp.ny < (1ull << 29);
+    auto look = [&](const ws_field &f) {
+        one = one && f.pitch == u.pitch;
+        small = small && (uint64_t)f.pitch * (uint64_t)vp.nyg < (1ull << 29);
+    };
+    for (const ws_field &f : {u, v, w, T}) look(f);
     if (MODE == VM_FIELDS) {
-        for (int q = 0; q < 9; ++q) fast = fast && mf.A[q].pitch == u.pitch;
-        fast = fast && mf.ajac.pitch == u.pitch;
+        for (int q = 0; q < 9; ++q) look(mf.A[q]);
+        look(mf.ajac);
     }
     const long columns = (long)((vp.nx + FZ::TX - 1) / FZ::TX) * ((vp.ny + FZ::TY - 1) / FZ::TY);
     const int zc = fused_chunk(columns, vp.nz, R, cus);
     const long ntiles = columns * ((vp.nz + zc - 1) / zc);
     const dim3 g((unsigned)(8 * ((ntiles + 7) / 8)));
     auto go = [&](auto kern) { hipLaunchKernelGGL(kern, g, dim3(FNT), 0, s, vp, wt, u, v, w, T, mf, du, zc); };
-    // the closure form's table holds the central weights too: it also serves the rare layouts
-    if (!fast) go(k_vis_fused<ORDER, MODE, VC_ALL, false>);
-    else if (bnd_z) go(k_vis_fused<ORDER, MODE, VC_ALL, true>);
-    else if (bnd_xy) go(k_vis_fused<ORDER, MODE, VC_XY, true>);
-    else go(k_vis_fused<ORDER, MODE, VC_NONE, true>);
+    // the closure form's table holds the central weights too: it also serves the largest planes,
+    // and with several pitches any closed face.  T's pitch its own, with 64-bit addresses in the
+    // closure form for every such layout / now / one pitch: 256x160x96 sixth order 467 / 207 / 202
+    // us, eighth 917 / 305 / 300, x faces closed 157x111x75 184 / 137 and 371 / 228, metric fields
+    // 237 / 111 and 677 / 166
+    if (!small) go(k_vis_fused<ORDER, MODE, VC_ALL, VL_BIG>);
+    else if (!one && (bnd_z || bnd_xy)) go(k_vis_fused<ORDER, MODE, VC_ALL, VL_PITCHES>);
+    else if (!one) go(k_vis_fused<ORDER, MODE, VC_NONE, VL_PITCHES>);
+    else if (bnd_z) go(k_vis_fused<ORDER, MODE, VC_ALL, VL_ONE>);
+    else if (bnd_xy) go(k_vis_fused<ORDER, MODE, VC_XY, VL_ONE>);
+    else go(k_vis_fused<ORDER, MODE, VC_NONE, VL_ONE>);
 }
 
 template <int ORDER, bool FIELDS, bool BND>
