@@ -631,17 +631,21 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
     uint32_t doff = cell ? 8u * ((uint32_t)fx + du.pitch * (uint32_t)fy) : 0u;
     const size_t vstride = (size_t)du.pitch * p.ny * p.nz, dplane = 8 * (size_t)du.pitch * p.ny;
     const size_t fplane = 8 * (size_t)u.pitch * nyg;          // VL_ONE: bytes of a field's plane
+    // VL_ONE; with closed z faces formed from the plane: the four running offsets would not fit the
+    // scalar registers, and what spills takes vector ones (eighth order over metric fields 368 ->
+    // 132 bytes of scratch per lane; all faces closed 211x93x67 sixth order 157 -> 143 us)
+    auto plane_off = [&](const PlaneWalk<!BNDZ> &z) { return BNDZ ? fplane * (size_t)(z.plane() + LAP) : z.off; };
     auto plane_of = [&](const ws_field &f, const PlaneWalk<!BNDZ> &z) {
         return (const char *)f.ptr + 8 * (size_t)f.pitch * (size_t)nyg * (size_t)(z.plane() + LAP);
     };
     // element of field f at this thread's point of the plane a walk stands on
     auto at = [&](const ws_field &f, const PlaneWalk<!BNDZ> &z) -> double {
-        if constexpr (LAYOUT == VL_ONE) return *(const double *)((const char *)f.ptr + z.off + off);
+        if constexpr (LAYOUT == VL_ONE) return *(const double *)((const char *)f.ptr + plane_off(z) + off);
         else if constexpr (LAYOUT == VL_PITCHES) return *(const double *)(plane_of(f, z) + (cx + 8u * f.pitch * cy));
         else return f.ptr[fidx(f.pitch, nyg, cxw + LAP, cyw + LAP, z.plane() + LAP)];
     };
     auto at_border = [&](const ws_field &f, const PlaneWalk<!BNDZ> &z) -> double {
-        if constexpr (LAYOUT == VL_ONE) return *(const double *)((const char *)f.ptr + z.off + boff);
+        if constexpr (LAYOUT == VL_ONE) return *(const double *)((const char *)f.ptr + plane_off(z) + boff);
         else if constexpr (LAYOUT == VL_PITCHES) return *(const double *)(plane_of(f, z) + (bx + 8u * f.pitch * by));
         else return f.ptr[fidx(f.pitch, nyg, bxw + LAP, byw + LAP, z.plane() + LAP)];
     };
