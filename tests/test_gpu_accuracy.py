@@ -157,3 +157,23 @@ def test_viscous_terms_of_a_cell_without_temperature(ws, fields):
     du = _viscous(prims, 6, metrics)
     assert np.isfinite(ref).all() and np.isfinite(du).all()
     assert rel_l2(du, ref) <= 1e-13
+
+
+@pytest.mark.parametrize("flow", [(0.0, 0.0, 0.0), (0.4, 0.0, 0.0)])
+@pytest.mark.parametrize("precision,tol", [(W.WS_PREC_FP64, 1e-12), (W.WS_PREC_MIXED, 1e-6)])
+def test_no_smoothing_of_eigenvalues_at_rest(orc, ws, flow, precision, tol):
+    """epsl_sw = 0 is accepted: gas at rest, and directions without flow, have eigenvalues of
+    exactly zero, of which the split takes |0| = 0 (tiles and one-launch kernel, as the oracle)."""
+    from tests.helpers import rel_l2
+    rng = np.random.default_rng(11)
+    nx, ny, nz = 31, 17, 19
+    a = lambda: 1.0 + 0.2 * rng.random((nz, ny, nx))
+    prims = [a(), *(np.full((nz, ny, nx), q) for q in flow), a()]
+    ref = oracle_du(orc, prims, eps=0.0)
+    for tile in [None, *W.TILE_SHAPES]:
+        ctx = make_ctx(nx, ny, nz, precision=precision, epsl_sw=0.0)
+        if tile is not None:
+            ctx.set_tile_shape(tile)
+        err = rel_l2(gpu_du_comput(ctx, upload_state(prims)), ref)
+        log(f"  flow {flow} precision {precision} tile {tile}: rel L2 {err:.3e}")
+        assert err <= tol

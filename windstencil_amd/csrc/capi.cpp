@@ -37,6 +37,7 @@ KParams make_kparams(const ws_config &c)
     k.c3h = 0.5 + k.c3;
     k.gm1 = c.gamma - 1.0;
     k.eps2 = c.epsl_sw * c.epsl_sw;
+    k.eps2n = std::fmax(k.eps2, 0x1p-1000);
     k.ama = c.ama; k.rcp_ama = 1.0 / c.ama;
     k.cv = 1.0 / (c.gamma * (c.gamma - 1.0) * c.ama * c.ama);  // OCFD_init.cpp:380
     const double h[3] = {c.hx, c.hy, c.hz};

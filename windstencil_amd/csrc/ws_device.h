@@ -659,10 +659,10 @@ __device__ __forceinline__ void split_fast(const KParams &k, double d, double u,
     const double vs = fma(A3, w, fma(A2, v, A1 * u));
     const double cs = cc * sn;
     const double E2 = vs - cs, E3 = vs + cs;
-    // eps2 > 0 keeps the radicands positive and normal
-    const double S1 = sqrt_h(fma(vs, vs, k.eps2));
-    const double S2 = sqrt_h(fma(E2, E2, k.eps2));
-    const double S3 = sqrt_h(fma(E3, E3, k.eps2));
+    // eps2n keeps the radicands positive and normal (a point at rest without smoothing too)
+    const double S1 = sqrt_h(fma(vs, vs, k.eps2n));
+    const double S2 = sqrt_h(fma(E2, E2, k.eps2n));
+    const double S3 = sqrt_h(fma(E3, E3, k.eps2n));
     const double t = d * k.quarter_rcp_gamma;
     const double cr = cc * rsn, cv = cr * vs, tc = t * cr;
     const double q = fma(w, w, fma(v, v, u * u));
@@ -692,10 +692,10 @@ __device__ __forceinline__ void split_mixed(const KParams &k, double d, double u
     const double vs = fma(A3, w, fma(A2, v, A1 * u));
     const double cs = cc * sn;
     const double E1 = vs, E2 = vs - cs, E3 = vs + cs;
-    // eps2 > 0 keeps the radicands positive and normal
-    const double E1P = 0.5 * (E1 + sqrt_nr(fma(E1, E1, k.eps2)));
-    const double E2P = 0.5 * (E2 + sqrt_nr(fma(E2, E2, k.eps2)));
-    const double E3P = 0.5 * (E3 + sqrt_nr(fma(E3, E3, k.eps2)));
+    // eps2n keeps the radicands positive and normal (a point at rest without smoothing too)
+    const double E1P = 0.5 * (E1 + sqrt_nr(fma(E1, E1, k.eps2n)));
+    const double E2P = 0.5 * (E2 + sqrt_nr(fma(E2, E2, k.eps2n)));
+    const double E3P = 0.5 * (E3 + sqrt_nr(fma(E3, E3, k.eps2n)));
     const double E1M = E1 - E1P, E2M = E2 - E2P, E3M = E3 - E3P;
     const double t0 = d * k.half_rcp_gamma;
     const double ck1 = cc * k1, ck2 = cc * k2, ck3 = cc * k3;

@@ -24,6 +24,7 @@ struct KParams {
     double c3h;                // 0.5 + c3
     double gm1;                // gamma-1
     double eps2;               // epsl_sw^2
+    double eps2n;              // the same, at least 2^-1000: the fast splits' radicands, positive and normal
     double ama, rcp_ama;
     double cv;                 // 1/(gamma (gamma-1) Ma^2)
     double h[3];               // grid spacings
