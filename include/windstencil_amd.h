@@ -179,7 +179,7 @@ int ws_ctx_get_config(const ws_ctx *ctx, ws_config *out);
 int ws_ctx_set_precision(ws_ctx *ctx, int32_t precision);
 int ws_ctx_set_kernel(ws_ctx *ctx, int32_t kernel);
 /* WS_TILE_*.  Until a tile shape, a stage shape or a schedule is set, RHS calls on small jobs
- * (at most 1200 cells per compute unit, no closures) run one launch over cubes of 4^3 cells
+ * (at most 1400 cells per compute unit, no closures) run one launch over cubes of 4^3 cells
  * instead of the directional tiles, with the same bits. */
 int ws_ctx_set_tile_shape(ws_ctx *ctx, int32_t shape);
 int ws_ctx_get_tile_shape(const ws_ctx *ctx, int32_t *shape);

@@ -282,11 +282,16 @@ bool box_serves(const Ctx &c, const ws_job &job)
 {
     if (!c.box || c.kp.bnd_any[0] || c.kp.bnd_any[1] || c.kp.bnd_any[2]) return false;
     const long n = (long)(job.end.x - job.start.x) * (long)(job.end.y - job.start.y) * (long)(job.end.z - job.start.z);
-    // 1200 cells per compute unit, 307 thousand on 256: at 48x48x48 the directional tiles take
-    // 35.1 us (FP64; mixed 37.5) and this kernel 20.8 (21.4), at 100x60x40 51.6 (54.0) and 38.0
-    // (41.1), at 96x96x64, 393 thousand cells, 79.0 (81.8) and 84.7 (94.7): there the tiles
-    // fill the chip, and split 1.27 points per cell and direction where a cube splits 3
-    return n <= 1200l * c.compute_units;
+    // 1400 cells per compute unit, 358 thousand on 256.  du_comput by cubes / by tiles, in us:
+    //   thousand cells      196        262        319        368        409        460        589
+    //   FP64             42.5/54.1  49.7/60.3  61.5/68.8  68.5/75.4  74.1/74.7  85.2/84.8  106/99.6
+    //   mixed            37.6/53.9  50.3/59.5  61.6/66.7  69.6/74.2  79.6/72.9  87.5/83.1  111/98.0
+    //   metric fields    45.2/54.1  55.4/59.1  66.0/68.9  77.0/77.2  83.8/76.3  94.3/90.3  117/104
+    // RK3 steps cross between 368 (203/220) and 422 (255/250).  Then the tiles fill the chip, and
+    // split 1.27 points per cell and direction where a cube splits 3.  Cells and not cubes are
+    // counted: a job thinner than a cube leaves cubes partly empty, but tiles more so (600x256x1
+    // 95/101, 300x128x1 29/39, 1x256x16 8/25).
+    return n <= 1400l * c.compute_units;
 }
 
 long box_launch_tiles(const ws_job &job)
