@@ -75,7 +75,7 @@ bool tune_stage(ws_ctx *c, const ws_state *st, const ws_job &job, int reps, hipE
         for (int o = 0; o < WS_ORDER_COUNT; ++o) {
             c->stage_shape = sh;
             c->stage_order = o;
-            const long n = stage_launch_tiles(*c);
+            const long n = stage_launch_tiles(*c, state_reach(c->kp, *st));
             if (n > tiles) tiles = n;
         }
     c->stage_order = saved;
@@ -96,6 +96,7 @@ bool tune_stage(ws_ctx *c, const ws_state *st, const ws_job &job, int reps, hipE
     f.ptr = scratch;
     StageArgs sa{f, st->f, nullptr, c->cfg.dt, 2};
     sa.planes = c->cfg.bc_planes != 0;
+    sa.big = state_reach(c->kp, *st);
     if (prims) {
         ws_field *out[6] = {&sa.pd, &sa.pu, &sa.pv, &sa.pw, &sa.pT, &sa.pcc};
         for (int q = 0; q < 6; ++q) *out[q] = ws_field{scratch + 5 * fper + q * pper, st->d.pitch, 0};

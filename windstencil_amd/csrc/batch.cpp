@@ -92,13 +92,16 @@ void block_tiles(int b, const int n[3], int shape, int dir, std::vector<int4> &o
 }
 
 // the tile shape of the batch's stage-applying RHS
-int stage_shape_of(const ws_batch *b) { return b->stage_shape >= 0 ? b->stage_shape : b->tile_shape; }
+int stage_shape_of(const ws_batch *b)
+{
+    return b->big == 2 ? WS_TILE_30x16_K2 : b->stage_shape >= 0 ? b->stage_shape : b->tile_shape;
+}
 
 // the launch tables of the batch's RHS, or with `stage` of its stage-applying RHS
 BatchTiles tiles_of(const ws_batch *b, bool stage = false)
 {
     BatchTiles t;
-    t.shape = b->big ? WS_TILE_30x16_K2 : stage ? stage_shape_of(b) : b->tile_shape;
+    t.shape = stage || b->big == 2 ? stage_shape_of(b) : b->tile_shape;
     t.schedule = b->schedule;
     t.blocks = b->d_blocks;
     t.stage = nullptr;
@@ -278,7 +281,7 @@ int ws_batch_create(const ws_config *base, int32_t nblocks, const int32_t *exten
     for (int i = 0; i < nblocks; ++i) {
         const ws_state &st = states[i];
         if (!same_pitch(st.d, st.u, st.v, st.w, st.cc)) b->same_own = 0;
-        if (!rel_state(b->ctx[i]->kp, st)) b->big = 1;
+        b->big = std::max(b->big, state_reach(b->ctx[i]->kp, st));
     }
     hipError_t e = hipMalloc(&b->d_blocks, sizeof(BatchBlock) * nblocks);
     if (e != hipSuccess) return fail(b, set_error(WS_ERR_NOMEM, "batch block table"));
@@ -495,7 +498,7 @@ static int batch_step(ws_batch *b, const double *dt_dev, hipStream_t s, bool cfl
     // block's f and fn as created, and whether they are exchanged now is the same for all
     // blocks (they swap together).
     bool fuse = b->kernel == WS_KERNEL_TILED && !b->base.viscous && b->schedule == WS_SCHED_GRID &&
-                !b->big && b->ctx[0]->fuse_stage;
+                b->ctx[0]->fuse_stage;
     const int swapped = b->st[0].f.ptr == b->fb0 ? 1 : 0;
     for (size_t i = 0; i < b->st.size() && fuse; ++i)
         fuse = b->st[i].f.ptr == (swapped ? b->fbs[i] : b->fas[i]);
@@ -590,7 +593,7 @@ int ws_batch_rk3_step(ws_batch *b, const double *dt_dev, hipStream_t s)
 static bool batch_alternating(ws_batch *b, hipStream_t s, bool cfl)
 {
     if (b->kernel != WS_KERNEL_TILED || b->base.viscous || b->schedule != WS_SCHED_GRID ||
-        b->big || b->ctx[0]->fuse_stage < 3)
+        b->ctx[0]->fuse_stage < 3)
         return false;
     if (!prim_tables(b, s) || !aux_table(b, s) || !b->aux_second) return false;
     if (!cfl || b->d_cfl_tiles) return true;
@@ -797,7 +800,7 @@ int ws_batch_autotune(ws_batch *b, int32_t reps, float *times_ms, hipStream_t s)
             if (times_ms) times_ms[shape * WS_SCHED_COUNT + sched] = ms;
             if (ms < best_ms) { best_ms = ms; best_shape = shape; best_sched = sched; }
         }
-    if (!r && best_sched == WS_SCHED_GRID && !b->base.viscous && !b->big && b->ctx[0]->fuse_stage) {
+    if (!r && best_sched == WS_SCHED_GRID && !b->base.viscous && b->ctx[0]->fuse_stage) {
         b->tile_shape = best_shape;
         b->schedule = best_sched;
         // the stage candidates differ by 1-3 %: three times the repetitions

@@ -283,7 +283,7 @@ bool fused_stage_ok(const ws_ctx *c, const ws_state *st)
 {
     const bool closures = c->kp.bnd_any[0] || c->kp.bnd_any[1] || c->kp.bnd_any[2];
     return c->fuse_stage && c->cfg.kernel == WS_KERNEL_TILED && !c->cfg.viscous &&
-           (c->schedule == WS_SCHED_GRID || box_serves(*c, interior_job(c))) && !closures && rel_state(c->kp, *st);
+           (c->schedule == WS_SCHED_GRID || (!state_reach(c->kp, *st) && box_serves(*c, interior_job(c)))) && !closures;
 }
 
 bool alternating_steps(ws_ctx *c, const ws_state *st, hipStream_t s, bool cfl)
@@ -293,7 +293,7 @@ bool alternating_steps(ws_ctx *c, const ws_state *st, hipStream_t s, bool cfl)
     if (c->fuse_stage < 3 || !fused_stage_ok(c, st) || !periodic || !prim_set(c, s, second)) return false;
     if (!cfl) return true;
     // room for either producer's count (tiles of the stage launch; stage-kernel work-groups)
-    const long tiles = stage_launch_tiles(*c), blocks = stage_blocks(*c);
+    const long tiles = stage_launch_tiles(*c, state_reach(c->kp, *st)), blocks = stage_blocks(*c);
     const long need = tiles > blocks ? tiles : blocks;
     if (c->cfl_tiles_n < need) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -330,6 +330,7 @@ int rk3_step_fused(ws_ctx *c, ws_state *st, const double *dt_dev, hipStream_t s,
     const ws_soa nolap{};
     const bool periodic = c->cfg.periodic[0] && c->cfg.periodic[1] && c->cfg.periodic[2];
     const bool fuse = fused_stage_ok(c, st);
+    const int big = state_reach(c->kp, *st);
     ws_field second[6];
     const bool prims = fuse && periodic && c->fuse_stage > 1 && prim_set(c, s, second);
     const ws_field g[6] = {st->d, st->u, st->v, st->w, st->T, st->cc};
@@ -344,6 +345,7 @@ int rk3_step_fused(ws_ctx *c, ws_state *st, const double *dt_dev, hipStream_t s,
             const ws_field *in = krk == 2 ? B : A, *out = krk == 2 ? A : B;
             StageArgs sa{st->f, st->fn, dt_dev, c->cfg.dt, krk};
             sa.planes = planes;
+            sa.big = big;
             sa.pd = out[0]; sa.pu = out[1]; sa.pv = out[2]; sa.pw = out[3]; sa.pT = out[4];
             if (krk == 3 && last) {
                 sa.pP = st->P;
@@ -368,6 +370,7 @@ int rk3_step_fused(ws_ctx *c, ws_state *st, const double *dt_dev, hipStream_t s,
             const ws_field *in = krk == 2 ? second : g;
             const ws_field *out = krk == 1 ? second : g;
             StageArgs sa{st->f, st->fn, dt_dev, c->cfg.dt, krk};
+            sa.big = big;
             if (krk < 3) {
                 sa.planes = planes;
                 sa.pd = out[0]; sa.pu = out[1]; sa.pv = out[2]; sa.pw = out[3]; sa.pT = out[4]; sa.pcc = out[5];
@@ -381,7 +384,8 @@ int rk3_step_fused(ws_ctx *c, ws_state *st, const double *dt_dev, hipStream_t s,
             continue;
         }
         if (fuse) {
-            const StageArgs sa{st->f, st->fn, dt_dev, c->cfg.dt, krk};
+            StageArgs sa{st->f, st->fn, dt_dev, c->cfg.dt, krk};
+            sa.big = big;
             if (!r)
                 r = c->cfg.precision == WS_PREC_MIXED
                         ? launch_rhs_mixed_stage(*c, st->d, st->u, st->v, st->w, st->cc, st->du, interior_job(c), sa, s)
@@ -805,7 +809,7 @@ int ws_rk3_run(ws_ctx *c, ws_state *st, int32_t nsteps, double cfl, int32_t use_
     // c->cfl_tiles, and the last step ends in the state's fields.
     const bool alt = nsteps > 1 && alternating_steps(c, st, s, dt_dev != nullptr);
     double *cfl_next = !dt_dev ? nullptr : alt ? c->cfl_tiles : cfl_stage_buffer(c);
-    const int cfl_n = alt ? (int)stage_launch_tiles(*c) : (int)c->cfl_stage_n;
+    const int cfl_n = alt ? (int)stage_launch_tiles(*c, state_reach(c->kp, *st)) : (int)c->cfl_stage_n;
     auto mode_of = [&](int n) {
         if (!alt) return STEP_PLAIN;
         if (n == nsteps - 1) return (n & 1) ? STEP_LAST_FROM_SECOND : STEP_PLAIN;

@@ -334,8 +334,8 @@ int launch_prepared_rhs(const Ctx &c, const ws_state &st, const ws_metric_fields
 {
     const ws_job job = interior_job(&c);
     KParams k = c.kp;
-    *done = c.cfg.kernel == WS_KERNEL_TILED && box_serves(c, job) && (!m || rel_planes(k, *m)) &&
-            rel_planes(k, {st.d, st.u, st.v, st.w, st.T, st.cc}, {st.du});
+    *done = c.cfg.kernel == WS_KERNEL_TILED && box_serves(c, job) && (!m || !plane_reach(k, *m)) &&
+            !plane_reach(k, {st.d, st.u, st.v, st.w, st.T, st.cc}, {st.du});
     if (!*done) return WS_OK;
     k.same_pitch = same_pitch(st.d, st.u, st.v, st.w, st.cc) ? 1 : 0;
     const BoxPrep prep{st.T, {c.cfg.periodic[0], c.cfg.periodic[1], c.cfg.periodic[2]}};

@@ -16,12 +16,12 @@ int launch_rhs_tiled_stage(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_
     return launch_rhs_tile<false>(c, d, u, v, w, cc, nullptr, du, job, 0, s, &sa);
 }
 
-long stage_launch_tiles(const Ctx &c)
+long stage_launch_tiles(const Ctx &c, int big)
 {
     const ws_job job = interior_job(&c);
-    if (box_serves(c, job)) return box_launch_tiles(job);
+    if (!big && box_serves(c, job)) return box_launch_tiles(job);
     const Box box = job_box(job);
-    switch (c.stage_shape >= 0 ? c.stage_shape : c.tile_shape) {
+    switch (big == 2 ? WS_TILE_30x16_K2 : c.stage_shape >= 0 ? c.stage_shape : c.tile_shape) {
     case 0: return stage_tiles_n<0>(box, c.stage_order);
     case 1: return stage_tiles_n<1>(box, c.stage_order);
     case 2: return stage_tiles_n<2>(box, c.stage_order);

@@ -112,8 +112,8 @@ __device__ __forceinline__ TileGeo tile_geo(const Box &box, int bx, int by, int 
 // lane's byte offset within the tile: 32 bits, formed with one 24-bit multiply-add and
 // taken as such by the memory instructions, so an access costs no vector address
 // arithmetic of its own and five fields of one pitch share one offset.  That holds while
-// the planes of every field a launch touches are below kTilePlane elements (rel_planes); BIG
-// kernels keep 64-bit lane offsets for larger ones.  Against 64-bit addresses per access: the
+// the planes (z tiles) or rows (x and y tiles) of every field a launch touches are below
+// kTilePlane elements (plane_reach); BIG kernels keep 64-bit lane offsets for larger ones.  Against 64-bit addresses per access: the
 // FP64 RHS of 256x160x96 392 -> 383 us, over metric fields 535 -> 507 us, of 600x256x128
 // 1850 -> 1822 us.  The mixed kernels, which wait on memory rather than on issue, load their
 // primitives by 64-bit offsets: 600x256x128 takes 1902 us so, 1963 us with 32-bit ones, whose
@@ -673,7 +673,7 @@ k_rhs_tile(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field c
 // the tiles in launch order (x tiles fastest), so neighbouring tiles, which share halo
 // lines, run on the same work-group and XCD.  With PREFETCH the next tile's loads are
 // issued as soon as this tile's split has consumed the load registers.
-template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool PREFETCH>
+template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool PREFETCH, bool BIG>
 __global__ void __launch_bounds__(320)
 k_rhs_persist(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc, ws_soa du, Box box,
               int gx, int gy, int ntiles, int chunk)
@@ -690,15 +690,16 @@ k_rhs_persist(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_fiel
     };
     TileLoads<DIR, L, W, K, false> ld;
     TileGeo g = geo(first);
-    if (PREFETCH) tile_load<DIR, L, W, K, MIX>(k.nyg, d, u, v, w, cc, nullptr, g, ld, k.same_pitch);
+    if (PREFETCH) tile_load<DIR, L, W, K, BIG || MIX>(k.nyg, d, u, v, w, cc, nullptr, g, ld, k.same_pitch);
     for (int i = first; i < last; ++i) {
-        if (!PREFETCH) tile_load<DIR, L, W, K, MIX>(k.nyg, d, u, v, w, cc, nullptr, g, ld, k.same_pitch);
+        if (!PREFETCH) tile_load<DIR, L, W, K, BIG || MIX>(k.nyg, d, u, v, w, cc, nullptr, g, ld, k.same_pitch);
         const bool more = i + 1 < last;
         const TileGeo gn = more ? geo(i + 1) : g;
         auto next = [&] {
-            if (PREFETCH && more) tile_load<DIR, L, W, K, MIX>(k.nyg, d, u, v, w, cc, nullptr, gn, ld, k.same_pitch);
+            if (PREFETCH && more)
+                tile_load<DIR, L, W, K, BIG || MIX>(k.nyg, d, u, v, w, cc, nullptr, gn, ld, k.same_pitch);
         };
-        tile_compute<DIR, L, W, K, false, ACC, MIX, false, false, false>(k, nomf, du, g, ld, sp, StageArgs{}, next);
+        tile_compute<DIR, L, W, K, false, ACC, MIX, false, false, BIG>(k, nomf, du, g, ld, sp, StageArgs{}, next);
         __syncthreads();   // the next tile reuses the LDS buffer
         g = gn;
     }
@@ -709,7 +710,7 @@ k_rhs_persist(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_fiel
 // of the tile list, so neighbouring tiles (which share halo lines) run on the same
 // work-group, hence the same XCD and L2.  Each block brings its own fields, extents
 // and spacing; the physics constants and metrics are the batch's.
-template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool PREFETCH>
+template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool PREFETCH, bool BIG>
 __global__ void __launch_bounds__(320)
 k_rhs_batch(KParams k, const BatchBlock *blocks, const int4 *tiles, int ntiles, int chunk)
 {
@@ -737,7 +738,7 @@ k_rhs_batch(KParams k, const BatchBlock *blocks, const int4 *tiles, int ntiles, 
     TileGeo g = tile_geo<DIR, L, W, K>(box_of(blocks[tl.x]), tl.y, tl.z, tl.w);
     if (PREFETCH) {
         const BatchBlock &b = blocks[tl.x];
-        tile_load<DIR, L, W, K, MIX>(b.n[1] + 2 * LAP, b.d, b.u, b.v, b.w, b.cc, nullptr, g, ld, k.same_pitch);
+        tile_load<DIR, L, W, K, BIG || MIX>(b.n[1] + 2 * LAP, b.d, b.u, b.v, b.w, b.cc, nullptr, g, ld, k.same_pitch);
     }
     for (int i = first; i < last; ++i) {
         const BatchBlock &b = blocks[tl.x];
@@ -745,7 +746,8 @@ k_rhs_batch(KParams k, const BatchBlock *blocks, const int4 *tiles, int ntiles, 
         kb.nx = b.n[0]; kb.ny = b.n[1]; kb.nz = b.n[2];
         kb.nyg = b.n[1] + 2 * LAP; kb.nzg = b.n[2] + 2 * LAP;
         kb.rh[DIR] = b.rh[DIR];
-        if (!PREFETCH) tile_load<DIR, L, W, K, MIX>(kb.nyg, b.d, b.u, b.v, b.w, b.cc, nullptr, g, ld, k.same_pitch);
+        if (!PREFETCH)
+            tile_load<DIR, L, W, K, BIG || MIX>(kb.nyg, b.d, b.u, b.v, b.w, b.cc, nullptr, g, ld, k.same_pitch);
         const bool more = i + 1 < last;
         const int4 tn = more ? tile_at(i + 1) : tl;
         const TileGeo gn = tile_geo<DIR, L, W, K>(box_of(blocks[tn.x]), tn.y, tn.z, tn.w);
@@ -754,11 +756,11 @@ k_rhs_batch(KParams k, const BatchBlock *blocks, const int4 *tiles, int ntiles, 
         auto next = [&] {
             if (PREFETCH && more) {
                 const BatchBlock &bn = blocks[tn.x];
-                tile_load<DIR, L, W, K, MIX>(bn.n[1] + 2 * LAP, bn.d, bn.u, bn.v, bn.w, bn.cc, nullptr, gn, ld,
-                                        k.same_pitch);
+                tile_load<DIR, L, W, K, BIG || MIX>(bn.n[1] + 2 * LAP, bn.d, bn.u, bn.v, bn.w, bn.cc, nullptr, gn, ld,
+                                                    k.same_pitch);
             }
         };
-        tile_compute<DIR, L, W, K, false, ACC, MIX, false, false, false>(kb, nomf, b.du, g, ld, sp, StageArgs{}, next);
+        tile_compute<DIR, L, W, K, false, ACC, MIX, false, false, BIG>(kb, nomf, b.du, g, ld, sp, StageArgs{}, next);
         __syncthreads();   // the next tile reuses the LDS buffer
         tl = tn;
         g = gn;
@@ -821,18 +823,18 @@ int resident_of(Kern kern, int threads)
     return cus * per;
 }
 
-template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool PF>
+template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool PF, bool BIG>
 void launch_persist(const KParams &k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc, ws_soa du,
                     const Box &box, int gx, int gy, int gz, hipStream_t s)
 {
     using TL = Tile<DIR, L, W, K>;
-    static const int resident = resident_of(k_rhs_persist<DIR, L, W, K, ACC, MIX, PF>, TL::NT);
+    static const int resident = resident_of(k_rhs_persist<DIR, L, W, K, ACC, MIX, PF, BIG>, TL::NT);
     const int n = gx * gy * gz;
     if (n <= 0) return;
     int grid = resident < n ? resident : n;
     const int chunk = (n + grid - 1) / grid;
     grid = (n + chunk - 1) / chunk;
-    hipLaunchKernelGGL((k_rhs_persist<DIR, L, W, K, ACC, MIX, PF>), dim3(grid), dim3(TL::NT), 0, s, k, d, u, v, w,
+    hipLaunchKernelGGL((k_rhs_persist<DIR, L, W, K, ACC, MIX, PF, BIG>), dim3(grid), dim3(TL::NT), 0, s, k, d, u, v, w,
                        cc, du, box, gx, gy, n, chunk);
 }
 
@@ -854,13 +856,13 @@ void launch_dir(const KParams &k, ws_field d, ws_field u, ws_field v, ws_field w
         // one-sided closures in this direction: the grid schedule with the closure code
         hipLaunchKernelGGL((k_rhs_tile<DIR, L, W, K, FIELDS, ACC, MIX, true, false, BIG>), grid1, dim3(TL::NT), 0, s, k, d, u, v,
                            w, cc, mf, du, box, (int)grid.x, (int)grid.y, ntiles, StageArgs{});
-    } else if (FIELDS || BIG || sched == WS_SCHED_GRID) {
+    } else if (FIELDS || sched == WS_SCHED_GRID) {
         hipLaunchKernelGGL((k_rhs_tile<DIR, L, W, K, FIELDS, ACC, MIX, false, false, BIG>), grid1, dim3(TL::NT), 0, s, k, d, u,
                            v, w, cc, mf, du, box, (int)grid.x, (int)grid.y, ntiles, StageArgs{});
     } else if (sched == WS_SCHED_PREFETCH) {
-        launch_persist<DIR, L, W, K, ACC, MIX, true>(k, d, u, v, w, cc, du, box, grid.x, grid.y, grid.z, s);
+        launch_persist<DIR, L, W, K, ACC, MIX, true, BIG>(k, d, u, v, w, cc, du, box, grid.x, grid.y, grid.z, s);
     } else {
-        launch_persist<DIR, L, W, K, ACC, MIX, false>(k, d, u, v, w, cc, du, box, grid.x, grid.y, grid.z, s);
+        launch_persist<DIR, L, W, K, ACC, MIX, false, BIG>(k, d, u, v, w, cc, du, box, grid.x, grid.y, grid.z, s);
     }
 }
 
@@ -878,7 +880,7 @@ dim3 tile_grid(const Box &box)
 
 // The last launch of an RK3 stage that applies the stage itself (grid schedule, constant
 // metrics, no closures).
-template <int DIR, int L, int W, int K, bool MIX>
+template <int DIR, int L, int W, int K, bool MIX, bool BIG>
 void launch_dir_stage(const KParams &k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc, ws_soa du,
                       const Box &box, const StageArgs &sa, hipStream_t s)
 {
@@ -886,7 +888,7 @@ void launch_dir_stage(const KParams &k, ws_field d, ws_field u, ws_field v, ws_f
     const dim3 grid = tile_grid<DIR, L, W, K>(box);
     const int ntiles = (int)(grid.x * grid.y * grid.z);
     const ws_metric_fields nomf{};
-    hipLaunchKernelGGL((k_rhs_tile<DIR, L, W, K, false, true, MIX, false, true>), dim3(8 * ((ntiles + 7) / 8)),
+    hipLaunchKernelGGL((k_rhs_tile<DIR, L, W, K, false, true, MIX, false, true, BIG>), dim3(8 * ((ntiles + 7) / 8)),
                        dim3(TL::NT), 0, s, k, d, u, v, w, cc, nomf, du, box, (int)grid.x, (int)grid.y, ntiles, sa);
 }
 
@@ -894,37 +896,43 @@ void launch_dir_stage(const KParams &k, ws_field d, ws_field u, ws_field v, ws_f
 // read-modify-write it.  Which direction pays for that read shifts the time differently
 // per precision, so the order is a tuning choice (WS_ORDER_*).  With a stage (sa) the last
 // launch applies it instead of writing du.
-template <int L0, int W0, int L1, int W1, int L2, int W2, int K, bool FIELDS, bool MIX, bool BIG>
+template <int L0, int W0, int L1, int W1, int L2, int W2, int K, bool FIELDS, bool MIX, int BIG>
 void launch_all(const KParams &k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc,
                 const ws_metric_fields &mf, ws_soa du, const Box &box, int accumulate, int sched, int order,
                 const StageArgs *sa, hipStream_t s)
 {
+    constexpr bool BXY = BIG == 2, BZ = BIG != 0;     // which tiles take 64-bit offsets (KParams::big)
     if (order == WS_ORDER_ZYX) {
-        if (accumulate) launch_dir<2, L2, W2, K, FIELDS, true, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
-        else launch_dir<2, L2, W2, K, FIELDS, false, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
-        launch_dir<1, L1, W1, K, FIELDS, true, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
+        if (accumulate) launch_dir<2, L2, W2, K, FIELDS, true, MIX, BZ>(k, d, u, v, w, cc, mf, du, box, sched, s);
+        else launch_dir<2, L2, W2, K, FIELDS, false, MIX, BZ>(k, d, u, v, w, cc, mf, du, box, sched, s);
+        launch_dir<1, L1, W1, K, FIELDS, true, MIX, BXY>(k, d, u, v, w, cc, mf, du, box, sched, s);
         if constexpr (!FIELDS) {
             if (sa) {
-                launch_dir_stage<0, L0, W0, K, MIX>(k, d, u, v, w, cc, du, box, *sa, s);
+                launch_dir_stage<0, L0, W0, K, MIX, BXY>(k, d, u, v, w, cc, du, box, *sa, s);
                 return;
             }
         }
-        launch_dir<0, L0, W0, K, FIELDS, true, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
+        launch_dir<0, L0, W0, K, FIELDS, true, MIX, BXY>(k, d, u, v, w, cc, mf, du, box, sched, s);
         return;
     }
-    if (accumulate) launch_dir<0, L0, W0, K, FIELDS, true, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
-    else launch_dir<0, L0, W0, K, FIELDS, false, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
-    launch_dir<1, L1, W1, K, FIELDS, true, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
+    if (accumulate) launch_dir<0, L0, W0, K, FIELDS, true, MIX, BXY>(k, d, u, v, w, cc, mf, du, box, sched, s);
+    else launch_dir<0, L0, W0, K, FIELDS, false, MIX, BXY>(k, d, u, v, w, cc, mf, du, box, sched, s);
+    launch_dir<1, L1, W1, K, FIELDS, true, MIX, BXY>(k, d, u, v, w, cc, mf, du, box, sched, s);
     if constexpr (!FIELDS) {
         if (sa) {
-            launch_dir_stage<2, L2, W2, K, MIX>(k, d, u, v, w, cc, du, box, *sa, s);
+            launch_dir_stage<2, L2, W2, K, MIX, BZ>(k, d, u, v, w, cc, du, box, *sa, s);
             return;
         }
     }
-    launch_dir<2, L2, W2, K, FIELDS, true, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, sched, s);
+    launch_dir<2, L2, W2, K, FIELDS, true, MIX, BZ>(k, d, u, v, w, cc, mf, du, box, sched, s);
 }
 
-template <int S, bool FIELDS, bool MIX, bool BIG = false>
+template <int N>
+struct Int {
+    static constexpr int value = N;
+};
+
+template <int S, bool FIELDS, bool MIX, int BIG>
 void launch_shape_n(const KParams &k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc,
                     const ws_metric_fields &mf, ws_soa du, const Box &box, int acc, int sched, int order,
                     const StageArgs *sa, hipStream_t s)
@@ -939,18 +947,27 @@ void launch_shape(int shape, const KParams &k, ws_field d, ws_field u, ws_field 
                   const ws_metric_fields &mf, ws_soa du, const Box &box, int acc, int sched, int order,
                   const StageArgs *sa, hipStream_t s)
 {
-    if (k.big) {
-        // planes beyond 32-bit tile offsets: one shape serves them (and no stage is fused)
-        launch_shape_n<WS_TILE_30x16_K2, FIELDS, MIX, true>(k, d, u, v, w, cc, mf, du, box, acc, sched, order, sa, s);
-        return;
-    }
-    switch (shape) {
-    case 0: launch_shape_n<0, FIELDS, MIX>(k, d, u, v, w, cc, mf, du, box, acc, sched, order, sa, s); break;
-    case 1: launch_shape_n<1, FIELDS, MIX>(k, d, u, v, w, cc, mf, du, box, acc, sched, order, sa, s); break;
-    case 2: launch_shape_n<2, FIELDS, MIX>(k, d, u, v, w, cc, mf, du, box, acc, sched, order, sa, s); break;
-    case 3: launch_shape_n<3, FIELDS, MIX>(k, d, u, v, w, cc, mf, du, box, acc, sched, order, sa, s); break;
-    default: launch_shape_n<4, FIELDS, MIX>(k, d, u, v, w, cc, mf, du, box, acc, sched, order, sa, s); break;
-    }
+    auto go = [&](auto big) {
+        constexpr int BIG = decltype(big)::value;
+        auto run = [&](auto shape_n) {
+            launch_shape_n<decltype(shape_n)::value, FIELDS, MIX, BIG>(k, d, u, v, w, cc, mf, du, box, acc, sched, order, sa,
+                                                                       s);
+        };
+        if constexpr (BIG == 2) {
+            run(Int<WS_TILE_30x16_K2>{});      // rows of 13.1 million points: one shape serves them
+        } else {
+            switch (shape) {
+            case 0: run(Int<0>{}); break;
+            case 1: run(Int<1>{}); break;
+            case 2: run(Int<2>{}); break;
+            case 3: run(Int<3>{}); break;
+            default: run(Int<4>{}); break;
+            }
+        }
+    };
+    if (k.big == 0) go(Int<0>{});
+    else if (k.big == 1) go(Int<1>{});
+    else go(Int<2>{});
 }
 
 // tiles of the stage-applying launch (the last direction of `order`) of tile shape S
@@ -964,80 +981,67 @@ long stage_tiles_n(const Box &box, int order)
 
 // ---- batched launches ------------------------------------------------------------------
 
-template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool PF>
+// one direction over its tile list; STG: this launch applies the RK3 stage bt.stage (grid
+// schedule)
+template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool PF, bool STG, bool BIG>
 void launch_batch_dir(const KParams &k, const BatchTiles &bt, hipStream_t s)
 {
     const int n = bt.ntiles[DIR];
     if (n <= 0) return;
-    if constexpr (DIR == 2 && ACC) {
-        if (bt.stage) {
-            // the last launch applies the RK3 stage (grid schedule only: the caller checks)
-            hipLaunchKernelGGL((k_rhs_batch_grid<DIR, L, W, K, true, MIX, true>), dim3(8 * ((n + 7) / 8)),
-                               dim3(Tile<DIR, L, W, K>::NT), 0, s, k, bt.blocks, bt.tiles[DIR], n, *bt.stage);
-            return;
-        }
-    }
-    if (bt.schedule == WS_SCHED_GRID) {
-        hipLaunchKernelGGL((k_rhs_batch_grid<DIR, L, W, K, ACC, MIX>), dim3(8 * ((n + 7) / 8)),
-                           dim3(Tile<DIR, L, W, K>::NT), 0, s, k, bt.blocks, bt.tiles[DIR], n, BatchStage{});
+    constexpr int NT = Tile<DIR, L, W, K>::NT;
+    if (STG || bt.schedule == WS_SCHED_GRID) {
+        hipLaunchKernelGGL((k_rhs_batch_grid<DIR, L, W, K, ACC, MIX, STG, BIG>), dim3(8 * ((n + 7) / 8)), dim3(NT), 0, s,
+                           k, bt.blocks, bt.tiles[DIR], n, STG ? *bt.stage : BatchStage{});
         return;
     }
-    static const int resident = resident_of(k_rhs_batch<DIR, L, W, K, ACC, MIX, PF>, Tile<DIR, L, W, K>::NT);
+    static const int resident = resident_of(k_rhs_batch<DIR, L, W, K, ACC, MIX, PF, BIG>, NT);
     int grid = resident < n ? resident : n;
     const int chunk = (n + grid - 1) / grid;
     grid = (n + chunk - 1) / chunk;
-    hipLaunchKernelGGL((k_rhs_batch<DIR, L, W, K, ACC, MIX, PF>), dim3(grid), dim3(Tile<DIR, L, W, K>::NT), 0, s,
-                       k, bt.blocks, bt.tiles[DIR], n, chunk);
+    hipLaunchKernelGGL((k_rhs_batch<DIR, L, W, K, ACC, MIX, PF, BIG>), dim3(grid), dim3(NT), 0, s, k, bt.blocks,
+                       bt.tiles[DIR], n, chunk);
 }
 
-// one tile per work-group over direction DIR's tile list (the grid schedule), STG: this
-// launch applies the RK3 stage bt.stage
-template <int DIR, int L, int W, int K, bool ACC, bool MIX, bool STG, bool BIG = false>
-void launch_batch_grid(const KParams &k, const BatchTiles &bt, hipStream_t s)
-{
-    const int n = bt.ntiles[DIR];
-    if (n <= 0) return;
-    hipLaunchKernelGGL((k_rhs_batch_grid<DIR, L, W, K, ACC, MIX, STG, BIG>), dim3(8 * ((n + 7) / 8)),
-                       dim3(Tile<DIR, L, W, K>::NT), 0, s, k, bt.blocks, bt.tiles[DIR], n,
-                       STG ? *bt.stage : BatchStage{});
-}
-
-template <int S, bool MIX, bool PF>
+template <int S, bool MIX, bool PF, int BIG>
 void launch_batch_shape_n(const KParams &k, const BatchTiles &bt, hipStream_t s)
 {
     constexpr TileShapeDef D = kTileShapes[S];
-    if (k.big) {
-        // planes beyond 32-bit tile offsets: the grid schedule in this one shape (the caller
-        // passes its tile lists)
-        if constexpr (S == WS_TILE_30x16_K2 && !PF) {
-            launch_batch_grid<0, D.L0, D.W0, D.K, false, MIX, false, true>(k, bt, s);
-            launch_batch_grid<1, D.L1, D.W1, D.K, true, MIX, false, true>(k, bt, s);
-            launch_batch_grid<2, D.L2, D.W2, D.K, true, MIX, false, true>(k, bt, s);
-        }
-        return;
-    }
+    constexpr bool BXY = BIG == 2, BZ = BIG != 0;     // which tiles take 64-bit offsets (KParams::big)
     if (bt.stage && bt.stage_order == WS_ORDER_ZYX) {
         // z writes du, y accumulates, x adds its terms and applies the stage
-        launch_batch_grid<2, D.L2, D.W2, D.K, false, MIX, false>(k, bt, s);
-        launch_batch_grid<1, D.L1, D.W1, D.K, true, MIX, false>(k, bt, s);
-        launch_batch_grid<0, D.L0, D.W0, D.K, true, MIX, true>(k, bt, s);
+        launch_batch_dir<2, D.L2, D.W2, D.K, false, MIX, PF, false, BZ>(k, bt, s);
+        launch_batch_dir<1, D.L1, D.W1, D.K, true, MIX, PF, false, BXY>(k, bt, s);
+        launch_batch_dir<0, D.L0, D.W0, D.K, true, MIX, PF, true, BXY>(k, bt, s);
         return;
     }
-    launch_batch_dir<0, D.L0, D.W0, D.K, false, MIX, PF>(k, bt, s);
-    launch_batch_dir<1, D.L1, D.W1, D.K, true, MIX, PF>(k, bt, s);
-    launch_batch_dir<2, D.L2, D.W2, D.K, true, MIX, PF>(k, bt, s);
+    launch_batch_dir<0, D.L0, D.W0, D.K, false, MIX, PF, false, BXY>(k, bt, s);
+    launch_batch_dir<1, D.L1, D.W1, D.K, true, MIX, PF, false, BXY>(k, bt, s);
+    if (bt.stage) launch_batch_dir<2, D.L2, D.W2, D.K, true, MIX, PF, true, BZ>(k, bt, s);
+    else launch_batch_dir<2, D.L2, D.W2, D.K, true, MIX, PF, false, BZ>(k, bt, s);
+}
+
+template <bool MIX, bool PF, int BIG>
+void launch_batch_big(const KParams &k, const BatchTiles &bt, hipStream_t s)
+{
+    if constexpr (BIG == 2) {
+        launch_batch_shape_n<WS_TILE_30x16_K2, MIX, PF, BIG>(k, bt, s);   // the shape of tiles_of then
+    } else {
+        switch (bt.shape) {
+        case 0: launch_batch_shape_n<0, MIX, PF, BIG>(k, bt, s); break;
+        case 1: launch_batch_shape_n<1, MIX, PF, BIG>(k, bt, s); break;
+        case 2: launch_batch_shape_n<2, MIX, PF, BIG>(k, bt, s); break;
+        case 3: launch_batch_shape_n<3, MIX, PF, BIG>(k, bt, s); break;
+        default: launch_batch_shape_n<4, MIX, PF, BIG>(k, bt, s); break;
+        }
+    }
 }
 
 template <bool MIX, bool PF>
 void launch_batch_pf(const KParams &k, const BatchTiles &bt, hipStream_t s)
 {
-    switch (bt.shape) {
-    case 0: launch_batch_shape_n<0, MIX, PF>(k, bt, s); break;
-    case 1: launch_batch_shape_n<1, MIX, PF>(k, bt, s); break;
-    case 2: launch_batch_shape_n<2, MIX, PF>(k, bt, s); break;
-    case 3: launch_batch_shape_n<3, MIX, PF>(k, bt, s); break;
-    default: launch_batch_shape_n<4, MIX, PF>(k, bt, s); break;
-    }
+    if (k.big == 0) launch_batch_big<MIX, PF, 0>(k, bt, s);
+    else if (k.big == 1) launch_batch_big<MIX, PF, 1>(k, bt, s);
+    else launch_batch_big<MIX, PF, 2>(k, bt, s);
 }
 
 template <bool MIX>
@@ -1051,7 +1055,7 @@ int launch_rhs_tile(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w
     const int order = sa ? c.stage_order : c.dir_order;
     KParams k = c.kp;
     k.same_pitch = same_pitch(d, u, v, w, cc) ? 1 : 0;
-    k.big = rel_planes(k, {d, u, v, w, cc}, {du}) && (!m || rel_planes(k, *m)) ? 0 : 1;
+    k.big = sa ? sa->big : std::max(plane_reach(k, {d, u, v, w, cc}, {du}), m ? plane_reach(k, *m) : 0);
     if (!k.big && box_serves(c, job)) {
         launch_rhs_box(MIX, k, d, u, v, w, cc, m, du, job, order, accumulate, sa, nullptr, s);
     } else if (m) {
@@ -1068,7 +1072,7 @@ int launch_rhs_tile(const Ctx &c, ws_field d, ws_field u, ws_field v, ws_field w
 template <bool MIX>
 int launch_rhs_batch_tile(const KParams &k, const BatchTiles &bt, hipStream_t s)
 {
-    if (bt.schedule == WS_SCHED_PREFETCH && !k.big) launch_batch_pf<MIX, true>(k, bt, s);
+    if (bt.schedule == WS_SCHED_PREFETCH) launch_batch_pf<MIX, true>(k, bt, s);
     else launch_batch_pf<MIX, false>(k, bt, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_error(e, MIX ? "batched mixed-precision RHS launch" : "batched RHS launch");

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstdint>
 #include <initializer_list>
 #include <string>
@@ -42,7 +43,8 @@ struct KParams {
     int nonref[6];
     int bnd_any[3];
     // set per launch: the RHS inputs d, u, v, w, cc share d's pitch, so one offset addresses
-    // all five; big: a field of the launch has planes of kTilePlane elements or more
+    // all five; big: 1 when a field of the launch has planes of kTilePlane elements or more (the
+    // z tiles take 64-bit offsets), 2 when it has rows of that length (all tiles do)
     int same_pitch = 0;
     int big = 0;
 };
@@ -55,35 +57,31 @@ inline bool same_pitch(const ws_field &d, const ws_field &u, const ws_field &v, 
 // The tiled kernels address a tile's points by 32-bit byte offsets from its first one, formed
 // with 24-bit products.  The longest reach is that of z tiles: at most 40 planes (L + 2 LAP
 // with L = 32) and one row, so planes below (2^32 / 8) / 41 elements, about 13.1 million, keep
-// every offset below 2^32 and every stride below 2^24.  x tiles reach 16 rows, y tiles 40, both
-// within a plane's rows or (few rows per plane) below 40 pitches.
+// every offset below 2^32 and every stride below 2^24.  x tiles reach 16 rows and y tiles 40,
+// so for them the same limit holds for a row.
 constexpr unsigned long long kTilePlane = (1ull << 29) / 41;
 
-inline bool rel_field(const ws_field &f, int rows)
+// KParams::big over the fields given (absent ones aside)
+template <typename Field>
+inline int reach_of(const Field &f, int rows)
 {
-    return !f.ptr || (unsigned long long)f.pitch * (unsigned long long)rows < kTilePlane;
+    if (!f.ptr) return 0;
+    return f.pitch >= kTilePlane ? 2 : (unsigned long long)f.pitch * (unsigned long long)rows >= kTilePlane ? 1 : 0;
 }
 
-inline bool rel_soa(const ws_soa &f, int rows)
+inline int plane_reach(const KParams &k, std::initializer_list<ws_field> fields, std::initializer_list<ws_soa> states)
 {
-    return !f.ptr || (unsigned long long)f.pitch * (unsigned long long)rows < kTilePlane;
+    int big = 0;
+    for (const ws_field &f : fields) big = std::max(big, reach_of(f, k.nyg));
+    for (const ws_soa &f : states) big = std::max(big, reach_of(f, k.ny));
+    return big;
 }
 
-// whether every field given has planes the tiles' 32-bit offsets reach
-inline bool rel_planes(const KParams &k, std::initializer_list<ws_field> fields, std::initializer_list<ws_soa> states)
+inline int plane_reach(const KParams &k, const ws_metric_fields &m)
 {
-    for (const ws_field &f : fields)
-        if (!rel_field(f, k.nyg)) return false;
-    for (const ws_soa &f : states)
-        if (!rel_soa(f, k.ny)) return false;
-    return true;
-}
-
-inline bool rel_planes(const KParams &k, const ws_metric_fields &m)
-{
-    for (const ws_field &f : m.A)
-        if (!rel_field(f, k.nyg)) return false;
-    return rel_field(m.ajac, k.nyg);
+    int big = reach_of(m.ajac, k.nyg);
+    for (const ws_field &f : m.A) big = std::max(big, reach_of(f, k.nyg));
+    return big;
 }
 
 // The SSP-RK3 stage the last directional RHS launch applies to its cells itself (f from fn,
@@ -107,14 +105,17 @@ struct StageArgs {
     // ghost fill of those fields would make from the interior cells written here (every
     // direction periodic)
     int halo = 0;
+    // KParams::big of the launch: state_reach, the same for every stage of a step, which
+    // decides what runs it (and so the entries of cfl_part)
+    int big = 0;
 };
 
-// whether the tiles' 32-bit offsets reach all of a state and the context's second primitive
-// set (its pitch: nx + 2 LAP rounded to 32)
-inline bool rel_state(const KParams &k, const ws_state &st)
+// KParams::big over all of a state and the context's second primitive set (its pitch: nx + 2 LAP
+// rounded to 32)
+inline int state_reach(const KParams &k, const ws_state &st)
 {
     const ws_field second{st.d.ptr, (uint32_t)((k.nx + 2 * LAP + 31) / 32 * 32), 0};
-    return rel_planes(k, {st.d, st.u, st.v, st.w, st.T, st.P, st.cc, second}, {st.f, st.fn, st.du});
+    return plane_reach(k, {st.d, st.u, st.v, st.w, st.T, st.P, st.cc, second}, {st.f, st.fn, st.du});
 }
 
 struct Ctx {
@@ -295,8 +296,9 @@ void launch_rhs_box(bool mixed, const KParams &k, ws_field d, ws_field u, ws_fie
                     const ws_metric_fields *m, ws_soa du, const ws_job &job, int order, int accumulate,
                     const StageArgs *sa, const BoxPrep *prep, hipStream_t s);
 // work-groups of the context's launch that applies an RK3 stage (the last direction of its
-// order, in its tile shape, or the one-launch kernel): the entries that launch writes to StageArgs::cfl_part
-long stage_launch_tiles(const Ctx &c);
+// order, in its tile shape, or the one-launch kernel) on a state of this state_reach: the entries
+// that launch writes to StageArgs::cfl_part
+long stage_launch_tiles(const Ctx &c, int big);
 // the RHS with the RK3 stage `sa` applied by its last launch (grid schedule; the caller
 // checks that the configuration allows it: tiled kernels, constant metrics, no closures,
 // no viscous terms); du holds partial sums afterwards, or what it held (one-launch kernel)
@@ -318,7 +320,7 @@ int rhs_for_ctx(ws_ctx *c, const ws_state *st, hipStream_t s);
 // RHS, plus the viscous terms when the configuration has them
 int du_from_prepared(ws_ctx *c, const ws_state *st, hipStream_t s);
 // whether RK3 steps can let the last RHS launch apply the stage (stage fusion on, tiled
-// kernels, grid schedule or one-launch kernel, no closures, no viscous terms, planes the tiles' offsets reach)
+// kernels, grid schedule or one-launch kernel, no closures, no viscous terms)
 bool fused_stage_ok(const ws_ctx *c, const ws_state *st);
 // How a step of stage fusion 3 treats the primitive sets (rk3_step_fused): STEP_PLAIN starts
 // and ends with the primitives in the state's fields (every level); STEP_FROM_STATE and
