@@ -479,23 +479,26 @@ __global__ void __launch_bounds__(NT) k_vis_div(VisParams p, EvFields ev, ws_fie
 // the two add up; issuing each stage's reads under the stage before it, and letting half the
 // wavefronts run half a step behind, were tried and measured no faster.  Before this form (z
 // fluxes and xy sums in LDS rings, closure forms branched per derivative, fixed 64-plane
-// chunks) and now, alone: 600x128x128 sixth order 638 -> 515 us, eighth 942 -> 734;
-// 157x111x75 193 -> 83 and 227 -> 133; x faces closed 211x93x67 461 -> 96 and 458 -> 180, all
-// faces closed 520 -> 164 and 522 -> 203; metric fields 256x160x96 (two kernels around a ghost
-// fill of twelve flux fields before) 445 -> 321 and 450 -> 387.
+// chunks) and now, alone: 600x128x128 sixth order 640 -> 466 us, eighth 943 -> 696;
+// 157x111x75 193 -> 69 and 227 -> 125; x faces closed 211x93x67 459 -> 98 and 458 -> 178, all
+// faces closed 521 -> 151 and 523 -> 197; metric fields 256x160x96 (two kernels around a ghost
+// fill of twelve flux fields before) 446 -> 320 and 450 -> 358.
+// Rounding against 64-bit-mantissa arithmetic, before and now: vortices 5.29e-16 -> 5.03e-16
+// (sixth order) and 6.18e-16 -> 5.91e-16, rough flow 1.87e-16 -> 1.87e-16 and 2.54e-16 ->
+// 2.54e-16.
 constexpr int FX = 32, FY = 16, FNT = FX * FY;
 enum { VM_DIAG, VM_CONST, VM_FIELDS };
 enum { VC_NONE, VC_XY, VC_ALL };
 enum { VL_ONE, VL_PITCHES, VL_BIG };
 
-// Weights of the differences f(c + q) - f(c - q), q = 1..4 at index q - 1.
+// Weights of the differences f(c + q) - f(c - q), q = 1..4 at index q - 1: whole numbers over one
+// denominator (60, or 840 for the eighth order), so that they carry no rounding, and what that
+// denominator, the spacing and the constant metric terms make of a derivative.
 struct VisWeights {
-    double g[3][4];          // gradient along d: coefficient / h_d (VM_DIAG: times A_dd)
-    double f[2][4];          // flux derivative along x and y: coefficient / h_d times the Jacobian factors
-    double row[5][4];        // coefficients at distance 0..3 from a closed face, and the central ones
-    double rg[5][4];         // the same times gs[2]
-    double z[4], rz[5][4];   // the W_j = W_(1-j), j = 1..4, of the central form and of each row, times fs[2]
-    double gs[3], fs[3];     // what g and f multiply the central coefficients by
+    double row[5][4];        // numerators at distance 0..3 from a closed face, and the central ones
+    double rz[5][4];         // of the W_j = W_(1-j), j = 1..4, of each row
+    double gs[3], fs[3];     // VM_DIAG: of a gradient along d and of a flux derivative; VM_FIELDS: gs alone, on the terms
+    double gA[9], fA[9];     // VM_CONST: the metric terms of the gradients and of the fluxes, times them
 };
 
 template <int R>
@@ -675,36 +678,40 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
             oy[q] = (q < closure_reach<R>(ry) ? q + 1 : 0) * PX;
         }
     }
-    // derivatives along x and y (rows of PX) at element e of an LDS array
+    // Undivided derivatives along x and y (rows of PX) at element e of an LDS array: the smallest
+    // difference's weight is one in the sixth-order central form.
+    constexpr double CD[4] = {ORDER == 8 ? 672.0 : 45.0, ORDER == 8 ? -168.0 : -9.0, ORDER == 8 ? 32.0 : 1.0, -3.0};
+    constexpr double CZ[4] = {ORDER == 8 ? 533.0 : 37.0, ORDER == 8 ? -139.0 : -8.0, ORDER == 8 ? 29.0 : 1.0, -3.0};
     int wtx = tx, wty = ty;
-    auto ddx = [&](const double *e, const double *wgt, double scale) {
+    auto ddx = [&](const double *e) {
         double t = 0.0;
 #pragma unroll
-        for (int q = 0; q < R; ++q) {
-            const double d = BND ? e[ox[q]] - e[-ox[q]] : e[q + 1] - e[-q - 1], a = BND ? wxl[q][wtx] : wgt[q];
-            t = q == 0 ? a * d : fma(a, d, t);
+        for (int q = R - 1; q >= 0; --q) {
+            const double d = BND ? e[ox[q]] - e[-ox[q]] : e[q + 1] - e[-q - 1], a = BND ? wxl[q][wtx] : CD[q];
+            t = q == R - 1 ? a * d : fma(a, d, t);
         }
-        return BND ? t * scale : t;
+        return t;
     };
-    auto ddy = [&](const double *e, const double *wgt, double scale) {
+    auto ddy = [&](const double *e) {
         double t = 0.0;
 #pragma unroll
-        for (int q = 0; q < R; ++q) {
+        for (int q = R - 1; q >= 0; --q) {
             const double d = BND ? e[oy[q]] - e[-oy[q]] : e[(q + 1) * PX] - e[-(q + 1) * PX];
-            const double a = BND ? wyl[q][wty] : wgt[q];
-            t = q == 0 ? a * d : fma(a, d, t);
+            const double a = BND ? wyl[q][wty] : CD[q];
+            t = q == R - 1 ? a * d : fma(a, d, t);
         }
-        return BND ? t * scale : t;
+        return t;
     };
     // flux planes zf0 .. zf1 - 1 produce the chunk's cells z0 .. z1 - 1
     const int zf0 = z0 - R, zf1 = z1 + R;
     // slot (P + R + k) % Q at the step of phase P: plane zf + k of the column (c), and the
     // derivative sum of cell zf + k (acc)
     double c[4][Q], acc[4][Q];
-    // the z flux of plane zf - 1: in registers, but where an eighth-order instance has none to
-    // spare in LDS, which costs less than the scratch they would take (x closed 211x93x67 198 ->
-    // 178 us, all faces 220 -> 200, metric fields 256x160x96 394 -> 388)
-    constexpr bool FZL = ORDER == 8 && (BND || FLD);
+    // the z flux of plane zf - 1: in registers, but in instances that have none to spare in LDS,
+    // which costs less than the scratch they would take (eighth order, x closed 211x93x67 198 ->
+    // 178 us, all faces 220 -> 200, metric fields 256x160x96 394 -> 388; sixth order, x closed 101
+    // -> 98)
+    constexpr bool FZL = BND || (ORDER == 8 && FLD);
     __shared__ double fzl[4][FZL ? FNT : 1];
     double fzr[4];
     auto last = [&](int m) -> double & {
@@ -789,34 +796,42 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
                     wm.next();
                 }
             }
-            gk[f] = ddx(pc + f * PN, wt.g[0], wt.gs[0]);
-            gi[f] = ddy(pc + f * PN, wt.g[1], wt.gs[1]);
+            gk[f] = ddx(pc + f * PN);
+            gi[f] = ddy(pc + f * PN);
             if constexpr (!BNDZ) {
-                gs[f] = wt.g[2][0] * (c[f][slot(1)] - c[f][slot(-1)]);
 #pragma unroll
-                for (int q = 2; q <= R; ++q) gs[f] = fma(wt.g[2][q - 1], c[f][slot(q)] - c[f][slot(-q)], gs[f]);
+                for (int q = R; q >= 1; --q) {
+                    const double d = c[f][slot(q)] - c[f][slot(-q)];
+                    gs[f] = q == R ? CD[q - 1] * d : fma(CD[q - 1], d, gs[f]);
+                }
             }
+            if constexpr (MODE == VM_DIAG) { gk[f] *= wt.gs[0]; gi[f] *= wt.gs[1]; if (!BNDZ) gs[f] *= wt.gs[2]; }
             __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (BNDZ) {
             // selects and not branches: the arrays stay in registers without copies at joins
             const int row = closure_row(min(max(zf, 0), p.nz - 1), p.nz, zlo, zhi), reach = closure_reach<R>(row);
 #pragma unroll
-            for (int q = 1; q <= R; ++q)
+            for (int q = R; q >= 1; --q)
 #pragma unroll
                 for (int f = 0; f < 4; ++f) {
                     const double d = q <= reach ? c[f][slot(q)] - c[f][slot(-q)] : 0.0;
-                    gs[f] = q == 1 ? wt.rg[row][0] * d : fma(wt.rg[row][q - 1], d, gs[f]);
+                    gs[f] = q == R ? wt.row[row][q - 1] * d : fma(wt.row[row][q - 1], d, gs[f]);
+                    if (MODE == VM_DIAG && q == 1) gs[f] *= wt.gs[2];
                 }
         }
+        if constexpr (FLD)
+#pragma unroll
+            for (int q = 0; q < 9; ++q) met[q] *= wt.gs[q / 3];
         const double uc = c[0][slot(0)], vc = c[1][slot(0)], wc = c[2][slot(0)], tc = c[3][slot(0)];
-        // T^3 with a summand below its last bit, except for T = 0, of which sqrt_h is not defined
-        const double amu = p.amu_c0 * sqrt_h(fma(tc * tc, tc, 0x1p-1000)) * recip_nr(p.tsb + tc);
+        // T^3 with a summand below its last bit, except for T = 0, of which sqrt_nr is not defined
+        const double amu = p.amu_c0 * sqrt_nr(fma(tc * tc, tc, 0x1p-1000)) * recip_nr(p.tsb + tc);
         auto A = [&](int q) {
             if constexpr (FLD) return met[q];
-            else return p.metric[q];
+            else return wt.gA[q];
         };
-        // physical derivatives from the computational ones (VM_DIAG: the weights carry A_dd)
+        // physical derivatives from the computational ones (the metric terms, or in VM_DIAG the
+        // scale before, carry the spacing)
         auto dot = [](double a, double x, double b, double y, double c, double z) { return fma(c, z, fma(b, y, a * x)); };
         auto px = [&](int f) { return MODE == VM_DIAG ? gk[f] : dot(gk[f], A(0), gi[f], A(3), gs[f], A(6)); };
         auto py = [&](int f) { return MODE == VM_DIAG ? gi[f] : dot(gk[f], A(1), gi[f], A(4), gs[f], A(7)); };
@@ -833,7 +848,8 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
         const double E1 = fma(amuk, Tx, dot(uc, s11, vc, s12, wc, s13));
         const double E2 = fma(amuk, Ty, dot(uc, s12, vc, s22, wc, s23));
         const double E3 = fma(amuk, Tz, dot(uc, s13, vc, s23, wc, s33));
-        // flux of direction d (the weights of its derivative carry the constant factors)
+        // flux of direction d (its metric terms, or in VM_DIAG the scale of its derivative, carry the
+        // spacing and the constant factors)
         auto flux = [&](int d, double out[4]) {
             if constexpr (MODE == VM_DIAG) {
                 out[0] = d == 0 ? s11 : d == 1 ? s12 : s13;
@@ -841,8 +857,8 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
                 out[2] = d == 0 ? s13 : d == 1 ? s23 : s33;
                 out[3] = d == 0 ? E1 : d == 1 ? E2 : E3;
             } else {
-                double a1 = A(3 * d), a2 = A(3 * d + 1), a3 = A(3 * d + 2);
-                if constexpr (FLD) { a1 *= met[9]; a2 *= met[9]; a3 *= met[9]; }
+                double a1 = wt.fA[3 * d], a2 = wt.fA[3 * d + 1], a3 = wt.fA[3 * d + 2];
+                if constexpr (FLD) { a1 = A(3 * d) * met[9]; a2 = A(3 * d + 1) * met[9]; a3 = A(3 * d + 2) * met[9]; }
                 out[0] = dot(a1, s11, a2, s12, a3, s13);
                 out[1] = dot(a1, s12, a2, s22, a3, s23);
                 out[2] = dot(a1, s13, a2, s23, a3, s33);
@@ -865,6 +881,7 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
             G[m] = F[m] - last(m);
+            if (MODE == VM_DIAG) G[m] *= wt.fs[2];
             last(m) = F[m];
         }
         if constexpr (BNDZ) {
@@ -890,8 +907,8 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
             for (int m = 0; m < 4; ++m)
 #pragma unroll
                 for (int q = 1; q <= R; ++q) {
-                    acc[m][slot(-q)] = fma(wt.z[q - 1], G[m], acc[m][slot(-q)]);
-                    acc[m][slot(q - 1)] = q == R ? wt.z[q - 1] * G[m] : fma(wt.z[q - 1], G[m], acc[m][slot(q - 1)]);
+                    acc[m][slot(-q)] = fma(CZ[q - 1], G[m], acc[m][slot(-q)]);
+                    acc[m][slot(q - 1)] = q == R ? CZ[q - 1] * G[m] : fma(CZ[q - 1], G[m], acc[m][slot(q - 1)]);
                 }
         }
         // du of the cell the coming step writes: here rather than with the other loads, whose
@@ -908,8 +925,9 @@ __global__ void __launch_bounds__(FNT) k_vis_fused(VisParams p, VisWeights wt, w
         if (cell)
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
-                acc[m][slot(-1)] += ddx(&fxa[nxt][m][(ty - R) * FX + tx], wt.f[0], wt.fs[0]) +
-                                    ddy(&fya[nxt][m][ty * PX + tx], wt.f[1], wt.fs[1]);
+                const double fx_x = ddx(&fxa[nxt][m][(ty - R) * FX + tx]), fy_y = ddy(&fya[nxt][m][ty * PX + tx]);
+                if constexpr (MODE == VM_DIAG) acc[m][slot(-1)] += fma(fx_x, wt.fs[0], fy_y * wt.fs[1]);
+                else acc[m][slot(-1)] += fx_x + fy_y;
                 __builtin_amdgcn_sched_barrier(0);
             }
         // the sums are formed here: used only where a cell is written, they would otherwise be
@@ -958,31 +976,29 @@ void launch_fused(const VisParams &vp, ws_field u, ws_field v, ws_field w, ws_fi
 {
     constexpr int R = ORDER / 2;
     using FZ = Fused<R>;
-    // coefficients over their denominators: the four rows beside a closed face, the central form
-    const double num[5][4] = {{1, 0, 0, 0}, {1, 0, 0, 0}, {8, -1, 0, 0}, {45, -9, 1, 0},
+    // the four rows beside a closed face and the central form, over 60 (sixth order) or 840
+    constexpr double C = ORDER == 8 ? 14.0 : 1.0;
+    const double num[5][4] = {{60 * C, 0, 0, 0}, {30 * C, 0, 0, 0}, {40 * C, -5 * C, 0, 0}, {45 * C, -9 * C, C, 0},
                               {ORDER == 8 ? 672.0 : 45.0, ORDER == 8 ? -168.0 : -9.0, ORDER == 8 ? 32.0 : 1.0,
                                ORDER == 8 ? -3.0 : 0.0}};
-    const double den[5] = {1, 2, 12, 60, ORDER == 8 ? 840.0 : 60.0};
     VisWeights wt{};
     const double aj = vp.metric[9];
     for (int d = 0; d < 3; ++d) {
-        const double A = MODE == VM_DIAG ? vp.metric[4 * d] : 1.0;
-        wt.gs[d] = A / vp.h[d];
-        wt.fs[d] = MODE == VM_FIELDS ? 1.0 / vp.h[d] : aj * (A * aj) / vp.h[d];
+        const double A = MODE == VM_DIAG ? vp.metric[4 * d] : 1.0, h = 60.0 * C * vp.h[d];
+        wt.gs[d] = A / h;
+        wt.fs[d] = aj * (A * aj) / h;
+        for (int q = 3 * d; q < 3 * d + 3; ++q) {
+            wt.gA[q] = vp.metric[q] / h;
+            wt.fA[q] = aj * (vp.metric[q] * aj) / h;
+        }
     }
     for (int r = 0; r < 5; ++r) {
         double sum = 0.0;
         for (int q = 3; q >= 0; --q) {
             sum += num[r][q];
-            wt.row[r][q] = num[r][q] / den[r];
-            wt.rg[r][q] = wt.row[r][q] * wt.gs[2];
-            wt.rz[r][q] = sum / den[r] * wt.fs[2];
+            wt.row[r][q] = num[r][q];
+            wt.rz[r][q] = sum;
         }
-    }
-    for (int q = 0; q < 4; ++q) {
-        wt.z[q] = wt.rz[4][q];
-        for (int d = 0; d < 3; ++d) wt.g[d][q] = wt.row[4][q] * wt.gs[d];
-        for (int d = 0; d < 2; ++d) wt.f[d][q] = wt.row[4][q] * wt.fs[d];
     }
     const bool bnd_xy = vp.bnd[0] || vp.bnd[1] || vp.bnd[2] || vp.bnd[3], bnd_z = vp.bnd[4] || vp.bnd[5];
     // the layout: shared pitch, planes of fewer than 2^32 bytes
@@ -1003,9 +1019,9 @@ void launch_fused(const VisParams &vp, ws_field u, ws_field v, ws_field w, ws_fi
     auto go = [&](auto kern) { hipLaunchKernelGGL(kern, g, dim3(FNT), 0, s, vp, wt, u, v, w, T, mf, du, zc); };
     // the closure form's table holds the central weights too: it also serves the largest planes,
     // and with several pitches any closed face.  T's pitch its own, with 64-bit addresses in the
-    // closure form for every such layout / now / one pitch: 256x160x96 sixth order 467 / 207 / 202
-    // us, eighth 917 / 305 / 300, x faces closed 157x111x75 184 / 137 and 371 / 228, metric fields
-    // 237 / 111 and 677 / 166
+    // closure form for every such layout / now / one pitch: 256x160x96 sixth order 467 / 179 / 177
+    // us, eighth 927 / 287 / 275; x faces closed 157x111x75 184 / 129 and 362 / 239, metric fields
+    // 237 / 107 and 680 / 168 before and now
     if (!small) go(k_vis_fused<ORDER, MODE, VC_ALL, VL_BIG>);
     else if (!one && (bnd_z || bnd_xy)) go(k_vis_fused<ORDER, MODE, VC_ALL, VL_PITCHES>);
     else if (!one) go(k_vis_fused<ORDER, MODE, VC_NONE, VL_PITCHES>);
