@@ -639,17 +639,18 @@ __device__ __forceinline__ bool closure_m(Cell cell, int n, int f, bool lo, int 
 }
 
 // Steger-Warming split in the form the tiled FP64 kernels use: A1..A3 the metric terms, sn = |A|
-// and rsn = 1/|A| supplied by the caller (constants when metrics are uniform).  With vs = A.u,
-// cs = c |A|, P_i twice the smoothed positive (or negative) eigenvalues of vs, vs - cs and
-// vs + cs, the mass flux is f0 = t (c1 P_1 + P_2 + P_3), the momentum flux f0 u_i + t c/|A| (P_3 -
-// P_2) A_i and the energy flux t (P_1 vv + P_2 (H - c vs/|A|) + P_3 (H + c vs/|A|)) with H =
-// |u|^2/2 + c^2/2 + W2.  75 FP64 instructions against the 108 of split_mixed (whose shifted
-// velocities u -+ c k are spelled out); a tile splits 25-31 % more points than it owns.  Both
-// halves are formed from their own eigenvalues: against 113-bit arithmetic the rounding of the
-// ten fluxes is 0.87 to 0.98 of split_mixed's form's (seven flows, at rest to Mach 10).  With the
-// negative ones as 2 vs - P_1 and so on, four instructions fewer, it is 0.93 to 1.09, and three
-// times that of its own in a supersonic stream's negative half (the RHS of 600x256x128 takes
-// 0.7 % longer than so).
+// and rsn = 1/|A| supplied by the caller (constants when metrics are uniform).  The smoothed
+// eigenvalues of a half are (E_i +- S_i) / 2 with E_i = vs, vs - cs, vs + cs (vs = A.u, cs = c |A|)
+// and S_i = sqrt(E_i^2 + eps^2).  Each half is half the physical flux plus or minus a term of the
+// S_i: the mass flux d vs / 2 +- t (c1 S_1 + S_2 + S_3), the momentum flux f0 u_i + t c/|A| (2 cs +-
+// (S_3 - S_2)) A_i, the energy flux t (vs vv + E_2 H_2 + E_3 H_3) +- t (S_1 vv + S_2 H_2 + S_3 H_3)
+// with t = d/(4 gamma), H_2,3 = |u|^2/2 + c^2/2 + W2 -+ c vs/|A|.  71 FP64 instructions against the
+// 108 of split_mixed (whose shifted velocities u -+ c k are spelled out); a tile splits 25-31 %
+// more points than it owns.  What the two halves share rounds alike in both and leaves the sum of
+// a face's two values: the RHS's error against 64-bit-mantissa arithmetic is 0.91, 0.90, 0.89 and
+// 1.00 of that with split_mixed's form (a jump at rest, Mach 2 blobs, vortices, rough flow); with
+// the eigenvalues of each half formed first 0.99, 0.98, 0.97 and 1.00, with the negative ones as
+// 2 vs - P_1 and so on 0.97, 0.99, 1.06 and 1.03.
 __device__ __forceinline__ void split_fast(const KParams &k, double d, double u, double v, double w,
                                            double cc, double A1, double A2, double A3, double sn,
                                            double rsn, double fp[5], double fm[5])
@@ -668,17 +669,20 @@ __device__ __forceinline__ void split_fast(const KParams &k, double d, double u,
     const double q = fma(w, w, fma(v, v, u * u));
     const double vv = k.gm1 * q, H = fma(0.5, q, k.c3h * (cc * cc));
     const double H2 = H - cv, H3 = H + cv;
-    auto half = [&](double P1, double P2, double P3, double f[5]) {
-#pragma clang fp contract(off)
-        const double g = tc * (P3 - P2);
-        f[0] = t * (fma(k.c1, P1, P2) + P3);
-        f[1] = fma(g, A1, f[0] * u);
-        f[2] = fma(g, A2, f[0] * v);
-        f[3] = fma(g, A3, f[0] * w);
-        f[4] = t * fma(P3, H3, fma(P2, H2, P1 * vv));
-    };
-    half(vs + S1, E2 + S2, E3 + S3, fp);
-    half(vs - S1, E2 - S2, E3 - S3, fm);
+    const double m = 0.5 * d * vs, ms = fma(k.c1, S1, S2 + S3);
+    const double e = t * fma(E3, H3, fma(E2, H2, vs * vv)), es = fma(S3, H3, fma(S2, H2, S1 * vv));
+    const double dS = S3 - S2;
+    const double gp = tc * fma(2.0, cs, dS), gm = tc * fma(2.0, cs, -dS);
+    fp[0] = fma(t, ms, m);
+    fp[1] = fma(gp, A1, fp[0] * u);
+    fp[2] = fma(gp, A2, fp[0] * v);
+    fp[3] = fma(gp, A3, fp[0] * w);
+    fp[4] = fma(t, es, e);
+    fm[0] = fma(-t, ms, m);
+    fm[1] = fma(gm, A1, fm[0] * u);
+    fm[2] = fma(gm, A2, fm[0] * v);
+    fm[3] = fma(gm, A3, fm[0] * w);
+    fm[4] = fma(-t, es, e);
 }
 
 // Steger-Warming split of the mixed-precision kernels: k1..k3 = A/|A|.  The mixed
