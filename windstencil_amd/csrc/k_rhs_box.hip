@@ -62,16 +62,16 @@ __device__ __forceinline__ bool box_point(int r, int &dir, int &l, int &p)
 // What bounds it: on a small grid the chain load - split - reconstruct - store of one cube,
 // with one to three cubes per compute unit to overlap it; on a larger one the FP64 issue.
 // Both want few operations, so one thread reconstructs all five faces of one line and
-// variable, which share the window's differences: 128 FP64 operations per face against 190 with
-// a thread per face (64x32x16 9.5 us so, 100x60x40 52).  Cubes of 8^3 cells through the three
+// variable, which share the window's differences: 135 FP64 operations per face (with a thread
+// per face 64x32x16 took 9.5 us, 100x60x40 52).  Cubes of 8^3 cells through the three
 // directions in turn took 19-23 us on a grid of any small size.
-// FP64 RHS, the directional launches before and this kernel: 64x32x16 23.1 -> 8.8 us,
-// 48x48x48 35.1 -> 20.8 us; an RK3 step of 64x32x16 85 -> 47 us.
+// FP64 RHS, the directional launches and this kernel: 64x32x16 24.0 / 8.9 us, 48x48x48 35.0 /
+// 20.5 us, 100x60x40 52.6 / 39.1; an RK3 step of 64x32x16 77.7 / 34.9 us.
 // PREP: the launch also prepares its inputs: these work-groups read the interior primitives, by
 // their periodic images past a periodic face, and take the sound speed of the T they read;
 // the work-groups after them write the ghost points and the sound speed (prepare_points),
-// which nothing in the launch reads (du_comput of 64x32x16 12.9 -> 9.8 us against preparing in a
-// launch before, of 100x60x40 47.2 -> 44.9).
+// which nothing in the launch reads (du_comput of 64x32x16 12.9 -> 9.6 us against preparing in a
+// launch before, of 100x60x40 47.2 -> 44.0).
 template <bool FIELDS, bool MIX, bool STG, bool PREP>
 __global__ void __launch_bounds__(BOX_NT, 3)
 k_rhs_box(KParams k, ws_field d, ws_field u, ws_field v, ws_field w, ws_field cc, ws_metric_fields mf, ws_soa du,

@@ -472,7 +472,10 @@ __global__ void __launch_bounds__(NT) k_vis_div(VisParams p, EvFields ev, ws_fie
 // planes of 4 GB and more (VL_BIG) take 64-bit addresses.
 //
 // Algorithmic traffic 96 B per cell (constant metrics): u, v, w, T in and du[1..4] read and
-// written.  512 threads of up to 256 VGPRs: one work-group per compute unit.
+// written.  512 threads of up to 256 VGPRs: one work-group per compute unit.  Sixth order and
+// periodic eighth order spill nothing with one pitch; scratch per lane of the others: eighth order
+// with closed faces 36-72 bytes, over metric fields 140-144; eighth order with several pitches
+// 8-52 (closed faces 64, over metric fields 156); planes of 4 GB 36-380.
 //
 // What bounds it: a step moves 84 values per thread through LDS at 128 B per cycle (3,100 of
 // about 5,300 cycles), and the eight wavefronts read LDS and compute in the same phases, so
